@@ -35,14 +35,57 @@ namespace medusa {
 
 constexpr uint32_t kBlock = 4096;  // elements per canonical block (64 lanes x 64 rounds)
 
-// Tree-merge of the (s, c) pairs held by groups of g lanes (g a power of two,
-// groups aligned within the wave); lane 0 of each group ends with the result.
-__device__ __forceinline__ void group_tree(float& s, float& c, uint32_t g) {
-    for (uint32_t off = g >> 1; off; off >>= 1) {
-        const float s2 = __shfl_down(s, off, kWave);
-        const float c2 = __shfl_down(c, off, kWave);
-        kahan_combine(s, c, s2, c2);
-    }
+// Lane exchanges of the canonical tree, in vector registers (v_permlane32_swap, v_permlane16_swap
+// and row shifts) instead of through the LDS crossbar.
+//
+// swap32 turns a, b into (a's lanes 0..31 | b's lanes 0..31) and (a's 32..63 | b's 32..63);
+// swap16 does the same with the 16-lane rows of each half: a = (a0 b0 a2 b2), b = (a1 b1 a3 b3).
+__device__ __forceinline__ void swap32(float& a, float& b) {
+    const auto r = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(uint32_t, a), __builtin_bit_cast(uint32_t, b),
+                                                    false, false);
+    const uint32_t lo = r[0], hi = r[1];  // a bit_cast of a vector element takes element 0
+    a = __builtin_bit_cast(float, lo);
+    b = __builtin_bit_cast(float, hi);
+}
+__device__ __forceinline__ void swap16(float& a, float& b) {
+    const auto r = __builtin_amdgcn_permlane16_swap(__builtin_bit_cast(uint32_t, a), __builtin_bit_cast(uint32_t, b),
+                                                    false, false);
+    const uint32_t lo = r[0], hi = r[1];  // a bit_cast of a vector element takes element 0
+    a = __builtin_bit_cast(float, lo);
+    b = __builtin_bit_cast(float, hi);
+}
+// x of the lane kOff above in the same 16-lane row (0 past the row's end).
+template <int kOff>
+__device__ __forceinline__ float row_above(float x) {
+    return __builtin_bit_cast(
+        float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), 0x100 | kOff, 0xf, 0xf, true));
+}
+
+// Two lanes' pairs as the tree's offset 32 (16) merges them, for two vertices at once: the lower
+// half (the even rows) of the result holds (s, c)'s vertex, the other half (the odd rows)
+// (s2, c2)'s.  With one vertex in both arguments both halves (both rows) end the same.
+__device__ __forceinline__ void merge32(float& s, float& c, float s2, float c2) {
+    swap32(s, s2);
+    swap32(c, c2);
+    kahan_combine(s, c, s2, c2);
+}
+__device__ __forceinline__ void merge16(float& s, float& c, float s2, float c2) {
+    swap16(s, s2);
+    swap16(c, c2);
+    kahan_combine(s, c, s2, c2);
+}
+// Offsets 8, 4, 2, 1 inside every 16-lane row; the row's lane 0 ends with its result.
+__device__ __forceinline__ void row_tree(float& s, float& c) {
+    kahan_combine(s, c, row_above<8>(s), row_above<8>(c));
+    kahan_combine(s, c, row_above<4>(s), row_above<4>(c));
+    kahan_combine(s, c, row_above<2>(s), row_above<2>(c));
+    kahan_combine(s, c, row_above<1>(s), row_above<1>(c));
+}
+// The whole 64-lane tree of one vertex; lane 0 ends with the result.
+__device__ __forceinline__ void wave_tree(float& s, float& c) {
+    merge32(s, c, s, c);
+    merge16(s, c, s, c);
+    row_tree(s, c);
 }
 
 // Canonical sum of `len` values x(k), computed by one whole wave; every lane
@@ -66,9 +109,9 @@ __device__ __forceinline__ float wave_segment_sum(uint32_t len, Load load) {
             for (uint32_t j = 0; j < 16; ++j)
                 if (lane + (r0 + j) * kWave < lim) kahan_add(s, c, x[j]);
         }
-        group_tree(s, c, kWave);
-        s = __shfl(s, 0, kWave);
-        c = __shfl(c, 0, kWave);
+        wave_tree(s, c);
+        s = __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, s)));
+        c = __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, c)));
         if (b0 == 0) {
             as = s;
             ac = c;
@@ -137,64 +180,46 @@ __device__ __forceinline__ float lane_vertex_sum(uint32_t deg, const uint32_t* _
     return s0 - c0;
 }
 
-// The same canonical sum for a lane whose elements come from a functor (LDS slots of the
-// binned variant).
-template <class Load>
-__device__ __forceinline__ void lane_subtree_at(float& S, float& C, uint32_t r, uint32_t st, uint32_t deg, Load load) {
-    float s[16], c[16];
-#pragma unroll
-    for (uint32_t j = 0; j < 16; ++j) {
-        s[j] = (r + st * j < deg) ? load(r + st * j) : 0.f;
-        c[j] = 0.f;
-    }
-    tree16(s, c);
-    S = s[0];
-    C = c[0];
-}
-// The canonical 64-slot tree over a lane's first L slots (L a power of two <= 16, deg <= L):
-// slot j absorbs slot j+off for off = L/2, ..., 1.  Every slot from deg on is (0,0), so the
-// 64-slot tree's levels above L/2 only merge (0,0) pairs, an exact identity, and this is the
-// whole sum.
-template <uint32_t L, class Load>
-__device__ __forceinline__ float lane_tree_small(uint32_t deg, Load load) {
+// Binned variant: the sums of one lane item (planned by pr_bins.h), whose lane l holds slots
+// at[64 j + l], j = 0, 1, ...: with `per` = pr_lane_group(deg) vertices the item's slots are
+// column-major, so that is element r + st j of vertex l mod per, with st = 64 / per and
+// r = l / per.  A lane reduces its (at most 16) elements by the tree's offsets down to st, then
+// the st lanes of a vertex merge by the offsets below it, and lane i < per ends with vertex i's
+// sum.  Slots past a vertex's own in-degree hold +0.0 and are not distinguished from elements:
+// (0, 0) pairs merge as the exact identity that the canonical tree uses for absent elements.
+template <uint32_t L>
+__device__ __forceinline__ void lane_item_leaves(float& S, float& C, uint32_t st, uint32_t deg, const float* at) {
+    const uint32_t r = st == 1 ? 0u : st == 2 ? lane_id() >> 5 : lane_id() >> 4;
     float s[L], c[L];
 #pragma unroll
     for (uint32_t j = 0; j < L; ++j) {
-        s[j] = j < deg ? load(j) : 0.f;
+        s[j] = r + st * j < deg ? at[64 * j] : 0.f;
         c[j] = 0.f;
     }
 #pragma unroll
     for (uint32_t off = L / 2; off >= 1; off >>= 1)
 #pragma unroll
         for (uint32_t j = 0; j < off; ++j) kahan_combine(s[j], c[j], s[j + off], c[j + off]);
-    return s[0] - c[0];
+    S = s[0];
+    C = c[0];
 }
-
-template <class Load>
-__device__ __forceinline__ float lane_vertex_sum_at(uint32_t deg, Load load) {
-    if (deg <= 1) return lane_tree_small<1>(deg, load);
-    if (deg <= 2) return lane_tree_small<2>(deg, load);
-    if (deg <= 4) return lane_tree_small<4>(deg, load);
-    if (deg <= 8) return lane_tree_small<8>(deg, load);
-    // the 1, 2 or 4 interleaved subtrees one at a time (a loop, so only one subtree's leaves
-    // are live), then merged as the 64-slot tree merges them
-    const uint32_t st = deg <= 16 ? 1u : deg <= 32 ? 2u : 4u;
-    float ss[4], cc[4];
-#pragma unroll 1
-    for (uint32_t r = 0; r < st; ++r) {
-        float S, C;
-        lane_subtree_at(S, C, r, st, deg, load);
-        ss[r] = S;
-        cc[r] = C;
+__device__ __forceinline__ float lane_item_sum(uint32_t deg, const float* at) {
+    float s, c;
+    if (deg <= 1) {
+        lane_item_leaves<1>(s, c, 1, deg, at);
+    } else if (deg <= 2) {
+        lane_item_leaves<2>(s, c, 1, deg, at);
+    } else if (deg <= 4) {
+        lane_item_leaves<4>(s, c, 1, deg, at);
+    } else if (deg <= 8) {
+        lane_item_leaves<8>(s, c, 1, deg, at);
+    } else {
+        const uint32_t st = 64 / pr_lane_group(deg);
+        lane_item_leaves<16>(s, c, st, deg, at);
+        if (st >= 2) merge32(s, c, s, c);
+        if (st == 4) merge16(s, c, s, c);
     }
-    if (st == 2) {
-        kahan_combine(ss[0], cc[0], ss[1], cc[1]);
-    } else if (st == 4) {
-        kahan_combine(ss[0], cc[0], ss[2], cc[2]);
-        kahan_combine(ss[1], cc[1], ss[3], cc[3]);
-        kahan_combine(ss[0], cc[0], ss[1], cc[1]);
-    }
-    return ss[0] - cc[0];
+    return s - c;
 }
 
 // One superstep for every vertex.  kFromMsg: values come from the message
@@ -258,7 +283,7 @@ __device__ __forceinline__ void dangle_block_sum(const float* __restrict__ rank,
         for (uint32_t j = 0; j < 16; ++j)
             if (lane + (r0 + j) * kWave < B.len) kahan_add(s, c, v[j]);
     }
-    group_tree(s, c, kWave);
+    wave_tree(s, c);
 }
 
 // Dangling mass, step 1: one wave per canonical block of a graph's dangling tail
@@ -346,7 +371,7 @@ __global__ __launch_bounds__(256) void k_pr_dangle_base(const float* __restrict_
             for (uint32_t j = 0; j < 16; ++j)
                 if (lane + (r0 + j) * kWave < B.len) kahan_add(s, c, v[j]);
         }
-        group_tree(s, c, kWave);
+        wave_tree(s, c);
         if (lane == 0) {
             s_s[b] = s;
             s_c[b] = c;
@@ -484,10 +509,12 @@ constexpr uint32_t kCombineUnroll = 4;  // groups of four entries per thread in 
 //      the host; a group never straddles two runs) and its four slots (8 bytes) load together,
 //      then its four messages (16 bytes); each message goes to its LDS slot (padding entries to
 //      a dummy slot);
-//   3. after the barrier, wave w sums its items from LDS in the canonical order.  A lane
-//      vertex sums as many slots as the largest in-degree of its group: the slots past its own
-//      in-degree hold +0.0, which merges as the exact identity the canonical tree uses for
-//      absent elements, so no per-vertex degree is read.
+//   3. after the barrier, wave w sums its items from LDS in the canonical order: lane items
+//      (lane_item_sum; at most 16 slots per lane) and wave vertices, four at a time.  A wave
+//      vertex alone spent most of its time in the tree's twelve dependent exchanges, and the bins
+//      of the heaviest destinations (about 90 wave vertices, or two 64-vertex lane items) ran
+//      long after the others; four trees now share seven merges in vector registers.  Combine
+//      of RMAT-16 (141 bins, one round) 18.8 -> 8.8 us, of RMAT-20 29.6 -> 25.1 us (5.3 TB/s).
 // Workgroups from nbins on sum the hub destinations (one wave each) by gathering r / outdeg of
 // their sources over the CSC, with the same division the send does.  kFold: a single graph with at most 64
 // dangling blocks, whose base every wave merges here from the send's block pairs; otherwise
@@ -608,22 +635,51 @@ __global__ __launch_bounds__(kCombineThreads) void k_pr_combine(
     const uint32_t mine = B.item_end > B.item_begin + wave
                               ? (B.item_end - B.item_begin - wave + kCombineWaves - 1) / kCombineWaves
                               : 0u;
-    for (uint32_t j = 0; j < mine; ++j) {
-        const uint32_t v = __builtin_amdgcn_readlane(iv, j), cnt = __builtin_amdgcn_readlane(icount, j);
-        const uint32_t kind = __builtin_amdgcn_readlane(ikind, j), at = __builtin_amdgcn_readlane(ilds, j);
-        const uint32_t deg = __builtin_amdgcn_readlane(ideg, j);
-        const float base = kFold ? base_all : base_p[__builtin_amdgcn_readlane(ipart, j)];
+    for (uint32_t j = 0; j < mine;) {
+        const uint32_t kind = __builtin_amdgcn_readlane(ikind, j);
         if (kind == kPrWave) {
-            const float S = wave_segment_sum(deg, [&](uint32_t k) { return lds[at + k]; });
-            if (lane == 0) finish(v, S, base);
-        } else if (lane < cnt) {
-            if (kind == kPrZero) {
-                finish(v + lane, 0.f, base);
-            } else {
-                const float* x = lds + at + lane;
-                finish(v + lane, lane_vertex_sum_at(deg, [&](uint32_t k) { return x[k * kWave]; }), base);
+            // up to four wave vertices at once: their Kahan chains overlap, and the tree's offsets
+            // 32 and 16 merge two and four of them per exchange
+            uint32_t at[4], deg[4], v[4], part[4], top = 0, cnt = 0;
+#pragma unroll
+            for (uint32_t q = 0; q < 4; ++q) {
+                at[q] = deg[q] = v[q] = part[q] = 0;
+                if (cnt == q && j + q < mine && __builtin_amdgcn_readlane(ikind, j + q) == kPrWave) {
+                    at[q] = __builtin_amdgcn_readlane(ilds, j + q);
+                    deg[q] = __builtin_amdgcn_readlane(ideg, j + q);
+                    v[q] = __builtin_amdgcn_readlane(iv, j + q);
+                    part[q] = __builtin_amdgcn_readlane(ipart, j + q);
+                    top = max(top, deg[q]);
+                    ++cnt;
+                }
             }
+            float s[4] = {0.f, 0.f, 0.f, 0.f}, c[4] = {0.f, 0.f, 0.f, 0.f};
+            for (uint32_t k = lane; k - lane < top; k += kWave) {  // uniform across the wave
+                float x[4];
+#pragma unroll
+                for (uint32_t q = 0; q < 4; ++q) x[q] = k < deg[q] ? lds[at[q] + k] : 0.f;
+#pragma unroll
+                for (uint32_t q = 0; q < 4; ++q)
+                    if (k < deg[q]) kahan_add(s[q], c[q], x[q]);
+            }
+            merge32(s[0], c[0], s[1], c[1]);
+            merge32(s[2], c[2], s[3], c[3]);
+            merge16(s[0], c[0], s[2], c[2]);  // rows: vertices 0, 2, 1, 3
+            row_tree(s[0], c[0]);
+            const uint32_t row = lane / 16;
+            const uint32_t mv = row == 0 ? v[0] : row == 1 ? v[2] : row == 2 ? v[1] : v[3];
+            const uint32_t mp = row == 0 ? part[0] : row == 1 ? part[2] : row == 2 ? part[1] : part[3];
+            const uint32_t mq = row == 1 ? 2u : row == 2 ? 1u : row;
+            if (lane % 16 == 0 && mq < cnt) finish(mv, s[0] - c[0], kFold ? base_all : base_p[mp]);
+            j += cnt;
+            continue;
         }
+        const uint32_t v = __builtin_amdgcn_readlane(iv, j), cnt = __builtin_amdgcn_readlane(icount, j);
+        const uint32_t at = __builtin_amdgcn_readlane(ilds, j), deg = __builtin_amdgcn_readlane(ideg, j);
+        const float base = kFold ? base_all : base_p[__builtin_amdgcn_readlane(ipart, j)];
+        const float S = kind == kPrZero ? 0.f : lane_item_sum(deg, lds + at + lane);
+        if (lane < cnt) finish(v + lane, S, base);
+        ++j;
     }
 }
 

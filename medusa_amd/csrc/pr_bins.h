@@ -45,9 +45,18 @@ static_assert(kPrTileEdges % kPrRunAlign == 0, "tiles keep the alignment of thei
 static_assert(kPrBinValues < 65536 && kPrChunkSources <= 65536, "slots and source offsets are 16-bit");
 static_assert(kPrHubDeg <= kPrBinValues, "a wave vertex must fit one bin");
 
+// Vertices of one lane item whose largest in-degree is `deg`: 64, or 32 (16) above 16 (32)
+// in-edges, so that a wave holds at most 16 messages per lane of every item, two (four) lanes
+// sharing a vertex.  With 64 vertices per item whatever the in-degree, a bin of in-degree 64 was
+// two items: two of the workgroup's eight waves each summed 64 messages per lane.
+#if defined(__HIPCC__)
+__host__ __device__
+#endif
+inline uint32_t pr_lane_group(uint32_t deg) { return deg <= 16 ? 64u : deg <= 32 ? 32u : 16u; }
+
 // One combine item: a wave vertex (kPrWave; its k-th message at LDS lds+k), a group of up to
-// 64 consecutive lane vertices (kPrLane; lane i's k-th message at lds + 64k + i), or up to 64
-// consecutive vertices without in-edges (kPrZero).
+// g = pr_lane_group(deg) consecutive lane vertices (kPrLane; vertex i's k-th message at
+// lds + g k + i), or up to 64 consecutive vertices without in-edges (kPrZero).
 struct PrItem {
     uint32_t v;      // first internal vertex
     uint32_t count;  // vertices (1 for kPrWave)
@@ -162,11 +171,12 @@ inline std::string plan_pr_bins(uint32_t n, const uint32_t* cptr, const uint32_t
                 used += deg;
                 group = -1;
             } else {
-                const bool extend = group >= 0 && P.items[group].kind == kind && P.items[group].count < 64 &&
+                const uint32_t most = kind == kPrLane ? pr_lane_group(group_max) : 64u;
+                const bool extend = group >= 0 && P.items[group].kind == kind && P.items[group].count < most &&
                                     P.items[group].v + P.items[group].count == p && deg <= group_max &&
                                     verts + 1 <= cap_verts;
                 if (!extend) {
-                    const uint32_t foot = kind == kPrLane ? 64u * deg : 0u;
+                    const uint32_t foot = kind == kPrLane ? pr_lane_group(deg) * deg : 0u;
                     if (full(foot)) close_bin();
                     group = (int64_t)P.items.size();
                     P.items.push_back({p, 0, kind, used, part, deg, {0, 0}});
@@ -237,7 +247,7 @@ inline std::string plan_pr_bins(uint32_t n, const uint32_t* cptr, const uint32_t
             const uint64_t cb = (u / kPrChunkSources) * B + b;
             const uint32_t i = fill[cb]++;
             P.srcloc[rstart[cb] + i] = (uint16_t)(u % kPrChunkSources);
-            const uint32_t lds = I.kind == kPrWave ? I.lds + k : I.lds + 64u * k + (p - I.v);
+            const uint32_t lds = I.kind == kPrWave ? I.lds + k : I.lds + pr_lane_group(I.deg) * k + (p - I.v);
             P.slot[slot_begin[b] + kstart[cb] + i] = (uint16_t)lds;
             ++P.nmsg;
         }
@@ -332,7 +342,8 @@ inline std::string check_pr_bins(uint32_t n, const uint32_t* cptr, const PrBinsP
         uint32_t verts = 0;
         for (uint32_t i = B.item_begin; i < B.item_end; ++i) {
             const PrItem& I = P.items[i];
-            if (I.count == 0 || I.count > 64 || (I.kind == kPrWave && I.count != 1)) return "bins: item count";
+            const uint32_t most = I.kind == kPrWave ? 1u : I.kind == kPrLane ? pr_lane_group(I.deg) : 64u;
+            if (I.count == 0 || I.count > most) return "bins: item count";
             if ((uint64_t)I.v + I.count > n) return "bins: item vertices";
             if (I.kind == kPrWave && I.deg != cptr[I.v + 1] - cptr[I.v]) return "bins: wave item degree";
             verts += I.count;
@@ -342,7 +353,7 @@ inline std::string check_pr_bins(uint32_t n, const uint32_t* cptr, const PrBinsP
                 if (I.kind == kPrLane && (deg == 0 || deg > kPrLaneMax || deg > I.deg)) return "bins: lane item degree";
             }
             const uint64_t top = I.kind == kPrWave ? (uint64_t)I.lds + I.deg
-                                 : I.kind == kPrLane ? (uint64_t)I.lds + 64ull * I.deg
+                                 : I.kind == kPrLane ? (uint64_t)I.lds + (uint64_t)most * I.deg
                                                      : 0;
             if (top > P.bin_slots[b]) return "bins: item beyond its LDS slots";
         }

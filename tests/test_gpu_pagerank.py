@@ -115,6 +115,27 @@ def test_pagerank_binned_shapes(oracle):
                     assert np.array_equal(_bits(r), _bits(want)), (len(rp) - 1, steps, use_graph)
 
 
+@pytest.mark.parametrize("deg", [1, 8, 9, 16, 17, 32, 33, 64, 65, 127, 192, 4096])
+def test_binned_item_shapes(oracle, deg):
+    """In-degrees at the edges of the combine's item classes (64, 32 or 16 vertices per lane item;
+    wave vertices four at a time), with vertex counts that leave every item and every group of
+    four partly filled, and neighbours of one in-edge fewer in the same items.  Bits equal."""
+    rng = np.random.default_rng(deg)
+    n = 9000  # two source chunks
+    counts = (1, 4, 5) if deg > 2000 else (5, 33, 67)
+    arcs, v = [], 0
+    for c in counts:
+        for d in (deg, max(deg - 1, 1)):
+            dst = np.repeat(np.arange(v, v + c), d)
+            arcs.append(np.stack([rng.integers(0, n, len(dst)), dst], 1))
+            v += c
+    rp, col, _ = csr_from_edges(n, np.concatenate(arcs))
+    with md.Graph(rp, col) as G:
+        want = oracle.pagerank_f32(rp, col, 0.85, 3)
+        r, _ = G.pagerank(0.85, 3, variant=md.PR_BINNED)
+        assert np.array_equal(_bits(r), _bits(want))
+
+
 def test_pagerank_damping_and_repeat(oracle):
     rp, col, _ = random_graph(8000, 50000, 4)
     with md.Graph(rp, col) as G:
