@@ -191,7 +191,9 @@ struct PrLayout {
     // work
     DBuf<float> rank, rank_prev, contrib0, contrib1, msg, base, unperm;
     DBuf<float> partials;   // (s, c) pairs of the dangling-sum blocks
-    DBuf<double> resid;
+    DBuf<double> resid;     // per-workgroup sums of the last two iterates' L1 distance
+    HBuf<double> h_resid;
+    DBuf<uint32_t> ticket;  // dangling blocks published by the running send (0 between launches)
     // captured superstep sequence, reused while (steps, variant, damping) stay the same
     hipGraphExec_t exec = nullptr;
     uint32_t exec_steps = 0;
@@ -299,6 +301,11 @@ namespace medusa {
 [[nodiscard]] std::unique_lock<std::recursive_mutex> enter(const medusa_graph* g);
 // Grows the timing-event pool to at least `count` events.
 void ensure_events(medusa_graph* g, size_t count);
+// Whether `p` is device memory (of any GPU); host pointers unknown to HIP are not.
+bool is_device_memory(const void* p);
+// Whether g's kernels may write 4-byte values at `p`: device memory of g's own GPU, aligned.
+// Other destinations (host, managed, another GPU) are copied to.
+bool kernels_can_write(const medusa_graph* g, const void* p);
 // Copies `bytes` from device pointer `src` to `dst`, which may be host or device memory.
 void copy_out(medusa_graph* g, void* dst, const void* src, size_t bytes);
 // Sums pairwise (start, stop) event intervals [0, pairs) in milliseconds.

@@ -55,12 +55,24 @@ double sum_event_pairs(medusa_graph* g, size_t pairs) {
     return ms;
 }
 
+bool is_device_memory(const void* p) {
+    hipPointerAttribute_t attr{};
+    const hipError_t e = hipPointerGetAttributes(&attr, p);
+    (void)hipGetLastError();  // host pointers unknown to HIP report an error; that is the "host" answer
+    return e == hipSuccess && attr.type == hipMemoryTypeDevice;
+}
+
+bool kernels_can_write(const medusa_graph* g, const void* p) {
+    hipPointerAttribute_t attr{};
+    const hipError_t e = hipPointerGetAttributes(&attr, p);
+    (void)hipGetLastError();
+    return e == hipSuccess && attr.type == hipMemoryTypeDevice && attr.device == g->device &&
+           reinterpret_cast<uintptr_t>(p) % 4 == 0;
+}
+
 void copy_out(medusa_graph* g, void* dst, const void* src, size_t bytes) {
     if (!bytes) return;
-    hipPointerAttribute_t attr{};
-    hipError_t e = hipPointerGetAttributes(&attr, dst);
-    (void)hipGetLastError();  // host pointers unknown to HIP report an error; that is the "host" answer
-    const bool dev = (e == hipSuccess && attr.type == hipMemoryTypeDevice);
+    const bool dev = is_device_memory(dst);
     MDS_HIP(hipMemcpyAsync(dst, src, bytes, dev ? hipMemcpyDeviceToDevice : hipMemcpyDeviceToHost, g->stream));
     MDS_HIP(hipStreamSynchronize(g->stream));
 }

@@ -345,6 +345,78 @@ __global__ __launch_bounds__(256) void k_pr_base(const float* __restrict__ parti
     if (lane == 0) base_out[w] = base;
 }
 
+// Dangling mass of several graphs (or of one with many blocks) inside the binned send: every
+// block's wave publishes its pair and takes a ticket, and the wave with the last ticket merges
+// the pairs of all graphs into their bases, so the combine needs no launch in between (4.5 us of
+// the 30 us superstep of a batch of 64 graphs, 8 M arcs).  The exchanges' results are waited for
+// before the ticket is drawn, and the merging wave reads the pairs with device-scope loads, so
+// no fence is needed.
+constexpr uint32_t kFoldParts = 256;      // graphs a single wave merges, one lane each
+constexpr uint32_t kFoldPartBlocks = 32;  // blocks per graph up to which one lane merges them
+
+// Whether the send merges the bases itself (above the limits a launch of k_pr_base does, one wave
+// per graph; nothing dangling leaves no wave to take a ticket).
+static bool pr_send_folds(const PrLayout& L) {
+    if (L.blocks.empty()) return false;
+    if (L.parts.size() == 1) return true;
+    uint32_t most = 0;
+    for (const PrPart& P : L.parts) most = std::max(most, P.nblocks);
+    return L.parts.size() <= kFoldParts && most <= kFoldPartBlocks;
+}
+
+// Bases of every graph from the published pairs, by one wave; graph order and merge order as in
+// k_pr_base.
+__device__ __forceinline__ void pr_fold_published(const float* __restrict__ partials, uint32_t nblk,
+                                                  const PrPart* __restrict__ parts, uint32_t nparts, float d,
+                                                  float* __restrict__ base_out) {
+    const uint32_t lane = lane_id();
+    float as = 0.f, ac = 0.f;
+    if (nparts == 1) {
+        for (uint32_t c0 = 0; c0 < nblk; c0 += kWave) {
+            const uint32_t i = c0 + lane;
+            const float ps = i < nblk ? load_now(partials + 2 * i) : 0.f;
+            const float pc = i < nblk ? load_now(partials + 2 * i + 1) : 0.f;
+            const uint32_t lim = min(nblk - c0, (uint32_t)kWave);
+            for (uint32_t j = 0; j < lim; ++j) {
+                const float s2 = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, ps), j));
+                const float c2 = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, pc), j));
+                if (c0 + j == 0) {
+                    as = s2;
+                    ac = c2;
+                } else {
+                    kahan_combine(as, ac, s2, c2);
+                }
+            }
+        }
+        if (lane == 0) base_out[0] = pr_base_value(as - ac, d, parts[0].n);
+        return;
+    }
+    for (uint32_t g = lane; g < nparts; g += kWave) {
+        const PrPart P = parts[g];
+        as = ac = 0.f;
+        for (uint32_t i0 = 0; i0 < P.nblocks; i0 += 8) {
+            float s2[8], c2[8];
+#pragma unroll
+            for (uint32_t j = 0; j < 8; ++j) {
+                const bool in = i0 + j < P.nblocks;
+                s2[j] = in ? load_now(partials + 2 * (P.first_block + i0 + j)) : 0.f;
+                c2[j] = in ? load_now(partials + 2 * (P.first_block + i0 + j) + 1) : 0.f;
+            }
+#pragma unroll
+            for (uint32_t j = 0; j < 8; ++j) {
+                if (i0 + j >= P.nblocks) continue;
+                if (i0 + j == 0) {
+                    as = s2[j];
+                    ac = c2[j];
+                } else {
+                    kahan_combine(as, ac, s2[j], c2[j]);
+                }
+            }
+        }
+        base_out[g] = pr_base_value(as - ac, d, P.n);
+    }
+}
+
 constexpr uint32_t kSmallBlocks = 64;  // dangling blocks up to which one workgroup does both steps
 
 // Both dangling-mass steps in one workgroup when there are at most kSmallBlocks blocks:
@@ -424,30 +496,48 @@ constexpr uint32_t kSendWaves = kSendThreads / kWave;
 // contributions c = r / outdeg into LDS and write one tile of the message array (contiguous;
 // runs are padded to 4 entries, so every access is 16-byte aligned).  Tiles of one chunk run on
 // one XCD, so the chunk's ranks are read from HBM once per XCD.
-// Workgroups from ntiles on write the (s, c) pairs of the dangling blocks of `rank` (one block
-// per wave), which the combine of the same superstep merges into its base.
+// The first `dwg` workgroups write the (s, c) pairs of the dangling blocks of `rank` (one block
+// per wave), which the combine of the same superstep merges into its base; with base_out (see
+// pr_send_folds) the last of those waves merges them here.  They come first so that the merge is
+// over before the tiles are.
 __global__ __launch_bounds__(kSendThreads) void k_pr_send(const PrTile* __restrict__ tiles, uint32_t ntiles,
                                                  const uint16_t* __restrict__ srcloc, const float* __restrict__ rank,
                                                  const uint32_t* __restrict__ outdeg, float* __restrict__ msg,
                                                  const PrBlock* __restrict__ blocks,
-                                                 uint32_t nblk, float* __restrict__ partials) {
+                                                 uint32_t nblk, uint32_t dwg, float* __restrict__ partials,
+                                                 const PrPart* __restrict__ parts, uint32_t nparts, float d,
+                                                 float* __restrict__ base_out, uint32_t* __restrict__ ticket) {
     __shared__ float s_c[kPrChunkSources];
     using u16x4 = unsigned short __attribute__((ext_vector_type(4)));
     using f32x4 = float __attribute__((ext_vector_type(4)));
     using u32x4 = uint32_t __attribute__((ext_vector_type(4)));
-    if (blockIdx.x >= ntiles) {
+    if (blockIdx.x < dwg) {
         const uint32_t lane = threadIdx.x & (kWave - 1);
-        const uint32_t b = (blockIdx.x - ntiles) * kSendWaves + threadIdx.x / kWave;
+        const uint32_t b = blockIdx.x * kSendWaves + threadIdx.x / kWave;
         if (b >= nblk) return;  // uniform across the wave
         float bs, bc;
         dangle_block_sum(rank, blocks[b], bs, bc);
-        if (lane == 0) {
-            partials[2 * b] = bs;
-            partials[2 * b + 1] = bc;
+        if (!base_out) {
+            if (lane == 0) {
+                partials[2 * b] = bs;
+                partials[2 * b + 1] = bc;
+            }
+            return;
         }
+        uint32_t t = 0;
+        if (lane == 0) {
+            const float r0 = atomicExch(&partials[2 * b], bs), r1 = atomicExch(&partials[2 * b + 1], bc);
+            uint32_t inc = 1;
+            asm volatile("" : "+v"(inc) : "v"(r0), "v"(r1));
+            t = atomicAdd(ticket, inc);
+        }
+        t = __builtin_amdgcn_readfirstlane(t);
+        if (t != nblk - 1) return;
+        pr_fold_published(partials, nblk, parts, nparts, d, base_out);
+        if (lane == 0) *ticket = 0;  // for the next superstep's send
         return;
     }
-    const PrTile T = tiles[xcd_major(blockIdx.x, ntiles)];
+    const PrTile T = tiles[xcd_major(blockIdx.x - dwg, ntiles)];
     const u16x4* __restrict__ sl = reinterpret_cast<const u16x4*>(srcloc + T.msg_begin);
     f32x4* __restrict__ out = reinterpret_cast<f32x4*>(msg + T.msg_begin);
     const uint32_t nq = (T.msg_end - T.msg_begin) / 4;
@@ -692,9 +782,12 @@ uint32_t pr_combine_slots(const medusa_graph* g) {
 }
 
 // r_0 = (float)(1 / n_g) for every vertex of graph g (graph found by binary search
-// over the range starts, which internal ids keep).
+// over the range starts, which internal ids keep), its contribution when the first superstep
+// reads one (contrib not null), and the send's ticket.
 __global__ void k_pr_init(uint32_t n, const uint32_t* __restrict__ part_begin, uint32_t nparts,
-                          const uint32_t* __restrict__ outdeg, float* __restrict__ rank, float* __restrict__ contrib) {
+                          const uint32_t* __restrict__ outdeg, float* __restrict__ rank, float* __restrict__ contrib,
+                          uint32_t* __restrict__ ticket) {
+    if (blockIdx.x == 0 && threadIdx.x == 0) *ticket = 0;
     for (uint32_t p = blockIdx.x * blockDim.x + threadIdx.x; p < n; p += gridDim.x * blockDim.x) {
         uint32_t lo = 0, hi = nparts;  // last graph with begin <= p
         while (hi - lo > 1) {
@@ -704,6 +797,7 @@ __global__ void k_pr_init(uint32_t n, const uint32_t* __restrict__ part_begin, u
         }
         const float r0 = (float)(1.0 / (double)(part_begin[lo + 1] - part_begin[lo]));
         rank[p] = r0;
+        if (!contrib) continue;
         const uint32_t od = outdeg[p];
         if (od) contrib[p] = r0 / (float)od;
     }
@@ -723,28 +817,25 @@ __global__ void k_pr_scatter(uint32_t n, const uint32_t* __restrict__ optr, cons
     }
 }
 
-__global__ void k_pr_unpermute(uint32_t n, const uint32_t* __restrict__ iperm, const float* __restrict__ rank,
-                               float* __restrict__ out) {
-    for (uint32_t v = blockIdx.x * blockDim.x + threadIdx.x; v < n; v += gridDim.x * blockDim.x)
-        out[v] = rank[iperm[v]];
-}
-
-__global__ void k_pr_resid(uint32_t n, const float* __restrict__ a, const float* __restrict__ b,
-                           double* __restrict__ out) {
+// End of a run: the ranks in original vertex order, and the L1 distance of the last two iterates
+// as one FP64 sum per workgroup, which the host adds up in order (512 atomics on one address took
+// as long as the rest of the pass).
+constexpr uint32_t kFinishWgs = 1024;
+__global__ __launch_bounds__(256) void k_pr_finish(uint32_t n, const uint32_t* __restrict__ iperm,
+                                                   const float* __restrict__ rank, const float* __restrict__ prev,
+                                                   float* __restrict__ out, double* __restrict__ resid) {
     __shared__ double s_part[4];
     double acc = 0.0;
-    for (uint32_t p = blockIdx.x * blockDim.x + threadIdx.x; p < n; p += gridDim.x * blockDim.x)
-        acc += fabs((double)a[p] - (double)b[p]);
+    for (uint32_t v = blockIdx.x * blockDim.x + threadIdx.x; v < n; v += gridDim.x * blockDim.x) {
+        out[v] = rank[iperm[v]];
+        acc += fabs((double)rank[v] - (double)prev[v]);
+    }
 #pragma unroll
     for (int off = kWave / 2; off >= 1; off >>= 1) acc += __shfl_xor(acc, off, kWave);
     if ((threadIdx.x & (kWave - 1)) == 0) s_part[threadIdx.x / kWave] = acc;
     __syncthreads();
-    if (threadIdx.x == 0) atomicAdd(out, s_part[0] + s_part[1] + s_part[2] + s_part[3]);
+    if (threadIdx.x == 0) resid[blockIdx.x] = s_part[0] + s_part[1] + s_part[2] + s_part[3];
 }
-
-__global__ void k_zero_f64(double* p) { *p = 0.0; }
-
-__global__ void k_set_f32(float* p, float v) { *p = v; }
 
 // A single graph with at most this many dangling blocks merges its base inside the binned
 // combine (every wave merges the block pairs itself) instead of in a launch of its own.
@@ -793,13 +884,16 @@ static void pr_run(medusa_graph* g, float damping, uint32_t steps, float* out, c
     L.contrib1.ensure(n);
     L.base.ensure(nparts);
     L.partials.ensure(2 * (size_t)std::max(nblk, 1u));
-    L.resid.ensure(1);
+    L.resid.ensure(kFinishWgs);
+    L.h_resid.ensure(kFinishWgs);
+    L.ticket.ensure(1);
     L.rank_prev.ensure(n);
-    L.unperm.ensure(n);
     if (push) L.msg.ensure(m);
     hipStream_t s = g->stream;
-    MDS_HIP(hipMemsetAsync(L.contrib0.p, 0, (size_t)n * 4, s));
-    MDS_HIP(hipMemsetAsync(L.contrib1.p, 0, (size_t)n * 4, s));
+    // an output the kernels can write is written by the last one itself
+    const bool direct = kernels_can_write(g, out);
+    if (!direct) L.unperm.ensure(n);
+    const bool send_folds = !fold && pr_send_folds(L);
 
     const float d_f = damping;
     const uint32_t dangle_wgs = (nblk + 3) / 4, base_wgs = (nparts + 3) / 4;
@@ -822,7 +916,8 @@ static void pr_run(medusa_graph* g, float damping, uint32_t steps, float* out, c
     };
 
     hipLaunchKernelGGL(k_pr_init, dim3(grid_for(n, 256)), dim3(256), 0, s, n, (const uint32_t*)L.d_part_begin.p,
-                       nparts, L.outdeg.p, L.rank.p, L.contrib0.p);
+                       nparts, L.outdeg.p, L.rank.p,
+                       steps > 0 && var[0] == MEDUSA_PR_BINNED ? nullptr : L.contrib0.p, L.ticket.p);
     MDS_LAUNCHED();
 
     const bool timing = o.timing != 0 || o.trace != 0;
@@ -848,11 +943,12 @@ static void pr_run(medusa_graph* g, float damping, uint32_t steps, float* out, c
                 if (dwg + Bn->ntiles) {  // none when nothing dangles and every in-edge goes to a hub
                     hipLaunchKernelGGL(k_pr_send, dim3(Bn->ntiles + dwg), dim3(kSendThreads), 0, s,
                                        (const PrTile*)Bn->tiles.p, Bn->ntiles, (const uint16_t*)Bn->srcloc.p, r_in,
-                                       (const uint32_t*)L.outdeg.p, Bn->msg.p, (const PrBlock*)L.d_blocks.p, nblk,
-                                       L.partials.p);
+                                       (const uint32_t*)L.outdeg.p, Bn->msg.p, (const PrBlock*)L.d_blocks.p, nblk, dwg,
+                                       L.partials.p, (const PrPart*)L.d_parts.p, nparts, d_f,
+                                       send_folds ? L.base.p : nullptr, L.ticket.p);
                     MDS_LAUNCHED();
                 }
-                if (!fold) {
+                if (!fold && !send_folds) {
                     hipLaunchKernelGGL(k_pr_base, dim3(base_wgs), dim3(256), 0, s, (const float*)L.partials.p,
                                        (const PrPart*)L.d_parts.p, nparts, d_f, L.base.p);
                     MDS_LAUNCHED();
@@ -925,17 +1021,15 @@ static void pr_run(medusa_graph* g, float damping, uint32_t steps, float* out, c
     MDS_HIP(hipEventRecord(g->ev_end, s));
     float* final_rank = rk[steps & 1];
     const float* prev_rank = rk[(steps + 1) & 1];
-    if (steps > 0) {
-        hipLaunchKernelGGL(k_zero_f64, dim3(1), dim3(1), 0, s, L.resid.p);
-        MDS_LAUNCHED();
-        hipLaunchKernelGGL(k_pr_resid, dim3(grid_for(n, 256, 512)), dim3(256), 0, s, n, (const float*)final_rank,
-                           prev_rank, L.resid.p);
-        MDS_LAUNCHED();
-    }
-    hipLaunchKernelGGL(k_pr_unpermute, dim3(grid_for(n, 256)), dim3(256), 0, s, n, L.iperm.p,
-                       (const float*)final_rank, L.unperm.p);
+    // without a superstep there is no previous iterate: the distance to itself is 0
+    const uint32_t fin = grid_for(n, 256, kFinishWgs);
+    hipLaunchKernelGGL(k_pr_finish, dim3(fin), dim3(256), 0, s, n, L.iperm.p, (const float*)final_rank,
+                       steps > 0 ? prev_rank : (const float*)final_rank, direct ? out : L.unperm.p, L.resid.p);
     MDS_LAUNCHED();
-    MDS_HIP(hipStreamSynchronize(s));
+    MDS_HIP(hipMemcpyAsync(L.h_resid.p, L.resid.p, fin * sizeof(double), hipMemcpyDeviceToHost, s));
+    if (!direct) copy_out(g, out, L.unperm.p, (size_t)n * 4);
+    else MDS_HIP(hipStreamSynchronize(s));
+    for (uint32_t i = 0; i < fin; ++i) st.residual_l1 += L.h_resid.p[i];
     float ms = 0;
     MDS_HIP(hipEventElapsedTime(&ms, g->ev_begin, g->ev_end));
     st.device_ms = ms;
@@ -972,8 +1066,6 @@ static void pr_run(medusa_graph* g, float damping, uint32_t steps, float* out, c
     st.edges_traversed = (uint64_t)steps * m;
     st.supersteps = steps;
     st.reached = n;
-    if (steps > 0) MDS_HIP(hipMemcpy(&st.residual_l1, L.resid.p, sizeof(double), hipMemcpyDeviceToHost));
-    copy_out(g, out, L.unperm.p, (size_t)n * 4);
 }
 
 }  // namespace medusa

@@ -113,6 +113,32 @@ def test_packed_pagerank_quarter_bins_large_items(oracle):
                     assert np.array_equal(_bits(r[begin[k]:begin[k + 1]]), _bits(want)), (k, steps, use_graph)
 
 
+@pytest.mark.parametrize("dangling", [
+    [300_000],                            # one graph, more than 64 blocks of 4096
+    [0, 5000, 0],                         # graphs with nothing dangling among others
+    [0, 0],                               # no dangling block at all
+    [40, 4096, 4097] + [30] * 67,         # more graphs than lanes, blocks at their edge
+    [131_072, 10], [131_073, 10],         # 32 and 33 blocks in one graph
+    [20] * 257,                           # more graphs than the send merges
+])
+def test_binned_dangling_bases(oracle, dangling):
+    """The bases of packed graphs merged by the send's last dangling wave, by a launch of their own
+    above its limits, or with no dangling block: per-graph bits equal the oracle's."""
+    graphs = []
+    for k, nd in enumerate(dangling):
+        rng = np.random.default_rng(100 + k)
+        core = 24  # vertices with out-edges; the others have none
+        arcs = np.stack([rng.integers(0, core, 96 + nd // 2), rng.integers(0, core + nd, 96 + nd // 2)], 1)
+        ring = np.stack([np.arange(core), (np.arange(core) + 1) % core], 1)
+        graphs.append(csr_from_edges(core + nd, np.concatenate([arcs, ring]))[:2])
+    with md.Graph.packed(graphs) as G:
+        begin = G.batch()
+        r, _ = G.pagerank(0.85, 4, variant=md.PR_BINNED)
+        for k, (rp, col) in enumerate(graphs):
+            want = oracle.pagerank_f32(rp, col, 0.85, 4)
+            assert np.array_equal(_bits(r[begin[k]:begin[k + 1]]), _bits(want)), k
+
+
 def test_set_batch_back_to_plain_graph(oracle):
     graphs = _mixed_batch()[:6]
     rp, col, _, begin = md.pack_graphs(graphs)
