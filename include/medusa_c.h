@@ -52,8 +52,9 @@ extern "C" {
 #define MEDUSA_DIR_PULL 2  /* bottom-up over CSC every superstep */
 
 /* PageRank kernel variant (opts.variant); all variants give bit-identical ranks. */
-#define MEDUSA_PR_DEFAULT 0 /* the engine's choice: MEDUSA_PR_BINNED, or MEDUSA_PR_PULL on a graph whose
-                               binned layout cannot be planned */
+#define MEDUSA_PR_DEFAULT 0 /* the engine's choice: MEDUSA_PR_PULL on a small graph (at most 2^19 arcs and 1024
+                               vertices without out-edges) or one whose binned layout cannot be planned,
+                               else MEDUSA_PR_BINNED */
 #define MEDUSA_PR_PUSH 1   /* scatter into per-in-edge message slots, then combine (reference style) */
 #define MEDUSA_PR_BINNED 2 /* message array blocked by source chunk and destination bin: streaming
                               writes of one message per out-edge, then a combine from LDS per bin */

@@ -201,7 +201,7 @@ void build_pr_layout(medusa_graph* g) {
         if (deg > kPrLaneMax) return kPrWave;
         return kPrLane;
     };
-    auto per_wg = [](uint32_t kind) -> uint32_t { return kind == kPrWave ? 4u : 256u; };
+    auto per_wg = [](uint32_t kind, uint32_t deg) -> uint32_t { return kind == kPrWave ? 4u : 4 * pr_lane_group(deg); };
     L->runs.clear();
     uint32_t wg = 0;
     uint64_t ell_size = 0;
@@ -227,7 +227,7 @@ void build_pr_layout(medusa_graph* g) {
             r.ell_base = ell_size;
             ell_size += (uint64_t)deg * r.ell_stride;
         }
-        wg += (r.count + per_wg(kind) - 1) / per_wg(kind);
+        wg += (r.count + per_wg(kind, r.deg) - 1) / per_wg(kind, r.deg);
         L->runs.push_back(r);
         p = q;
     }

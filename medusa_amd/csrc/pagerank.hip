@@ -155,31 +155,6 @@ __device__ __forceinline__ void lane_subtree(float& S, float& C, uint32_t r, uin
     C = c[0];
 }
 
-// Canonical sum of one vertex of in-degree deg <= 64 held by a single lane.
-// The 64-slot tree splits into 1, 2 or 4 interleaved 16-leaf subtrees.
-template <bool kFromMsg>
-__device__ __forceinline__ float lane_vertex_sum(uint32_t deg, const uint32_t* __restrict__ col, uint32_t stride,
-                                                 const float* __restrict__ vals, uint32_t seg) {
-    float s0, c0, s1, c1;
-    if (deg <= 16) {
-        lane_subtree<kFromMsg>(s0, c0, 0, 1, deg, col, stride, vals, seg);
-    } else if (deg <= 32) {
-        lane_subtree<kFromMsg>(s0, c0, 0, 2, deg, col, stride, vals, seg);
-        lane_subtree<kFromMsg>(s1, c1, 1, 2, deg, col, stride, vals, seg);
-        kahan_combine(s0, c0, s1, c1);
-    } else {
-        float s2, c2, s3, c3;
-        lane_subtree<kFromMsg>(s0, c0, 0, 4, deg, col, stride, vals, seg);
-        lane_subtree<kFromMsg>(s2, c2, 2, 4, deg, col, stride, vals, seg);
-        kahan_combine(s0, c0, s2, c2);
-        lane_subtree<kFromMsg>(s1, c1, 1, 4, deg, col, stride, vals, seg);
-        lane_subtree<kFromMsg>(s3, c3, 3, 4, deg, col, stride, vals, seg);
-        kahan_combine(s1, c1, s3, c3);
-        kahan_combine(s0, c0, s1, c1);
-    }
-    return s0 - c0;
-}
-
 // Binned variant: the sums of one lane item (planned by pr_bins.h), whose lane l holds slots
 // at[64 j + l], j = 0, 1, ...: with `per` = pr_lane_group(deg) vertices the item's slots are
 // column-major, so that is element r + st j of vertex l mod per, with st = 64 / per and
@@ -222,50 +197,6 @@ __device__ __forceinline__ float lane_item_sum(uint32_t deg, const float* at) {
     return s - c;
 }
 
-// One superstep for every vertex.  kFromMsg: values come from the message
-// array in slot order (push variant) instead of contrib[src] (pull variant).
-template <bool kFromMsg>
-__global__ __launch_bounds__(256) void k_pr_main(const PrRun* __restrict__ runs, const uint32_t* __restrict__ wg_run,
-                                                 const uint32_t* __restrict__ ell, const uint32_t* __restrict__ cptr,
-                                                 const uint32_t* __restrict__ crow,
-                                                 const float* __restrict__ vals,
-                                                 const uint32_t* __restrict__ outdeg,
-                                                 const float* __restrict__ base_p, float d,
-                                                 float* __restrict__ rank_out, float* __restrict__ contrib_out) {
-    const uint32_t wg = blockIdx.x;
-    const PrRun R = runs[wg_run[wg]];  // a table lookup, not a search at every workgroup's start
-    const uint32_t local = wg - R.wg_begin;
-    const uint32_t lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
-    const float base = base_p[R.part];
-
-    auto finish = [&](uint32_t p, float S) {
-        const float r = fmaf(d, S, base);
-        rank_out[p] = r;
-        const uint32_t od = outdeg[p];
-        if (od) contrib_out[p] = r / (float)od;
-    };
-
-    if (R.kind == kPrWave) {
-        const uint32_t p = R.begin + local * 4 + wave;
-        if (p >= R.begin + R.count) return;  // uniform across the wave
-        const uint32_t b = cptr[p], len = cptr[p + 1] - b;
-        const float S = wave_segment_sum(len, [&](uint32_t k) {
-            return kFromMsg ? vals[b + k] : vals[crow[b + k]];
-        });
-        if (lane == 0) finish(p, S);
-        return;
-    }
-    const uint32_t i = local * 256 + threadIdx.x;
-    if (i >= R.count) return;
-    const uint32_t p = R.begin + i;
-    if (R.kind == kPrZero) {
-        finish(p, 0.f);
-        return;
-    }
-    const uint32_t seg = kFromMsg ? cptr[p] : 0u;
-    finish(p, lane_vertex_sum<kFromMsg>(R.deg, ell + R.ell_base + i, R.ell_stride, vals, seg));
-}
-
 // Canonical (s, c) pair of one dangling block, computed by one wave (lane 0 holds it).
 __device__ __forceinline__ void dangle_block_sum(const float* __restrict__ rank, const PrBlock B, float& s, float& c) {
     const uint32_t lane = threadIdx.x & (kWave - 1);
@@ -286,6 +217,81 @@ __device__ __forceinline__ void dangle_block_sum(const float* __restrict__ rank,
     wave_tree(s, c);
 }
 
+// base = fmaf(d, D / (float)n_g, (float)((1 - d) / n_g)) for dangling mass D.
+__device__ __forceinline__ float pr_base_value(float D, float d, uint32_t n_g) {
+    const float tele = (float)((1.0 - (double)d) / (double)n_g);
+    return fmaf(d, D / (float)n_g, tele);
+}
+
+// A single graph with at most this many dangling vertices (one block): every wave of the pull or
+// push superstep sums them itself (16 loads a lane) instead of a launch of one workgroup doing it
+// before.  RMAT-16 (547 dangling), pull: 10.8 -> 9.2 us per superstep.  The
+// limit is one round of the sum's loads; each further round would add about as much to every wave
+// as the launch costs.
+constexpr uint32_t kOwnBaseVertices = 1024;
+
+// One superstep for every vertex.  kFromMsg: values come from the message
+// array in slot order (push variant) instead of contrib[src] (pull variant).  kOwnBase: every
+// wave sums the dangling block `dangling` of rank_in itself; otherwise base_p was written before.
+template <bool kFromMsg, bool kOwnBase>
+__global__ __launch_bounds__(256) void k_pr_main(const PrRun* __restrict__ runs, const uint32_t* __restrict__ wg_run,
+                                                 const uint32_t* __restrict__ ell, const uint32_t* __restrict__ cptr,
+                                                 const uint32_t* __restrict__ crow,
+                                                 const float* __restrict__ vals,
+                                                 const uint32_t* __restrict__ outdeg,
+                                                 const float* __restrict__ base_p,
+                                                 const float* __restrict__ rank_in, PrBlock dangling, uint32_t n,
+                                                 float d, float* __restrict__ rank_out,
+                                                 float* __restrict__ contrib_out) {
+    const uint32_t wg = blockIdx.x;
+    const PrRun R = runs[wg_run[wg]];  // a table lookup, not a search at every workgroup's start
+    const uint32_t local = wg - R.wg_begin;
+    const uint32_t lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
+    float base;
+    if constexpr (kOwnBase) {
+        float s, c;
+        dangle_block_sum(rank_in, dangling, s, c);
+        const float D = s - c;
+        base = pr_base_value(
+            __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, D))), d, n);
+    } else {
+        base = base_p[R.part];
+    }
+
+    auto finish = [&](uint32_t p, float S) {
+        const float r = fmaf(d, S, base);
+        rank_out[p] = r;
+        const uint32_t od = outdeg[p];
+        if (od) contrib_out[p] = r / (float)od;
+    };
+
+    if (R.kind == kPrWave) {
+        const uint32_t p = R.begin + local * 4 + wave;
+        if (p >= R.begin + R.count) return;  // uniform across the wave
+        const uint32_t b = cptr[p], len = cptr[p + 1] - b;
+        const float S = wave_segment_sum(len, [&](uint32_t k) {
+            return kFromMsg ? vals[b + k] : vals[crow[b + k]];
+        });
+        if (lane == 0) finish(p, S);
+        return;
+    }
+    // kPrLane (and kPrZero, whose deg is 0): a wave takes `per` vertices, 64 / per lanes each, so
+    // no lane gathers more than 16 values, in one round of loads.  With one lane per vertex
+    // whatever the in-degree, a vertex of 33..64 in-edges was four rounds of index loads and
+    // gathers in one lane: pull superstep of
+    // RMAT-16 9.2 -> 7.5 us, RMAT-18 32 -> 27 us (41 registers instead of 94).
+    const uint32_t per = pr_lane_group(R.deg), st = kWave / per;
+    const uint32_t i = local * 4 * per + wave * per + (lane & (per - 1));
+    const bool in = i < R.count;  // the lanes of a vertex agree
+    const uint32_t p = R.begin + (in ? i : 0u);
+    float S, C;
+    lane_subtree<kFromMsg>(S, C, lane / per, st, in ? R.deg : 0u, ell + R.ell_base + (in ? i : 0u), R.ell_stride, vals,
+                           kFromMsg ? cptr[p] : 0u);
+    if (st >= 2) merge32(S, C, S, C);
+    if (st == 4) merge16(S, C, S, C);
+    if (in && lane < per) finish(p, S - C);
+}
+
 // Dangling mass, step 1: one wave per canonical block of a graph's dangling tail
 // writes the block's (s, c) pair.
 __global__ __launch_bounds__(256) void k_pr_dangle(const float* __restrict__ rank, const PrBlock* __restrict__ blocks,
@@ -299,12 +305,6 @@ __global__ __launch_bounds__(256) void k_pr_dangle(const float* __restrict__ ran
         partials[2 * b] = s;
         partials[2 * b + 1] = c;
     }
-}
-
-// base = fmaf(d, D / (float)n_g, (float)((1 - d) / n_g)) for dangling mass D.
-__device__ __forceinline__ float pr_base_value(float D, float d, uint32_t n_g) {
-    const float tele = (float)((1.0 - (double)d) / (double)n_g);
-    return fmaf(d, D / (float)n_g, tele);
 }
 
 // base = fmaf(d, D / (float)n_g, (float)((1 - d) / n_g)) of a graph whose `nblocks` block pairs
@@ -841,6 +841,14 @@ __global__ __launch_bounds__(256) void k_pr_finish(uint32_t n, const uint32_t* _
 // combine (every wave merges the block pairs itself) instead of in a launch of its own.
 constexpr uint32_t kFoldBlocks = 64;
 
+// In-edges up to which the default variant is the pull, when its superstep is one launch
+// (kOwnBaseVertices); us per superstep, pull against binned: R-MAT 12 (66 K arcs) 4.7 and 8.0,
+// 14 (262 K) 5.2 and 8.3, 15 (524 K) 5.6 and 9.1, 16 (1.05 M) 7.5 and 10.9, 17 (2.1 M) 14.0 and
+// 18.0, 18 (4.2 M) 27.5 and 25.6.  From here to about 3 M in-edges the pull is still the faster,
+// but what decides there (dangling share, in-degree spread) is what the variant policy learns,
+// and its measured gain is defined against the fixed binned variant.
+constexpr uint64_t kPullDefaultEdges = 1u << 19;
+
 static void pr_run(medusa_graph* g, float damping, uint32_t steps, float* out, const medusa_opts& o,
                    medusa_stats& st) {
     build_pr_layout(g);
@@ -853,10 +861,13 @@ static void pr_run(medusa_graph* g, float damping, uint32_t steps, float* out, c
     MDS_CHECK(o.variant == MEDUSA_PR_DEFAULT || o.variant == MEDUSA_PR_PULL || o.variant == MEDUSA_PR_PUSH ||
                   o.variant == MEDUSA_PR_BINNED,
               MEDUSA_ERR_ARG, "pagerank: unknown variant %d", o.variant);
-    // the engine's default: the binned exchange wherever its layout can be planned
-    const int dflt = o.variant != MEDUSA_PR_DEFAULT       ? o.variant
-                     : build_pr_bins(g, /*required=*/false) ? MEDUSA_PR_BINNED
-                                                            : MEDUSA_PR_PULL;
+    // the engine's default: the pull on small graphs, else the binned exchange wherever its layout
+    // can be planned
+    const bool own_base = L.parts.size() == 1 && nd <= kOwnBaseVertices;
+    const int dflt = o.variant != MEDUSA_PR_DEFAULT             ? o.variant
+                     : own_base && m <= kPullDefaultEdges       ? MEDUSA_PR_PULL
+                     : build_pr_bins(g, /*required=*/false)     ? MEDUSA_PR_BINNED
+                                                                : MEDUSA_PR_PULL;
     // kernel variant of every superstep: the caller's, or the learned policy's per superstep
     // (it keeps the caller's unless it predicts a clear gain); the ranks are the same bits
     uint64_t wave_vertices = 0, lane_vertices = 0;
@@ -967,21 +978,19 @@ static void pr_run(medusa_graph* g, float damping, uint32_t steps, float* out, c
                 if (with_events) MDS_HIP(hipEventRecord(g->events[3 * t + 2], s));
                 continue;
             }
-            enqueue_base(r_in);
+            if (!own_base) enqueue_base(r_in);
             if (step_push) {
                 hipLaunchKernelGGL(k_pr_scatter, dim3(grid_for(n, 4, 16384)), dim3(256), 0, s, n, L.optr.p,
                                    L.oslot.p, c_in, L.msg.p);
                 MDS_LAUNCHED();
             }
             if (with_events) MDS_HIP(hipEventRecord(g->events[3 * t + 1], s));
-            if (step_push)
-                hipLaunchKernelGGL(k_pr_main<true>, dim3(L.total_wgs), dim3(256), 0, s, (const PrRun*)L.d_runs.p,
-                                   (const uint32_t*)L.d_wg_run.p, (const uint32_t*)L.ell.p, L.cptr.p, L.crow.p,
-                                   (const float*)L.msg.p, L.outdeg.p, (const float*)L.base.p, d_f, r_out, c_out);
-            else
-                hipLaunchKernelGGL(k_pr_main<false>, dim3(L.total_wgs), dim3(256), 0, s, (const PrRun*)L.d_runs.p,
-                                   (const uint32_t*)L.d_wg_run.p, (const uint32_t*)L.ell.p, L.cptr.p, L.crow.p, c_in,
-                                   L.outdeg.p, (const float*)L.base.p, d_f, r_out, c_out);
+            auto kern = step_push ? (own_base ? k_pr_main<true, true> : k_pr_main<true, false>)
+                                  : (own_base ? k_pr_main<false, true> : k_pr_main<false, false>);
+            hipLaunchKernelGGL(kern, dim3(L.total_wgs), dim3(256), 0, s, (const PrRun*)L.d_runs.p,
+                               (const uint32_t*)L.d_wg_run.p, (const uint32_t*)L.ell.p, L.cptr.p, L.crow.p,
+                               step_push ? (const float*)L.msg.p : c_in, L.outdeg.p, (const float*)L.base.p, r_in,
+                               nblk ? L.blocks[0] : PrBlock{0, 0}, n, d_f, r_out, c_out);
             MDS_LAUNCHED();
             if (with_events) MDS_HIP(hipEventRecord(g->events[3 * t + 2], s));
         }

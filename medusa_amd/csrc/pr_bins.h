@@ -38,6 +38,7 @@ constexpr uint32_t kPrBinMaxItems = 512;      // items of one bin (8 waves hold 
 constexpr uint32_t kPrBinRuns = 2048;         // runs (chunks sending to it) one bin may have
 constexpr uint32_t kPrChunkSources = 8192;    // sources of one send chunk (their contributions fit LDS)
 constexpr uint32_t kPrTileEdges = 16384;      // message entries written by one send workgroup (at least)
+constexpr uint32_t kPrTileSmall = 4096;       // ... on graphs whose tiles take at most a quarter of one round
 constexpr uint32_t kPrHubDeg = 4096;          // in-degree above which a destination is summed by gather
 constexpr uint32_t kPrRunAlign = 4;           // runs start and end on multiples of this many entries
 constexpr uint16_t kPrDummySlot = (uint16_t)kPrBinValues;  // LDS slot of padding entries
@@ -194,9 +195,14 @@ inline std::string plan_pr_bins(uint32_t n, const uint32_t* cptr, const uint32_t
     // The combine runs its bins in rounds of combine_slots workgroups.  When the last round is
     // short (at most a quarter of the slots: RMAT-20, 2231 bins for 1024), its bins would run
     // nearly alone at the end; the vertices of those bins are planned again into quarter-size
-    // bins, which spread that work over the workgroups as they free up.
+    // bins, which spread that work over the workgroups as they free up.  A graph whose bins take
+    // at most a quarter of one round gets quarter-size bins throughout: four times as many
+    // workgroups, each with a quarter of the entries and sums (RMAT-16, 141 bins: combine 8.8 ->
+    // 5.0 us).
     plan_items(n);
-    if (combine_slots && P.bins.size() > combine_slots) {
+    if (combine_slots && P.bins.size() <= combine_slots / 4) {
+        plan_items(0);
+    } else if (combine_slots && P.bins.size() > combine_slots) {
         const uint64_t r = P.bins.size() % combine_slots;
         if (r && r <= combine_slots / 4) plan_items(P.items[P.bins[P.bins.size() - r].item_begin].v);
     }
@@ -281,7 +287,9 @@ inline std::string plan_pr_bins(uint32_t n, const uint32_t* cptr, const uint32_t
     // send) tiles, so T = nentry / (slots - those chunks) fits one round.  A larger T is not
     // taken: tiles of many small chunks would then differ widely in length, the longest alone at
     // the end (a batch of 128 graphs, 789 chunks for 1023 slots, ran 17 % slower that way).
-    // Tiles never get smaller: each recomputes its chunk's contributions.
+    // Smaller tiles repeat the computation of their chunk's contributions, which only pays where the
+    // tiles take at most a quarter of a round (RMAT-16, 64 tiles of 16,384 or 256 of 4096: 381 or
+    // 360 us per 30 supersteps; a batch of 64 graphs, half a round, with 9,300: 551 instead of 545).
     uint64_t sending = 0, fixed_tiles = 0;
     for (uint64_t c = 0; c < C; ++c) {
         sending += chunk_start[c + 1] > chunk_start[c];
@@ -291,6 +299,8 @@ inline std::string plan_pr_bins(uint32_t n, const uint32_t* cptr, const uint32_t
         const uint64_t even = (P.nentry + (send_slots - sending) - 1) / (send_slots - sending);
         const uint64_t T = (even + kPrRunAlign - 1) / kPrRunAlign * kPrRunAlign;
         if (T > kPrTileEdges && T <= 2ull * kPrTileEdges) P.tile_edges = (uint32_t)T;
+    } else if (fixed_tiles <= send_slots / 4) {
+        P.tile_edges = kPrTileSmall;
     }
     for (uint64_t c = 0; c < C; ++c) {
         const uint32_t src = (uint32_t)(c * kPrChunkSources);
@@ -360,7 +370,7 @@ inline std::string check_pr_bins(uint32_t n, const uint32_t* cptr, const PrBinsP
         if (verts > kPrBinMaxVertices) return "bins: vertices per bin";
     }
     if (real != P.nmsg) return "bins: message count";
-    if (P.tile_edges < kPrTileEdges || P.tile_edges % kPrRunAlign) return "bins: tile size";
+    if (P.tile_edges < kPrTileSmall || P.tile_edges % kPrRunAlign) return "bins: tile size";
     for (const PrTile& T : P.tiles) {
         if (T.msg_begin > T.msg_end || T.msg_end > P.nentry || T.msg_end - T.msg_begin > P.tile_edges)
             return "bins: tile entries";

@@ -115,6 +115,24 @@ def test_pagerank_binned_shapes(oracle):
                     assert np.array_equal(_bits(r), _bits(want)), (len(rp) - 1, steps, use_graph)
 
 
+@pytest.mark.parametrize("dangling", [0, 1, 63, 1024, 1025])
+def test_own_base_and_default_variant(oracle, dangling):
+    """Pull and push supersteps that sum up to 1024 dangling vertices themselves, the launch above
+    that, and the default variant on either side of both limits; bits equal throughout."""
+    rng = np.random.default_rng(7 + dangling)
+    core = 3000
+    for m in (1 << 19, (1 << 19) + 1):
+        ring = np.stack([np.arange(core), (np.arange(core) + 1) % core], 1)
+        arcs = np.stack([rng.integers(0, core, m - core), rng.integers(0, core + dangling, m - core)], 1)
+        rp, col, _ = csr_from_edges(core + dangling, np.concatenate([ring, arcs]))
+        want = oracle.pagerank_f32(rp, col, 0.85, 4)
+        with md.Graph(rp, col) as G:
+            for v in (md.PR_PULL, md.PR_PUSH, md.PR_BINNED, md.PR_DEFAULT):
+                r, st = G.pagerank(0.85, 4, variant=v)
+                assert np.array_equal(_bits(r), _bits(want)), (m, v)
+            assert st.pull_steps == (4 if dangling <= 1024 and m <= 1 << 19 else 0)
+
+
 @pytest.mark.parametrize("deg", [1, 8, 9, 16, 17, 32, 33, 64, 65, 127, 192, 4096])
 def test_binned_item_shapes(oracle, deg):
     """In-degrees at the edges of the combine's item classes (64, 32 or 16 vertices per lane item;

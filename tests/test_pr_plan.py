@@ -106,6 +106,23 @@ def test_long_last_combine_round_kept(checker, tmp_path, random_csc):
     assert out["bins1"] == b0
 
 
+def test_bins_of_a_small_graph_are_quarter_size(checker, tmp_path, random_csc):
+    """Bins that take at most a quarter of one combine round are all planned at a quarter of the
+    size; one bin more than that keeps the full size."""
+    b0 = _plan(checker, tmp_path, random_csc, 0, 0)["bins0"]
+    out = _plan(checker, tmp_path, random_csc, 0, 4 * b0)
+    assert out["bins1"] == out["tail_bins"] > 3 * b0 and out["tail_max_slots"] <= BIN // 4
+    assert _plan(checker, tmp_path, random_csc, 0, 4 * b0 - 1)["bins1"] == b0
+
+
+def test_send_tiles_of_a_small_graph(checker, tmp_path, random_csc):
+    """Tiles that take at most a quarter of one send round are cut to 4096 entries."""
+    t0 = _plan(checker, tmp_path, random_csc, 0, 0)["tiles0"]
+    out = _plan(checker, tmp_path, random_csc, 4 * t0, 0)
+    assert out["tile_edges1"] == out["max_tile1"] == TILE // 4 and out["tiles1"] > 3 * t0
+    assert _plan(checker, tmp_path, random_csc, 4 * t0 - 1, 0)["tile_edges1"] == TILE
+
+
 def test_quarter_bins_hold_larger_items_alone(checker, tmp_path):
     """A packed batch whose last graph (in the tail) has wave vertices of in-degree 2100-4000 and
     lane groups of in-degree 40-64, whose slots exceed a quarter-size bin: each gets a bin of its
