@@ -258,6 +258,7 @@ struct medusa_graph {
     uint32_t n = 0;
     uint64_t m = 0;
     bool weighted = false;
+    uint32_t max_outdeg = 0;
     int device = 0;
     hipStream_t stream = nullptr;
     // host copies (layouts are derived from them)
@@ -277,6 +278,7 @@ struct medusa_graph {
     medusa::DBuf<unsigned long long> bitmap;
     medusa::DBuf<unsigned long long> near_q;  // SSSP near queues of (slice << 32 | vertex) entries
     medusa::DBuf<unsigned long long> sssp_phases;  // SSSP device-loop phase marks (trace on)
+    medusa::DBuf<uint4> sssp_rec;  // SSSP vertex records (local rounds without hubs), 64 bytes each
     // per-superstep counters (device) and their pinned host mirror; each engine
     // views the 256 bytes as its own counter struct
     medusa::DBuf<unsigned long long> ctr_raw;
@@ -359,15 +361,25 @@ __device__ __forceinline__ uint32_t lane_id() {
 __device__ __forceinline__ uint32_t lanes_below(unsigned long long mask) {
     return __builtin_amdgcn_mbcnt_hi((uint32_t)(mask >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)mask, 0u));
 }
+// x of another lane through the vector unit's data-parallel primitives; 0 where kCtrl has no
+// source lane or kRows leaves the row out.
+template <int kCtrl, int kRows = 0xf>
+__device__ __forceinline__ uint32_t dpp_or_zero(uint32_t x) {
+    return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, kCtrl, kRows, 0xf, false);
+}
+// Inclusive prefix sum over the wave (every lane active): a scan of every 16-lane row by row
+// shifts, then the rows' totals by the two row broadcasts; six additions and no LDS crossbar.
 __device__ __forceinline__ uint32_t wave_incl_scan(uint32_t x) {
-    const uint32_t lane = lane_id();
-#pragma unroll
-    for (int off = 1; off < kWave; off <<= 1) {
-        const uint32_t y = __shfl_up(x, off, kWave);
-        if (lane >= (uint32_t)off) x += y;
-    }
+    x += dpp_or_zero<0x111>(x);        // row_shr:1
+    x += dpp_or_zero<0x112>(x);        // row_shr:2
+    x += dpp_or_zero<0x114>(x);        // row_shr:4
+    x += dpp_or_zero<0x118>(x);        // row_shr:8
+    x += dpp_or_zero<0x142, 0xa>(x);   // row_bcast:15 into rows 1 and 3
+    x += dpp_or_zero<0x143, 0xc>(x);   // row_bcast:31 into rows 2 and 3
     return x;
 }
+// Orders this wave's LDS accesses for the compiler (the hardware keeps them in order).
+__device__ __forceinline__ void wave_lds_fence() { __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront"); }
 __device__ __forceinline__ unsigned long long wave_sum_u64(unsigned long long x) {
 #pragma unroll
     for (int off = kWave / 2; off >= 1; off >>= 1) x += __shfl_xor(x, off, kWave);

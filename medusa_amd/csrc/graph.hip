@@ -352,6 +352,7 @@ extern "C" int medusa_graph_create(uint32_t n, uint64_t m, const uint32_t* row_p
         g->n = n;
         g->m = m;
         g->weighted = weight != nullptr;
+        for (uint32_t v = 0; v < n; ++v) g->max_outdeg = std::max(g->max_outdeg, row_ptr[v + 1] - row_ptr[v]);
         MDS_HIP(hipGetDevice(&g->device));
         MDS_HIP(hipStreamCreateWithFlags(&g->stream, hipStreamNonBlocking));
         MDS_HIP(hipEventCreate(&g->ev_begin));

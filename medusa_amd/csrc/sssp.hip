@@ -26,7 +26,8 @@
 // so the frontier advances several hops per superstep.  This stays exact: a vertex kept
 // here is relaxed at the distance this workgroup wrote into it (if its atomicMin found a
 // lower one, that value's writer relaxes the vertex), and any later, lower offer from
-// another workgroup puts it in the near queue by stamp as usual.
+// another workgroup puts it in the near queue by stamp as usual.  On graphs without hubs every
+// wave does this on its own (wave rounds, below).
 
 #include <algorithm>
 #include <chrono>
@@ -399,6 +400,293 @@ __device__ __forceinline__ uint32_t wave_min_u32(uint32_t x) {
     return x;
 }
 
+// ---- wave rounds -------------------------------------------------------------------------
+// Local rounds on graphs without hubs (largest out-degree at most kSlice; a road network).  Such a
+// run is bound by the latency of one hop after the other, so a hop is kept to one memory round
+// trip.  A wave works through a ring of offers (target, distance) in LDS, 64 at a time: the
+// returning atomicMin on the target's distance and the load of the target's record (its
+// out-degree and up to kRecEdges out-edges in 64 bytes) are issued together, and a target lowered
+// below the threshold puts the offers of its own out-edges into the ring.  No barrier, no search
+// for an edge's owner, no second round trip for the edges, and only the offer that lowered a
+// vertex goes on (1.7 relaxations per edge of the 1400^2 lattice; 2.6 with plain reads of the
+// distance, whose line in this XCD's L2 may be old).  About 0.9 us per hop against 2.1 in the
+// block-wide tiles: 1400^2 lattice 7.73 -> 3.95 ms, 173 x 211 0.91 -> 0.50 ms, uniform random
+// graphs of mean out-degree 2 and 4 (262 K vertices) 0.47 -> 0.23 and 0.77 -> 0.46 ms.  With hubs
+// the rings of a few waves hold the frontier and the others idle (2.4 M-vertex Chung-Lu graph,
+// out-degrees up to 100 K: 1.3 ms against 0.75 in the block-wide tiles), hence the rule.
+constexpr uint32_t kRecEdges = 7;
+constexpr uint32_t kRecWords = 4;        // uint4 per record: {out-degree, row_ptr, (target, weight) x 7}
+constexpr uint32_t kRing = 512;          // offers per wave
+constexpr uint32_t kKeep = 128;          // offers past which a wave hands vertices to the near queue, so
+                                         // a growing frontier spreads over all waves (64: lattice 5.3 ms)
+constexpr uint32_t kWaveFar = 128;       // staged far appends per wave
+constexpr uint32_t kWide = 4;            // out-edges per lane in flight of vertices beyond their record
+constexpr uint32_t kWaveThreads = 1024;  // few workgroups, so few atomics on the queue counters
+constexpr uint32_t kBlockWaves = kWaveThreads / kWave;
+constexpr uint32_t kSsspGridWave = 256;  // a workgroup per CU (LDS)
+static_assert(kRing >= kWave * kRecEdges && kRing >= kWave * kWide && kRing >= kKeep && (kRing & (kRing - 1)) == 0,
+              "a tile's offers fit");
+
+__global__ __launch_bounds__(256) void k_sssp_records(uint32_t n, const uint32_t* __restrict__ row_ptr,
+                                                      const uint32_t* __restrict__ col,
+                                                      const uint32_t* __restrict__ w, uint4* __restrict__ rec) {
+    for (uint64_t v = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x; v < n; v += (uint64_t)gridDim.x * blockDim.x) {
+        const uint32_t b = row_ptr[v], deg = row_ptr[v + 1] - b;
+        uint32_t x[16] = {deg, b};
+#pragma unroll
+        for (uint32_t k = 0; k < kRecEdges; ++k)
+            if (k < deg) {
+                x[2 + 2 * k] = col[b + k];
+                x[3 + 2 * k] = w[b + k];
+            }
+#pragma unroll
+        for (uint32_t q = 0; q < kRecWords; ++q)
+            rec[v * kRecWords + q] = uint4{x[4 * q], x[4 * q + 1], x[4 * q + 2], x[4 * q + 3]};
+    }
+}
+
+struct WaveLds {
+    unsigned long long ring[kBlockWaves][kRing];  // distance << 32 | target
+    uint32_t far[kBlockWaves][kWaveFar];
+    uint32_t off[kBlockWaves][kWave], beg[kBlockWaves][kWave], du[kBlockWaves][kWave];  // push_wide
+    uint32_t n_far[kBlockWaves], fmin[kBlockWaves];
+    unsigned long long relax[kBlockWaves];
+};
+
+struct WaveIn {
+    const uint4* rec;
+    const uint32_t *col, *w;
+    uint32_t *dist, *stamp;
+    uint32_t epoch;          // stamp of the vertices that the rounds hand to the near queue
+    uint32_t thr, rounds;
+    // relaxation superstep: near entries q[0, count); split: far entries (or every vertex)
+    const unsigned long long* q;
+    const uint32_t* far_in;
+    uint32_t count, rescan, split_epoch, old_thr;
+};
+
+// Entries per wave: so many that every wave of the grid gets some, at most 64.
+__device__ __forceinline__ uint32_t wave_tile_entries(uint32_t qn, uint32_t waves) {
+    const uint32_t per = (uint32_t)(((uint64_t)qn + waves - 1) / waves);
+    return per < 1u ? 1u : (per > (uint32_t)kWave ? (uint32_t)kWave : per);
+}
+
+// One superstep by the whole block, each wave on its own: seeds (a tile of near
+// entries; with kSplit the far entries that the new threshold moves) put the offers of their
+// out-edges into the wave's ring, then the wave works the ring off.  The offers that the seeds
+// make are the superstep's own relaxation; the vertices that they and up to `rounds` - 1 further
+// generations of offers lower are expanded here, those of the last generation, and any beyond
+// kKeep offers, go to the near queue (once per superstep, by stamp).  `relax` counts the offers and
+// `fmin` is the smallest distance appended to the far queue, both for the block in thread 0;
+// every other counter atomic of the block has returned when this does.
+template <bool kSplit>
+__device__ __forceinline__ void wave_superstep(const WaveIn& a, WaveLds& L, const Sinks& k,
+                                                unsigned long long& relax, uint32_t& fmin) {
+    const uint32_t lane = threadIdx.x & (kWave - 1), wv = threadIdx.x / kWave;
+    unsigned long long* ring = L.ring[wv];
+    uint32_t* far = L.far[wv];
+    uint32_t head = 0, tail = 0, nfar = 0, offers = 0, gen = 0, gen_end = 0;  // uniform in the wave
+    uint32_t least = 0xFFFFFFFFu;
+    bool draining = false;
+
+    auto flush_far = [&](uint32_t base) {
+        for (uint32_t i = lane; i < nfar; i += kWave)
+            if (base + i < k.far_cap) k.far[base + i] = far[i];
+    };
+    auto put_far = [&](bool p, uint32_t v) {
+        const unsigned long long m = __ballot(p);
+        if (!m) return;
+        if (nfar + kWave > kWaveFar) {
+            uint32_t base = 0;
+            if (lane == 0) base = atomicAdd(k.far_cnt, nfar);
+            flush_far(__builtin_amdgcn_readfirstlane(base));
+            wave_lds_fence();
+            nfar = 0;
+        }
+        if (p) far[nfar + lanes_below(m)] = v;
+        wave_lds_fence();
+        nfar += (uint32_t)__popcll(m);
+    };
+    // every lane calls it: the lanes' vertices with p, once per superstep (by stamp), to the near queue
+    auto put_near = [&](bool p, uint32_t v) {
+        p = p && atomicMax(&a.stamp[v], a.epoch) < a.epoch;
+        const unsigned long long m = __ballot(p);
+        if (!m) return;
+        uint32_t base = 0;
+        if (lane == 0) base = atomicAdd(k.near_cnt, (uint32_t)__popcll(m));
+        base = __builtin_amdgcn_readfirstlane(base) + lanes_below(m);
+        if (p && base < k.near_cap) k.near[base] = v;  // slice 0, its only one
+    };
+    // offer of an edge of weight w from distance d (a sum past 32 bits never lowers anything)
+    auto offer = [](uint32_t v, uint32_t d, uint32_t w) {
+        const unsigned long long s = (unsigned long long)d + w;
+        return (s < 0xFFFFFFFFull ? s << 32 : 0xFFFFFFFFull << 32) | v;
+    };
+    auto load_rec = [&](uint32_t v, uint4 (&r)[kRecWords]) {
+#pragma unroll
+        for (uint32_t q = 0; q < kRecWords; ++q) r[q] = a.rec[(size_t)v * kRecWords + q];
+    };
+    // the offers of the records of the lanes with c > 0 (c <= kRecEdges out-edges; all fit)
+    auto push_rec = [&](uint32_t c, uint32_t d, const uint4 (&r)[kRecWords]) {
+        const uint32_t incl = wave_incl_scan(c), total = __builtin_amdgcn_readlane(incl, kWave - 1);
+        const uint32_t e[2 * kRecEdges] = {r[0].z, r[0].w, r[1].x, r[1].y, r[1].z, r[1].w, r[2].x,
+                                           r[2].y, r[2].z, r[2].w, r[3].x, r[3].y, r[3].z, r[3].w};
+        const uint32_t at = tail + incl - c;
+#pragma unroll
+        for (uint32_t j = 0; j < kRecEdges; ++j)
+            if (j < c) ring[(at + j) & (kRing - 1)] = offer(e[2 * j], d, e[2 * j + 1]);
+        wave_lds_fence();
+        tail += total;
+    };
+    // the offers of out-edges [beg, beg + cnt) of every lane from its distance d: the wave shares
+    // the edges through a prefix sum, kWide * 64 at a time, their loads issued together; `room`
+    // makes space for that many or is a no-op where all are known to fit
+    auto push_wide = [&](uint32_t beg, uint32_t cnt, uint32_t d, auto room) {
+        const uint32_t incl = wave_incl_scan(cnt), total = __builtin_amdgcn_readlane(incl, kWave - 1);
+        if (!total) return;
+        L.off[wv][lane] = incl - cnt;
+        L.beg[wv][lane] = beg;
+        L.du[wv][lane] = d;
+        wave_lds_fence();
+        for (uint32_t e0 = 0; e0 < total; e0 += kWide * kWave) {
+            room();
+            uint32_t v[kWide], wt[kWide], from[kWide];
+#pragma unroll
+            for (uint32_t j = 0; j < kWide; ++j) {
+                const uint32_t e = e0 + j * kWave + lane;
+                if (e >= total) continue;
+                uint32_t lo = 0;  // the last lane whose first edge is <= e (it has edges)
+#pragma unroll
+                for (uint32_t step = kWave / 2; step; step >>= 1)
+                    if (L.off[wv][lo + step] <= e) lo += step;
+                const uint32_t x = L.beg[wv][lo] + (e - L.off[wv][lo]);
+                v[j] = a.col[x];
+                wt[j] = a.w[x];
+                from[j] = L.du[wv][lo];
+            }
+#pragma unroll
+            for (uint32_t j = 0; j < kWide; ++j) {
+                const uint32_t e = e0 + j * kWave + lane;
+                if (e < total) ring[(tail + j * kWave + lane) & (kRing - 1)] = offer(v[j], from[j], wt[j]);
+            }
+            wave_lds_fence();
+            tail += min(total - e0, kWide * kWave);
+        }
+    };
+    // up to 64 offers of the current generation
+    auto batch = [&]() {
+        if (head == gen_end) {
+            gen_end = tail;
+            ++gen;
+        }
+        const bool expand = gen <= a.rounds;
+        const uint32_t cnt = min(gen_end - head, (uint32_t)kWave);
+        const bool on = lane < cnt;
+        const unsigned long long o = on ? ring[(head + lane) & (kRing - 1)] : 0ull;
+        wave_lds_fence();
+        head += cnt;
+        offers += cnt;
+        const uint32_t v = (uint32_t)o, nd = (uint32_t)(o >> 32);
+        const bool below = on && nd < a.thr;
+        uint4 r[kRecWords] = {};
+        if (below && expand) load_rec(v, r);
+        const bool low = on && nd < atomicMin(&a.dist[v], nd);
+        const bool beyond = low && nd >= a.thr;
+        if (beyond) least = min(least, nd);
+        put_far(beyond, v);
+        const bool grow = low && below;
+        if (!__ballot(grow)) return;
+        const uint32_t deg = grow ? r[0].x : 0u;
+        const uint32_t total = __builtin_amdgcn_readlane(wave_incl_scan(deg), kWave - 1);
+        const bool any_wide = __ballot(deg > kRecEdges) != 0;
+        // (a drain inside push_wide must not enter push_wide again: its LDS is in use)
+        if (!expand || tail - head + total > kKeep || (draining && any_wide)) {  // uniform
+            put_near(expand ? deg > 0 : grow, v);
+            return;
+        }
+        push_rec(deg <= kRecEdges ? deg : 0u, nd, r);
+        if (any_wide) push_wide(r[0].y, deg > kRecEdges ? deg : 0u, nd, [] {});
+    };
+    auto make_room = [&](uint32_t need) {
+        draining = true;
+        while (tail - head + need > kRing) batch();
+        draining = false;
+    };
+
+    const uint32_t waves = gridDim.x * kBlockWaves, T = wave_tile_entries(a.count, waves);
+    for (uint32_t chunk = blockIdx.x * kBlockWaves + wv; (uint64_t)chunk * T < a.count; chunk += waves) {
+        const uint64_t i = (uint64_t)chunk * T + lane;
+        const bool in = lane < T && i < a.count;
+        uint32_t v = 0, d = 0, deg = 0;
+        uint4 r[kRecWords] = {};
+        if constexpr (kSplit) {
+            if (in) {
+                v = a.rescan ? (uint32_t)i : a.far_in[i];
+                d = a.dist[v];
+                load_rec(v, r);
+            }
+            const bool open = in && d != 0xFFFFFFFFu && d >= a.old_thr;
+            const bool mine = open && atomicMax(&a.stamp[v], a.split_epoch) < a.split_epoch;
+            const bool keep = mine && d >= a.thr;
+            if (keep) least = min(least, d);
+            put_far(keep, v);
+            deg = mine && !keep ? r[0].x : 0u;
+        } else if (in) {
+            v = (uint32_t)a.q[i];
+            d = a.dist[v];
+            load_rec(v, r);
+            deg = r[0].x;
+        }
+        make_room(kWave * kRecEdges);
+        push_rec(deg <= kRecEdges ? deg : 0u, d, r);
+        push_wide(r[0].y, deg > kRecEdges ? deg : 0u, d, [&] { make_room(kWide * kWave); });
+    }
+    while (head != tail) batch();
+
+#pragma unroll
+    for (int off = kWave / 2; off >= 1; off >>= 1) least = min(least, (uint32_t)__shfl_xor(least, off, kWave));
+    if (lane == 0) {
+        L.n_far[wv] = nfar;
+        L.relax[wv] = offers;
+        L.fmin[wv] = least;
+    }
+    __syncthreads();
+    // one far append for the block
+    uint32_t before = 0, total = 0;
+    for (uint32_t w = 0; w < kBlockWaves; ++w) {
+        if (w < wv) before += L.n_far[w];
+        total += L.n_far[w];
+    }
+    relax = 0;
+    fmin = 0xFFFFFFFFu;
+    __shared__ uint32_t s_base;
+    if (threadIdx.x == 0) {
+        s_base = total ? atomicAdd(k.far_cnt, total) : 0u;
+        for (uint32_t w = 0; w < kBlockWaves; ++w) {
+            relax += L.relax[w];
+            fmin = min(fmin, L.fmin[w]);
+        }
+    }
+    __syncthreads();
+    flush_far(s_base + before);
+}
+
+// One relaxation superstep over the near queue with wave rounds (host-driven loop).
+__global__ __launch_bounds__(kWaveThreads) void k_sssp_relax_wave(
+    const unsigned long long* __restrict__ q, uint32_t qn, const uint32_t* __restrict__ row_ptr,
+    const uint32_t* __restrict__ col, const uint32_t* __restrict__ w, const uint4* __restrict__ rec, uint32_t* dist,
+    uint32_t* __restrict__ stamp, uint32_t epoch, uint32_t thr, unsigned long long* __restrict__ near_next,
+    uint32_t near_cap, uint32_t* __restrict__ far_q, uint32_t far_cap, SsspCounters* __restrict__ ctr,
+    uint32_t rounds) {
+    __shared__ WaveLds lds;
+    const Sinks k{near_next, &ctr->n_near, near_cap, far_q, &ctr->n_far, far_cap, row_ptr};
+    const WaveIn in{rec, col, w, dist, stamp, epoch, thr, rounds, q, nullptr, qn, 0, 0, 0};
+    unsigned long long relax;
+    uint32_t fmin;
+    wave_superstep<false>(in, lds, k, relax, fmin);
+    if (threadIdx.x == 0 && relax) atomicAdd(&ctr->relax, relax);
+}
+
 // One relaxation superstep over the near queue (host-driven loop); kLoc: with the local list
 // (its LDS is allocated only in that variant).
 template <bool kLoc>
@@ -496,19 +784,19 @@ __device__ __forceinline__ void phase_mark(unsigned long long* marks, uint32_t i
 
 // Tickets of the last-workgroup election: workgroup b takes a ticket on line b mod kSsspSlots,
 // and the last of a line's workgroups one on `top`, so no address sees more than
-// grid / kSsspSlots atomics (same-address device atomics serialise).
+// grid / kSsspSlots atomics (same-address device atomics serialise).  A ticket also adds the
+// workgroup's relaxed edges: the low 16 bits count, the rest sum.
 constexpr uint32_t kSsspSlots = 32;
 struct SsspTicket {
-    alignas(128) uint32_t v;
+    alignas(128) unsigned long long v;
 };
 struct SsspDevCounters {
     MDS_COUNTER(uint32_t, n_near);   // near entries written by this slot's work kernel
     MDS_COUNTER(uint32_t, n_far);    // far queue length (relax appends after the current entries)
     MDS_COUNTER(uint32_t, far_out);  // far entries kept by a split
     MDS_COUNTER(uint32_t, far_min);  // smallest distance kept by a split
-    MDS_COUNTER(unsigned long long, relax);
     SsspTicket sub[kSsspSlots];
-    MDS_COUNTER(uint32_t, top);
+    MDS_COUNTER(unsigned long long, top);
 };
 // storage units of the device-driven loop: the control block, then the counters
 constexpr size_t kSsspCtlUnits = 1 + (sizeof(SsspDevCounters) + sizeof(CtlStorage) - 1) / sizeof(CtlStorage);
@@ -522,14 +810,17 @@ __device__ __forceinline__ uint32_t sat_add(uint32_t a, uint32_t b) {
 // workgroup's counter atomics were performed before its ticket): folds the counters into the
 // control block and clears them and the tickets for the next slot.  The next work kernel reads
 // both after the kernel boundary.
-__device__ void sssp_decide(SsspCtl* ctl, SsspDevCounters* ctr, uint32_t far_cap, uint32_t near_cap,
-                            unsigned long long* __restrict__ marks) {
-    SsspDevCounters k;
+__device__ void sssp_decide(SsspCtl* ctl, SsspDevCounters* ctr, unsigned long long relaxed, uint32_t far_cap,
+                            uint32_t near_cap, unsigned long long* __restrict__ marks) {
+    struct {
+        uint32_t n_near, n_far, far_out, far_min;
+        unsigned long long relax;
+    } k;
     k.n_near = load_now(&ctr->n_near);
     k.n_far = load_now(&ctr->n_far);
     k.far_out = load_now(&ctr->far_out);
     k.far_min = load_now(&ctr->far_min);
-    k.relax = load_now(&ctr->relax);
+    k.relax = relaxed;
     SsspCtl c = load_now_block(ctl);
     if (k.n_near > near_cap) {
         // entries past the queue were dropped by the writers (near_capacity rules this out):
@@ -620,7 +911,6 @@ __device__ void sssp_decide(SsspCtl* ctl, SsspDevCounters* ctr, uint32_t far_cap
     ctr->n_far = n_far;
     ctr->far_out = 0;
     ctr->far_min = 0xFFFFFFFFu;
-    ctr->relax = 0;
     for (uint32_t i = 0; i < kSsspSlots; ++i) ctr->sub[i].v = 0;
     ctr->top = 0;
 }
@@ -628,21 +918,26 @@ __device__ void sssp_decide(SsspCtl* ctl, SsspDevCounters* ctr, uint32_t far_cap
 // End of a work kernel's workgroup: thread 0 takes the tickets after every counter atomic of
 // the block has returned (the callers wait for their results before the barrier here, and
 // `dep` carries thread 0's last one), so the workgroup that takes the last ticket sees every
-// other workgroup's counts.  Returns true in every thread of that workgroup.
-__device__ __forceinline__ bool sssp_last_block(SsspDevCounters* __restrict__ ctr, unsigned long long dep) {
+// other workgroup's counts.  `relax` (thread 0's) is the block's relaxed edges; the last
+// workgroup's thread 0 gets the launch's sum in its place.  Returns true in every thread of
+// that workgroup.
+__device__ __forceinline__ bool sssp_last_block(SsspDevCounters* __restrict__ ctr, unsigned long long dep,
+                                                unsigned long long& relax) {
     __shared__ uint32_t s_last;
     __syncthreads();
     if (threadIdx.x == 0) {
-        uint32_t inc = 1;
+        unsigned long long inc = (relax << 16) | 1;
         asm volatile("" : "+v"(inc) : "v"(dep));
         const uint32_t sl = blockIdx.x % kSsspSlots;
         const uint32_t members = (gridDim.x - sl + kSsspSlots - 1) / kSsspSlots;  // workgroups of line sl
         const uint32_t nslots = gridDim.x < kSsspSlots ? gridDim.x : kSsspSlots;
         bool last = false;
-        if (atomicAdd(&ctr->sub[sl].v, inc) == members - 1) {
-            uint32_t inc2 = 1;
-            asm volatile("" : "+v"(inc2) : "v"(members));
-            last = atomicAdd(&ctr->top, inc2) == nslots - 1;
+        const unsigned long long line = atomicAdd(&ctr->sub[sl].v, inc) + inc;
+        if ((line & 0xFFFF) == members) {
+            const unsigned long long inc2 = (line & ~0xFFFFull) | 1;
+            const unsigned long long all = atomicAdd(&ctr->top, inc2) + inc2;
+            last = (all & 0xFFFF) == nslots;
+            relax = all >> 16;
         }
         s_last = last ? 1u : 0u;
     }
@@ -682,7 +977,7 @@ __global__ __launch_bounds__(256) void k_sssp_work(SsspCtl* ctl,
     keep_here((uint32_t)c.n);
     if (c.done) return;  // uniform: no workgroup takes a ticket
     const uint32_t epoch = c.epoch, thr = c.thr;
-    unsigned long long ndeg = 0;
+    unsigned long long ndeg = 0, relax = 0;
     unsigned long long dep = 0;  // thread 0's last counter atomic result
     if (c.split_pending) {
         const bool rescan = c.overflow != 0;
@@ -698,9 +993,7 @@ __global__ __launch_bounds__(256) void k_sssp_work(SsspCtl* ctl,
             // the moved vertices this block kept are relaxed at once; their stamps use the next
             // epoch, so a vertex this split kept far still enters the near queue if it is lowered
             // below the threshold
-            const unsigned long long relax =
-                local_rounds<kLoc>(sl, c.local_rounds, col, w, dist, stamp, epoch + 1, thr, st, k, ndeg, fmin);
-            if (threadIdx.x == 0 && relax) dep += atomicAdd(&ctr->relax, relax);
+            relax = local_rounds<kLoc>(sl, c.local_rounds, col, w, dist, stamp, epoch + 1, thr, st, k, ndeg, fmin);
         }
         stage_flush(st, k, true);  // thread 0 stored its atomics' results in LDS
         fmin = wave_min_u32(fmin);
@@ -708,23 +1001,64 @@ __global__ __launch_bounds__(256) void k_sssp_work(SsspCtl* ctl,
             const uint32_t r = atomicMin(&ctr->far_min, fmin);
             asm volatile("" ::"v"(r));  // wait for it before the barrier in sssp_last_block
         }
-        if (sssp_last_block(ctr, dep) && threadIdx.x == 0) sssp_decide(ctl, ctr, far_cap, near_cap, marks);
+        if (sssp_last_block(ctr, dep, relax) && threadIdx.x == 0)
+            sssp_decide(ctl, ctr, relax, far_cap, near_cap, marks);
         return;
     }
-    const uint32_t N = c.n_near;
-    if (N == 0) {  // not reached: a decision leaves either a split pending or entries to relax
-        if (sssp_last_block(ctr, dep) && threadIdx.x == 0) sssp_decide(ctl, ctr, far_cap, near_cap, marks);
-        return;
-    }
+    const uint32_t N = c.n_near;  // a decision leaves either a split pending or entries to relax
     const Sinks k{c.near_sel ? near0 : near1, &ctr->n_near, near_cap, c.far_sel ? far1 : far0, &ctr->n_far,
                   far_cap, row_ptr};
     if (loc && threadIdx.x == 0) loc->n[0] = 0;
     stage_init(st);  // its barrier publishes loc->n[0]
-    const unsigned long long relax = relax_block<kLoc>(c.near_sel ? near1 : near0, N, col, w, dist, stamp, epoch,
-                                                       thr, st, k, ndeg, loc, kLoc ? c.local_rounds : 0u);
+    relax = relax_block<kLoc>(c.near_sel ? near1 : near0, N, col, w, dist, stamp, epoch, thr, st, k, ndeg, loc,
+                              kLoc ? c.local_rounds : 0u);
     stage_flush(st, k, true);  // thread 0 stored its atomics' results in LDS
-    if (threadIdx.x == 0 && relax) dep += atomicAdd(&ctr->relax, relax);
-    if (sssp_last_block(ctr, dep) && threadIdx.x == 0) sssp_decide(ctl, ctr, far_cap, near_cap, marks);
+    if (sssp_last_block(ctr, dep, relax) && threadIdx.x == 0) sssp_decide(ctl, ctr, relax, far_cap, near_cap, marks);
+}
+
+// The same slot with wave rounds.
+__global__ __launch_bounds__(kWaveThreads) void k_sssp_work_wave(
+    SsspCtl* ctl, unsigned long long* __restrict__ near0, unsigned long long* __restrict__ near1, uint32_t near_cap,
+    uint32_t* __restrict__ far0, uint32_t* __restrict__ far1, uint32_t far_cap, const uint32_t* __restrict__ row_ptr,
+    const uint32_t* __restrict__ col, const uint32_t* __restrict__ w, const uint4* __restrict__ rec, uint32_t* dist,
+    uint32_t* __restrict__ stamp, SsspDevCounters* __restrict__ ctr, unsigned long long* __restrict__ marks) {
+    __shared__ WaveLds lds;
+    const SsspCtl c = *ctl;
+    // every field this kernel reads, loaded in one round trip
+    keep_here(c.done);
+    keep_here(c.local_cfg);
+    keep_here(c.split_pending);
+    keep_here(c.n_near);
+    keep_here(c.epoch);
+    keep_here(c.thr);
+    keep_here(c.old_thr);
+    keep_here(c.near_sel);
+    keep_here(c.far_sel);
+    keep_here(c.overflow);
+    keep_here(c.n_far);
+    keep_here((uint32_t)c.n);
+    if (c.done) return;  // uniform: no workgroup takes a ticket
+    unsigned long long relax = 0;
+    unsigned long long dep = 0;  // thread 0's last counter atomic result
+    uint32_t fmin;
+    if (c.split_pending) {
+        // the moved vertices are relaxed at once; what that lowers is stamped with the next epoch, so
+        // a vertex this split kept far still enters the near queue if it falls below the threshold
+        const Sinks k{c.near_sel ? near1 : near0, &ctr->n_near, near_cap, c.far_sel ? far0 : far1,
+                      &ctr->far_out, far_cap, row_ptr};
+        const uint32_t rescan = c.overflow != 0;
+        const WaveIn in{rec, col, w, dist, stamp, c.epoch + 1, c.thr, c.local_cfg, nullptr, c.far_sel ? far1 : far0,
+                        rescan ? (uint32_t)c.n : c.n_far, rescan, c.epoch, c.old_thr};
+        wave_superstep<true>(in, lds, k, relax, fmin);
+        if (threadIdx.x == 0 && fmin != 0xFFFFFFFFu) dep += atomicMin(&ctr->far_min, fmin);
+    } else {
+        const Sinks k{c.near_sel ? near0 : near1, &ctr->n_near, near_cap, c.far_sel ? far1 : far0, &ctr->n_far,
+                      far_cap, row_ptr};
+        const WaveIn in{rec, col, w, dist, stamp, c.epoch, c.thr, c.local_cfg, c.near_sel ? near1 : near0, nullptr,
+                        c.n_near, 0, 0, 0};
+        wave_superstep<false>(in, lds, k, relax, fmin);
+    }
+    if (sssp_last_block(ctr, dep, relax) && threadIdx.x == 0) sssp_decide(ctl, ctr, relax, far_cap, near_cap, marks);
 }
 
 __global__ void k_sssp_seed_ctl(SsspCtl* ctl, SsspDevCounters* c, uint32_t n, unsigned long long m, uint32_t thr,
@@ -748,7 +1082,6 @@ __global__ void k_sssp_seed_ctl(SsspCtl* ctl, SsspDevCounters* c, uint32_t n, un
     c->n_far = 0;
     c->far_out = 0;
     c->far_min = 0xFFFFFFFFu;
-    c->relax = 0;
     for (uint32_t i = 0; i < kSsspSlots; ++i) c->sub[i].v = 0;
     c->top = 0;
 }
@@ -761,6 +1094,26 @@ static uint32_t sssp_local_cfg(const medusa_graph* g, const medusa_opts& o) {
     if (o.local_rounds == 0xFFFFFFFFu) return 0;
     if (o.local_rounds) return o.local_rounds;
     return g->m <= (uint64_t)kLocalMeanDeg * g->n ? kLocalRounds : 0u;
+}
+
+// The vertex records of the wave rounds, built once per handle, when the run uses them: local
+// rounds on a graph without hubs.  Null otherwise, and where there is no memory for them (the
+// block-wide rounds take their place).
+static const uint4* sssp_records(medusa_graph* g, const medusa_opts& o) {
+    if (!sssp_local_cfg(g, o) || g->max_outdeg > kSlice) return nullptr;
+    if (!g->sssp_rec.p) {
+        try {
+            g->sssp_rec.alloc((size_t)g->n * kRecWords);
+        } catch (const Error& e) {
+            if (e.code != MEDUSA_ERR_NOMEM) throw;
+            (void)hipGetLastError();
+            return nullptr;
+        }
+        hipLaunchKernelGGL(k_sssp_records, dim3(grid_for(g->n, 256, 8192)), dim3(256), 0, g->stream, g->n, g->row_ptr.p,
+                           g->col.p, g->w.p, g->sssp_rec.p);
+        MDS_LAUNCHED();
+    }
+    return g->sssp_rec.p;
 }
 
 // Far-queue capacity: m + n entries, or the caller's smaller limit (a full queue is rebuilt
@@ -860,17 +1213,23 @@ static void sssp_run_device(medusa_graph* g, uint32_t src, uint32_t* out, const 
     GraphCache& gc = g->sssp_graph;
     unsigned long long* marks = g->sssp_phases.p;
     const uint32_t local_cfg = sssp_local_cfg(g, o);
-    // the marks buffer is 256-byte aligned, so its low bit can carry the kernel variant
+    const uint4* rec = sssp_records(g, o);
+    // the marks buffer is 256-byte aligned, so its low bits can carry the kernel variant
     const uintptr_t key[6] = {(uintptr_t)g->dist.p, (uintptr_t)g->near_q.p, (uintptr_t)g->q_aux.p,
-                              (uintptr_t)g->w.p, (uintptr_t)marks | (local_cfg ? 1u : 0u), (uintptr_t)ctl};
+                              (uintptr_t)g->w.p, (uintptr_t)marks | (rec ? 2u : local_cfg ? 1u : 0u), (uintptr_t)ctl};
     if (!gc.exec || !std::equal(key, key + 6, gc.key)) {
         gc.reset();
         MDS_HIP(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
         for (uint32_t k = 0; k < kSsspBatch; ++k) {
-            hipLaunchKernelGGL(local_cfg ? k_sssp_work<true> : k_sssp_work<false>,
-                               dim3(local_cfg ? kSsspGridLocal : kSsspGrid), dim3(256), 0, s,
-                               ctl, near0, near1, (uint32_t)near_cap, far0, far1, (uint32_t)far_cap,
-                               g->row_ptr.p, g->col.p, g->w.p, g->dist.p, g->stamp.p, ctr, marks);
+            if (rec)
+                hipLaunchKernelGGL(k_sssp_work_wave, dim3(kSsspGridWave), dim3(kWaveThreads), 0, s, ctl, near0, near1,
+                                   (uint32_t)near_cap, far0, far1, (uint32_t)far_cap, g->row_ptr.p, g->col.p, g->w.p,
+                                   rec, g->dist.p, g->stamp.p, ctr, marks);
+            else
+                hipLaunchKernelGGL(local_cfg ? k_sssp_work<true> : k_sssp_work<false>,
+                                   dim3(local_cfg ? kSsspGridLocal : kSsspGrid), dim3(256), 0, s,
+                                   ctl, near0, near1, (uint32_t)near_cap, far0, far1, (uint32_t)far_cap,
+                                   g->row_ptr.p, g->col.p, g->w.p, g->dist.p, g->stamp.p, ctr, marks);
         }
         hipGraph_t graph = nullptr;
         hipError_t e = hipStreamEndCapture(s, &graph);
@@ -945,6 +1304,7 @@ static void sssp_run_host(medusa_graph* g, uint32_t src, uint32_t* out, const me
     const bool timing = o.timing != 0;
     if (timing) ensure_events(g, 2);
     const uint32_t local_cfg = sssp_local_cfg(g, o);
+    const uint4* rec = sssp_records(g, o);
     Frontier f{};
     f.n = n;
     f.m = m;
@@ -1011,10 +1371,15 @@ static void sssp_run_host(medusa_graph* g, uint32_t src, uint32_t* out, const me
         if (timing) MDS_HIP(hipEventRecord(g->events[0], s));  // brackets the relaxation launch alone
         // 256 entries per workgroup chunk; the far queue keeps growing at far_a[n_far..)
         const uint32_t rounds = n_near <= kLocalQueue ? local_cfg : 0u;
-        hipLaunchKernelGGL(rounds ? k_sssp_relax<true> : k_sssp_relax<false>,
-                           dim3(grid_for(n_near, 1, local_cfg ? kSsspGridLocal : kSsspGrid)),
-                           dim3(256), 0, s, near_cur, n_near, g->row_ptr.p, g->col.p, g->w.p, g->dist.p, g->stamp.p,
-                           epoch, thr, near_nxt, (uint32_t)near_cap, far_a, (uint32_t)far_cap, C, rounds);
+        if (rec)
+            hipLaunchKernelGGL(k_sssp_relax_wave, dim3(kSsspGridWave), dim3(kWaveThreads), 0, s, near_cur, n_near,
+                               g->row_ptr.p, g->col.p, g->w.p, rec, g->dist.p, g->stamp.p, epoch, thr, near_nxt,
+                               (uint32_t)near_cap, far_a, (uint32_t)far_cap, C, local_cfg);
+        else
+            hipLaunchKernelGGL(rounds ? k_sssp_relax<true> : k_sssp_relax<false>,
+                               dim3(grid_for(n_near, 1, local_cfg ? kSsspGridLocal : kSsspGrid)), dim3(256), 0, s,
+                               near_cur, n_near, g->row_ptr.p, g->col.p, g->w.p, g->dist.p, g->stamp.p, epoch, thr,
+                               near_nxt, (uint32_t)near_cap, far_a, (uint32_t)far_cap, C, rounds);
         MDS_LAUNCHED();
         if (timing) MDS_HIP(hipEventRecord(g->events[1], s));
         const SsspCounters c = read_counters<SsspCounters>(g);

@@ -311,6 +311,27 @@ def test_sssp_local_rounds(oracle, case):
             G.sssp(src, local_rounds=65)
 
 
+@pytest.mark.parametrize("deg", [1, 7, 8, 63, 128, 129])
+def test_sssp_wave_rounds(oracle, deg):
+    """Local rounds at the edges of the wave rounds: out-degrees up to a record's 7 edges, beyond it,
+    the largest (128) and one past it (block-wide rounds instead), zero and large weights, a source
+    whose neighbours all have that degree (rings that overflow into the near queue), few and many
+    rounds, and a far queue that overflows; both drivers, distances equal Dijkstra's."""
+    rng = np.random.default_rng(deg)
+    n = 6000
+    src = [np.zeros(deg, np.int64), np.repeat(np.arange(1, 600), deg), rng.integers(600, n, 3 * n)]
+    dst = [np.arange(1, deg + 1), rng.integers(0, n, 599 * deg), rng.integers(0, n, 3 * n)]
+    rp, col, _ = csr_from_edges(n, np.stack([np.concatenate(src), np.concatenate(dst)], 1))
+    w = rng.integers(0, 1001, len(col)).astype(np.uint32)
+    w[rng.integers(0, len(w), 20)] = 0xF0000000  # sums past 32 bits
+    want = oracle.sssp_dijkstra(rp, col, w, 0)
+    with md.Graph(rp, col, w) as G:
+        for rounds in (1, 2, 64):
+            for timing, delta, far in ((0, 0, 0), (1, 300, 0), (0, 50, 40), (0, 0xFFFFFFFF, 0)):
+                d, st = G.sssp(0, local_rounds=rounds, timing=timing, delta=delta, far_limit=far)
+                assert np.array_equal(d, want), (rounds, timing, delta, far)
+
+
 def test_sssp_sparse_power_law_local_rounds(oracle):
     """A sparse skewed graph (Chung-Lu, mean out-degree about 2, so local rounds are on by
     default) whose hubs span many near-queue slices and are never kept locally, and whose
