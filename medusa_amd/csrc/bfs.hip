@@ -46,7 +46,13 @@
 
 namespace medusa {
 
-constexpr uint32_t kLargeDefault = 2048;
+// Out-degree above which a frontier vertex is split over workgroups.  Below it one wave walks the
+// whole list, 256 out-edges at a time, and the superstep waits for the longest: BFS of the
+// 2.4 M-vertex Chung-Lu graph takes 588 us at 2048, 461 at 1024, 424 at 512; of a batch of 64
+// Chung-Lu graphs 144, 136 and 132; RMAT-20 has no such vertex.  The line is at 1024: at 512 the
+// Chung-Lu pushes come out level with its pulls, and the learned direction, which gains 4 % there
+// over the heuristic at 1024, loses 2 % to its own evaluation.
+constexpr uint32_t kLargeDefault = 1024;
 constexpr uint32_t kLargeSplit = 16;  // workgroups per hub in the large-vertex push
 constexpr uint32_t kBfsBatch = 8;     // supersteps per captured graph
 constexpr uint32_t kExpandGrid = 1024;
@@ -147,9 +153,11 @@ __host__ __device__ constexpr uint32_t bfs_span(uint32_t n) {
 
 // A push claims exactly (compare-and-swap, no compaction) when the frontier has at most
 // `exact_edges` out-edges: 1, or 2 when it also has at most 64 vertices (every wave then reads
-// all of them and takes an equal share of their out-edges).  Its winners all go to segment 0 of
-// the next queue, which may then run on over the other segments' space (kBfsSlots * span >= n
-// entries, and no other segment receives any).
+// all of them and takes an equal share of their out-edges).  Workgroup b appends its winners to
+// segment b mod kBfsSlots of the next queue whatever their ids: exact_edges is at most a
+// segment's span, so any segment could hold them all.  (With every winner in segment 0, 4096
+// waves added to one counter: 94 us for a superstep of 44 K vertices and 68 K out-edges of the
+// 2.4 M-vertex Chung-Lu graph, 24 us with the segments.)
 __host__ __device__ inline uint32_t bfs_small(bool pull, unsigned long long n_f, unsigned long long m_f,
                                               unsigned long long exact_edges) {
     return pull || m_f > exact_edges ? 0u : (n_f <= (unsigned long long)kWave ? 2u : 1u);
@@ -298,12 +306,12 @@ __device__ __forceinline__ uint32_t bfs_queue_at(const BfsArgs& a, const uint32_
     return q[(size_t)s * a.span + (i - pre[s])];
 }
 
-// Output of an exact-claim push: its winners go to segment 0 of the next queue (which may run on
-// over the space of the others), the next bitmap and the hub queue.
+// Output of an exact-claim push: its winners go to the workgroup's segment of the next queue, the
+// next bitmap and the hub queue.
 struct BfsExactOut {
     unsigned long long* nxt;
-    uint32_t* q_next;
-    BfsLine* seg_next;
+    uint32_t* q_next;   // the workgroup's segment
+    BfsLine* seg_next;  // its counter
     uint32_t* hub_next;
 };
 
@@ -330,8 +338,8 @@ __device__ __forceinline__ bool bfs_claim(const BfsArgs& a, uint32_t v, int32_t 
 constexpr uint32_t kPushUnroll = 4;  // out-edges per lane per round of the push, loads issued together
 
 // Winners of a round of an exact-claim push (the calling wave is converged; won[j] / v[j] for
-// the round's kPushUnroll edges of this lane): one packed atomic per wave appends them to
-// segment 0 of the next queue and counts them with their out-degrees; each sets its bit in the
+// the round's kPushUnroll edges of this lane): one packed atomic per wave appends them to the
+// workgroup's segment of the next queue and counts them with their out-degrees; each sets its bit in the
 // next bitmap; hubs also go to the next hub queue.
 __device__ __forceinline__ void bfs_record_round(const BfsArgs& a, const BfsExactOut& o, const bool* won,
                                                  const uint32_t* v, unsigned long long& hacc) {
@@ -354,7 +362,7 @@ __device__ __forceinline__ void bfs_record_round(const BfsArgs& a, const BfsExac
     }
     const unsigned long long dtot = wave_sum_u64(dsum);
     uint32_t base = 0;
-    if (lane == 0) base = (uint32_t)atomicAdd(&o.seg_next[0].v, bfs_pack(cnt, (uint32_t)dtot));
+    if (lane == 0) base = (uint32_t)atomicAdd(&o.seg_next->v, bfs_pack(cnt, (uint32_t)dtot));
     base = __shfl(base, 0, kWave);
     unsigned long long hm[kPushUnroll], hany = 0;
     uint32_t hcnt = 0;
@@ -507,81 +515,97 @@ __device__ __forceinline__ void push_hubs(const BfsArgs& a, const uint32_t* __re
 constexpr uint32_t kPullLane = 32;  // in-degree up to which one lane scans a vertex alone
 constexpr uint32_t kPullGroup = 4;  // in-edges a lane probes per round
 
-// Bottom-up over 64 consecutive vertices from `base` (one per lane; the wave is converged): an
-// unvisited vertex (visited bitmap) joins if any in-neighbour is in the frontier bitmap.  A lane scans a vertex
-// of in-degree <= kPullLane alone; above that the whole wave scans it 64 in-edges at a time and
-// stops at the first hit (ballot), so one high in-degree vertex does not hold its wave for
-// hundreds of sequential probes.  Returns the join mask, which is also written as the chunk's
-// word of the next bitmap.  `probes` counts in-edges examined up to and including the first
-// hit in either case.
-__device__ __forceinline__ unsigned long long pull_chunk(const BfsArgs& a, const unsigned long long* __restrict__ cur,
-                                                         unsigned long long* __restrict__ nxt, uint64_t base,
-                                                         int32_t next, unsigned long long& probes) {
+// Bottom-up over this wave's kRoundChunks chunks of 64 consecutive vertices from `base` (one vertex
+// of each chunk per lane; the wave is converged): an unvisited vertex (visited bitmap) joins if any
+// in-neighbour is in the frontier bitmap.  The chunks go through the chain of dependent loads
+// (visited word, in-offsets, sources, bitmap words) together, so a round of the workgroup costs one
+// such chain and not one per chunk (2.4 M-vertex Chung-Lu graph, pulls of 1.2 M to 0.5 M unvisited
+// vertices: 37 .. 31 us -> 34 .. 26).  A lane scans a vertex of in-degree <= kPullLane
+// alone, kPullGroup in-edges of every chunk per round; above that the whole wave scans it 64
+// in-edges at a time and stops at the first hit (ballot), so one high in-degree vertex does not
+// hold its wave for hundreds of sequential probes.  jm[k] receives chunk k's join mask, which is
+// also written as the chunk's word of the next bitmap.  `probes` counts in-edges examined up to and
+// including the first hit in either case.
+__device__ __forceinline__ void pull_chunks(const BfsArgs& a, const unsigned long long* __restrict__ cur,
+                                            unsigned long long* __restrict__ nxt, uint64_t base, int32_t next,
+                                            const unsigned long long (&vis)[kRoundChunks],
+                                            const uint32_t (&b)[kRoundChunks], const uint32_t (&e)[kRoundChunks],
+                                            unsigned long long (&jm)[kRoundChunks], unsigned long long& probes) {
     const uint32_t lane = threadIdx.x & (kWave - 1);
-    const uint32_t n = a.n;
-    if (base >= n) return 0;  // uniform across the wave
-    const uint32_t v = (uint32_t)base + lane;
-    const unsigned long long vis = a.visited[base / kWave];
-    uint32_t b = 0, e = 0;
-    bool todo = false, joined = false;
-    if (v < n && !((vis >> lane) & 1ull)) {
-        b = a.cptr[v];
-        e = a.cptr[v + 1];
-        todo = b < e;
+    const uint64_t word0 = base / kWave;
+    unsigned long long joined[kRoundChunks];
+    unsigned long long big[kRoundChunks];
+    uint32_t sb[kRoundChunks], se[kRoundChunks];
+    bool more = false;
+#pragma unroll
+    for (uint32_t k = 0; k < kRoundChunks; ++k) {
+        big[k] = __ballot(e[k] - b[k] > kPullLane);
+        joined[k] = 0;
+        sb[k] = b[k];
+        se[k] = e[k] - b[k] > kPullLane ? b[k] : e[k];
+        more |= sb[k] < se[k];
     }
-    const bool big = todo && e - b > kPullLane;
-    if (todo && !big) {
-        // kPullGroup in-edges per round: their source and bitmap loads are issued together,
-        // so a round costs two memory round trips instead of two per in-edge
-        for (uint32_t k0 = b; k0 < e; k0 += kPullGroup) {
-            uint32_t u[kPullGroup];
-            unsigned long long word[kPullGroup];
+    while (__ballot(more)) {  // uniform across the wave
+        uint32_t u[kRoundChunks][kPullGroup];
 #pragma unroll
-            for (uint32_t j = 0; j < kPullGroup; ++j) u[j] = k0 + j < e ? a.csrc[k0 + j] : 0u;
+        for (uint32_t k = 0; k < kRoundChunks; ++k)
 #pragma unroll
-            for (uint32_t j = 0; j < kPullGroup; ++j) word[j] = k0 + j < e ? cur[u[j] >> 6] : 0ull;
+            for (uint32_t j = 0; j < kPullGroup; ++j) u[k][j] = sb[k] + j < se[k] ? a.csrc[sb[k] + j] : 0u;
+        unsigned long long word[kRoundChunks][kPullGroup];
+#pragma unroll
+        for (uint32_t k = 0; k < kRoundChunks; ++k)
+#pragma unroll
+            for (uint32_t j = 0; j < kPullGroup; ++j) word[k][j] = sb[k] + j < se[k] ? cur[u[k][j] >> 6] : 0ull;
+        more = false;
+#pragma unroll
+        for (uint32_t k = 0; k < kRoundChunks; ++k) {
             uint32_t hit = kPullGroup;
 #pragma unroll
             for (uint32_t j = kPullGroup; j-- > 0;)
-                if ((word[j] >> (u[j] & 63)) & 1ull) hit = j;
+                if ((word[k][j] >> (u[k][j] & 63)) & 1ull) hit = j;
+            const uint32_t left = min(se[k] - sb[k], kPullGroup);
             if (hit < kPullGroup) {
                 probes += hit + 1;
-                a.level[v] = next;
-                joined = true;
-                break;
+                a.level[base + k * kWave + lane] = next;
+                joined[k] = 1;
+                sb[k] = se[k];
+            } else {
+                probes += left;
+                sb[k] += left;
             }
-            probes += min(e - k0, kPullGroup);
+            more |= sb[k] < se[k];
         }
     }
-    unsigned long long bigjoin = 0;
-    for (unsigned long long bm = __ballot(big); bm; bm &= bm - 1) {
-        const uint32_t owner = __builtin_ctzll(bm);
-        const uint32_t vb = __shfl(b, owner, kWave), ve = __shfl(e, owner, kWave);
-        for (uint32_t k0 = vb; k0 < ve; k0 += kWave) {
-            const uint32_t k = k0 + lane;
-            bool hit = false;
-            if (k < ve) {
-                const uint32_t u = a.csrc[k];
-                hit = (cur[u >> 6] >> (u & 63)) & 1ull;
-            }
-            const unsigned long long hm = __ballot(hit);
-            if (hm) {
-                if (lane == 0) {
-                    probes += __builtin_ctzll(hm) + 1;
-                    a.level[(uint32_t)base + owner] = next;
+#pragma unroll
+    for (uint32_t k = 0; k < kRoundChunks; ++k) {
+        jm[k] = __ballot(joined[k] != 0);
+        for (unsigned long long bm = big[k]; bm; bm &= bm - 1) {
+            const uint32_t owner = __builtin_ctzll(bm);
+            const uint32_t vb = __shfl(b[k], owner, kWave), ve = __shfl(e[k], owner, kWave);
+            for (uint32_t k0 = vb; k0 < ve; k0 += kWave) {
+                const uint32_t i = k0 + lane;
+                bool hit = false;
+                if (i < ve) {
+                    const uint32_t u = a.csrc[i];
+                    hit = (cur[u >> 6] >> (u & 63)) & 1ull;
                 }
-                bigjoin |= 1ull << owner;
-                break;
+                const unsigned long long hm = __ballot(hit);
+                if (hm) {
+                    if (lane == 0) {
+                        probes += __builtin_ctzll(hm) + 1;
+                        a.level[base + k * kWave + owner] = next;
+                    }
+                    jm[k] |= 1ull << owner;
+                    break;
+                }
+                if (lane == 0) probes += min(ve - k0, (uint32_t)kWave);
             }
-            if (lane == 0) probes += min(ve - k0, (uint32_t)kWave);
+        }
+        if (lane == 0 && word0 + k < a.nwords) {
+            nxt[word0 + k] = jm[k];
+            a.visited[word0 + k] = vis[k] | jm[k];  // the wave owns this word in a pull
         }
     }
-    const unsigned long long jm = __ballot(joined) | bigjoin;
-    if (lane == 0) {
-        nxt[base / kWave] = jm;
-        a.visited[base / kWave] = vis | jm;  // the wave owns this word in a pull
-    }
-    return jm;
 }
 
 // Pull superstep: workgroup rounds of kBfsRound consecutive vertices, wave w taking chunks
@@ -591,13 +615,39 @@ __device__ __forceinline__ void pull_all(const BfsArgs& a, const unsigned long l
                                          unsigned long long* __restrict__ nxt, uint32_t* __restrict__ q_next,
                                          BfsLine* __restrict__ seg_next, uint32_t* __restrict__ hub_next, int32_t next,
                                          unsigned long long& hacc, unsigned long long& probes, BfsAppendLds& L) {
-    const uint32_t wv = threadIdx.x / kWave;
-    for (uint64_t blk = (uint64_t)blockIdx.x * kBfsRound; blk < a.n; blk += (uint64_t)gridDim.x * kBfsRound) {
-        unsigned long long jm[kRoundChunks];
-#pragma unroll 1
-        for (uint32_t k = 0; k < kRoundChunks; ++k)
-            jm[k] = pull_chunk(a, cur, nxt, blk + (wv * kRoundChunks + k) * kWave, next, probes);
-        bfs_append_round(a, jm, blk, q_next, seg_next, hub_next, hacc, L);
+    const uint32_t lane = threadIdx.x & (kWave - 1), wv = threadIdx.x / kWave;
+    const uint64_t step = (uint64_t)gridDim.x * kBfsRound;
+    const uint64_t first = (uint64_t)blockIdx.x * kBfsRound + (uint64_t)wv * kRoundChunks * kWave;
+    // the visited words of 64 / kRoundChunks rounds, one per lane, in one load: lane r * kRoundChunks
+    // + k holds round r's chunk k
+    constexpr uint32_t kAhead = kWave / kRoundChunks;
+    uint64_t blk = (uint64_t)blockIdx.x * kBfsRound;
+    for (uint64_t r0 = 0; blk < a.n; r0 += kAhead) {
+        const uint64_t w = (first + (r0 + lane / kRoundChunks) * step) / kWave + lane % kRoundChunks;
+        const unsigned long long mine = w < a.nwords ? a.visited[w] : ~0ull;
+        unsigned long long vis[kRoundChunks];
+        uint32_t b[kRoundChunks], e[kRoundChunks];  // in-edges of the lane's unvisited vertices
+        auto offsets = [&](uint32_t r) {
+            const uint64_t base = first + (r0 + r) * step;
+#pragma unroll
+            for (uint32_t k = 0; k < kRoundChunks; ++k) {
+                vis[k] = bfs_pack(__builtin_amdgcn_readlane((uint32_t)mine, r * kRoundChunks + k),
+                                  __builtin_amdgcn_readlane((uint32_t)(mine >> 32), r * kRoundChunks + k));
+                const uint64_t v = base + k * kWave + lane;
+                b[k] = e[k] = 0;
+                if (v < a.n && !((vis[k] >> lane) & 1ull)) {
+                    b[k] = a.cptr[v];
+                    e[k] = a.cptr[v + 1];
+                }
+            }
+        };
+        offsets(0);
+        for (uint32_t r = 0; r < kAhead && blk < a.n; ++r, blk += step) {
+            unsigned long long jm[kRoundChunks];
+            pull_chunks(a, cur, nxt, first + (r0 + r) * step, next, vis, b, e, jm, probes);
+            if (r + 1 < kAhead) offsets(r + 1);  // in flight while this round's joins are appended
+            bfs_append_round(a, jm, blk, q_next, seg_next, hub_next, hacc, L);
+        }
     }
 }
 
@@ -956,7 +1006,8 @@ __global__ __launch_bounds__(256) void k_bfs_super(BfsArgs a) {
         if (bfs_finish<kDecide>(a.ctr, hacc + (probes << 32))) bfs_decide(a);
         return;
     }
-    const BfsExactOut o{nxt, q_next, seg_next, hub_next};
+    const uint32_t own = blockIdx.x % kBfsSlots;
+    const BfsExactOut o{nxt, q_next + (size_t)own * a.span, seg_next + own, hub_next};
     const uint32_t hub = ctl->hub_wgs, small = ctl->small;
     if (!small && blockIdx.x == 0 && threadIdx.x == 0) a.ctl->pending = 1;  // the only writer of ctl in this launch
     if (small == 2) {

@@ -64,6 +64,27 @@ def test_bfs_hubs_use_large_path(oracle):
                 assert np.array_equal(lv, oracle.bfs_queue(rp, col, s)), (large, s)
 
 
+@pytest.mark.parametrize("n", [1023, 1024, 2049, 40_001])
+def test_bfs_rounds_per_workgroup(oracle, n):
+    """Two workgroups walk the vertex rounds of the pull and the compaction (20 rounds each at the
+    largest size, past the 16 whose visited words load at once), with in-degrees on both sides of
+    the lane limit of 32 and winners of exact claims in both workgroups' segments."""
+    rng = np.random.default_rng(n)
+    src = [rng.integers(0, n, 3 * n)]
+    dst = [rng.integers(0, n, 3 * n)]
+    for d in (31, 32, 33, 200):
+        v = rng.integers(0, n, 8)
+        src.append(rng.integers(0, n, 8 * d))
+        dst.append(np.repeat(v, d))
+    rp, col, _ = csr_from_edges(n, np.stack([np.concatenate(src), np.concatenate(dst)], 1))
+    s = wl.max_outdeg_vertex(rp)
+    want = oracle.bfs_queue(rp, col, s)
+    with md.Graph(rp, col) as G:
+        for d in _dirs():
+            for grid in (2, 0):
+                assert np.array_equal(G.bfs(s, direction=d, grid=grid, large_degree=4)[0], want), (d, grid)
+
+
 def test_bfs_edge_cases(oracle):
     with md.Graph(np.array([0, 0], np.uint32), np.array([], np.uint32)) as G:
         lv, st = G.bfs(0)
