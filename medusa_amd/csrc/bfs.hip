@@ -48,11 +48,12 @@ namespace medusa {
 
 // Out-degree above which a frontier vertex is split over workgroups.  Below it one wave walks the
 // whole list, 256 out-edges at a time, and the superstep waits for the longest: BFS of the
-// 2.4 M-vertex Chung-Lu graph takes 588 us at 2048, 461 at 1024, 424 at 512; of a batch of 64
-// Chung-Lu graphs 144, 136 and 132; RMAT-20 has no such vertex.  The line is at 1024: at 512 the
-// Chung-Lu pushes come out level with its pulls, and the learned direction, which gains 4 % there
-// over the heuristic at 1024, loses 2 % to its own evaluation.
-constexpr uint32_t kLargeDefault = 1024;
+// 2.4 M-vertex Chung-Lu graph takes 588 us at 2048, 514 at 1280, 461 at 1024, 424 at 512; RMAT-20
+// has no such vertex.  Further down the heuristic's pushes on that graph come out level with its
+// pulls, and the learned direction, which gains 5 % over the heuristic at 1280 (490 us), gains
+// 1..4 % at 1024 and loses 2 % to its own evaluation at 512; the autotuner finds the lower
+// thresholds for a caller's graph.
+constexpr uint32_t kLargeDefault = 1280;
 constexpr uint32_t kLargeSplit = 16;  // workgroups per hub in the large-vertex push
 constexpr uint32_t kBfsBatch = 8;     // supersteps per captured graph
 constexpr uint32_t kExpandGrid = 1024;
