@@ -29,17 +29,22 @@
 // In the reference every writer stores the same level, so its claim is a plain store; here the
 // first setter of the bit also writes the level, which gives the same levels.
 //
+//   solo:  while a frontier has few out-edges one workgroup runs superstep after superstep by
+//          itself, with the frontier in LDS, instead of a launch of the whole grid for each.
+//
 // Two drivers run the same kernel:
 //   device-driven (default): the last workgroup of each superstep (by a ticket taken after
 //     its counters) decides the next one (direction, hub queue split, the termination vote)
-//     into a control block in HBM; batches of superstep slots are captured once as hipGraphs
-//     and replayed until the control block says done, so the host waits once per batch, not
-//     per superstep (the first batch has as many slots as the previous run on the handle had
-//     supersteps, then kBfsBatch);
+//     into a control block in HBM.  A run is one hipGraph: the reset, a starting kernel that
+//     reads the run's parameters from pinned host memory, a number of superstep slots (as many as
+//     the previous run on the handle used) and a closing kernel that copies the levels out and
+//     the control block to pinned memory; the host launches it and waits once, and replays
+//     batches of kBfsBatch slots if the control block does not say done;
 //   host-driven (timing or trace requested): the host reads the counters after every
 //     superstep, times it with hipEvents and logs the trace record.
 
 #include <algorithm>
+#include <cstddef>
 
 #include "engine.h"
 #include "sched.h"
@@ -58,7 +63,9 @@ constexpr uint32_t kLargeSplit = 16;  // workgroups per hub in the large-vertex 
 constexpr uint32_t kBfsBatch = 8;     // supersteps per captured graph
 constexpr uint32_t kExpandGrid = 1024;
 
-// Control block of the device-driven loop.
+// Control block of the device-driven loop.  There are two: launch k of a batch reads block k % 2
+// and leaves the next launch's in the other, so a workgroup that starts late never sees what an
+// early one of the same launch has written.
 struct BfsCtl {
     int32_t step;       // superstep being run (= level of the frontier)
     uint32_t pull;      // direction of this superstep
@@ -70,9 +77,23 @@ struct BfsCtl {
     uint32_t pending;   // a push with plain claims has run and its compaction has not
     uint32_t small;     // push with exact (atomic) claims: the frontier's out-edges fit one queue segment
     uint32_t slots;     // kernel launches the loop has used (a push with plain claims takes two)
-    uint32_t pad;
+    uint32_t rot;       // which bitmap holds the frontier; the next one is built in bm[(rot + 1) % 3]
     unsigned long long n, m, n_f, m_f, n_u, m_u, reached, reached_edges, kernel_bytes, alg_bytes;
+    int32_t* out;              // where the closing kernel copies the levels (null: nowhere)
+    unsigned long long t_begin;  // wall clock at the reset
 };
+
+// Pinned host memory of a device-driven run.
+constexpr uint32_t kBfsHostSources = 4096;    // sources the starting kernel takes from here
+constexpr size_t kBfsStageBytes = 1u << 20;   // levels up to which a host output goes through pinned memory
+struct BfsHost {
+    BfsCtl ctl;                // written by the closing kernel
+    unsigned long long t_end;  // wall clock after the last superstep
+    int32_t* out;              // the run's parameters, read by the starting kernel
+    uint32_t count, mode;
+    uint32_t src[kBfsHostSources];
+};
+size_t bfs_host_words() { return (sizeof(BfsHost) + 7) / 8; }
 
 // Workgroups of a push expansion given to the hub queue: in proportion to its share of
 // the frontier's out-edges, at least one for each non-empty queue.
@@ -97,6 +118,10 @@ __global__ void k_bfs_set_ctl(BfsCtl* ctl, int32_t step, uint32_t pull, uint32_t
     ctl->n_large = n_large;
     ctl->hub_wgs = hub_wgs;
     ctl->pending = 0;
+    ctl->rot = (uint32_t)step % 3u;
+    BfsCtl c = *ctl;  // for the compaction, if one follows
+    c.pending = 1;
+    ctl[1] = c;
 }
 
 // Counters of one superstep.  Atomics on one address serialise (about 10 ns each on this
@@ -127,10 +152,11 @@ struct BfsCounters {
 };
 
 // Buffers and shape of a BFS run, passed by value to every superstep kernel.  Superstep t
-// reads the frontier as bitmap bm[t % 3] (pull), queue q[t % 2] (push) and hub queue
-// hub[t % 2], builds the next frontier's in bm[(t + 1) % 3], q[(t + 1) % 2] and
-// hub[(t + 1) % 2], and clears bm[(t + 2) % 3] for superstep t + 1 (an exact-claim push sets
-// bits in its next bitmap).
+// reads the frontier as bitmap bm[rot] (pull), queue q[t % 2] (push) and hub queue
+// hub[t % 2], builds the next frontier's in bm[(rot + 1) % 3], q[(t + 1) % 2] and
+// hub[(t + 1) % 2], and clears bm[(rot + 2) % 3] for superstep t + 1 (an exact-claim push sets
+// bits in its next bitmap).  The control block's rot advances by one with every superstep of the
+// whole grid and with every run of solo supersteps.
 struct BfsArgs {
     const uint32_t *row_ptr, *col, *cptr, *csrc;
     int32_t* level;
@@ -150,6 +176,18 @@ __host__ __device__ constexpr uint32_t bfs_span(uint32_t n) {
     const uint64_t per = ((uint64_t)n + kBfsSlots - 1) / kBfsSlots;
     const uint64_t span = (per + kBfsRound - 1) / kBfsRound * kBfsRound;
     return (uint32_t)(span ? span : kBfsRound);
+}
+
+// Whether a superstep is run by one workgroup (as a push, whatever the direction heuristic or the
+// policy would say of the whole grid) whose LDS holds frontiers of `cap` vertices: the frontier
+// and every vertex it may reach must fit, and its out-edges take at most kSoloRounds rounds of cap
+// (one, unless the whole graph fits, and so its visited bitmap too).  Erdos-Renyi, 4096 vertices and
+// 33 K arcs: 74 us a run with eight rounds, 84 with one (two supersteps of the whole grid then), 130
+// with none and no run in one graph.
+constexpr uint32_t kSoloRounds = 8;
+__host__ __device__ inline bool bfs_solo_fits(uint32_t cap, unsigned long long n, unsigned long long n_f,
+                                              unsigned long long m_f) {
+    return n_f <= cap && (m_f <= cap || (n <= cap && m_f <= (unsigned long long)kSoloRounds * cap));
 }
 
 // A push claims exactly (compare-and-swap, no compaction) when the frontier has at most
@@ -678,14 +716,90 @@ __device__ __forceinline__ void bfs_clear_counters(BfsCounters* __restrict__ ctr
     }
 }
 
-// The next superstep from this one's counters (the deciding workgroup's first wave, after
-// every workgroup of the superstep has added its counters): direction by the heuristic or the
-// learned policy, hub queue split and the termination vote, written into the control block;
-// the counters are cleared for the next superstep.  The updated control block waits in LDS
-// while the policy is evaluated, so it holds no registers there.
-__device__ __forceinline__ void bfs_decide(const BfsArgs& a) {
-    __shared__ BfsCtl s_c;
-    __shared__ float s_params[kMlpWaveLds];
+// LDS frontier capacity of a superstep slot's workgroup 0, and of the starting kernel's workgroup:
+// one round of kPushUnroll out-edges per thread.
+constexpr uint32_t kSoloSlot = 256 * kPushUnroll;
+constexpr uint32_t kSoloStart = 1024 * kPushUnroll;
+
+// Counts of a finished superstep.
+struct BfsCounts {
+    uint32_t n_new, n_hub;
+    unsigned long long deg_sum, deg_large, probes;
+    uint32_t slots;  // launches it took
+};
+
+// The counts of the superstep just finished folded into the control block; true if another follows.
+__device__ __forceinline__ bool bfs_fold(const BfsArgs& a, BfsCtl& c, const BfsCounts& k) {
+    const uint32_t n = a.n, n_new = k.n_new;
+    // bytes of the superstep just finished (every expansion clears one bitmap: 8 per word):
+    // push = queue entry and out-offsets per frontier vertex (12) + target id and visited bit
+    // per out-edge (8); exact claims then add compare-and-swap (4), two bit ORs (16),
+    // out-offsets (8) and queue entry (4) per join, plain claims the store per join (4) and the compaction's level
+    // pass (4n), next and visited bitmaps (16 per word), out-offsets and queue entry per join
+    // (12); pull = visited word per 64 vertices and in-offsets of unvisited vertices (8) +
+    // source id and bitmap word per probed in-edge (8) + next and visited bitmaps (16 per
+    // word) + level, out-offsets and queue entry per join (16)
+    const unsigned long long kb =
+        c.pull    ? 8ull * c.n_u + 8ull * k.probes + 32ull * a.nwords + 16ull * n_new
+        : c.small ? 12ull * c.n_f + 8ull * c.m_f + 8ull * a.nwords + 32ull * n_new
+                  : 12ull * c.n_f + 8ull * c.m_f + 4ull * n + 24ull * a.nwords + 16ull * n_new;
+    c.kernel_bytes += kb;
+    c.alg_bytes += kb;
+    c.slots += k.slots;
+    if (n_new == 0) {
+        c.done = 1;
+        return false;
+    }
+    c.step += 1;
+    c.n_f = n_new;
+    c.m_f = k.deg_sum;
+    c.n_u -= n_new;
+    c.m_u -= k.deg_sum;
+    c.reached += n_new;
+    c.reached_edges += k.deg_sum;
+    c.n_small = n_new - k.n_hub;
+    c.n_large = k.n_hub;
+    c.hub_wgs = bfs_hub_wgs(a.grid, c.n_small, k.n_hub, k.deg_large, k.deg_sum);
+    return true;
+}
+
+// The heuristic's direction of the next superstep (Beamer, Asanovic, Patterson, SC'12) after one in
+// direction `pull`.
+__device__ __forceinline__ bool bfs_heuristic(const BfsCtl& c, bool pull) {
+    return !pull ? (double)c.m_f > (double)c.m_u / Sched::kAlphaBfs : !((double)c.n_f < (double)c.n / Sched::kBeta);
+}
+// Whether the learned policy is asked for it.
+__device__ __forceinline__ bool bfs_asks(const BfsArgs& a, const BfsCtl& c, bool pull) {
+    return c.mode == 3 && a.policy &&
+           bfs_policy_consulted(pull, (double)c.n_f, (double)c.m_f, (double)c.m_u, (double)c.n, Sched::kAlphaBfs,
+                                Sched::kBeta);
+}
+__device__ __forceinline__ void bfs_record(const BfsCtl& c, double (&rec)[MEDUSA_TRACE_FIELDS]) {
+    rec[0] = (double)c.step;
+    rec[1] = (double)c.n_f;
+    rec[2] = (double)c.m_f;
+    rec[3] = (double)c.n_u;
+    rec[4] = (double)c.m_u;
+    rec[5] = (double)c.n;
+    rec[6] = (double)c.m;
+    rec[7] = rec[8] = 0.0;
+}
+__device__ __forceinline__ void bfs_set_direction(const BfsArgs& a, BfsCtl& c, bool pull, bool solo) {
+    c.pull = pull ? 1u : 0u;
+    c.small = solo ? 3u : bfs_small(pull, c.n_f, c.m_f, a.exact_edges);
+    c.supersteps += 1;
+    if (pull)
+        c.pull_steps += 1;
+    else
+        c.push_steps += 1;
+}
+
+// The decision after a superstep of the whole grid (the deciding workgroup, after every workgroup
+// of the superstep has added its counters; its first wave does the work): counters folded in and
+// cleared for the next superstep, direction by the heuristic or the learned policy, hub queue split
+// and the termination vote, written into the control block.  The updated control block waits in
+// LDS while the policy is evaluated, so it holds no registers there.
+__device__ __forceinline__ void bfs_decide(const BfsArgs& a, uint32_t slot, BfsCtl* s_c, float* s_params) {
     if (threadIdx.x >= kWave) return;
     // with a policy, its parameters start for LDS now, behind the counter loads, holding no
     // registers; a decision that does not consult it only waits for them at the end
@@ -693,76 +807,32 @@ __device__ __forceinline__ void bfs_decide(const BfsArgs& a) {
     BfsCounters* ctr = a.ctr;
     const uint32_t lane = threadIdx.x;
     uint32_t par;
-    bool pull, ask = false, plain = false, done;
+    bool pull = false, ask = false, plain = false, solo = false, more;
     double rec[MEDUSA_TRACE_FIELDS] = {};
     {
-        BfsCtl c = load_now_block(a.ctl);
+        BfsCtl c = load_now_block(a.ctl + slot);
         par = (uint32_t)c.step & 1u;
         unsigned long long joined, work;
         bfs_sum_counters(ctr, par ^ 1u, joined, work);
         const uint32_t n_hub = load_now(&ctr->n_hub);
-        const uint32_t n = a.n, n_new = (uint32_t)joined;
-        const unsigned long long deg_sum = joined >> 32, deg_large = (uint32_t)work, probes = work >> 32;
-        // bytes of the superstep just finished (every expansion clears one bitmap: 8 per word):
-        // push = queue entry and out-offsets per frontier vertex (12) + target id and visited bit
-        // per out-edge (8); exact claims then add compare-and-swap (4), two bit ORs (16),
-        // out-offsets (8) and queue entry (4) per join, plain claims the store per join (4) and the compaction's level
-        // pass (4n), next and visited bitmaps (16 per word), out-offsets and queue entry per join
-        // (12); pull = visited word per 64 vertices and in-offsets of unvisited vertices (8) +
-        // source id and bitmap word per probed in-edge (8) + next and visited bitmaps (16 per
-        // word) + level, out-offsets and queue entry per join (16)
-        const unsigned long long kb =
-            c.pull    ? 8ull * c.n_u + 8ull * probes + 32ull * a.nwords + 16ull * n_new
-            : c.small ? 12ull * c.n_f + 8ull * c.m_f + 8ull * a.nwords + 32ull * n_new
-                      : 12ull * c.n_f + 8ull * c.m_f + 4ull * n + 24ull * a.nwords + 16ull * n_new;
-        c.kernel_bytes += kb;
-        c.alg_bytes += kb;
-        c.slots += c.pending ? 2u : 1u;
+        const BfsCounts k{(uint32_t)joined, n_hub, joined >> 32, (uint32_t)work, work >> 32,
+                          c.pending ? 2u : 1u};
+        c.rot = c.rot == 2 ? 0 : c.rot + 1;
         c.pending = 0;
-        if (n_new == 0) {
-            c.done = 1;
-        } else {
-            c.step += 1;
-            c.n_f = n_new;
-            c.m_f = deg_sum;
-            c.n_u -= n_new;
-            c.m_u -= deg_sum;
-            c.reached += n_new;
-            c.reached_edges += deg_sum;
-            c.n_small = n_new - n_hub;
-            c.n_large = n_hub;
-            c.hub_wgs = bfs_hub_wgs(a.grid, c.n_small, n_hub, deg_large, deg_sum);
-        }
-        done = c.done != 0;
-        pull = c.pull != 0;
-        if (!done) {
-            if (c.mode == 1) {
-                pull = false;
-            } else if (c.mode == 2) {
+        more = bfs_fold(a, c, k);
+        if (more) {
+            solo = c.mode != 2 && bfs_solo_fits(kSoloSlot, c.n, c.n_f, c.m_f);
+            if (c.mode == 2) {
                 pull = true;
-            } else if (c.mode == 3 && a.policy &&
-                       bfs_policy_consulted(pull, (double)c.n_f, (double)c.m_f, (double)c.m_u, (double)c.n,
-                                            Sched::kAlphaBfs, Sched::kBeta)) {
-                ask = true;
+            } else if (c.mode != 1 && !solo) {
+                ask = bfs_asks(a, c, c.pull != 0);
                 // the heuristic's choice stands unless the policy predicts a clear gain
-                plain = !pull ? (double)c.m_f > (double)c.m_u / Sched::kAlphaBfs
-                              : !((double)c.n_f < (double)c.n / Sched::kBeta);
-                rec[0] = (double)c.step;
-                rec[1] = (double)c.n_f;
-                rec[2] = (double)c.m_f;
-                rec[3] = (double)c.n_u;
-                rec[4] = (double)c.m_u;
-                rec[5] = (double)c.n;
-                rec[6] = (double)c.m;
-            } else {
-                // direction-optimising heuristic (Beamer, Asanovic, Patterson, SC'12)
-                if (!pull)
-                    pull = (double)c.m_f > (double)c.m_u / Sched::kAlphaBfs;
-                else
-                    pull = !((double)c.n_f < (double)c.n / Sched::kBeta);
+                pull = plain = bfs_heuristic(c, c.pull != 0);
+                if (ask) bfs_record(c, rec);
             }
         }
-        if (lane == 0) s_c = c;
+        if (lane == 0) *s_c = c;
+        wave_lds_fence();
     }
     if (ask) {  // uniform across the wave
         float c_push, c_pull;
@@ -773,65 +843,236 @@ __device__ __forceinline__ void bfs_decide(const BfsArgs& a) {
     }
     bfs_clear_counters(ctr, par);  // this wave read them above
     if (lane == 0) {
-        BfsCtl c = s_c;
-        if (!done) {
-            c.pull = pull ? 1u : 0u;
-            c.small = bfs_small(pull, c.n_f, c.m_f, a.exact_edges);
-            c.supersteps += 1;
-            if (pull)
-                c.pull_steps += 1;
-            else
-                c.push_steps += 1;
-        }
-        *a.ctl = c;
+        BfsCtl c = *s_c;
+        if (more) bfs_set_direction(a, c, pull, solo);
+        a.ctl[slot ^ 1u] = c;
     }
+}
+
+// ---- solo supersteps ------------------------------------------------------------------
+// One workgroup, the others idle or not launched: a thin frontier's superstep costs two dependent
+// global round trips and a few barriers (2 us, and 4 to 5 for each full round of 4096 scattered
+// out-edges, which one CU issues line by line) instead of a launch, 1024 workgroups' tickets and the
+// counters' round trips (8..11 us).  The supersteps of Erdos-Renyi with 65536 vertices: 105 us a run
+// before, 84 now; RMAT-20 183 and 164; the 2.4 M-vertex Chung-Lu graph, whose tail of thin
+// supersteps took a launch each, 500 and 481.
+
+template <uint32_t kThreads>
+struct BfsSoloLds {
+    static constexpr uint32_t kCap = kThreads * kPushUnroll;
+    uint32_t off[kCap], beg[kCap];            // the frontier's out-edge prefix and offsets
+    uint32_t v[kCap], vbeg[kCap], deg[kCap];  // the next frontier as it is claimed
+    unsigned long long vis[kCap / 64];        // the visited bitmap of a graph of at most kCap vertices
+    uint32_t wsum[kThreads / kWave];
+    uint32_t n, n_hub;
+    unsigned long long deg_sum, deg_large;
+};
+
+template <uint32_t kThreads>
+__device__ __forceinline__ void solo_reset(BfsSoloLds<kThreads>& L) {
+    if (threadIdx.x == 0) {
+        L.n = L.n_hub = 0;
+        L.deg_sum = L.deg_large = 0;
+    }
+}
+
+// Claims up to kPushUnroll vertices v[j] (0xFFFFFFFF: none) per thread for `level` and appends the
+// ones this thread won to the next frontier.  No other workgroup touches the bitmap in this launch,
+// so workgroup scope is enough; the targets' row offsets load beside the claims.  kLdsVis: the
+// bitmap is L.vis (a small graph's few lines of global memory would take one atomic at a time:
+// 33 K out-edges of 4096 vertices 80 us instead of 49).
+template <bool kLdsVis, uint32_t kThreads, uint32_t kN>
+__device__ __forceinline__ void solo_claim(const BfsArgs& a, BfsSoloLds<kThreads>& L, const uint32_t (&v)[kN],
+                                           int32_t level) {
+    unsigned long long old[kN];
+    uint32_t b[kN], e[kN];
+#pragma unroll
+    for (uint32_t j = 0; j < kN; ++j) {
+        b[j] = e[j] = 0;
+        old[j] = ~0ull;
+        if (v[j] != 0xFFFFFFFFu) {
+            b[j] = a.row_ptr[v[j]];
+            e[j] = a.row_ptr[v[j] + 1];
+            old[j] = __hip_atomic_fetch_or(kLdsVis ? &L.vis[v[j] >> 6] : &a.visited[v[j] >> 6], 1ull << (v[j] & 63),
+                                           __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        }
+    }
+    // one LDS atomic per wave and counter: hundreds of lanes on one LDS address would serialise
+    unsigned long long wm[kN];
+    uint32_t cnt = 0, dsum = 0, hubs = 0, hsum = 0;  // out-degrees of distinct vertices: below 2^32 in all
+#pragma unroll
+    for (uint32_t j = 0; j < kN; ++j) {
+        const bool won = !((old[j] >> (v[j] & 63)) & 1ull);
+        wm[j] = __ballot(won);
+        cnt += (uint32_t)__popcll(wm[j]);
+        if (won) {
+            const uint32_t d = e[j] - b[j];
+            dsum += d;
+            hubs += d > a.large;
+            hsum += d > a.large ? d : 0u;
+        }
+    }
+    if (!cnt) return;  // uniform across the wave
+    dsum = __builtin_amdgcn_readlane(wave_incl_scan(dsum), kWave - 1);
+    uint32_t i = 0;
+    if (lane_id() == 0) {
+        i = atomicAdd(&L.n, cnt);
+        atomicAdd(&L.deg_sum, (unsigned long long)dsum);
+    }
+    i = __builtin_amdgcn_readfirstlane(i);
+    if (hubs) {
+        atomicAdd(&L.n_hub, hubs);
+        atomicAdd(&L.deg_large, (unsigned long long)hsum);
+    }
+#pragma unroll
+    for (uint32_t j = 0; j < kN; ++j) {
+        if ((wm[j] >> lane_id()) & 1ull) {
+            const uint32_t at = i + lanes_below(wm[j]);
+            a.level[v[j]] = level;
+            L.v[at] = v[j];
+            L.vbeg[at] = b[j];
+            L.deg[at] = e[j] - b[j];
+        }
+        i += (uint32_t)__popcll(wm[j]);
+    }
+}
+
+// Supersteps of the frontier in L (v, vbeg, deg; L.n vertices, complete behind a barrier) and of the
+// ones after it while they fit; c (the same in every thread) follows.  Ends with c.done, or with the
+// first frontier that does not fit in L and no direction chosen for it.  Every thread calls it.
+template <bool kLdsVis, uint32_t kThreads>
+__device__ __forceinline__ void bfs_solo(const BfsArgs& a, BfsSoloLds<kThreads>& L, BfsCtl& c) {
+    constexpr uint32_t kCap = BfsSoloLds<kThreads>::kCap, kPer = kPushUnroll;
+    const uint32_t t = threadIdx.x, lane = t & (kWave - 1), wv = t / kWave;
+    for (;;) {
+        // the frontier's offsets, kPer consecutive entries per thread
+        const uint32_t n = L.n;
+        uint32_t d[kPer], sum = 0;
+#pragma unroll
+        for (uint32_t j = 0; j < kPer; ++j) {
+            const uint32_t i = t * kPer + j;
+            d[j] = i < n ? L.deg[i] : 0u;
+            sum += d[j];
+            if (i < n) L.beg[i] = L.vbeg[i];
+        }
+        const uint32_t incl = wave_incl_scan(sum);
+        if (lane == kWave - 1) L.wsum[wv] = incl;
+        __syncthreads();
+        uint32_t at = incl - sum, total = 0;
+#pragma unroll
+        for (uint32_t w = 0; w < kThreads / kWave; ++w) {
+            if (w < wv) at += L.wsum[w];
+            total += L.wsum[w];
+        }
+#pragma unroll
+        for (uint32_t j = 0; j < kPer; ++j) {
+            L.off[t * kPer + j] = at;  // past n: total
+            at += d[j];
+        }
+        solo_reset(L);
+        __syncthreads();
+        for (uint32_t e0 = 0; e0 < total; e0 += kCap) {  // uniform
+            // kPushUnroll consecutive out-edges per thread: one search for the first one's owner, the
+            // last entry whose offset is at most e (it has out-edges), then steps to the next
+            uint32_t v[kPushUnroll], x[kPushUnroll];
+            const uint32_t first = e0 + t * kPushUnroll;
+            uint32_t lo = 0;
+            if (first < total) {
+#pragma unroll
+                for (uint32_t step = kCap / 2; step; step >>= 1)
+                    if (L.off[lo + step] <= first) lo += step;
+            }
+#pragma unroll
+            for (uint32_t j = 0; j < kPushUnroll; ++j) {
+                x[j] = 0;
+                if (first + j < total) {
+                    while (lo + 1 < n && L.off[lo + 1] <= first + j) ++lo;
+                    x[j] = L.beg[lo] + (first + j - L.off[lo]);
+                }
+            }
+#pragma unroll
+            for (uint32_t j = 0; j < kPushUnroll; ++j) v[j] = first + j < total ? a.col[x[j]] : 0xFFFFFFFFu;
+            solo_claim<kLdsVis>(a, L, v, c.step + 1);
+        }
+        __syncthreads();
+        if (!bfs_fold(a, c, BfsCounts{L.n, L.n_hub, L.deg_sum, L.deg_large, 0, 0})) return;
+        if (!bfs_solo_fits(kCap, c.n, c.n_f, c.m_f)) return;
+        bfs_set_direction(a, c, false, true);
+    }
+}
+
+// The frontier in L handed to the next launch, in bm[c.rot] (all zero), queue step % 2 (segment 0,
+// which may run on over the others' space), its hub queue and its counters; the control block goes
+// to *ctl.  (Counters other than the queues' are zero: nobody adds to them in this launch.)
+template <uint32_t kThreads>
+__device__ __forceinline__ void solo_publish(const BfsArgs& a, BfsSoloLds<kThreads>& L, const BfsCtl& c,
+                                             BfsCtl* ctl) {
+    const uint32_t t = threadIdx.x, par = (uint32_t)c.step & 1u;
+    if (!c.done) {
+        const uint32_t n = L.n;
+        unsigned long long* bm = a.bm[c.rot];
+        if (t < kBfsSlots) {
+            a.ctr->seg[par][t].v = t == 0 ? bfs_pack(n, (uint32_t)L.deg_sum) : 0ull;
+            a.ctr->seg[par ^ 1u][t].v = 0;
+        }
+        __syncthreads();
+        if (t == 0) L.n_hub = 0;
+        __syncthreads();
+        for (uint32_t i = t; i < n; i += kThreads) {
+            const uint32_t v = L.v[i];
+            a.q[par][i] = v;
+            __hip_atomic_fetch_or(&bm[v >> 6], 1ull << (v & 63), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+            if (L.deg[i] > a.large) a.hub[par][atomicAdd(&L.n_hub, 1u)] = v;
+        }
+    }
+    if (t == 0) *ctl = c;
 }
 
 // ---- kernels (both drivers) ---------------------------------------------------------
 
-// First decision (superstep 0) from the first frontier's counts, by the calling workgroup's
-// first wave (the others return; every thread passes the same values): the control block is
-// written and the work slots, tickets and hub count are cleared (queue 0's counters stay:
-// superstep 0 reads them).
-__device__ __forceinline__ void bfs_first_decision(const BfsArgs& a, unsigned long long joined,
-                                                   unsigned long long work, uint32_t n_hub, unsigned long long m,
-                                                   uint32_t mode) {
-    if (threadIdx.x >= kWave) return;
-    BfsCounters* ctr = a.ctr;
+// The control block of superstep 0 from the first frontier's counts, no direction chosen yet.
+__device__ __forceinline__ BfsCtl bfs_first(const BfsArgs& a, const BfsCounts& k, unsigned long long m, uint32_t mode,
+                                            int32_t* out) {
     BfsCtl c{};
     c.mode = mode;
     c.n = a.n;
     c.m = m;
-    c.step = 0;
-    c.n_f = (uint32_t)joined;
-    c.m_f = joined >> 32;
+    c.n_f = k.n_new;
+    c.m_f = k.deg_sum;
     c.n_u = a.n - c.n_f;
     c.m_u = m - c.m_f;
     c.reached = c.n_f;
     c.reached_edges = c.m_f;
-    c.n_small = (uint32_t)c.n_f - n_hub;
-    c.n_large = n_hub;
-    c.hub_wgs = bfs_hub_wgs(a.grid, c.n_small, c.n_large, (uint32_t)work, c.m_f);
-    bool pull = false;
-    if (c.mode == 2) {
-        pull = true;
-    } else if (c.mode == 3 && a.policy &&
-               bfs_policy_consulted(false, (double)c.n_f, (double)c.m_f, (double)c.m_u, (double)c.n,
-                                    Sched::kAlphaBfs, Sched::kBeta)) {
-        const double rec[MEDUSA_TRACE_FIELDS] = {0.0, (double)c.n_f, (double)c.m_f, (double)c.n_u, (double)c.m_u,
-                                                 (double)c.n, (double)c.m, 0.0, 0.0};
-        __shared__ float s_params[kMlpWaveLds];
-        float c_push, c_pull;
-        policy_direction_costs_wave(rec, a.policy, s_params, c_push, c_pull);
-        pull = policy_pull(c_push, c_pull, (double)c.m_f > (double)c.m_u / Sched::kAlphaBfs);
-    } else if (c.mode == 0 || c.mode == 3) {  // heuristic, or the policy far from its switching point
-        pull = (double)c.m_f > (double)c.m_u / Sched::kAlphaBfs;
-    }
-    c.pull = pull ? 1u : 0u;
-    c.small = bfs_small(pull, c.n_f, c.m_f, a.exact_edges);
-    c.supersteps = 1;
-    c.push_steps = pull ? 0 : 1;
-    c.pull_steps = pull ? 1 : 0;
+    c.n_small = k.n_new - k.n_hub;
+    c.n_large = k.n_hub;
+    c.hub_wgs = bfs_hub_wgs(a.grid, c.n_small, c.n_large, k.deg_large, c.m_f);
+    c.out = out;
+    c.t_begin = a.ctl->t_begin;
+    return c;
+}
+// Direction of a superstep after a push (or the first), by one wave.
+__device__ __forceinline__ bool bfs_next_pull(const BfsArgs& a, const BfsCtl& c, float* s_params) {
+    if (c.mode == 1) return false;
+    if (c.mode == 2) return true;
+    const bool plain = bfs_heuristic(c, false);
+    if (!bfs_asks(a, c, false)) return plain;
+    double rec[MEDUSA_TRACE_FIELDS];
+    bfs_record(c, rec);
+    float c_push, c_pull;
+    policy_direction_costs_wave(rec, a.policy, s_params, c_push, c_pull);
+    return policy_pull(c_push, c_pull, plain);
+}
+
+// First decision after k_bfs_mark placed the sources; one workgroup.  The work slots, tickets and
+// hub count are cleared (queue 0's counters stay: superstep 0 reads them).
+__global__ __launch_bounds__(kWave) void k_bfs_first_decide(BfsArgs a, unsigned long long m, uint32_t mode, int32_t* out) {
+    __shared__ float s_params[kMlpWaveLds];
+    BfsCounters* ctr = a.ctr;
+    unsigned long long joined, work;
+    bfs_sum_counters(ctr, 0, joined, work);
+    const uint32_t n_hub = load_now(&ctr->n_hub);
+    BfsCtl c = bfs_first(a, BfsCounts{(uint32_t)joined, n_hub, joined >> 32, (uint32_t)work, 0, 0}, m, mode, out);
+    bfs_set_direction(a, c, bfs_next_pull(a, c, s_params), false);
     if (threadIdx.x < kBfsSlots) {
         ctr->work[threadIdx.x].v = 0;
         ctr->sub[threadIdx.x].v = 0;
@@ -843,22 +1084,84 @@ __device__ __forceinline__ void bfs_first_decision(const BfsArgs& a, unsigned lo
     }
 }
 
-// First decision after k_bfs_mark placed several sources; one workgroup.
-__global__ __launch_bounds__(256) void k_bfs_first_decide(BfsArgs a, unsigned long long m, uint32_t mode) {
-    unsigned long long joined, work;
-    bfs_sum_counters(a.ctr, 0, joined, work);
-    bfs_first_decision(a, joined, work, a.ctr->n_hub, m, mode);
+// Start of a device-driven run, one workgroup, after the reset: the sources (any duplicates counted
+// once) at level 0 and the supersteps from there on that one workgroup runs fastest; then the
+// first decision for the whole grid, and the frontier is handed to the superstep slots.
+__global__ __launch_bounds__(1024) void k_bfs_start(BfsArgs a, const BfsHost* __restrict__ host, unsigned long long m) {
+    __shared__ BfsSoloLds<1024> L;
+    __shared__ float s_params[kMlpWaveLds];
+    __shared__ uint32_t s_pull;
+    static_assert(kBfsHostSources <= BfsSoloLds<1024>::kCap, "the sources fit the LDS frontier");
+    const uint32_t t = threadIdx.x;
+    auto param = [](const auto* p) { return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM); };
+    // one trip over the bus: the first sources with the parameters that say how many there are
+    uint32_t src = param(&host->src[t]);
+    const uint32_t count = param(&host->count), mode = param(&host->mode);
+    int32_t* out = param(&host->out);
+    solo_reset(L);
+    __syncthreads();
+    for (uint32_t i0 = 0; i0 < count; i0 += 1024) {
+        if (i0) src = i0 + t < count ? param(&host->src[i0 + t]) : 0u;
+        const uint32_t v[1] = {i0 + t < count ? src : 0xFFFFFFFFu};
+        solo_claim<false>(a, L, v, 0);
+    }
+    __syncthreads();
+    BfsCtl c = bfs_first(a, BfsCounts{L.n, L.n_hub, L.deg_sum, L.deg_large, 0, 0}, m, mode, out);
+    if (c.mode != 2 && bfs_solo_fits(kSoloStart, c.n, c.n_f, c.m_f)) {
+        bfs_set_direction(a, c, false, true);
+        if (a.n <= BfsSoloLds<1024>::kCap) {
+            if (t < a.nwords) L.vis[t] = a.visited[t];  // behind the barrier above
+            bfs_solo<true>(a, L, c);
+            if (t < a.nwords) a.visited[t] = L.vis[t];
+        } else {
+            bfs_solo<false>(a, L, c);
+        }
+    }
+    if (!c.done) {
+        if (t < kWave) {
+            const bool pull = bfs_next_pull(a, c, s_params);
+            if (t == 0) s_pull = pull ? 1u : 0u;
+        }
+        __syncthreads();
+        bfs_set_direction(a, c, s_pull != 0, false);
+    }
+    solo_publish(a, L, c, a.ctl);  // into bitmap 0, which the reset cleared
 }
 
-// Level reset, counters and bitmap 1 cleared, and the first frontier when there is one source:
-// with `single` < n that vertex is placed at level 0, in bitmap 0 and in queue 0 here, and with
-// kDecide workgroup 0 also makes the first decision (the device-driven loop); otherwise
-// k_bfs_mark places the sources.
-template <bool kDecide>
-__global__ __launch_bounds__(256) void k_bfs_seed(BfsArgs a, uint32_t single, unsigned long long m, uint32_t mode) {
-    __shared__ uint32_t s_deg;
+// End of a batch of slots: the control block to the host, and the levels to their destination when
+// the run is done.
+// `odd`: the batch had an odd number of slots, so it left the control block in the second place;
+// the next batch starts from the first.
+__global__ __launch_bounds__(256) void k_bfs_close(BfsArgs a, BfsHost* __restrict__ host, uint32_t odd) {
+    const BfsCtl* ctl = a.ctl + odd;
+    if (blockIdx.x == 0) {
+        if (odd && threadIdx.x < sizeof(BfsCtl) / 4)
+            reinterpret_cast<uint32_t*>(a.ctl)[threadIdx.x] = reinterpret_cast<const uint32_t*>(ctl)[threadIdx.x];
+        if (threadIdx.x == 0) host->t_end = (unsigned long long)wall_clock64();
+        if (threadIdx.x < sizeof(BfsCtl) / 8)
+            reinterpret_cast<unsigned long long*>(&host->ctl)[threadIdx.x] =
+                reinterpret_cast<const unsigned long long*>(ctl)[threadIdx.x];
+    }
+    int32_t* out = ctl->out;
+    if (!ctl->done || !out) return;
+    const uint64_t tid = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x, stride = (uint64_t)gridDim.x * blockDim.x;
+    uint64_t i = tid;
+    if (reinterpret_cast<uintptr_t>(out) % 16 == 0) {
+        const uint64_t n4 = a.n / 4;
+        for (uint64_t q = tid; q < n4; q += stride)
+            reinterpret_cast<int4*>(out)[q] = reinterpret_cast<const int4*>(a.level)[q];
+        i = 4 * n4 + tid;
+    }
+    for (; i < a.n; i += stride) out[i] = a.level[i];
+}
+
+// Level reset, counters, bitmaps 0 and 1 and the visited bitmap cleared; with `single` < n that
+// vertex is placed at level 0, in bitmap 0 and in queue 0 with its counters (the host-driven loop;
+// otherwise k_bfs_start or k_bfs_mark places the sources).
+__global__ __launch_bounds__(256) void k_bfs_seed(BfsArgs a, uint32_t single) {
     const uint32_t n = a.n;
     const bool one = single < n;
+    if (blockIdx.x == 0 && threadIdx.x == 0) a.ctl->t_begin = (unsigned long long)wall_clock64();
     const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
     for (uint64_t v = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; v < n; v += stride)
         a.level[v] = v == single ? 0 : -1;
@@ -870,26 +1173,15 @@ __global__ __launch_bounds__(256) void k_bfs_seed(BfsArgs a, uint32_t single, un
     bfs_clear_counters(a.ctr, 0);
     bfs_clear_counters(a.ctr, 1);
     __syncthreads();
-    if (threadIdx.x == 0) {
-        const uint32_t deg = one ? a.row_ptr[single + 1] - a.row_ptr[single] : 0u;
-        const bool hub = one && deg > a.large;
-        s_deg = deg;
-        if (one) {
-            const uint32_t sg = single / a.span;
-            a.ctr->seg[0][sg].v = bfs_pack(1u, deg);
-            a.q[0][(size_t)sg * a.span] = single;
+    if (threadIdx.x == 0 && one) {
+        const uint32_t deg = a.row_ptr[single + 1] - a.row_ptr[single], sg = single / a.span;
+        a.ctr->seg[0][sg].v = bfs_pack(1u, deg);
+        a.q[0][(size_t)sg * a.span] = single;
+        if (deg > a.large) {
+            a.hub[0][0] = single;
+            a.ctr->work[0].v = deg;
+            a.ctr->n_hub = 1u;
         }
-        if (hub) a.hub[0][0] = single;
-        if (!kDecide) {  // the host reads the first frontier's counters
-            a.ctr->work[0].v = hub ? deg : 0ull;
-            a.ctr->n_hub = hub ? 1u : 0u;
-        }
-    }
-    if constexpr (kDecide) {
-        __syncthreads();
-        const uint32_t deg = s_deg;
-        const bool hub = deg > a.large;
-        bfs_first_decision(a, bfs_pack(1u, deg), hub ? deg : 0ull, hub ? 1u : 0u, m, mode);
     }
 }
 
@@ -972,22 +1264,37 @@ __device__ __forceinline__ void compact_level(const BfsArgs& a, int32_t next, un
 //   pending: the compaction after a push with plain claims;
 //   pull:    every unvisited vertex; the next frontier's bitmap, queue, hub queue and
 //            counters come out of the same pass;
-//   small:   push with exact claims (the frontier's out-edges fit one queue segment); the
+//   small:   3: workgroup 0 runs this superstep and the ones after it solo; else push with exact
+//            claims (the frontier's out-edges fit one queue segment); the
 //            winners are recorded as they are claimed; with at most 64 frontier vertices every
 //            wave takes an equal share of their out-edges (hubs included);
-//   else:    push with plain claims; it sets `pending`, so the next launch compacts.
+//   else:    push with plain claims; it leaves `pending` set, so the next launch compacts.
 // The first hub_wgs workgroups of a push take the hub queue, the rest the frontier queue.  Every
 // expansion clears the bitmap that superstep + 1 builds.  With kDecide the last workgroup to
 // finish a counting phase decides the next superstep; otherwise the host reads the counters.
 template <bool kDecide>
-__global__ __launch_bounds__(256) void k_bfs_super(BfsArgs a) {
+__global__ __launch_bounds__(256) void k_bfs_super(BfsArgs a, uint32_t slot) {
     __shared__ uint32_t s_beg[4][kWave], s_off[4][kWave];
     __shared__ uint32_t s_pre[kBfsSlots + 1];
     __shared__ BfsAppendLds s_app;
-    const BfsCtl* ctl = a.ctl;
-    if (ctl->done) return;
+    __shared__ BfsCtl s_c;
+    __shared__ float s_params[kDecide ? kMlpWaveLds : 4];
+    const BfsCtl* ctl = a.ctl + slot;
+    // the control block as it is, with `pending` set or not, for the next launch
+    auto pass_on = [&](uint32_t pending) {
+        if (!kDecide || blockIdx.x != 0) return;
+        if (threadIdx.x < sizeof(BfsCtl) / 4) {
+            uint32_t x = reinterpret_cast<const uint32_t*>(ctl)[threadIdx.x];
+            if (threadIdx.x == offsetof(BfsCtl, pending) / 4) x = pending;
+            reinterpret_cast<uint32_t*>(a.ctl + (slot ^ 1u))[threadIdx.x] = x;
+        }
+    };
+    if (ctl->done) {
+        pass_on(0);
+        return;
+    }
     const int32_t step = ctl->step, next = step + 1;
-    const uint32_t par = (uint32_t)step & 1u, t3 = (uint32_t)step % 3u;
+    const uint32_t par = (uint32_t)step & 1u, t3 = ctl->rot;
     unsigned long long* nxt = a.bm[t3 == 2 ? 0 : t3 + 1];
     uint32_t* q_next = a.q[par ^ 1u];
     BfsLine* seg_next = a.ctr->seg[par ^ 1u];
@@ -995,7 +1302,7 @@ __global__ __launch_bounds__(256) void k_bfs_super(BfsArgs a) {
     unsigned long long hacc = 0;
     if (ctl->pending) {
         compact_level(a, next, nxt, q_next, seg_next, hub_next, hacc, s_app);
-        if (bfs_finish<kDecide>(a.ctr, hacc)) bfs_decide(a);
+        if (bfs_finish<kDecide>(a.ctr, hacc)) bfs_decide(a, slot, &s_c, s_params);
         return;
     }
     unsigned long long* clr = a.bm[t3 == 0 ? 2 : t3 - 1];
@@ -1004,13 +1311,36 @@ __global__ __launch_bounds__(256) void k_bfs_super(BfsArgs a) {
     if (ctl->pull) {
         unsigned long long probes = 0;
         pull_all(a, a.bm[t3], nxt, q_next, seg_next, hub_next, next, hacc, probes, s_app);
-        if (bfs_finish<kDecide>(a.ctr, hacc + (probes << 32))) bfs_decide(a);
+        if (bfs_finish<kDecide>(a.ctr, hacc + (probes << 32))) bfs_decide(a, slot, &s_c, s_params);
         return;
     }
     const uint32_t own = blockIdx.x % kBfsSlots;
     const BfsExactOut o{nxt, q_next + (size_t)own * a.span, seg_next + own, hub_next};
     const uint32_t hub = ctl->hub_wgs, small = ctl->small;
-    if (!small && blockIdx.x == 0 && threadIdx.x == 0) a.ctl->pending = 1;  // the only writer of ctl in this launch
+    if constexpr (kDecide) {
+        if (small == 3) {
+            if (blockIdx.x != 0) return;  // (each cleared its share of the bitmap above)
+            __shared__ BfsSoloLds<256> L;
+            bfs_queue_prefix(a.ctr->seg[par], s_pre);
+            const uint32_t qn = s_pre[kBfsSlots];
+            for (uint32_t i = threadIdx.x; i < qn; i += 256) {
+                const uint32_t u = bfs_queue_at(a, a.q[par], s_pre, i);
+                const uint32_t b = a.row_ptr[u];
+                L.vbeg[i] = b;
+                L.deg[i] = a.row_ptr[u + 1] - b;
+            }
+            if (threadIdx.x == 0) L.n = qn;
+            BfsCtl c = *ctl;
+            __syncthreads();
+            bfs_solo<false>(a, L, c);
+            c.slots += 1;
+            c.rot = t3 == 2 ? 0 : t3 + 1;  // cleared by the launch before this one
+            if (!c.done) bfs_set_direction(a, c, c.mode != 1 && bfs_heuristic(c, false), false);
+            solo_publish(a, L, c, a.ctl + (slot ^ 1u));
+            return;
+        }
+    }
+    if (!small) pass_on(1);
     if (small == 2) {
         bfs_queue_prefix(a.ctr->seg[par], s_pre);
         push_tiny(a, a.q[par], s_pre, next, s_beg, s_off, o, hacc);
@@ -1027,7 +1357,7 @@ __global__ __launch_bounds__(256) void k_bfs_super(BfsArgs a) {
         else
             push_queue<false>(a, a.q[par], s_pre, next, w0, nwg * 4, s_beg, s_off, o, hacc);
     }
-    if (small && bfs_finish<kDecide>(a.ctr, hacc)) bfs_decide(a);
+    if (small && bfs_finish<kDecide>(a.ctr, hacc)) bfs_decide(a, slot, &s_c, s_params);
 }
 
 // Degree threshold of the hub queue and workgroups of the expansion: the caller's value,
@@ -1059,11 +1389,11 @@ struct BfsBufs {
     BfsCounters* ctr;
 };
 static size_t bfs_queue_cap(uint32_t n) { return (size_t)kBfsSlots * bfs_span(n); }
-// Control block and counters share one allocation: the control block, then the counters.
-constexpr size_t kBfsCtlUnits = 1 + (sizeof(BfsCounters) + sizeof(CtlStorage) - 1) / sizeof(CtlStorage);
+// Control blocks and counters share one allocation: the control blocks, then the counters.
+constexpr size_t kBfsCtlUnits = 2 + (sizeof(BfsCounters) + sizeof(CtlStorage) - 1) / sizeof(CtlStorage);
 static BfsBufs handle_bufs(medusa_graph* g) {
     g->bfs_ctl.ensure(kBfsCtlUnits);
-    static_assert(sizeof(BfsCtl) <= sizeof(BfsCtlStorage), "control block storage");
+    static_assert(sizeof(BfsCtl) <= sizeof(CtlStorage), "control block storage");
     const size_t nwords = ((size_t)g->n + 63) / 64;
     const size_t qcap = bfs_queue_cap(g->n);
     return {g->level.p,
@@ -1073,7 +1403,7 @@ static BfsBufs handle_bufs(medusa_graph* g) {
             g->bitmap.p + 3 * nwords,
             g->q_aux.p,
             reinterpret_cast<BfsCtl*>(g->bfs_ctl.p),
-            reinterpret_cast<BfsCounters*>(g->bfs_ctl.p + 1)};
+            reinterpret_cast<BfsCounters*>(g->bfs_ctl.p + 2)};
 }
 
 // Frontier out-edges up to which a push claims exactly instead of compacting after it.
@@ -1104,33 +1434,24 @@ static BfsArgs bfs_args(medusa_graph* g, const BfsBufs& B, uint32_t large, uint3
     return a;
 }
 
-// Seeding: every source at level 0 and in bitmap 0 (one source by value, several from
-// B.sources), the first queue, hub queue and counters; with `decide` also the first decision
-// (inside the seed kernel when there is one source).
-static void bfs_seed(medusa_graph* g, const BfsBufs& B, const BfsArgs& a, uint32_t nsrc, uint32_t single, bool decide,
-                     uint32_t mode) {
+// Seeding of the host-driven loop, and of a device-driven run of more sources than the starting
+// kernel takes: every source at level 0 and in bitmap 0 (one source by value, several from
+// B.sources), the first queue, hub queue and counters.
+static void bfs_seed(medusa_graph* g, const BfsBufs& B, const BfsArgs& a, uint32_t nsrc, uint32_t single) {
     hipStream_t s = g->stream;
-    const dim3 grid(grid_for(g->n, 256, 4096));
-    const unsigned long long m = g->m;
-    if (nsrc == 1 && decide)
-        hipLaunchKernelGGL(k_bfs_seed<true>, grid, dim3(256), 0, s, a, single, m, mode);
-    else
-        hipLaunchKernelGGL(k_bfs_seed<false>, grid, dim3(256), 0, s, a, nsrc == 1 ? single : 0xFFFFFFFFu, m, mode);
+    hipLaunchKernelGGL(k_bfs_seed, dim3(grid_for(g->n, 256, 4096)), dim3(256), 0, s, a,
+                       nsrc == 1 ? single : 0xFFFFFFFFu);
     MDS_LAUNCHED();
     if (nsrc > 1) {
         hipLaunchKernelGGL(k_bfs_mark, dim3(grid_for(nsrc, 256, 1024)), dim3(256), 0, s, a, B.sources, nsrc);
         MDS_LAUNCHED();
-        if (decide) {
-            hipLaunchKernelGGL(k_bfs_first_decide, dim3(1), dim3(256), 0, s, a, m, mode);
-            MDS_LAUNCHED();
-        }
     }
 }
 
 // One device-driven slot: one launch of the superstep kernel (a push with plain claims takes two
 // slots, its expansion and its compaction; every other superstep one).
-static void bfs_enqueue_slot(medusa_graph* g, const BfsArgs& a) {
-    hipLaunchKernelGGL(k_bfs_super<true>, dim3(a.grid), dim3(256), 0, g->stream, a);
+static void bfs_enqueue_slot(medusa_graph* g, const BfsArgs& a, uint32_t parity) {
+    hipLaunchKernelGGL(k_bfs_super<true>, dim3(a.grid), dim3(256), 0, g->stream, a, parity);
 }
 
 // Bytes of the seeding: the level reset (4 per vertex), bitmaps 0 and 1 and the visited bitmap
@@ -1139,70 +1460,90 @@ static uint64_t bfs_seed_bytes(uint32_t n, uint32_t nwords, uint32_t nsrc) {
     return 4ull * n + 24ull * nwords + 16ull * nsrc;
 }
 
-// Device-driven run: seed, first decision, then batches of superstep slots until the control
-// block says done.  capture: the batches are captured once as hipGraphs and replayed; without
-// it (medusa_bfs_noalloc, which may not allocate) the same slots are launched one by one.
-static void bfs_run_device(medusa_graph* g, const BfsBufs& B, uint32_t nsrc, uint32_t single, int32_t* out,
+// Device-driven run: reset, start, superstep slots and close, then batches of slots and a close until
+// the control block says done.  capture: each sequence is captured once as a hipGraph and replayed;
+// without it (medusa_bfs_noalloc, which may not allocate) the same kernels are launched one by one.
+static void bfs_run_device(medusa_graph* g, const BfsBufs& B, uint32_t nsrc, const uint32_t* sources, int32_t* out,
                            const medusa_opts& o, medusa_stats& st, bool capture = true) {
     const uint32_t n = g->n;
-    const uint64_t m = g->m;
+    const unsigned long long m = g->m;
     const uint32_t nwords = (n + 63) / 64;
     const uint32_t large = bfs_large(g, o), grid = bfs_grid(g, o);
     hipStream_t s = g->stream;
     const uint32_t mode = bfs_mode(o);
     const float* policy = mode == 3 ? policy_device_params(o.policy) : nullptr;
     const BfsArgs a = bfs_args(g, B, large, grid, policy);
+    BfsHost* host = reinterpret_cast<BfsHost*>(g->h_bfs.p);
 
-    // capture (once per graph, threshold, policy buffer and slot count) a batch of supersteps
-    auto captured = [&](GraphCache& gc, uint32_t slots) -> hipGraphExec_t {
-        const uintptr_t key[4] = {(uintptr_t)B.level ^ ((uintptr_t)B.hub[0] << 16), (uintptr_t)policy,
-                                  ((uintptr_t)grid << 32) | large, (uintptr_t)B.bm[0] ^ ((uintptr_t)slots << 48)};
-        if (gc.exec && std::equal(key, key + 4, gc.key)) return gc.exec;
+    // where the closing kernel puts the levels: the output itself, or pinned memory for a small host
+    // output; larger host outputs are copied afterwards
+    const bool in_place = out == B.level, direct = !in_place && kernels_can_write(g, out);
+    const bool staged = !in_place && !direct && (size_t)n * 4 <= kBfsStageBytes && !is_device_memory(out);
+    if (staged) g->h_levels.ensure(n);
+    int32_t* target = direct ? out : staged ? g->h_levels.p : nullptr;
+
+    const bool by_start = nsrc <= kBfsHostSources;
+    auto launch = [&](bool start, uint32_t slots) {
+        if (start) {
+            hipLaunchKernelGGL(k_bfs_seed, dim3(grid_for(n, 256, 4096)), dim3(256), 0, s, a, 0xFFFFFFFFu);
+            hipLaunchKernelGGL(k_bfs_start, dim3(1), dim3(1024), 0, s, a, (const BfsHost*)host, m);
+        }
+        for (uint32_t k = 0; k < slots; ++k) bfs_enqueue_slot(g, a, k & 1u);
+        hipLaunchKernelGGL(k_bfs_close, dim3(grid_for(n, 1024, 1024)), dim3(256), 0, s, a, host, slots & 1u);
+        MDS_LAUNCHED();
+    };
+    // capture (once per graph, threshold, policy buffer and slot count) a run's kernels
+    auto captured = [&](GraphCache& gc, bool start, uint32_t slots) -> hipGraphExec_t {
+        const uintptr_t key[6] = {(uintptr_t)B.level, (uintptr_t)B.hub[0], (uintptr_t)policy,
+                                  ((uintptr_t)grid << 32) | large, (uintptr_t)B.bm[0], (uintptr_t)B.q[0]};
+        if (gc.exec && std::equal(key, key + 6, gc.key)) return gc.exec;
         gc.reset();
         MDS_HIP(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
-        for (uint32_t k = 0; k < slots; ++k) bfs_enqueue_slot(g, a);
         hipGraph_t graph = nullptr;
-        hipError_t e = hipStreamEndCapture(s, &graph);
+        hipError_t e = hipSuccess;
+        try {
+            launch(start, slots);
+        } catch (...) {
+            (void)hipStreamEndCapture(s, &graph);
+            if (graph) (void)hipGraphDestroy(graph);
+            throw;
+        }
+        e = hipStreamEndCapture(s, &graph);
         if (e == hipSuccess) e = hipGraphInstantiate(&gc.exec, graph, nullptr, nullptr, 0);
         if (graph) (void)hipGraphDestroy(graph);
         MDS_HIP(e);
-        std::copy(key, key + 4, gc.key);
+        std::copy(key, key + 6, gc.key);
         return gc.exec;
     };
-    const uint32_t head = head_slots(g->bfs_last_steps, kBfsBatch);
-    const hipGraphExec_t head_exec = capture ? captured(head == kBfsBatch ? g->bfs_graph : g->bfs_head, head) : nullptr;
+    const uint32_t head = g->bfs_next_head == kNoHead ? kBfsBatch : g->bfs_next_head;
+    hipGraphExec_t exec = nullptr;
+    if (capture) exec = by_start ? captured(g->bfs_heads[head], true, head) : captured(g->bfs_graph, false, kBfsBatch);
 
-    // A device output is copied behind every batch, so the usual run (one batch) waits for the
-    // stream once; a run that takes more batches copies again after the next one.
-    hipPointerAttribute_t attr{};
-    const bool out_dev = out != B.level && hipPointerGetAttributes(&attr, out) == hipSuccess &&
-                         attr.type == hipMemoryTypeDevice;
-    (void)hipGetLastError();  // host pointers unknown to HIP report an error
-
-    MDS_HIP(hipEventRecord(g->ev_begin, s));
-    bfs_seed(g, B, a, nsrc, single, true, mode);
-    BfsCtl h{};
+    host->out = target;
+    host->count = nsrc;
+    host->mode = mode;
+    host->ctl.done = 0;
+    if (by_start) {
+        std::copy(sources, sources + nsrc, host->src);
+    } else {
+        bfs_seed(g, B, a, nsrc, sources[0]);
+        hipLaunchKernelGGL(k_bfs_first_decide, dim3(1), dim3(kWave), 0, s, a, m, mode, target);
+        MDS_LAUNCHED();
+    }
     for (uint32_t batch = 0;; ++batch) {
-        // the tail batch is captured after the timed region has started only on a handle's
-        // first runs; later runs find it cached
         if (capture) {
-            MDS_HIP(hipGraphLaunch(batch == 0 ? head_exec : captured(g->bfs_graph, kBfsBatch), s));
+            if (batch > 0) exec = captured(g->bfs_graph, false, kBfsBatch);
+            MDS_HIP(hipGraphLaunch(exec, s));
         } else {
-            for (uint32_t k = 0; k < kBfsBatch; ++k) bfs_enqueue_slot(g, a);
-            MDS_LAUNCHED();
+            launch(by_start && batch == 0, kBfsBatch);
         }
-        MDS_HIP(hipEventRecord(g->ev_end, s));
-        if (out_dev) MDS_HIP(hipMemcpyAsync(out, B.level, (size_t)n * 4, hipMemcpyDeviceToDevice, s));
-        MDS_HIP(hipMemcpyAsync(g->h_ctr_raw.p, B.ctl, sizeof(BfsCtl), hipMemcpyDeviceToHost, s));
         MDS_HIP(hipStreamSynchronize(s));
-        std::memcpy(&h, g->h_ctr_raw.p, sizeof(BfsCtl));
-        if (h.done) break;
+        if (host->ctl.done) break;
         MDS_CHECK(batch < (2ull * n + 2) / kBfsBatch + 2, MEDUSA_ERR_INTERNAL, "bfs: superstep loop did not end");
     }
-    if (capture) g->bfs_last_steps = h.slots;
-    float ms = 0;
-    MDS_HIP(hipEventElapsedTime(&ms, g->ev_begin, g->ev_end));
-    st.device_ms = ms;
+    const BfsCtl h = host->ctl;
+    if (capture) g->bfs_next_head = std::min(h.slots, kMaxHeadSlots);
+    st.device_ms = (double)(host->t_end - h.t_begin) / (double)g->wall_khz;
     st.supersteps = h.supersteps;
     st.push_steps = h.push_steps;
     st.pull_steps = h.pull_steps;
@@ -1210,7 +1551,8 @@ static void bfs_run_device(medusa_graph* g, const BfsBufs& B, uint32_t nsrc, uin
     st.reached = (uint32_t)h.reached;
     st.kernel_bytes = h.kernel_bytes;
     st.alg_bytes = h.alg_bytes + bfs_seed_bytes(n, nwords, nsrc);
-    if (out != B.level && !out_dev) copy_out(g, out, B.level, (size_t)n * 4);
+    if (staged) std::memcpy(out, g->h_levels.p, (size_t)n * 4);
+    else if (!in_place && !direct) copy_out(g, out, B.level, (size_t)n * 4);
 }
 
 // Sums of the counter slots, read back to the host (waits for the stream).
@@ -1254,7 +1596,7 @@ static void bfs_run_host(medusa_graph* g, uint32_t nsrc, uint32_t single, int32_
     g->trace.clear();
 
     MDS_HIP(hipEventRecord(g->ev_begin, s));
-    bfs_seed(g, B, a, nsrc, single, false, 0);
+    bfs_seed(g, B, a, nsrc, single);
     BfsSums c = read_bfs_counters(g, B.ctr, 0);
 
     Frontier f{};
@@ -1266,13 +1608,16 @@ static void bfs_run_host(medusa_graph* g, uint32_t nsrc, uint32_t single, int32_
     f.m_u = m - f.m_f;
     uint64_t reached_edges = f.m_f, reached = f.n_f, bytes = bfs_seed_bytes(n, nwords, nsrc);
     bool pull = false;
+    uint32_t solo_cap = nsrc <= kBfsHostSources ? kSoloStart : kSoloSlot;
     Sched sched(o, Sched::kBfs);
     if (timing) ensure_events(g, 2);
     for (uint32_t t = 0;; ++t) {
         f.step = t;
+        // the device-driven loop's solo supersteps are pushes, here of the whole grid
+        if (o.direction != MEDUSA_DIR_PULL && !bfs_solo_fits(solo_cap, n, f.n_f, f.m_f)) solo_cap = kSoloSlot;
         if (o.direction == MEDUSA_DIR_PUSH) pull = false;
         else if (o.direction == MEDUSA_DIR_PULL) pull = true;
-        else pull = sched.bfs_pull(f, pull);
+        else pull = bfs_solo_fits(solo_cap, n, f.n_f, f.m_f) ? false : sched.bfs_pull(f, pull);
         const uint32_t n_small = c.n_new - c.n_hub;
         const uint32_t hub = bfs_hub_wgs(grid, n_small, c.n_hub, c.deg_large, c.deg_sum);
         const uint32_t small = bfs_small(pull, f.n_f, f.m_f, a.exact_edges);
@@ -1282,10 +1627,10 @@ static void bfs_run_host(medusa_graph* g, uint32_t nsrc, uint32_t single, int32_
         hipLaunchKernelGGL(k_zero_counters, dim3(1), dim3(kWave), 0, s, a.ctr, (t & 1u) ^ 1u);
         MDS_LAUNCHED();
         if (timing) MDS_HIP(hipEventRecord(g->events[0], s));
-        hipLaunchKernelGGL(k_bfs_super<false>, dim3(grid), dim3(256), 0, s, a);
+        hipLaunchKernelGGL(k_bfs_super<false>, dim3(grid), dim3(256), 0, s, a, 0u);
         MDS_LAUNCHED();
-        if (!pull && !small) {  // the compaction (the push set `pending`)
-            hipLaunchKernelGGL(k_bfs_super<false>, dim3(grid), dim3(256), 0, s, a);
+        if (!pull && !small) {  // the compaction
+            hipLaunchKernelGGL(k_bfs_super<false>, dim3(grid), dim3(256), 0, s, a, 1u);
             MDS_LAUNCHED();
         }
         if (timing) MDS_HIP(hipEventRecord(g->events[1], s));
@@ -1350,11 +1695,11 @@ static void bfs_entry(medusa_graph* g, const uint32_t* sources, uint32_t count, 
     g->q_large.ensure(2 * (size_t)n);
     g->q_aux.ensure(std::max(n, count));
     g->bitmap.ensure(4 * (((size_t)n + 63) / 64));
-    if (count > 1)
+    if (count > (o.timing || o.trace ? 1u : kBfsHostSources))
         MDS_HIP(hipMemcpyAsync(g->q_aux.p, sources, (size_t)count * 4, hipMemcpyHostToDevice, g->stream));
     medusa_stats st{};
     if (o.timing || o.trace) bfs_run_host(g, count, sources[0], levels, o, st);
-    else bfs_run_device(g, handle_bufs(g), count, sources[0], levels, o, st);
+    else bfs_run_device(g, handle_bufs(g), count, sources, levels, o, st);
     if (stats) *stats = st;
 }
 
@@ -1417,12 +1762,11 @@ static void bfs_noalloc(medusa_graph* g, uint32_t source, int32_t* levels, medus
     B.visited = reinterpret_cast<unsigned long long*>(base + 4 * kNoAllocQueueBytes + 3 * kNoAllocBitmapBytes);
     CtlStorage* ctl = reinterpret_cast<CtlStorage*>(base + 4 * kNoAllocQueueBytes + 4 * kNoAllocBitmapBytes);
     B.ctl = reinterpret_cast<BfsCtl*>(ctl);
-    B.ctr = reinterpret_cast<BfsCounters*>(ctl + 1);
+    B.ctr = reinterpret_cast<BfsCounters*>(ctl + 2);
     B.sources = nullptr;  // one source: not used
-    static_assert(sizeof(BfsCtl) <= sizeof(CtlStorage), "control block storage");
     medusa_opts o{};  // heuristic direction, default or tuned launch shape
     medusa_stats st{};
-    bfs_run_device(g, B, 1, source, levels, o, st, /*capture=*/false);
+    bfs_run_device(g, B, 1, &source, levels, o, st, /*capture=*/false);
     if (stats) *stats = st;
 }
 

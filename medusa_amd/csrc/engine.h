@@ -240,6 +240,7 @@ struct GraphCache {
 // the same handle (capped), or the regular batch when there is none.  Slots after the
 // loop's end return at once, so the choice changes only the time, never the result.
 constexpr uint32_t kMaxHeadSlots = 64;
+constexpr uint32_t kNoHead = 0xFFFFFFFFu;  // no previous run
 inline uint32_t head_slots(uint32_t last_steps, uint32_t batch) {
     return last_steps ? (last_steps < kMaxHeadSlots ? last_steps : kMaxHeadSlots) : batch;
 }
@@ -287,9 +288,15 @@ struct medusa_graph {
     medusa::DBuf<medusa::CtlStorage> bfs_ctl, mbfs_ctl, sssp_ctl;
     medusa::GraphCache bfs_graph, mbfs_graph, sssp_graph;
     // first replay of the BFS / MBFS loops: as many slots as the previous run on this handle
-    // took supersteps, so a repeated traversal ends after one replay with no idle slots
-    medusa::GraphCache bfs_head, mbfs_head;
-    uint32_t bfs_last_steps = 0, mbfs_last_steps = 0;
+    // used, so a repeated traversal ends after one replay with no idle slots (BFS: one graph per
+    // slot count, so runs of different lengths do not capture again)
+    medusa::GraphCache bfs_heads[medusa::kMaxHeadSlots + 1], mbfs_head;
+    uint32_t bfs_next_head = medusa::kNoHead, mbfs_last_steps = 0;
+    // pinned: parameters of a BFS run and its control block afterwards; levels on their way to a
+    // small host output
+    medusa::HBuf<unsigned long long> h_bfs;
+    medusa::HBuf<int32_t> h_levels;
+    int wall_khz = 0;  // rate of the device's wall clock
     std::unique_ptr<medusa::PrLayout> pr;
     std::unique_ptr<medusa::PullLayout> pull;  // built on the first MBFS run
     std::vector<medusa::TraceRec> trace;
@@ -329,6 +336,8 @@ uint32_t pr_send_tile_slots(const medusa_graph* g, uint32_t nblk);
 // Binned-combine workgroups that run at once on g's device.
 uint32_t pr_combine_slots(const medusa_graph* g);
 void build_pull_layout(medusa_graph* g);
+// 8-byte words of the pinned memory that BFS runs use (bfs.hip).
+size_t bfs_host_words();
 
 constexpr size_t kCounterWords = 256;  // 2 KiB
 template <class T>

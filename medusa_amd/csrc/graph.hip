@@ -338,8 +338,11 @@ extern "C" int medusa_graph_create(uint32_t n, uint64_t m, const uint32_t* row_p
         MDS_CHECK(row_ptr && (m == 0 || col), MEDUSA_ERR_ARG, "graph_create: null CSR array");
         MDS_CHECK(row_ptr[0] == 0 && row_ptr[n] == m, MEDUSA_ERR_ARG,
                   "graph_create: row_ptr[0] must be 0 and row_ptr[n] must equal m");
-        for (uint32_t v = 0; v < n; ++v)
+        uint32_t max_outdeg = 0;
+        for (uint32_t v = 0; v < n; ++v) {
             MDS_CHECK(row_ptr[v] <= row_ptr[v + 1], MEDUSA_ERR_ARG, "graph_create: row_ptr decreases at %u", v);
+            max_outdeg = std::max(max_outdeg, row_ptr[v + 1] - row_ptr[v]);
+        }
         for (uint64_t e = 0; e < m; ++e)
             MDS_CHECK(col[e] < n, MEDUSA_ERR_ARG, "graph_create: col[%llu]=%u out of range", (unsigned long long)e,
                       col[e]);
@@ -352,7 +355,7 @@ extern "C" int medusa_graph_create(uint32_t n, uint64_t m, const uint32_t* row_p
         g->n = n;
         g->m = m;
         g->weighted = weight != nullptr;
-        for (uint32_t v = 0; v < n; ++v) g->max_outdeg = std::max(g->max_outdeg, row_ptr[v + 1] - row_ptr[v]);
+        g->max_outdeg = max_outdeg;
         MDS_HIP(hipGetDevice(&g->device));
         MDS_HIP(hipStreamCreateWithFlags(&g->stream, hipStreamNonBlocking));
         MDS_HIP(hipEventCreate(&g->ev_begin));
@@ -389,6 +392,9 @@ extern "C" int medusa_graph_create(uint32_t n, uint64_t m, const uint32_t* row_p
         }
         g->ctr_raw.alloc(kCounterWords);
         g->h_ctr_raw.ensure(kCounterWords);
+        g->h_bfs.ensure(bfs_host_words());
+        MDS_HIP(hipDeviceGetAttribute(&g->wall_khz, hipDeviceAttributeWallClockRate, g->device));
+        MDS_CHECK(g->wall_khz > 0, MEDUSA_ERR_HIP, "graph_create: no wall clock rate");
         MDS_HIP(hipStreamSynchronize(s));
         *out = g.release();
     });

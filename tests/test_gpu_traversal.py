@@ -85,6 +85,45 @@ def test_bfs_rounds_per_workgroup(oracle, n):
                 assert np.array_equal(G.bfs(s, direction=d, grid=grid, large_degree=4)[0], want), (d, grid)
 
 
+@pytest.mark.parametrize("n", [4096, 4097, 20000])
+@pytest.mark.parametrize("width,fan", [(1023, 1), (1024, 1), (1025, 1), (4095, 1), (341, 3), (342, 3), (1365, 3),
+                                       (1366, 3), (7, 585), (7, 586), (64, 600)])
+def test_bfs_frontiers_of_one_workgroup(oracle, n, width, fan):
+    """Second frontiers of `width` vertices with `fan` out-edges each, on both sides of the 1024 and
+    4096 out-edges that one workgroup takes, then a chain (thin supersteps to the end); hubs in the
+    frontiers handed over; host outputs, device-driven and host-driven runs, runs of different
+    lengths on one handle, and more sources than the starting kernel takes."""
+    rng = np.random.default_rng(width * fan + n)
+    width = min(width, n - 2)
+    first = np.arange(1, width + 1)
+    chain = np.arange(n - 41, n - 1)
+    edges = np.concatenate([
+        np.stack([np.zeros(width, np.int64), first], 1),
+        np.stack([np.repeat(first, fan), rng.integers(0, n - 40, width * fan)], 1),
+        np.stack([chain, chain + 1], 1),
+    ])
+    rp, col, _ = csr_from_edges(n, edges)
+    sources = rng.integers(0, n, 4000).astype(np.uint32)
+    with md.Graph(rp, col) as G:
+        for s in (0, n - 41, 1, 0):
+            want = oracle.bfs_queue(rp, col, s)
+            for d in _dirs():
+                for large in (0, 100):
+                    lv, st = G.bfs(s, direction=d, large_degree=large)
+                    assert np.array_equal(lv, want), (s, d, large)
+            host = G.bfs(s, timing=True)[1]
+            dev = G.bfs(s)[1]
+            assert (host.supersteps, host.push_steps, host.pull_steps) == (dev.supersteps, dev.push_steps, dev.pull_steps)
+            assert (host.reached, host.edges_traversed) == (dev.reached, dev.edges_traversed)
+        # as many sources as the starting kernel takes, and more (duplicates): one edge short of a
+        # search from a vertex that points at all of them
+        rp2 = np.append(rp, rp[-1] + len(np.unique(sources))).astype(np.uint32)
+        col2 = np.append(col, np.unique(sources)).astype(np.uint32)
+        want = np.maximum(oracle.bfs_queue(rp2, col2, n) - 1, -1)[:n]
+        for k in (4096, 5000):
+            assert np.array_equal(G.bfs_multi(np.resize(sources, k))[0], want), k
+
+
 def test_bfs_edge_cases(oracle):
     with md.Graph(np.array([0, 0], np.uint32), np.array([], np.uint32)) as G:
         lv, st = G.bfs(0)
