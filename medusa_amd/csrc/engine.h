@@ -225,7 +225,7 @@ struct TraceRec {
 // An instantiated hipGraph of captured supersteps and the buffers it was captured with.
 struct GraphCache {
     hipGraphExec_t exec = nullptr;
-    uintptr_t key[6] = {0, 0, 0, 0, 0, 0};
+    uintptr_t key[8] = {};
     GraphCache() = default;
     GraphCache(const GraphCache&) = delete;
     GraphCache& operator=(const GraphCache&) = delete;
@@ -279,6 +279,7 @@ struct medusa_graph {
     medusa::DBuf<unsigned long long> bitmap;
     medusa::DBuf<unsigned long long> near_q;  // SSSP near queues of (slice << 32 | vertex) entries
     medusa::DBuf<unsigned long long> sssp_phases;  // SSSP device-loop phase marks (trace on)
+    medusa::DBuf<uint32_t> mbfs_rows;  // MBFS: level rows on their way to a host output
     medusa::DBuf<uint4> sssp_rec;  // SSSP vertex records (local rounds without hubs), 64 bytes each
     // per-superstep counters (device) and their pinned host mirror; each engine
     // views the 256 bytes as its own counter struct

@@ -14,15 +14,15 @@
 //         in-neighbours, stopping early once every missing bit has been found; vertices are
 //         visited in in-degree order over ELL slabs of source ids (the pull layout), so the
 //         index loads are coalesced;
-//   update: new = next & ~visited; visited |= new; frontier = new; level[s][v] =
-//         step+1 for each new bit s; the two active queues and the counters are rebuilt
-//         with ballot + in-workgroup prefix scan.  Seeding is the same update at level 0
-//         after the sources' bits are placed in next[].
+//   update: new = next & ~visited; visited |= new; frontier = new; the level of the new bits goes
+//         into bit planes (plane p holds bit p of every (vertex, source) level); the two active
+//         queues and the counters are rebuilt with ballot + in-workgroup prefix scan;
+//   finish: once, after the last superstep: the planes as one level byte per (source, vertex).
 //
-// Drivers as for BFS: device-driven (a one-workgroup decide kernel after each update
-// writes the next superstep into a control block; batches of supersteps are captured as
-// hipGraphs and replayed until done, the first batch sized by the previous run on the
-// handle) and host-driven (timing or tracing) over the same kernels.
+// Drivers as for BFS: device-driven (the last workgroup of each update writes the next superstep
+// into a control block; batches of supersteps are captured as hipGraphs and replayed until done,
+// the first batch sized by the previous run on the handle, and each ends with the finish, which
+// returns at once unless the run is done) and host-driven (timing or tracing) over the same kernels.
 
 #include <algorithm>
 #include <cstring>
@@ -37,53 +37,64 @@ constexpr uint32_t kMbfsGridDefault = 2048;
 constexpr uint32_t kMbfsBatch = 8;
 constexpr uint32_t kMbfsSplit = 8;  // minimum workgroup items per hub
 
+constexpr uint32_t kMbfsProbeLines = 8;
+
+// Sums of an update, on lines of their own.
+enum { kMbfsActive, kMbfsActiveDeg, kMbfsNewBits, kMbfsReachedEdges, kMbfsLargeDeg, kMbfsSums };
+struct MbfsLine {
+    alignas(128) unsigned long long v;
+};
 struct MbfsCounters {
-    MDS_COUNTER(uint32_t, n_small);    // active vertices with 1 <= outdeg <= large
-    MDS_COUNTER(uint32_t, n_large);    // active vertices with outdeg > large
-    MDS_COUNTER(uint32_t, n_active);   // all active vertices
-    MDS_COUNTER(uint32_t, saturated);  // a level >= 255 was clamped to 0xFF
-    MDS_COUNTER(unsigned long long, active_deg);
-    MDS_COUNTER(unsigned long long, new_bits);
-    MDS_COUNTER(unsigned long long, reached_edges);  // sum over new (source, vertex) pairs of outdeg(vertex)
-    MDS_COUNTER(unsigned long long, probes);
-    MDS_COUNTER(unsigned long long, deg_large);      // out-degree sum of the hub queue
+    MDS_COUNTER(uint32_t, n_small);   // active vertices with 1 <= outdeg <= large
+    MDS_COUNTER(uint32_t, n_large);   // active vertices with outdeg > large
+    MDS_COUNTER(uint32_t, ticket);    // workgroups of the update that are done
+    MbfsLine sum[kMbfsSums];
+    MbfsLine probes[kMbfsProbeLines];  // in-edges examined, by workgroup number
 };
 
 struct MbfsCtl {
     int32_t step;
     uint32_t pull, done, n_small, n_large, hub_wgs, mode, saturated;
-    uint32_t supersteps, push_steps, pull_steps, n_active;
+    uint32_t supersteps, push_steps, pull_steps, k;
     unsigned long long n, m, n_f, m_f, n_u, m_u, reached, reached_edges, kernel_bytes, alg_bytes, full;
+    uint8_t* out;  // where the finish of a device-driven run writes the levels, or null
 };
 
-__global__ void k_mbfs_zero(MbfsCounters* c) {
-    c->n_small = 0;
-    c->n_large = 0;
-    c->n_active = 0;
-    c->saturated = 0;
-    c->active_deg = 0;
-    c->new_bits = 0;
-    c->reached_edges = 0;
-    c->probes = 0;
-    c->deg_large = 0;
-}
+struct MbfsArgs {
+    const uint32_t *row_ptr, *col, *cptr, *csrc;
+    uint32_t *q_small, *q_large;
+    unsigned long long *visited, *frontier, *next;
+    const PrRun* runs;
+    const uint32_t *wg_run, *perm, *ell;
+    MbfsCounters* ctr;
+    MbfsCtl* ctl;
+    const float* policy;
+    void* planes;  // kMbfsPlanes of n words each, of the width that holds k bits
+    uint32_t n, large, items, grid;
+};
+constexpr uint32_t kMbfsPlanes = 8;
 
-__global__ void k_mbfs_fill(uint32_t n, uint64_t level_words, uint32_t* __restrict__ level32,
-                            unsigned long long* __restrict__ visited, unsigned long long* __restrict__ frontier,
-                            unsigned long long* __restrict__ next) {
+// Masks cleared, counters and control block set up.
+__global__ __launch_bounds__(256) void k_mbfs_fill(MbfsArgs a, unsigned long long m, uint32_t k, uint32_t mode,
+                                                   uint8_t* out) {
     const uint64_t tid = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x, stride = (uint64_t)gridDim.x * blockDim.x;
-    for (uint64_t i = tid; i < level_words; i += stride) level32[i] = 0xFFFFFFFFu;
-    for (uint64_t v = tid; v < n; v += stride) {
-        visited[v] = 0;
-        frontier[v] = 0;
-        next[v] = 0;
+    // visited, frontier and next follow each other
+    for (uint64_t i = tid; i < 3ull * a.n; i += stride) a.visited[i] = 0;
+    if (blockIdx.x != 0) return;
+    for (uint32_t i = threadIdx.x; i < sizeof(MbfsCounters) / 8; i += blockDim.x)
+        reinterpret_cast<unsigned long long*>(a.ctr)[i] = 0;
+    if (threadIdx.x == 0) {
+        MbfsCtl z{};
+        z.mode = mode;
+        z.n = a.n;
+        z.m = m;
+        z.k = k;
+        z.n_u = (unsigned long long)a.n * k;
+        z.m_u = m * k;
+        z.full = k == 64 ? ~0ull : ((1ull << k) - 1);
+        z.out = out;
+        *a.ctl = z;
     }
-}
-
-// Places the k source bits (k <= 64, one thread) into next[]; the level-0 update does the rest.
-__global__ void k_mbfs_seed(const uint32_t* __restrict__ srcs, uint32_t k, unsigned long long* __restrict__ next) {
-    if (blockIdx.x != 0 || threadIdx.x != 0) return;
-    for (uint32_t s = 0; s < k; ++s) next[srcs[s]] |= 1ull << s;
 }
 
 // Workgroups of a push expansion given to the hub queue (as for BFS).
@@ -236,254 +247,350 @@ __device__ __forceinline__ void mbfs_pull_ell(unsigned long long full, const PrR
     __syncthreads();
     if (threadIdx.x == 0) {
         const unsigned long long t = s_probe[0] + s_probe[1] + s_probe[2] + s_probe[3];
-        if (t) atomicAdd(&ctr->probes, t);
+        if (t) atomicAdd(&ctr->probes[blockIdx.x % kMbfsProbeLines].v, t);
     }
 }
 
-__global__ __launch_bounds__(256) void k_mbfs_expand(const MbfsCtl* __restrict__ ctl,
-                                                     const uint32_t* __restrict__ q_small,
-                                                     const uint32_t* __restrict__ q_large,
-                                                     const uint32_t* __restrict__ row_ptr,
-                                                     const uint32_t* __restrict__ col, const uint32_t* __restrict__ cptr,
-                                                     const uint32_t* __restrict__ csrc,
-                                                     const unsigned long long* __restrict__ frontier,
-                                                     const unsigned long long* __restrict__ visited,
-                                                     unsigned long long* __restrict__ next,
-                                                     const PrRun* __restrict__ runs, const uint32_t* __restrict__ wg_run,
-                                                     uint32_t items, const uint32_t* __restrict__ perm,
-                                                     const uint32_t* __restrict__ ell, MbfsCounters* __restrict__ ctr) {
+__global__ __launch_bounds__(256) void k_mbfs_expand(MbfsArgs a) {
+    const MbfsCtl* ctl = a.ctl;
     if (ctl->done) return;
     if (ctl->pull) {
-        mbfs_pull_ell(ctl->full, runs, wg_run, items, perm, ell, cptr, csrc, frontier, visited, next, ctr);
+        mbfs_pull_ell(ctl->full, a.runs, a.wg_run, a.items, a.perm, a.ell, a.cptr, a.csrc, a.frontier, a.visited,
+                      a.next, a.ctr);
         return;
     }
     const uint32_t hub = ctl->hub_wgs;
     if (blockIdx.x < hub) {
-        mbfs_push_large(q_large, ctl->n_large, row_ptr, col, frontier, visited, next, blockIdx.x, hub);
+        mbfs_push_large(a.q_large, ctl->n_large, a.row_ptr, a.col, a.frontier, a.visited, a.next, blockIdx.x, hub);
         return;
     }
     const uint32_t wg = blockIdx.x - hub, nwg = gridDim.x - hub;
-    mbfs_push_small(q_small, ctl->n_small, row_ptr, col, frontier, visited, next, wg * 4 + threadIdx.x / kWave,
-                    nwg * 4);
+    mbfs_push_small(a.q_small, ctl->n_small, a.row_ptr, a.col, a.frontier, a.visited, a.next,
+                    wg * 4 + threadIdx.x / kWave, nwg * 4);
 }
 
-constexpr uint32_t kMbfsTile = 4 * kWave * 4;  // vertices per workgroup tile (4 chunks per wave)
-
-// new = next & ~visited for every vertex: levels, masks, the two active queues, counters.
-__global__ __launch_bounds__(256) void k_mbfs_update(const MbfsCtl* __restrict__ ctl, int32_t level_fixed,
-                                                     uint32_t n, uint32_t large, const uint32_t* __restrict__ row_ptr,
-                                                     unsigned long long* __restrict__ visited,
-                                                     unsigned long long* __restrict__ frontier,
-                                                     unsigned long long* __restrict__ next,
-                                                     uint8_t* __restrict__ level, uint32_t* __restrict__ q_small,
-                                                     uint32_t* __restrict__ q_large, MbfsCounters* __restrict__ ctr) {
-    __shared__ uint32_t s_cnt[4][3];
-    __shared__ unsigned long long s_sum[4][4];
-    __shared__ uint32_t s_base[2];
-    if (ctl && ctl->done) return;
-    const int32_t level_val = ctl ? ctl->step + 1 : level_fixed;
-    const uint32_t lane = threadIdx.x & (kWave - 1), wv = threadIdx.x / kWave;
-    const uint8_t lv = level_val >= 255 ? (uint8_t)0xFF : (uint8_t)level_val;
-    for (uint32_t tile = blockIdx.x; (uint64_t)tile * kMbfsTile < n; tile += gridDim.x) {
-        unsigned long long msm[4], mlg[4];
-        uint32_t csm = 0, clg = 0, cact = 0;
-        unsigned long long adeg = 0, bits = 0, redges = 0, dlg = 0;
-        // loads of the tile first (independent across chunks, so they overlap)
-        unsigned long long raw[4], fr[4], vis[4];
-        uint32_t dg[4];
-#pragma unroll
-        for (uint32_t c = 0; c < 4; ++c) {
-            const uint32_t v = (tile * 16 + c * 4 + wv) * kWave + lane;
-            raw[c] = v < n ? next[v] : 0ull;
-            fr[c] = v < n ? frontier[v] : 0ull;
-        }
-#pragma unroll
-        for (uint32_t c = 0; c < 4; ++c) {
-            const uint32_t v = (tile * 16 + c * 4 + wv) * kWave + lane;
-            vis[c] = raw[c] ? visited[v] : 0ull;
-        }
-#pragma unroll
-        for (uint32_t c = 0; c < 4; ++c) {
-            const uint32_t v = (tile * 16 + c * 4 + wv) * kWave + lane;
-            dg[c] = (raw[c] & ~vis[c]) ? row_ptr[v + 1] - row_ptr[v] : 0u;
-        }
-#pragma unroll
-        for (uint32_t c = 0; c < 4; ++c) {
-            const uint32_t v = (tile * 16 + c * 4 + wv) * kWave + lane;
-            unsigned long long nx = 0;
-            if (v < n) {
-                if (raw[c]) {
-                    next[v] = 0;
-                    nx = raw[c] & ~vis[c];
-                }
-                if (nx) visited[v] = vis[c] | nx;
-                if (fr[c] != nx) frontier[v] = nx;
-            }
-            const unsigned long long amask = __ballot(nx != 0);
-            msm[c] = 0;
-            mlg[c] = 0;
-            if (amask) {
-                const uint32_t deg = nx ? dg[c] : 0u;
-                msm[c] = __ballot(nx != 0 && deg > 0 && deg <= large);
-                mlg[c] = __ballot(nx != 0 && deg > large);
-                adeg += deg;
-                dlg += deg > large ? deg : 0u;
-                bits += __popcll(nx);
-                redges += (unsigned long long)__popcll(nx) * deg;
-                // level bytes: row s gets this wave's 64 consecutive vertices
-                unsigned long long any = nx;
-#pragma unroll
-                for (int off = kWave / 2; off >= 1; off >>= 1) any |= __shfl_xor(any, off, kWave);
-                while (any) {
-                    const uint32_t s = __builtin_ctzll(any);
-                    any &= any - 1;
-                    if ((nx >> s) & 1ull) level[(size_t)s * n + v] = lv;
-                }
-                cact += __popcll(amask);
-                csm += __popcll(msm[c]);
-                clg += __popcll(mlg[c]);
-            }
-        }
-        adeg = wave_sum_u64(adeg);
-        bits = wave_sum_u64(bits);
-        redges = wave_sum_u64(redges);
-        dlg = wave_sum_u64(dlg);
-        if (lane == 0) {
-            s_cnt[wv][0] = csm;
-            s_cnt[wv][1] = clg;
-            s_cnt[wv][2] = cact;
-            s_sum[wv][0] = adeg;
-            s_sum[wv][1] = bits;
-            s_sum[wv][2] = redges;
-            s_sum[wv][3] = dlg;
-        }
-        __syncthreads();
-        if (threadIdx.x == 0) {  // one set of atomics per tile
-            uint32_t tsm = 0, tlg = 0, tact = 0;
-            unsigned long long t[4] = {0, 0, 0, 0};
-            for (int w = 0; w < 4; ++w) {
-                tsm += s_cnt[w][0];
-                tlg += s_cnt[w][1];
-                tact += s_cnt[w][2];
-                for (int j = 0; j < 4; ++j) t[j] += s_sum[w][j];
-            }
-            s_base[0] = tsm ? atomicAdd(&ctr->n_small, tsm) : 0u;
-            s_base[1] = tlg ? atomicAdd(&ctr->n_large, tlg) : 0u;
-            if (tact) {
-                atomicAdd(&ctr->n_active, tact);
-                atomicAdd(&ctr->active_deg, t[0]);
-                atomicAdd(&ctr->new_bits, t[1]);
-                atomicAdd(&ctr->reached_edges, t[2]);
-                if (t[3]) atomicAdd(&ctr->deg_large, t[3]);
-            }
-            if (level_val >= 255 && tact) ctr->saturated = 1;
-        }
-        __syncthreads();
-        uint32_t osm = s_base[0], olg = s_base[1];
-        for (uint32_t w = 0; w < wv; ++w) {
-            osm += s_cnt[w][0];
-            olg += s_cnt[w][1];
-        }
-#pragma unroll
-        for (uint32_t c = 0; c < 4; ++c) {
-            const uint32_t v = (tile * 16 + c * 4 + wv) * kWave + lane;
-            if ((msm[c] >> lane) & 1ull) q_small[osm + lanes_below(msm[c])] = v;
-            if ((mlg[c] >> lane) & 1ull) q_large[olg + lanes_below(mlg[c])] = v;
-            osm += __popcll(msm[c]);
-            olg += __popcll(mlg[c]);
-        }
-        __syncthreads();
-    }
-}
-
-// Direction of the next superstep: fixed, learned (two MLP evaluations by the block), or the
-// direction-optimising heuristic.  All threads of the block call it.
-__device__ bool mbfs_direction(const MbfsCtl& c, bool pull, const float* __restrict__ policy, MlpShared& m,
-                               bool staged) {
+// Direction of the next superstep, by one wave: fixed, learned, or the direction-optimising
+// heuristic.
+__device__ __forceinline__ bool mbfs_direction(const MbfsCtl& c, bool pull, const float* __restrict__ policy,
+                                               float* s_params) {
     if (c.mode == 1) return false;
     if (c.mode == 2) return true;
-    if (c.mode == 3 && policy &&
-        bfs_policy_consulted(pull, (double)c.n_f, (double)c.m_f, (double)c.m_u, (double)c.n, Sched::kAlphaMbfs,
-                             Sched::kBeta)) {
-        const double rec[MEDUSA_TRACE_FIELDS] = {(double)c.step, (double)c.n_f, (double)c.m_f, (double)c.n_u,
-                                                 (double)c.m_u, (double)c.n, (double)c.m, 0.0, 0.0};
-        policy_direction_costs(rec, policy, m, staged);
-        const bool plain = !pull ? (double)c.m_f > (double)c.m_u / Sched::kAlphaMbfs
-                                 : !((double)c.n_f < (double)c.n / Sched::kBeta);
-        return policy_pull(m.out[0], m.out[1], plain);
-    }
-    if (!pull) return (double)c.m_f > (double)c.m_u / Sched::kAlphaMbfs;
-    return !((double)c.n_f < (double)c.n / Sched::kBeta);
+    const bool plain = !pull ? (double)c.m_f > (double)c.m_u / Sched::kAlphaMbfs
+                             : !((double)c.n_f < (double)c.n / Sched::kBeta);
+    if (c.mode != 3 || !policy ||
+        !bfs_policy_consulted(pull, (double)c.n_f, (double)c.m_f, (double)c.m_u, (double)c.n, Sched::kAlphaMbfs,
+                              Sched::kBeta))
+        return plain;
+    const double rec[MEDUSA_TRACE_FIELDS] = {(double)c.step, (double)c.n_f, (double)c.m_f, (double)c.n_u,
+                                             (double)c.m_u, (double)c.n, (double)c.m, 0.0, 0.0};
+    float c_push, c_pull;
+    policy_direction_costs_wave(rec, policy, s_params, c_push, c_pull);
+    return policy_pull(c_push, c_pull, plain);
 }
 
-// One workgroup after an update (or the seeding update when `first`): folds the counters
-// into the control block and decides the next superstep.
-__global__ __launch_bounds__(256) void k_mbfs_decide(MbfsCtl* __restrict__ ctl, MbfsCounters* __restrict__ ctr,
-                                                     const float* __restrict__ policy, uint32_t grid, uint32_t first) {
-    __shared__ MlpShared s_mlp;
-    MbfsCounters k;
-    k.n_small = load_now(&ctr->n_small);
-    k.n_large = load_now(&ctr->n_large);
-    k.n_active = load_now(&ctr->n_active);
-    k.saturated = load_now(&ctr->saturated);
-    k.active_deg = load_now(&ctr->active_deg);
-    k.new_bits = load_now(&ctr->new_bits);
-    k.reached_edges = load_now(&ctr->reached_edges);
-    k.probes = load_now(&ctr->probes);
-    k.deg_large = load_now(&ctr->deg_large);
-    MbfsCtl c = load_now_block(ctl);
-    if (c.done) return;
+// One wave, after every workgroup of an update (or the start, when `first`) has added its counters:
+// folds them into the control block, decides the next superstep and clears them.
+__device__ __forceinline__ void mbfs_decide(const MbfsArgs& a, bool first, float* s_params) {
+    MbfsCounters* ctr = a.ctr;
+    const uint32_t lane = threadIdx.x & (kWave - 1);
+    const uint32_t n_small = load_now(&ctr->n_small), n_large = load_now(&ctr->n_large);
+    unsigned long long sum[kMbfsSums];
+#pragma unroll
+    for (int i = 0; i < kMbfsSums; ++i) sum[i] = load_now(&ctr->sum[i].v);
+    const unsigned long long probe = lane < kMbfsProbeLines ? load_now(&ctr->probes[lane].v) : 0ull;
+    MbfsCtl c = load_now_block(a.ctl);
+    const unsigned long long probes = wave_sum_u64(probe);
     const unsigned long long n = c.n;
     if (!first) {
         // byte model of the superstep just finished: push = queue + offsets + mask per active
         // vertex, col + visited + next probe per edge; pull = offsets + visited per vertex,
         // source + frontier mask per probe; update = 24n
-        const unsigned long long kb = c.pull ? 4ull * (n + 1) + 8ull * n + 12ull * k.probes
+        const unsigned long long kb = c.pull ? 4ull * (n + 1) + 8ull * n + 12ull * probes
                                              : 20ull * c.n_f + 20ull * c.m_f;
         c.kernel_bytes += kb;
-        c.alg_bytes += kb + 24ull * n + k.new_bits;
+        c.alg_bytes += kb + 24ull * n + sum[kMbfsNewBits];
         c.supersteps += 1;
         if (c.pull) c.pull_steps += 1; else c.push_steps += 1;
         c.step += 1;
     }
-    c.saturated |= k.saturated;
-    c.reached += k.new_bits;
-    c.reached_edges += k.reached_edges;
-    c.n_u -= k.new_bits;
-    c.m_u -= k.reached_edges;
-    c.n_f = k.n_active;
-    c.m_f = k.active_deg;
-    c.n_small = k.n_small;
-    c.n_large = k.n_large;
-    c.n_active = k.n_active;
-    c.hub_wgs = mbfs_hub_wgs(grid, k.n_small, k.n_large, k.deg_large, k.active_deg);
-    if (k.n_active == 0) c.done = 1;
-    const bool pull = c.done ? false : mbfs_direction(c, first ? false : c.pull != 0, policy, s_mlp, false);
-    c.pull = pull ? 1u : 0u;
-    __syncthreads();  // every wave has read the control block and counters
-    if (threadIdx.x == 0) {
-        *ctl = c;
-        ctr->n_small = 0;
-        ctr->n_large = 0;
-        ctr->n_active = 0;
-        ctr->saturated = 0;
-        ctr->active_deg = 0;
-        ctr->new_bits = 0;
-        ctr->reached_edges = 0;
-        ctr->probes = 0;
-        ctr->deg_large = 0;
+    const unsigned long long n_active = sum[kMbfsActive];
+    if (c.step >= 255 && n_active) c.saturated = 1;
+    c.reached += sum[kMbfsNewBits];
+    c.reached_edges += sum[kMbfsReachedEdges];
+    c.n_u -= sum[kMbfsNewBits];
+    c.m_u -= sum[kMbfsReachedEdges];
+    c.n_f = n_active;
+    c.m_f = sum[kMbfsActiveDeg];
+    c.n_small = n_small;
+    c.n_large = n_large;
+    c.hub_wgs = mbfs_hub_wgs(a.grid, n_small, n_large, sum[kMbfsLargeDeg], c.m_f);
+    if (n_active == 0) c.done = 1;
+    c.pull = !c.done && mbfs_direction(c, first ? false : c.pull != 0, a.policy, s_params) ? 1u : 0u;
+    if (lane == 0) {
+        *a.ctl = c;
+        ctr->n_small = ctr->n_large = ctr->ticket = 0;
+    }
+    if (lane < kMbfsSums) ctr->sum[lane].v = 0;
+    if (lane < kMbfsProbeLines) ctr->probes[lane].v = 0;
+}
+
+struct MbfsSources {
+    uint32_t v[64];
+};
+
+// The k sources (any of them repeated) at level 0: masks, queues and counters; one workgroup of one
+// wave.  `decide`: and the first decision.
+__global__ __launch_bounds__(kWave) void k_mbfs_start(MbfsArgs a, MbfsSources src, uint32_t k, uint32_t decide) {
+    __shared__ float s_params[kMlpWaveLds];
+    const uint32_t lane = threadIdx.x;
+    const uint32_t v = lane < k ? src.v[lane] : 0xFFFFFFFFu;  // (vertices are below 2^32 - 1)
+    unsigned long long mask = 0;
+    for (uint32_t j = 0; j < k; ++j)
+        if (v == (uint32_t)__builtin_amdgcn_readlane(v, j)) mask |= 1ull << j;
+    const bool one = lane < k && (uint32_t)__builtin_ctzll(mask) == lane;  // the first of its vertex
+    uint32_t deg = 0;
+    if (one) {
+        deg = a.row_ptr[v + 1] - a.row_ptr[v];
+        a.frontier[v] = mask;
+        a.visited[v] = mask;
+    }
+    const bool large = deg > a.large, small = deg > 0 && !large;
+    const unsigned long long sm = __ballot(small), lm = __ballot(large);
+    if (small) a.q_small[lanes_below(sm)] = v;
+    if (large) a.q_large[lanes_below(lm)] = v;
+    const unsigned long long sum[kMbfsSums] = {(unsigned long long)__popcll(__ballot(one)), wave_sum_u64(deg), k,
+                                               wave_sum_u64((unsigned long long)__popcll(mask) * deg),
+                                               wave_sum_u64(large ? deg : 0u)};
+    if (lane == 0) {
+        MbfsCounters* ctr = a.ctr;
+        __hip_atomic_store(&ctr->n_small, (uint32_t)__popcll(sm), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __hip_atomic_store(&ctr->n_large, (uint32_t)__popcll(lm), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+#pragma unroll
+        for (int i = 0; i < kMbfsSums; ++i)
+            __hip_atomic_store(&ctr->sum[i].v, sum[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    if (!decide) return;
+    __threadfence();
+    mbfs_decide(a, true, s_params);
+}
+
+constexpr uint32_t kMbfsWg = 1024, kMbfsTile = 4 * kMbfsWg;  // vertices per workgroup tile (4 chunks per wave)
+
+// new = next & ~visited for every vertex: masks, level planes, the two active queues, counters.
+// kDecide: the last workgroup to add its counters decides the next superstep (one launch less per
+// superstep, 5 us).  Bound by its passes over next and frontier and the joins' plane words, and on
+// few vertices by the chain of atomics on each counter, hence workgroups of 1024 threads: 256 chains
+// of one add for 2^20 vertices.  Levels go into bit planes: as one byte store per joining (source,
+// vertex) with the wave's other lanes masked, this kernel took 36..46 us in the five supersteps of RMAT-20
+// with 64 sources that join most, and 20..24 with planes.
+template <class T, bool kDecide>
+__global__ __launch_bounds__(kMbfsWg) void k_mbfs_update(MbfsArgs a, int32_t level_fixed) {
+    constexpr uint32_t kWaves = kMbfsWg / kWave;
+    __shared__ uint32_t s_sm[kWaves], s_lg[kWaves], s_bsm[kWaves], s_blg[kWaves];
+    __shared__ unsigned long long s_sum[kMbfsSums];
+    __shared__ uint32_t s_last;
+    __shared__ float s_params[kDecide ? kMlpWaveLds : 4];
+    if (kDecide && a.ctl->done) return;
+    const int32_t level = kDecide ? a.ctl->step + 1 : level_fixed;
+    const uint32_t lv = level >= 255 ? 255u : (uint32_t)level;  // 255: saturated, reported as unreached
+    const uint32_t n = a.n, lane = threadIdx.x & (kWave - 1), wv = threadIdx.x / kWave;
+    T* planes = static_cast<T*>(a.planes);
+    if (threadIdx.x < kMbfsSums) s_sum[threadIdx.x] = 0;  // read behind the first tile's barriers
+    uint32_t cact = 0;
+    unsigned long long adeg = 0, bits = 0, redges = 0, dlg = 0;
+    for (uint64_t base = (uint64_t)blockIdx.x * kMbfsTile; base < n; base += (uint64_t)gridDim.x * kMbfsTile) {
+        const uint64_t v0 = base + wv * 4 * kWave + lane;
+        unsigned long long raw[4], fr[4], nx[4], vis[4];
+        uint32_t dg[4];
+#pragma unroll
+        for (uint32_t c = 0; c < 4; ++c) {
+            const uint64_t v = v0 + c * kWave;
+            raw[c] = v < n ? a.next[v] : 0ull;
+            fr[c] = v < n ? a.frontier[v] : 0ull;
+        }
+#pragma unroll
+        for (uint32_t c = 0; c < 4; ++c) vis[c] = raw[c] ? a.visited[v0 + c * kWave] : 0ull;
+#pragma unroll
+        for (uint32_t c = 0; c < 4; ++c) {
+            const uint64_t v = v0 + c * kWave;
+            nx[c] = raw[c] & ~vis[c];
+            dg[c] = nx[c] ? a.row_ptr[v + 1] - a.row_ptr[v] : 0u;
+        }
+#pragma unroll
+        for (uint32_t c = 0; c < 4; ++c) {
+            const uint64_t v = v0 + c * kWave;
+            if (raw[c]) a.next[v] = 0;
+            if (nx[c]) a.visited[v] = vis[c] | nx[c];
+            if (fr[c] != nx[c]) a.frontier[v] = nx[c];
+        }
+        for (uint32_t p = 0; p < kMbfsPlanes; ++p) {  // uniform
+            if (!((lv >> p) & 1u)) continue;
+            T* plane = planes + (size_t)p * n;
+            if (lv == 1u << p) {  // the plane's first use: every word written, none read
+#pragma unroll
+                for (uint32_t c = 0; c < 4; ++c)
+                    if (v0 + c * kWave < n) plane[v0 + c * kWave] = (T)nx[c];
+                continue;
+            }
+            T x[4];
+#pragma unroll
+            for (uint32_t c = 0; c < 4; ++c) x[c] = nx[c] ? plane[v0 + c * kWave] : (T)0;
+#pragma unroll
+            for (uint32_t c = 0; c < 4; ++c)
+                if (nx[c]) plane[v0 + c * kWave] = (T)(x[c] | (T)nx[c]);
+        }
+        unsigned long long msm[4], mlg[4];
+        uint32_t csm = 0, clg = 0;
+#pragma unroll
+        for (uint32_t c = 0; c < 4; ++c) {
+            const uint32_t deg = dg[c];
+            cact += (uint32_t)__popcll(__ballot(nx[c] != 0));
+            msm[c] = __ballot(deg > 0 && deg <= a.large);
+            mlg[c] = __ballot(deg > a.large);
+            csm += (uint32_t)__popcll(msm[c]);
+            clg += (uint32_t)__popcll(mlg[c]);
+            adeg += deg;
+            dlg += deg > a.large ? deg : 0u;
+            bits += __popcll(nx[c]);
+            redges += (unsigned long long)__popcll(nx[c]) * deg;
+        }
+        if (lane == 0) {
+            s_sm[wv] = csm;
+            s_lg[wv] = clg;
+        }
+        __syncthreads();
+        if (wv == 0) {
+            const uint32_t sm = lane < kWaves ? s_sm[lane] : 0u, lg = lane < kWaves ? s_lg[lane] : 0u;
+            const uint32_t ism = wave_incl_scan(sm), ilg = wave_incl_scan(lg);
+            uint32_t got = 0;
+            if (lane == kWave - 2 && ism) got = atomicAdd(&a.ctr->n_small, ism);
+            if (lane == kWave - 1 && ilg) got = atomicAdd(&a.ctr->n_large, ilg);
+            const uint32_t bsm = __builtin_amdgcn_readlane(got, kWave - 2), blg = __builtin_amdgcn_readlane(got, kWave - 1);
+            if (lane < kWaves) {
+                s_bsm[lane] = bsm + ism - sm;
+                s_blg[lane] = blg + ilg - lg;
+            }
+        }
+        __syncthreads();
+        uint32_t osm = s_bsm[wv], olg = s_blg[wv];
+#pragma unroll
+        for (uint32_t c = 0; c < 4; ++c) {
+            const uint32_t v = (uint32_t)(v0 + c * kWave);
+            if ((msm[c] >> lane) & 1ull) a.q_small[osm + lanes_below(msm[c])] = v;
+            if ((mlg[c] >> lane) & 1ull) a.q_large[olg + lanes_below(mlg[c])] = v;
+            osm += (uint32_t)__popcll(msm[c]);
+            olg += (uint32_t)__popcll(mlg[c]);
+        }
+    }
+    if (cact) {  // uniform across the wave
+        adeg = wave_sum_u64(adeg);
+        bits = wave_sum_u64(bits);
+        redges = wave_sum_u64(redges);
+        dlg = wave_sum_u64(dlg);
+        if (lane == 0) {
+            atomicAdd(&s_sum[kMbfsActive], (unsigned long long)cact);
+            atomicAdd(&s_sum[kMbfsActiveDeg], adeg);
+            atomicAdd(&s_sum[kMbfsNewBits], bits);
+            atomicAdd(&s_sum[kMbfsReachedEdges], redges);
+            atomicAdd(&s_sum[kMbfsLargeDeg], dlg);
+        }
+    }
+    __syncthreads();
+    if (wv != 0) return;
+    const unsigned long long sum = lane < kMbfsSums ? s_sum[lane] : 0ull;
+    if (sum) atomicAdd(&a.ctr->sum[lane].v, sum);
+    if constexpr (kDecide) {
+        // the wave's atomics have been performed before its ticket is taken
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        uint32_t t = 0;
+        if (lane == 0) t = atomicAdd(&a.ctr->ticket, 1u);
+        if ((uint32_t)__builtin_amdgcn_readfirstlane(t) == gridDim.x - 1) mbfs_decide(a, false, s_params);
     }
 }
 
-__global__ void k_mbfs_init_ctl(MbfsCtl* ctl, uint32_t n, unsigned long long m, uint32_t k, uint32_t mode) {
-    MbfsCtl z{};
-    z.mode = mode;
-    z.n = n;
-    z.m = m;
-    z.n_u = (unsigned long long)n * k;
-    z.m_u = m * k;
-    z.full = k == 64 ? ~0ull : ((1ull << k) - 1);
-    *ctl = z;
+// Bit j, j + 4, .. j + 28 of four planes' words as the nibbles of a word.
+__device__ __forceinline__ uint32_t mbfs_nibbles(uint32_t x0, uint32_t x1, uint32_t x2, uint32_t x3, uint32_t j) {
+    constexpr uint32_t kLow = 0x11111111u;
+    return ((x0 >> j) & kLow) | (((x1 >> j) & kLow) << 1) | (((x2 >> j) & kLow) << 2) | (((x3 >> j) & kLow) << 3);
+}
+
+// The planes as level bytes, one row of n per source, 0xFF where the source does not reach the
+// vertex: rows [row0, row1) at `out` (by the control block of a finished run: every row, at ctl->out).
+// A lane takes 4 vertices: the planes' words become nibbles, then bytes, 32 sources at a time, and 4
+// words of 4 sources each are transposed into 4 stores of 4 vertices each.  Bound by the stores: a
+// wave writes 256 contiguous bytes of a row at a time.  RMAT-20, 64 sources:
+// 25 us for 64 MiB of levels from 40 of planes and masks.
+template <class T>
+__global__ __launch_bounds__(256) void k_mbfs_finish(MbfsArgs a, MbfsCtl* __restrict__ host, uint8_t* out, uint32_t row0,
+                                                     uint32_t row1) {
+    const MbfsCtl* ctl = a.ctl;
+    if (host) {
+        if (blockIdx.x == 0 && threadIdx.x < sizeof(MbfsCtl) / 8)
+            reinterpret_cast<unsigned long long*>(host)[threadIdx.x] =
+                reinterpret_cast<const unsigned long long*>(ctl)[threadIdx.x];
+        if (!ctl->done || !ctl->out) return;
+        out = ctl->out;
+        row0 = 0;
+        row1 = ctl->k;
+    }
+    const uint32_t n = a.n;
+    const uint32_t last = ctl->step < 255 ? (uint32_t)ctl->step : 255u;  // the planes up to its bits were written
+    const uint32_t np = 32 - __builtin_clz(last | 1u);
+    const T* planes = static_cast<const T*>(a.planes);
+    const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
+    for (uint64_t q = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; q * 4 < n; q += stride) {
+        const uint64_t v0 = q * 4;
+        const uint32_t cnt = n - v0 < 4 ? (uint32_t)(n - v0) : 4u;
+        T x[kMbfsPlanes][4];
+        unsigned long long vis[4];
+#pragma unroll
+        for (uint32_t i = 0; i < 4; ++i) {
+            vis[i] = i < cnt ? a.visited[v0 + i] : 0ull;
+#pragma unroll
+            for (uint32_t p = 0; p < kMbfsPlanes; ++p)
+                x[p][i] = p < np && i < cnt ? planes[(size_t)p * n + v0 + i] : (T)0;
+        }
+#pragma unroll
+        for (uint32_t h = 0; h < (sizeof(T) == 8 ? 2u : 1u); ++h) {
+            auto word = [h](unsigned long long w) { return (uint32_t)(w >> (32 * h)); };
+#pragma unroll
+            for (uint32_t j = 0; j < 4; ++j) {
+                uint32_t lo[4], hi[4];  // nibbles of sources 32h + j + 4i
+#pragma unroll
+                for (uint32_t i = 0; i < 4; ++i) {
+                    const uint32_t u = ~word(vis[i]);
+                    lo[i] = mbfs_nibbles(word(x[0][i]) | u, word(x[1][i]) | u, word(x[2][i]) | u, word(x[3][i]) | u, j);
+                    hi[i] = np > 4 ? mbfs_nibbles(word(x[4][i]) | u, word(x[5][i]) | u, word(x[6][i]) | u,
+                                                  word(x[7][i]) | u, j)
+                                   : ((u >> j) & 0x11111111u) * 15u;
+                }
+#pragma unroll
+                for (uint32_t odd = 0; odd < 2; ++odd) {
+                    uint32_t b[4];  // bytes of sources s0, s0 + 8, s0 + 16, s0 + 24, vertex i
+#pragma unroll
+                    for (uint32_t i = 0; i < 4; ++i) {
+                        constexpr uint32_t kNib = 0x0F0F0F0Fu;
+                        b[i] = odd ? ((lo[i] >> 4) & kNib) | (hi[i] & ~kNib) : (lo[i] & kNib) | ((hi[i] & kNib) << 4);
+                    }
+                    const uint32_t s0 = 32 * h + j + 4 * odd;
+#pragma unroll
+                    for (uint32_t t = 0; t < 4; ++t) {
+                        const uint32_t s = s0 + 8 * t;
+                        if (8 * t + j + 4 * odd >= 8 * sizeof(T) || s < row0 || s >= row1) continue;
+                        uint32_t w = 0;
+#pragma unroll
+                        for (uint32_t i = 0; i < 4; ++i) w |= ((b[i] >> (8 * t)) & 0xFFu) << (8 * i);
+                        uint8_t* to = out + (uint64_t)(s - row0) * n + v0;
+                        if (cnt == 4) {
+                            __builtin_memcpy(to, &w, 4);  // rows of any alignment
+                        } else {
+                            for (uint32_t i = 0; i < cnt; ++i) to[i] = (uint8_t)(w >> (8 * i));
+                        }
+                    }
+                }
+            }
+        }
+    }
 }
 
 // Host-driven superstep: the host's decision written into the control block.
@@ -491,10 +598,12 @@ __global__ void k_mbfs_set_ctl(MbfsCtl* ctl, int32_t step, uint32_t pull, uint32
                                uint32_t hub_wgs) {
     ctl->step = step;
     ctl->pull = pull;
-    ctl->done = 0;
     ctl->n_small = n_small;
     ctl->n_large = n_large;
     ctl->hub_wgs = hub_wgs;
+}
+__global__ void k_mbfs_zero(MbfsCounters* c) {
+    if (threadIdx.x < sizeof(MbfsCounters) / 8) reinterpret_cast<unsigned long long*>(c)[threadIdx.x] = 0;
 }
 
 static uint32_t mbfs_large(const medusa_graph* g, const medusa_opts& o) {
@@ -504,6 +613,10 @@ static uint32_t mbfs_grid(const medusa_graph* g, const medusa_opts& o) {
     return o.grid ? o.grid : (g->tuned.mbfs_grid ? g->tuned.mbfs_grid : kMbfsGridDefault);
 }
 
+// Bytes of device memory for the rows of a host output on their way there.
+constexpr size_t kMbfsRowBytes = 256u << 20;
+
+template <class T>
 static void mbfs_run(medusa_graph* g, const uint32_t* srcs, uint32_t k, uint8_t* out, const medusa_opts& o,
                      medusa_stats& st) {
     const uint32_t n = g->n;
@@ -511,20 +624,15 @@ static void mbfs_run(medusa_graph* g, const uint32_t* srcs, uint32_t k, uint8_t*
     const uint32_t large = mbfs_large(g, o), grid = mbfs_grid(g, o);
     g->q_small.ensure(n);
     g->q_large.ensure(n);
-    g->q_aux.ensure(64);
     DBuf<unsigned long long>& masks = g->bitmap;
     masks.ensure(3 * (size_t)n);
-    unsigned long long* visited = masks.p;
-    unsigned long long* frontier = masks.p + n;
-    unsigned long long* next = masks.p + 2 * (size_t)n;
-    const size_t level_bytes = (size_t)k * n;
-    DBuf<uint32_t>& lvbuf = g->stamp;  // reused as byte storage for the levels
-    lvbuf.ensure((level_bytes + 3) / 4);
-    uint8_t* level = reinterpret_cast<uint8_t*>(lvbuf.p);
+    DBuf<uint32_t>& planes = g->stamp;  // reused as the storage of the level planes
+    planes.ensure((kMbfsPlanes * sizeof(T) * (size_t)n + 3) / 4);
     MbfsCounters* C = dev_counters<MbfsCounters>(g);
     static_assert(sizeof(MbfsCtl) <= sizeof(CtlStorage), "control block storage");
     g->mbfs_ctl.ensure(1);
     MbfsCtl* ctl = reinterpret_cast<MbfsCtl*>(g->mbfs_ctl.p);
+    MbfsCtl* host = reinterpret_cast<MbfsCtl*>(g->h_ctr_raw.p);
     hipStream_t s = g->stream;
     const bool host_driven = o.timing || o.trace;
     uint32_t mode = 0;
@@ -532,75 +640,93 @@ static void mbfs_run(medusa_graph* g, const uint32_t* srcs, uint32_t k, uint8_t*
     else if (o.direction == MEDUSA_DIR_PULL) mode = 2;
     else if (o.policy && policy_kind(o.policy) == MEDUSA_POLICY_DIRECTION) mode = 3;
     const float* policy = (mode == 3 && !host_driven) ? policy_device_params(o.policy) : nullptr;
-    MDS_HIP(hipMemcpyAsync(g->q_aux.p, srcs, (size_t)k * 4, hipMemcpyHostToDevice, s));
     g->trace.clear();
 
     build_pull_layout(g);
     const PullLayout& PL = *g->pull;
-    auto expand = [&]() {
-        hipLaunchKernelGGL(k_mbfs_expand, dim3(grid), dim3(256), 0, s, (const MbfsCtl*)ctl,
-                           (const uint32_t*)g->q_small.p, (const uint32_t*)g->q_large.p, g->row_ptr.p, g->col.p,
-                           g->cptr.p, g->csrc.p, (const unsigned long long*)frontier,
-                           (const unsigned long long*)visited, next, (const PrRun*)PL.d_runs.p,
-                           (const uint32_t*)PL.wg_run.p, PL.total_wgs, (const uint32_t*)PL.perm.p,
-                           (const uint32_t*)PL.ell.p, C);
-        MDS_LAUNCHED();
-    };
-    auto update = [&](const MbfsCtl* c, int32_t lv) {
-        hipLaunchKernelGGL(k_mbfs_update, dim3(grid_for(n, kMbfsTile, 4096)), dim3(256), 0, s, c, lv, n, large,
-                           g->row_ptr.p, visited, frontier, next, level, g->q_small.p, g->q_large.p, C);
-        MDS_LAUNCHED();
-    };
+    MbfsArgs a{};
+    a.row_ptr = g->row_ptr.p;
+    a.col = g->col.p;
+    a.cptr = g->cptr.p;
+    a.csrc = g->csrc.p;
+    a.q_small = g->q_small.p;
+    a.q_large = g->q_large.p;
+    a.visited = masks.p;
+    a.frontier = masks.p + n;
+    a.next = masks.p + 2 * (size_t)n;
+    a.runs = PL.d_runs.p;
+    a.wg_run = PL.wg_run.p;
+    a.perm = PL.perm.p;
+    a.ell = PL.ell.p;
+    a.ctr = C;
+    a.ctl = ctl;
+    a.policy = policy;
+    a.planes = planes.p;
+    a.n = n;
+    a.large = large;
+    a.items = PL.total_wgs;
+    a.grid = grid;
+    const dim3 update_grid(grid_for(n, kMbfsTile, 512)), finish_grid(grid_for(n, 1024, 8192));
+    const bool direct = kernels_can_write(g, out);  // else the rows are copied out at the end
 
-    // capture (once per graph, launch shape, policy buffer and slot count) a batch of supersteps
+    auto expand = [&]() {
+        hipLaunchKernelGGL(k_mbfs_expand, dim3(grid), dim3(256), 0, s, a);
+        MDS_LAUNCHED();
+    };
+    // capture (once per buffers, launch shape, policy buffer and slot count) a batch of supersteps
     auto captured = [&](GraphCache& gc, uint32_t slots) -> hipGraphExec_t {
-        const uintptr_t key[4] = {(uintptr_t)masks.p, (uintptr_t)policy, ((uintptr_t)grid << 32) | large,
-                                  ((uintptr_t)lvbuf.p ^ (uintptr_t)n) ^ ((uintptr_t)slots << 48)};
-        if (gc.exec && std::equal(key, key + 4, gc.key)) return gc.exec;
+        const uintptr_t key[8] = {(uintptr_t)masks.p,   (uintptr_t)policy,
+                                  ((uintptr_t)grid << 32) | large,
+                                  (uintptr_t)planes.p,  (uintptr_t)host,
+                                  (uintptr_t)a.q_small, (uintptr_t)a.q_large,
+                                  ((uintptr_t)sizeof(T) << 32) | slots};
+        if (gc.exec && std::equal(key, key + 8, gc.key)) return gc.exec;
         gc.reset();
         MDS_HIP(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
-        for (uint32_t b = 0; b < slots; ++b) {
-            expand();
-            update(ctl, 0);
-            hipLaunchKernelGGL(k_mbfs_decide, dim3(1), dim3(256), 0, s, ctl, C, policy, grid, 0u);
-        }
         hipGraph_t graph = nullptr;
+        try {
+            for (uint32_t b = 0; b < slots; ++b) {
+                expand();
+                hipLaunchKernelGGL((k_mbfs_update<T, true>), update_grid, dim3(kMbfsWg), 0, s, a, 0);
+            }
+            hipLaunchKernelGGL(k_mbfs_finish<T>, finish_grid, dim3(256), 0, s, a, host, (uint8_t*)nullptr, 0u, 0u);
+            MDS_LAUNCHED();
+        } catch (...) {
+            (void)hipStreamEndCapture(s, &graph);
+            if (graph) (void)hipGraphDestroy(graph);
+            throw;
+        }
         hipError_t e = hipStreamEndCapture(s, &graph);
         if (e == hipSuccess) e = hipGraphInstantiate(&gc.exec, graph, nullptr, nullptr, 0);
         if (graph) (void)hipGraphDestroy(graph);
         MDS_HIP(e);
-        std::copy(key, key + 4, gc.key);
+        std::copy(key, key + 8, gc.key);
         return gc.exec;
     };
     const uint32_t head = head_slots(g->mbfs_last_steps, kMbfsBatch);
     hipGraphExec_t head_exec = nullptr;
     if (!host_driven) head_exec = captured(head == kMbfsBatch ? g->mbfs_graph : g->mbfs_head, head);
 
+    MbfsSources sources{};
+    std::copy(srcs, srcs + k, sources.v);
     MDS_HIP(hipEventRecord(g->ev_begin, s));
-    hipLaunchKernelGGL(k_mbfs_fill, dim3(grid_for(std::max<uint64_t>(n, (level_bytes + 3) / 4), 256, 8192)),
-                       dim3(256), 0, s, n, (uint64_t)((level_bytes + 3) / 4), lvbuf.p, visited, frontier, next);
+    hipLaunchKernelGGL(k_mbfs_fill, dim3(grid_for(3ull * n, 256, 4096)), dim3(256), 0, s, a, (unsigned long long)m, k,
+                       mode, direct ? out : nullptr);
     MDS_LAUNCHED();
-    hipLaunchKernelGGL(k_mbfs_zero, dim3(1), dim3(1), 0, s, C);
-    MDS_LAUNCHED();
-    hipLaunchKernelGGL(k_mbfs_seed, dim3(1), dim3(1), 0, s, (const uint32_t*)g->q_aux.p, k, next);
-    MDS_LAUNCHED();
-    update(nullptr, 0);
-    hipLaunchKernelGGL(k_mbfs_init_ctl, dim3(1), dim3(1), 0, s, ctl, n, (unsigned long long)m, k, mode);
+    hipLaunchKernelGGL(k_mbfs_start, dim3(1), dim3(kWave), 0, s, a, sources, k, host_driven ? 0u : 1u);
     MDS_LAUNCHED();
 
     MbfsCtl h{};
     if (!host_driven) {
-        hipLaunchKernelGGL(k_mbfs_decide, dim3(1), dim3(256), 0, s, ctl, C, policy, grid, 1u);
-        MDS_LAUNCHED();
         for (uint32_t batch = 0;; ++batch) {
             MDS_HIP(hipGraphLaunch(batch == 0 ? head_exec : captured(g->mbfs_graph, kMbfsBatch), s));
-            MDS_HIP(hipMemcpyAsync(g->h_ctr_raw.p, ctl, sizeof(MbfsCtl), hipMemcpyDeviceToHost, s));
+            MDS_HIP(hipEventRecord(g->ev_end, s));
             MDS_HIP(hipStreamSynchronize(s));
-            std::memcpy(&h, g->h_ctr_raw.p, sizeof(MbfsCtl));
-            if (h.done) break;
+            if (host->done) break;
             MDS_CHECK(batch < (n + kMbfsBatch) / kMbfsBatch + 2, MEDUSA_ERR_INTERNAL,
                       "mbfs: superstep loop did not end");
         }
+        h = *host;
         g->mbfs_last_steps = h.supersteps;
     } else {
         Sched sched(o, Sched::kMbfs);
@@ -610,31 +736,30 @@ static void mbfs_run(medusa_graph* g, const uint32_t* srcs, uint32_t k, uint8_t*
         Frontier f{};
         f.n = n;
         f.m = m;
-        h.n_u = (uint64_t)n * k - c.new_bits;
-        h.m_u = (uint64_t)m * k - c.reached_edges;
-        h.reached = c.new_bits;
-        h.reached_edges = c.reached_edges;
-        h.saturated = c.saturated;
+        h.n_u = (uint64_t)n * k - c.sum[kMbfsNewBits].v;
+        h.m_u = (uint64_t)m * k - c.sum[kMbfsReachedEdges].v;
+        h.reached = c.sum[kMbfsNewBits].v;
+        h.reached_edges = c.sum[kMbfsReachedEdges].v;
         bool pull = false;
-        for (uint32_t t = 0; c.n_active; ++t) {
+        for (uint32_t t = 0; c.sum[kMbfsActive].v; ++t) {
             f.step = t;
-            f.n_f = c.n_active;
-            f.m_f = c.active_deg;
+            f.n_f = c.sum[kMbfsActive].v;
+            f.m_f = c.sum[kMbfsActiveDeg].v;
             f.n_u = h.n_u;
             f.m_u = h.m_u;
             if (o.direction == MEDUSA_DIR_PUSH) pull = false;
             else if (o.direction == MEDUSA_DIR_PULL) pull = true;
             else pull = sched.bfs_pull(f, pull);
             hipLaunchKernelGGL(k_mbfs_set_ctl, dim3(1), dim3(1), 0, s, ctl, (int32_t)t, pull ? 1u : 0u, c.n_small,
-                               c.n_large, mbfs_hub_wgs(grid, c.n_small, c.n_large, c.deg_large, c.active_deg));
+                               c.n_large, mbfs_hub_wgs(grid, c.n_small, c.n_large, c.sum[kMbfsLargeDeg].v, f.m_f));
             MDS_LAUNCHED();
-            hipLaunchKernelGGL(k_mbfs_zero, dim3(1), dim3(1), 0, s, C);
+            hipLaunchKernelGGL(k_mbfs_zero, dim3(1), dim3(sizeof(MbfsCounters) / 8), 0, s, C);
             MDS_LAUNCHED();
             if (timing) MDS_HIP(hipEventRecord(g->events[0], s));
             expand();
             if (timing) MDS_HIP(hipEventRecord(g->events[1], s));
-            update(nullptr, (int32_t)(t + 1));
-            const MbfsCounters prev = c;
+            hipLaunchKernelGGL((k_mbfs_update<T, false>), update_grid, dim3(kMbfsWg), 0, s, a, (int32_t)(t + 1));
+            MDS_LAUNCHED();
             c = read_counters<MbfsCounters>(g);
             double kms = 0;
             if (timing) {
@@ -644,22 +769,31 @@ static void mbfs_run(medusa_graph* g, const uint32_t* srcs, uint32_t k, uint8_t*
                 st.kernel_ms += ms;
                 ++st.kernel_launches;
             }
-            const uint64_t kb = pull ? 4ull * (n + 1) + 8ull * n + 12ull * c.probes
-                                     : 20ull * prev.n_active + 20ull * prev.active_deg;
+            uint64_t probes = 0;
+            for (const MbfsLine& l : c.probes) probes += l.v;
+            const uint64_t kb = pull ? 4ull * (n + 1) + 8ull * n + 12ull * probes : 20ull * f.n_f + 20ull * f.m_f;
+            const uint64_t new_bits = c.sum[kMbfsNewBits].v;
             h.kernel_bytes += kb;
-            h.alg_bytes += kb + 24ull * n + c.new_bits;
+            h.alg_bytes += kb + 24ull * n + new_bits;
             if (pull) ++h.pull_steps; else ++h.push_steps;
             sched.record(g, f, pull ? 1.0 : 0.0, kms);
             ++h.supersteps;
-            h.saturated |= c.saturated;
-            h.reached += c.new_bits;
-            h.reached_edges += c.reached_edges;
-            h.n_u -= c.new_bits;
-            h.m_u -= c.reached_edges;
+            if (t + 1 >= 255 && new_bits) h.saturated = 1;
+            h.reached += new_bits;
+            h.reached_edges += c.sum[kMbfsReachedEdges].v;
+            h.n_u -= new_bits;
+            h.m_u -= c.sum[kMbfsReachedEdges].v;
         }
+        // the last update's level, for the finish
+        hipLaunchKernelGGL(k_mbfs_set_ctl, dim3(1), dim3(1), 0, s, ctl, (int32_t)h.supersteps, 0u, 0u, 0u, 0u);
+        MDS_LAUNCHED();
+        if (direct) {
+            hipLaunchKernelGGL(k_mbfs_finish<T>, finish_grid, dim3(256), 0, s, a, (MbfsCtl*)nullptr, out, 0u, k);
+            MDS_LAUNCHED();
+        }
+        MDS_HIP(hipEventRecord(g->ev_end, s));
+        MDS_HIP(hipStreamSynchronize(s));
     }
-    MDS_HIP(hipEventRecord(g->ev_end, s));
-    MDS_HIP(hipStreamSynchronize(s));
     float ms = 0;
     MDS_HIP(hipEventElapsedTime(&ms, g->ev_begin, g->ev_end));
     st.device_ms = ms;
@@ -667,11 +801,21 @@ static void mbfs_run(medusa_graph* g, const uint32_t* srcs, uint32_t k, uint8_t*
     st.push_steps = h.push_steps;
     st.pull_steps = h.pull_steps;
     st.kernel_bytes = h.kernel_bytes;
-    st.alg_bytes = h.alg_bytes + level_bytes + 24ull * n;
+    st.alg_bytes = h.alg_bytes + (uint64_t)k * n + 24ull * n;
     st.edges_traversed = h.reached_edges;
     st.reached = (uint32_t)std::min<uint64_t>(h.reached, 0xFFFFFFFFull);
     st.reserved[0] = h.saturated;
-    copy_out(g, out, level, level_bytes);
+    if (direct) return;
+    // as many rows at a time as the row buffer holds
+    const uint32_t rows = (uint32_t)std::min<uint64_t>(k, std::max<uint64_t>(1, kMbfsRowBytes / n));
+    g->mbfs_rows.ensure(((size_t)rows * n + 3) / 4);
+    for (uint32_t r = 0; r < k; r += rows) {
+        const uint32_t r1 = std::min(k, r + rows);
+        uint8_t* buf = reinterpret_cast<uint8_t*>(g->mbfs_rows.p);
+        hipLaunchKernelGGL(k_mbfs_finish<T>, finish_grid, dim3(256), 0, s, a, (MbfsCtl*)nullptr, buf, r, r1);
+        MDS_LAUNCHED();
+        copy_out(g, out + (size_t)r * n, buf, (size_t)(r1 - r) * n);
+    }
 }
 
 }  // namespace medusa
@@ -691,7 +835,10 @@ extern "C" int medusa_mbfs(medusa_graph* g, const uint32_t* sources, uint32_t k,
         MDS_CHECK(o.direction >= 0 && o.direction <= 2, MEDUSA_ERR_ARG, "mbfs: bad direction %d", o.direction);
         MDS_CHECK(o.grid == 0 || (o.grid >= 2 && o.grid <= 65535), MEDUSA_ERR_ARG, "mbfs: grid must be 0 or 2..65535");
         medusa_stats st{};
-        mbfs_run(g, sources, k, levels, o, st);
+        if (k <= 8) mbfs_run<uint8_t>(g, sources, k, levels, o, st);
+        else if (k <= 16) mbfs_run<uint16_t>(g, sources, k, levels, o, st);
+        else if (k <= 32) mbfs_run<uint32_t>(g, sources, k, levels, o, st);
+        else mbfs_run<unsigned long long>(g, sources, k, levels, o, st);
         if (stats) *stats = st;
     });
 }

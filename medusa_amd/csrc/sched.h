@@ -135,23 +135,6 @@ __device__ inline void policy_direction_costs_wave(const double* rec, const floa
     if (staged) mlp_stage_wave_wait();
     mlp_eval_wave2(sP, x, c_push, c_pull);
 }
-
-// Predicted costs of push (out[0]) and pull (out[1]) for the superstep described by `rec`.
-// Every thread of the block calls it; `staged`: the kernel already ran mlp_stage into m.P.
-// Threads 0 and 1 build the push and pull rows with FP32 logarithms (direction_row's rows, up
-// to their rounding); mlp_eval_rows' first barrier publishes them.
-__device__ inline void policy_direction_costs(const double* rec, const float* __restrict__ policy, MlpShared& m,
-                                              bool staged = false) {
-    float x[MEDUSA_POLICY_INPUTS];
-    if (threadIdx.x < 2) {
-        float L[kDirectionLogs];  // in FP32, as the one-wave form does
-#pragma unroll
-        for (int i = 0; i < kDirectionLogs; ++i) L[i] = direction_log_f32(rec, i);
-        direction_fill(rec, L, (double)threadIdx.x, x);
-        for (int i = 0; i < MEDUSA_POLICY_INPUTS; ++i) m.x[threadIdx.x * MEDUSA_POLICY_INPUTS + i] = x[i];
-    }
-    mlp_eval_rows(policy, m.P, m.x, 2, m.a1, m.a2, m.out, staged);  // its first barrier publishes the rows
-}
 #endif
 
 // Frontier features at the start of a superstep.

@@ -256,6 +256,45 @@ def test_mbfs_small(oracle):
                 assert np.array_equal(out, want), (len(srcs), d)
 
 
+@pytest.mark.parametrize("n", [1, 3, 1023, 4095, 4097, 12290])
+@pytest.mark.parametrize("k", [1, 8, 9, 16, 17, 32, 33, 64])
+def test_mbfs_level_planes(oracle, n, k):
+    """Every width of the level planes, vertex counts around the update's tile of 4096 and the 4
+    vertices of a finishing lane, levels on both sides of 16 (the fifth plane) and 255 (saturated),
+    repeated sources, host and device outputs, both drivers, and a BFS in between whose buffers
+    replace the ones the supersteps were captured with."""
+    torch = pytest.importorskip("torch")
+    rng = np.random.default_rng(n * 64 + k)
+    chain = np.arange(min(n - 1, 300))  # levels past 255, the rest at random behind its ends
+    src = np.concatenate([chain, rng.integers(n // 2, n, 2 * n)])
+    dst = np.concatenate([chain + 1, rng.integers(n // 2, n, 2 * n)])
+    rp, col, _ = csr_from_edges(n, np.stack([src, dst], 1))
+    srcs = rng.integers(0, n, k).astype(np.uint32)
+    srcs[0], srcs[k // 2] = 0, min(n - 1, 284)
+    want = oracle.mbfs(rp, col, srcs)
+    dev = torch.full((k, n), 7, dtype=torch.uint8, device="cuda")
+    with md.Graph(rp, col) as G:
+        for opts in ({}, {"timing": 1}, {"direction": md.DIR_PULL, "large_degree": 2}, {}):
+            out, st = G.mbfs(srcs, **opts)
+            assert np.array_equal(out, want), opts
+            G.mbfs(srcs, out=dev, **opts)
+            assert np.array_equal(dev.cpu().numpy(), want), opts
+            G.bfs(0)
+        saturated = any(oracle.bfs_queue(rp, col, int(v)).max() >= 255 for v in np.unique(srcs))
+        assert G.mbfs(srcs)[1].reserved[0] == int(saturated)
+
+
+def test_mbfs_rows_in_pieces():
+    """A host output of more bytes than the row buffer holds: no vertex but the sources is reached."""
+    n, k = 5_000_001, 64
+    with md.Graph(np.zeros(n + 1, np.uint32), np.zeros(0, np.uint32)) as G:
+        srcs = (np.arange(k) * 70_001).astype(np.uint32)
+        out, _ = G.mbfs(srcs)
+    assert np.array_equal(out[np.arange(k), srcs], np.zeros(k))
+    out[np.arange(k), srcs] = 255
+    assert (out == 255).all()
+
+
 def test_mbfs_matches_plain_bfs(oracle):
     rp, col = wl.er_graph(8192, 65536, seed=1)
     srcs = wl.mbfs_sources(rp, 64, seed=4)
