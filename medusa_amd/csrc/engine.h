@@ -260,6 +260,7 @@ struct medusa_graph {
     uint64_t m = 0;
     bool weighted = false;
     uint32_t max_outdeg = 0;
+    uint32_t w_mean = 0;  // of sampled weights, 0 until an SSSP run needs it
     int device = 0;
     hipStream_t stream = nullptr;
     // host copies (layouts are derived from them)
@@ -287,16 +288,18 @@ struct medusa_graph {
     medusa::HBuf<unsigned long long> h_ctr_raw;
     // device-driven superstep loops: control blocks and captured superstep batches
     medusa::DBuf<medusa::CtlStorage> bfs_ctl, mbfs_ctl, sssp_ctl;
-    medusa::GraphCache bfs_graph, mbfs_graph, sssp_graph;
+    medusa::GraphCache bfs_graph, mbfs_graph;
+    medusa::GraphCache sssp_heads[medusa::kMaxHeadSlots / 4 + 1];  // by slot count / 4
     // first replay of the BFS / MBFS loops: as many slots as the previous run on this handle
     // used, so a repeated traversal ends after one replay with no idle slots (BFS: one graph per
     // slot count, so runs of different lengths do not capture again)
     medusa::GraphCache bfs_heads[medusa::kMaxHeadSlots + 1], mbfs_head;
-    uint32_t bfs_next_head = medusa::kNoHead, mbfs_last_steps = 0;
+    uint32_t bfs_next_head = medusa::kNoHead, mbfs_last_steps = 0, sssp_last_slots = 0;
     // pinned: parameters of a BFS run and its control block afterwards; levels on their way to a
     // small host output
     medusa::HBuf<unsigned long long> h_bfs;
     medusa::HBuf<int32_t> h_levels;
+    medusa::HBuf<unsigned long long> h_sssp;  // pinned: control block and sums of an SSSP run
     int wall_khz = 0;  // rate of the device's wall clock
     std::unique_ptr<medusa::PrLayout> pr;
     std::unique_ptr<medusa::PullLayout> pull;  // built on the first MBFS run

@@ -30,6 +30,7 @@
 // wave does this on its own (wave rounds, below).
 
 #include <algorithm>
+#include <numeric>
 #include <chrono>
 
 #include "engine.h"
@@ -56,14 +57,19 @@ __host__ __device__ inline uint32_t slices_of(uint32_t deg) { return deg <= kSli
 // by the split and lowered again by a local round is appended under both.
 __host__ inline size_t near_capacity(uint32_t n, uint64_t m) { return 2 * ((size_t)n + m / kSlice) + 64; }
 
-__global__ void k_sssp_init(uint32_t n, uint32_t* __restrict__ dist, uint32_t* __restrict__ stamp, uint32_t src,
-                            uint32_t src_slices, unsigned long long* __restrict__ near_q) {
+// Distances and stamps of vertex v at the start of a run; the source's near-queue entries.
+__device__ __forceinline__ void sssp_init(uint32_t n, uint32_t* __restrict__ dist, uint32_t* __restrict__ stamp,
+                                          uint32_t src, uint32_t src_slices, unsigned long long* __restrict__ near_q) {
     for (uint32_t v = blockIdx.x * blockDim.x + threadIdx.x; v < n; v += gridDim.x * blockDim.x) {
         dist[v] = v == src ? 0u : 0xFFFFFFFFu;
         stamp[v] = 0;
     }
     for (uint32_t k = blockIdx.x * blockDim.x + threadIdx.x; k < src_slices; k += gridDim.x * blockDim.x)
         near_q[k] = ((unsigned long long)k << 32) | src;
+}
+__global__ void k_sssp_init(uint32_t n, uint32_t* __restrict__ dist, uint32_t* __restrict__ stamp, uint32_t src,
+                            uint32_t src_slices, unsigned long long* __restrict__ near_q) {
+    sssp_init(n, dist, stamp, src, src_slices, near_q);
 }
 
 __global__ void k_sssp_zero(SsspCounters* c, uint32_t keep_far) {
@@ -753,6 +759,7 @@ __global__ __launch_bounds__(256) void k_sssp_split(const uint32_t* __restrict__
 // kSsspBatch slots are captured once as a hipGraph and replayed until done.
 
 constexpr uint32_t kSsspBatch = 32;
+constexpr uint32_t kSsspStep = 4;  // granularity of a replay's slots: one captured graph per multiple
 // Workgroups of a work launch: about the resident count (5 per CU at this LDS size) without local
 // rounds, so every tile is in flight at once (RMAT-20 at width 250: 1.51 ms against 1.79 with
 // 2048; ER 2^20/2^24: 1.15 against 1.36); twice that with local rounds, whose short queues spread
@@ -765,6 +772,8 @@ struct SsspCtl {
     uint32_t overflow, phase, supersteps, local_rounds, width, near_sel;
     uint32_t far_sel, local_cfg, trace, lost;  // lost: near entries beyond the queue
     unsigned long long n, m, relaxed, kernel_bytes;
+    unsigned long long out;  // where the closing kernel writes the distances (0: nowhere)
+    uint32_t slots, pad;     // work launches so far
 };
 
 // Phase marks of the device-driven loop when tracing: mark i (3 words) holds the features at
@@ -822,6 +831,7 @@ __device__ void sssp_decide(SsspCtl* ctl, SsspDevCounters* ctr, unsigned long lo
     k.far_min = load_now(&ctr->far_min);
     k.relax = relaxed;
     SsspCtl c = load_now_block(ctl);
+    c.slots += 1;
     if (k.n_near > near_cap) {
         // entries past the queue were dropped by the writers (near_capacity rules this out):
         // stop, and let the host report it, rather than read past the queue
@@ -1061,9 +1071,27 @@ __global__ __launch_bounds__(kWaveThreads) void k_sssp_work_wave(
     if (sssp_last_block(ctr, dep, relax) && threadIdx.x == 0) sssp_decide(ctl, ctr, relax, far_cap, near_cap, marks);
 }
 
-__global__ void k_sssp_seed_ctl(SsspCtl* ctl, SsspDevCounters* c, uint32_t n, unsigned long long m, uint32_t thr,
-                                uint32_t width, uint32_t src_slices, uint32_t local_cfg, uint32_t trace,
-                                unsigned long long* marks) {
+// What a device-driven run leaves in pinned memory: its control block and, by the closing kernel's
+// workgroups, the reached vertices and the out-edges they own (summed by the host: no counter to
+// clear, and none that all workgroups would queue up on).
+constexpr uint32_t kSsspCloseGrid = 256;
+struct SsspHost {
+    SsspCtl ctl;
+    unsigned long long t_begin, t_end;
+    unsigned long long edges[kSsspCloseGrid], reached[kSsspCloseGrid];
+};
+
+// Start of a device-driven run: distances, stamps and queue; control block and counters (by the first
+// workgroup).
+__global__ void k_sssp_start(uint32_t n, uint32_t* __restrict__ dist, uint32_t* __restrict__ stamp, uint32_t src,
+                             uint32_t src_slices, unsigned long long* __restrict__ near_q, SsspCtl* ctl,
+                             SsspDevCounters* c, unsigned long long m, uint32_t thr, uint32_t width, uint32_t local_cfg,
+                             uint32_t trace, unsigned long long* marks, SsspHost* host, uint32_t* out) {
+    sssp_init(n, dist, stamp, src, src_slices, near_q);
+    if (blockIdx.x != 0) return;
+    if (threadIdx.x < kSsspSlots) c->sub[threadIdx.x].v = 0;
+    if (threadIdx.x != 0) return;
+    host->t_begin = (unsigned long long)wall_clock64();
     SsspCtl z{};
     z.trace = trace;
     // phase 0: one source vertex, threshold 0 before the first advance
@@ -1077,13 +1105,61 @@ __global__ void k_sssp_seed_ctl(SsspCtl* ctl, SsspDevCounters* c, uint32_t n, un
     z.width = width;
     z.n = n;
     z.m = m;
+    z.out = reinterpret_cast<unsigned long long>(out);
     *ctl = z;
     c->n_near = 0;
     c->n_far = 0;
     c->far_out = 0;
     c->far_min = 0xFFFFFFFFu;
-    for (uint32_t i = 0; i < kSsspSlots; ++i) c->sub[i].v = 0;
     c->top = 0;
+}
+
+// End of a batch of slots: the control block to the host and, once the run is done (`ctl` null: it
+// is), the distances to `out` (null: the host copies them) with the reached vertices and the
+// out-edges they own, which are the GTEPS numerator (the same for every bucket width).  One pass over
+// the distances; in separate launches with a copy, two clears and two waits of their own these took
+// 120 us after a run on RMAT-20, now 8: 2177 us a run before, 2049 now; 173 x 211 lattice 582
+// and 510 (there a quarter of it is the replay's idle slots, sized by the run before).
+__global__ __launch_bounds__(1024) void k_sssp_close(const SsspCtl* __restrict__ ctl, SsspHost* __restrict__ host,
+                                                     uint32_t n, const uint32_t* __restrict__ dist,
+                                                     const uint32_t* __restrict__ row_ptr, uint32_t* __restrict__ out) {
+    __shared__ unsigned long long s_e[16], s_v[16];
+    if (ctl) {
+        if (blockIdx.x == 0) {
+            if (threadIdx.x < sizeof(SsspCtl) / 8)
+                reinterpret_cast<unsigned long long*>(&host->ctl)[threadIdx.x] =
+                    reinterpret_cast<const unsigned long long*>(ctl)[threadIdx.x];
+            if (threadIdx.x == 0) host->t_end = (unsigned long long)wall_clock64();
+        }
+        if (!ctl->done) return;
+        out = reinterpret_cast<uint32_t*>(ctl->out);
+    }
+    unsigned long long e = 0, c = 0;
+    const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
+    for (uint64_t v = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; v < n; v += stride) {
+        const uint32_t d = dist[v], deg = row_ptr[v + 1] - row_ptr[v];
+        if (d != 0xFFFFFFFFu) {
+            e += deg;
+            ++c;
+        }
+        if (out) out[v] = d;
+    }
+    e = wave_sum_u64(e);
+    c = wave_sum_u64(c);
+    if ((threadIdx.x & (kWave - 1)) == 0) {
+        s_e[threadIdx.x / kWave] = e;
+        s_v[threadIdx.x / kWave] = c;
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        e = c = 0;
+        for (uint32_t w = 0; w < 16; ++w) {
+            e += s_e[w];
+            c += s_v[w];
+        }
+        host->edges[blockIdx.x] = e;
+        host->reached[blockIdx.x] = c;
+    }
 }
 
 // Local rounds per superstep (while the near queue is short): the caller's count, or by
@@ -1127,12 +1203,15 @@ static size_t sssp_far_cap(const medusa_graph* g, const medusa_opts& o) {
 // Mean weight (sampled) and the default bucket width, a multiple of it: 8x with local rounds,
 // which absorb the extra hops of a wider bucket (1400x1400 lattice, 32 rounds: 8.0 ms at 8x,
 // 8.6 ms at 6x, 11.5 ms at 3x), else 2x.
-static void sssp_widths(const medusa_graph* g, const medusa_opts& o, uint32_t& wmean, uint32_t& dflt) {
-    uint64_t wsum = 0, wcnt = 0;
-    const uint64_t m = g->m;
-    const uint64_t wstride = std::max<uint64_t>(1, m / 4096);
-    for (uint64_t e = 0; e < m; e += wstride, ++wcnt) wsum += g->h_w[e];
-    wmean = (uint32_t)std::max<uint64_t>(1, wcnt ? wsum / wcnt : 1);
+static void sssp_widths(medusa_graph* g, const medusa_opts& o, uint32_t& wmean, uint32_t& dflt) {
+    if (!g->w_mean) {  // once per graph: 4096 cache misses, 60 us on 64 MiB of weights
+        uint64_t wsum = 0, wcnt = 0;
+        const uint64_t m = g->m;
+        const uint64_t wstride = std::max<uint64_t>(1, m / 4096);
+        for (uint64_t e = 0; e < m; e += wstride, ++wcnt) wsum += g->h_w[e];
+        g->w_mean = (uint32_t)std::max<uint64_t>(1, wcnt ? wsum / wcnt : 1);
+    }
+    wmean = g->w_mean;
     const uint64_t mult = sssp_local_cfg(g, o) ? 8 : 2;
     dflt = (uint32_t)std::min<uint64_t>(0xFFFFFFFEull, mult * wmean);
 }
@@ -1164,9 +1243,6 @@ static void sssp_device_trace(medusa_graph* g, uint32_t phases, uint32_t wmean) 
     std::vector<unsigned long long> h(3ull * nmarks);
     MDS_HIP(hipMemcpyAsync(h.data(), g->sssp_phases.p, h.size() * 8, hipMemcpyDeviceToHost, g->stream));
     MDS_HIP(hipStreamSynchronize(g->stream));
-    int khz = 0;
-    MDS_HIP(hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, g->device));
-    MDS_CHECK(khz > 0, MEDUSA_ERR_HIP, "sssp: no wall clock rate");
     g->trace.clear();
     for (uint32_t i = 0; i + 1 < nmarks; ++i) {
         Frontier f{};
@@ -1175,7 +1251,7 @@ static void sssp_device_trace(medusa_graph* g, uint32_t phases, uint32_t wmean) 
         f.n = g->n;
         f.m = g->m;
         const uint32_t thr = (uint32_t)h[3 * i + 1], delta = (uint32_t)(h[3 * i + 1] >> 32);
-        const double ms = (double)(h[3 * (i + 1) + 2] - h[3 * i + 2]) / (double)khz;
+        const double ms = (double)(h[3 * (i + 1) + 2] - h[3 * i + 2]) / (double)g->wall_khz;
         TraceRec r;
         Sched::to_sssp_record(f, wmean, thr, (double)delta, ms, r.f);
         g->trace.push_back(r);
@@ -1201,7 +1277,7 @@ static void sssp_run_device(medusa_graph* g, uint32_t src, uint32_t* out, const 
     // control block in unit 0 of the storage, counters and tickets after it
     g->sssp_ctl.ensure(kSsspCtlUnits);
     SsspCtl* ctl = reinterpret_cast<SsspCtl*>(g->sssp_ctl.p);
-    static_assert(sizeof(SsspCtl) <= sizeof(CtlStorage) - 16, "control block storage (its last 16 bytes: reached counts)");
+    static_assert(sizeof(SsspCtl) <= sizeof(CtlStorage), "control block storage");
     SsspDevCounters* ctr = reinterpret_cast<SsspDevCounters*>(g->sssp_ctl.p + 1);
     uint32_t* far0 = g->q_aux.p;
     uint32_t* far1 = g->q_aux.p + sssp_far_alloc(g);
@@ -1210,17 +1286,25 @@ static void sssp_run_device(medusa_graph* g, uint32_t src, uint32_t* out, const 
     unsigned long long* near1 = g->near_q.p + near_cap;
     const uint32_t src_slices = slices_of(g->h_row_ptr[src + 1] - g->h_row_ptr[src]);
 
-    GraphCache& gc = g->sssp_graph;
     unsigned long long* marks = g->sssp_phases.p;
     const uint32_t local_cfg = sssp_local_cfg(g, o);
     const uint4* rec = sssp_records(g, o);
-    // the marks buffer is 256-byte aligned, so its low bits can carry the kernel variant
-    const uintptr_t key[6] = {(uintptr_t)g->dist.p, (uintptr_t)g->near_q.p, (uintptr_t)g->q_aux.p,
-                              (uintptr_t)g->w.p, (uintptr_t)marks | (rec ? 2u : local_cfg ? 1u : 0u), (uintptr_t)ctl};
-    if (!gc.exec || !std::equal(key, key + 6, gc.key)) {
+    SsspHost* host = reinterpret_cast<SsspHost*>(g->h_sssp.p);
+    auto close = [&]() {
+        hipLaunchKernelGGL(k_sssp_close, dim3(grid_for(n, 1024, kSsspCloseGrid)), dim3(1024), 0, s, (const SsspCtl*)ctl,
+                           host, n, (const uint32_t*)g->dist.p, g->row_ptr.p, (uint32_t*)nullptr);
+    };
+    // `slots` work launches and the closing kernel, captured once per slot count
+    auto captured = [&](uint32_t slots) -> hipGraphExec_t {
+        GraphCache& gc = g->sssp_heads[slots / kSsspStep];
+        // the marks buffer is 256-byte aligned, so its low bits can carry the kernel variant
+        const uintptr_t key[7] = {(uintptr_t)g->dist.p, (uintptr_t)g->near_q.p, (uintptr_t)g->q_aux.p,
+                                  (uintptr_t)g->stamp.p, (uintptr_t)marks | (rec ? 2u : local_cfg ? 1u : 0u),
+                                  (uintptr_t)ctl, (uintptr_t)far_cap};
+        if (gc.exec && std::equal(key, key + 7, gc.key)) return gc.exec;
         gc.reset();
         MDS_HIP(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
-        for (uint32_t k = 0; k < kSsspBatch; ++k) {
+        for (uint32_t k = 0; k < slots; ++k) {
             if (rec)
                 hipLaunchKernelGGL(k_sssp_work_wave, dim3(kSsspGridWave), dim3(kWaveThreads), 0, s, ctl, near0, near1,
                                    (uint32_t)near_cap, far0, far1, (uint32_t)far_cap, g->row_ptr.p, g->col.p, g->w.p,
@@ -1231,38 +1315,42 @@ static void sssp_run_device(medusa_graph* g, uint32_t src, uint32_t* out, const 
                                    ctl, near0, near1, (uint32_t)near_cap, far0, far1, (uint32_t)far_cap,
                                    g->row_ptr.p, g->col.p, g->w.p, g->dist.p, g->stamp.p, ctr, marks);
         }
+        close();
         hipGraph_t graph = nullptr;
         hipError_t e = hipStreamEndCapture(s, &graph);
         if (e == hipSuccess) e = hipGraphInstantiate(&gc.exec, graph, nullptr, nullptr, 0);
         if (graph) (void)hipGraphDestroy(graph);
         MDS_HIP(e);
-        std::copy(key, key + 6, gc.key);
-    }
+        std::copy(key, key + 7, gc.key);
+        return gc.exec;
+    };
+    // slots of the next replay: what the previous run on the handle still took from here, in steps of
+    // kSsspStep; a batch where there is no previous run or this one is longer
+    auto next_slots = [&](uint64_t done) {
+        const uint64_t left = g->sssp_last_slots > done ? g->sssp_last_slots - done : kSsspBatch;
+        return (uint32_t)std::min<uint64_t>(kMaxHeadSlots, (left + kSsspStep - 1) / kSsspStep * kSsspStep);
+    };
+    uint32_t slots = next_slots(0);
+    hipGraphExec_t exec = captured(slots);
+    const bool direct = kernels_can_write(g, out);
 
-    MDS_HIP(hipEventRecord(g->ev_begin, s));
-    hipLaunchKernelGGL(k_sssp_init, dim3(grid_for(n, 256, 4096)), dim3(256), 0, s, n, g->dist.p, g->stamp.p, src,
-                       src_slices, near0);
+    hipLaunchKernelGGL(k_sssp_start, dim3(grid_for(n, 256, 4096)), dim3(256), 0, s, n, g->dist.p, g->stamp.p, src,
+                       src_slices, near0, ctl, ctr, (unsigned long long)m, thr0, d0, local_cfg, o.trace ? 1u : 0u, marks,
+                       host, direct ? out : nullptr);
     MDS_LAUNCHED();
-    hipLaunchKernelGGL(k_sssp_seed_ctl, dim3(1), dim3(1), 0, s, ctl, ctr, n, (unsigned long long)m, thr0, d0,
-                       src_slices, local_cfg, o.trace ? 1u : 0u, marks);
-    MDS_LAUNCHED();
-    SsspCtl h{};
     // every replay either relaxes a non-empty queue or raises the threshold
-    const uint64_t max_batches = 4ull * n / kSsspBatch + 1024;
-    for (uint64_t batch = 0;; ++batch) {
-        MDS_HIP(hipGraphLaunch(gc.exec, s));
-        MDS_HIP(hipMemcpyAsync(g->h_ctr_raw.p, ctl, sizeof(SsspCtl), hipMemcpyDeviceToHost, s));
+    const uint64_t max_slots = 4ull * n + 1024ull * kSsspBatch;
+    for (uint64_t done = 0;; exec = captured(slots = next_slots(done))) {
+        MDS_HIP(hipGraphLaunch(exec, s));
         MDS_HIP(hipStreamSynchronize(s));
-        std::memcpy(&h, g->h_ctr_raw.p, sizeof(SsspCtl));
-        MDS_CHECK(!h.lost, MEDUSA_ERR_INTERNAL, "sssp: near queue overflow");
-        if (h.done) break;
-        MDS_CHECK(batch < max_batches, MEDUSA_ERR_INTERNAL, "sssp: superstep loop did not end");
+        MDS_CHECK(!host->ctl.lost, MEDUSA_ERR_INTERNAL, "sssp: near queue overflow");
+        if (host->ctl.done) break;
+        done += slots;
+        MDS_CHECK(done < max_slots, MEDUSA_ERR_INTERNAL, "sssp: superstep loop did not end");
     }
-    MDS_HIP(hipEventRecord(g->ev_end, s));
-    MDS_HIP(hipStreamSynchronize(s));
-    float ms = 0;
-    MDS_HIP(hipEventElapsedTime(&ms, g->ev_begin, g->ev_end));
-    st.device_ms = ms;
+    const SsspCtl h = host->ctl;
+    g->sssp_last_slots = h.slots;
+    st.device_ms = (double)(host->t_end - host->t_begin) / (double)g->wall_khz;
     st.supersteps = h.supersteps;
     st.push_steps = h.supersteps;
     st.kernel_bytes = h.kernel_bytes;
@@ -1270,7 +1358,7 @@ static void sssp_run_device(medusa_graph* g, uint32_t src, uint32_t* out, const 
     st.reserved[0] = (uint32_t)std::min<uint64_t>(h.relaxed, 0xFFFFFFFFull);
     st.reserved[1] = h.phase;
     if (o.trace) sssp_device_trace(g, h.phase, wmean);
-    copy_out(g, out, g->dist.p, (size_t)n * 4);
+    if (!direct) copy_out(g, out, g->dist.p, (size_t)n * 4);
 }
 
 static void sssp_run_host(medusa_graph* g, uint32_t src, uint32_t* out, const medusa_opts& o, medusa_stats& st) {
@@ -1409,6 +1497,10 @@ static void sssp_run_host(medusa_graph* g, uint32_t src, uint32_t* out, const me
     close_phase();
     st.reserved[1] = phase;
     MDS_HIP(hipEventRecord(g->ev_end, s));
+    hipLaunchKernelGGL(k_sssp_close, dim3(grid_for(n, 1024, kSsspCloseGrid)), dim3(1024), 0, s, (const SsspCtl*)nullptr,
+                       reinterpret_cast<SsspHost*>(g->h_sssp.p), n, (const uint32_t*)g->dist.p, g->row_ptr.p,
+                       (uint32_t*)nullptr);
+    MDS_LAUNCHED();
     MDS_HIP(hipStreamSynchronize(s));
     float ms = 0;
     MDS_HIP(hipEventElapsedTime(&ms, g->ev_begin, g->ev_end));
@@ -1416,36 +1508,6 @@ static void sssp_run_host(medusa_graph* g, uint32_t src, uint32_t* out, const me
     copy_out(g, out, g->dist.p, (size_t)n * 4);
     st.alg_bytes = st.kernel_bytes + 8ull * n;
     st.reserved[0] = (uint32_t)std::min<uint64_t>(relaxed, 0xFFFFFFFFull);
-}
-
-// GTEPS numerator on the GPU: reached vertices and the out-edges they own (the same
-// for every bucket width).
-__global__ __launch_bounds__(256) void k_sssp_reached(uint32_t n, const uint32_t* __restrict__ dist,
-                                                      const uint32_t* __restrict__ row_ptr,
-                                                      unsigned long long* __restrict__ out) {
-    __shared__ unsigned long long s_e[4], s_v[4];
-    unsigned long long e = 0, c = 0;
-    for (uint32_t v = blockIdx.x * blockDim.x + threadIdx.x; v < n; v += gridDim.x * blockDim.x)
-        if (dist[v] != 0xFFFFFFFFu) {
-            e += row_ptr[v + 1] - row_ptr[v];
-            ++c;
-        }
-    e = wave_sum_u64(e);
-    c = wave_sum_u64(c);
-    if ((threadIdx.x & (kWave - 1)) == 0) {
-        s_e[threadIdx.x / kWave] = e;
-        s_v[threadIdx.x / kWave] = c;
-    }
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        atomicAdd(&out[0], s_e[0] + s_e[1] + s_e[2] + s_e[3]);
-        atomicAdd(&out[1], s_v[0] + s_v[1] + s_v[2] + s_v[3]);
-    }
-}
-
-__global__ void k_zero_u64x2(unsigned long long* p) {
-    p[0] = 0;
-    p[1] = 0;
 }
 
 }  // namespace medusa
@@ -1470,27 +1532,17 @@ extern "C" int medusa_sssp(medusa_graph* g, uint32_t source, uint32_t* dist, con
         g->near_q.ensure(2 * near_capacity(n, g->m));  // near queues A and B ((vertex, slice) entries)
         g->sssp_phases.ensure(3ull * kMaxPhaseMarks);     // phase marks of a traced device-driven run
         g->q_aux.ensure(2 * far_cap);                   // far queues A and B
+        g->h_sssp.ensure((sizeof(SsspHost) + 7) / 8);
         medusa_stats st{};
         // timing: host-driven, every relaxation launch timed; otherwise device-driven (traced
         // by phase marks when trace is on)
         if (o.timing) sssp_run_host(g, source, dist, o, st);
         else sssp_run_device(g, source, dist, o, st);
         if (o.trace) sssp_trace_settled(g);
-        unsigned long long* red = reinterpret_cast<unsigned long long*>(g->sssp_ctl.p) + 30;
-        if (!g->sssp_ctl.p) {
-            g->sssp_ctl.ensure(1);
-            red = reinterpret_cast<unsigned long long*>(g->sssp_ctl.p) + 30;
-        }
-        hipLaunchKernelGGL(k_zero_u64x2, dim3(1), dim3(1), 0, g->stream, red);
-        MDS_LAUNCHED();
-        hipLaunchKernelGGL(k_sssp_reached, dim3(grid_for(n, 256, 1024)), dim3(256), 0, g->stream, n,
-                           (const uint32_t*)g->dist.p, g->row_ptr.p, red);
-        MDS_LAUNCHED();
-        unsigned long long hr[2];
-        MDS_HIP(hipMemcpyAsync(hr, red, sizeof hr, hipMemcpyDeviceToHost, g->stream));
-        MDS_HIP(hipStreamSynchronize(g->stream));
-        st.edges_traversed = hr[0];
-        st.reached = (uint32_t)hr[1];
+        const SsspHost* h = reinterpret_cast<const SsspHost*>(g->h_sssp.p);
+        const uint32_t wgs = grid_for(n, 1024, kSsspCloseGrid);
+        st.edges_traversed = std::accumulate(h->edges, h->edges + wgs, 0ull);
+        st.reached = (uint32_t)std::accumulate(h->reached, h->reached + wgs, 0ull);
         if (stats) *stats = st;
     });
 }

@@ -329,6 +329,31 @@ def test_mbfs_rmat20_config(oracle, mbfs_policy):
             assert st.edges_traversed == reached
 
 
+@pytest.mark.parametrize("n", [1, 1023, 1025, 9000])
+def test_sssp_runs_of_different_lengths(oracle, n):
+    """Runs on one handle whose slot counts differ by more than a replay (a path of `n` vertices
+    from its start, its middle and its end), so the first replay is too short, too long and
+    right; between them a multi-source BFS, whose level planes replace the stamps; host and device
+    outputs, reached counts on both sides of a closing workgroup's 1024 vertices."""
+    torch = pytest.importorskip("torch")
+    rp, col, _ = csr_from_edges(n, np.stack([np.arange(n - 1), np.arange(1, n)], 1))
+    w = np.random.default_rng(n).integers(1, 1001, len(col)).astype(np.uint32)
+    dev = torch.empty(n, dtype=torch.int32, device="cuda")
+    with md.Graph(rp, col, w) as G:
+        for s in (0, n - 1, n // 2, 0, 0, n - 1):
+            want = oracle.sssp_dijkstra(rp, col, w, s)
+            for opts in ({}, {"local_rounds": 0xFFFFFFFF, "delta": 100000}, {"far_limit": 1}, {"timing": 1}):
+                if n > 1025 and "delta" not in opts and "timing" in opts:
+                    continue  # thousands of host-driven supersteps
+                got, st = G.sssp(s, **opts)
+                assert np.array_equal(got, want), (s, opts)
+                assert (st.reached, st.edges_traversed) == (n - s, n - 1 - s), (s, opts)
+                st = G.sssp(s, out=dev, **opts)[1]
+                assert np.array_equal(dev.cpu().numpy().view(np.uint32), want), (s, opts)
+                assert (st.reached, st.edges_traversed) == (n - s, n - 1 - s), (s, opts)
+            G.mbfs(np.arange(min(n, 64), dtype=np.uint32))
+
+
 @pytest.mark.parametrize("far_limit", [1, 7, 64])
 def test_sssp_far_queue_limit_rebuilds(oracle, far_limit):
     """A far queue capped far below its need is rebuilt from the distances at every split;
