@@ -204,19 +204,22 @@ struct PrLayout {
     }
 };
 
-// Layout for pull supersteps over 64-bit masks (MBFS): vertices with in-edges in in-degree-
-// descending order, cut into runs as in PrLayout (equal in-degree 1..64: a lane per vertex
-// over an ELL slab of ORIGINAL source ids, so the k-th sources of 64 vertices are one coalesced
-// load; in-degree > 64: a wave per vertex over the CSC segment).  Vertices without in-edges
-// never join through a pull and are left out.
+// Layout of the multi-source BFS (built on its first run): vertices in an internal order, sorted by
+// in-degree inside windows of kPullWindow consecutive ids, so that the 64 vertices of a wave (a
+// slice) have nearly equal in-degrees while masks and levels stay close to their place; every
+// slice's in-edges as columns of 64 source ids, a vertex of more than kPullLaneMax in-edges (a hub)
+// by itself.  All ids in it are internal.
+constexpr uint32_t kPullWindow = 4096, kPullLaneMax = 64;
 struct PullLayout {
-    std::vector<PrRun> runs;
-    uint32_t total_wgs = 0;  // work items of 256 lane-vertices or 4 wave-vertices
-    DBuf<PrRun> d_runs;
-    DBuf<uint32_t> wg_run;   // run of every work item
-    DBuf<uint32_t> perm;     // sorted position -> original vertex id
-    DBuf<uint32_t> ell;      // ELL slabs (original source ids)
+    uint32_t nslices = 0, nhubs = 0;
+    DBuf<uint32_t> pos;       // original id -> internal id
+    DBuf<uint2> out;          // per vertex: first out-edge, out-degree
+    DBuf<uint8_t> indeg;      // per vertex: in-degree, kPullHub for a hub
+    DBuf<uint64_t> base;      // per slice: first column (length: up to the next slice's base / 64)
+    DBuf<uint4> hub;          // vertex, in-degree, first in-edge (low, high word)
+    DBuf<uint32_t> src;       // slices' columns, then the hubs' in-edges
 };
+constexpr uint8_t kPullHub = 255;
 
 struct TraceRec {
     double f[MEDUSA_TRACE_FIELDS];
@@ -241,8 +244,13 @@ struct GraphCache {
 // loop's end return at once, so the choice changes only the time, never the result.
 constexpr uint32_t kMaxHeadSlots = 64;
 constexpr uint32_t kNoHead = 0xFFFFFFFFu;  // no previous run
-inline uint32_t head_slots(uint32_t last_steps, uint32_t batch) {
-    return last_steps ? (last_steps < kMaxHeadSlots ? last_steps : kMaxHeadSlots) : batch;
+constexpr uint32_t kHeadStep = 4;  // SSSP, MBFS: granularity of a replay's slots, one captured graph per multiple
+// Slots of the next replay: what the previous run on the handle (`last` slots in all) still took
+// after `done`, or a batch where there is no previous run or this one is longer.
+inline uint32_t next_slots(uint64_t last, uint64_t done, uint32_t batch) {
+    const uint64_t left = last > done ? last - done : batch;
+    const uint64_t up = (left + kHeadStep - 1) / kHeadStep * kHeadStep;
+    return (uint32_t)(up < kMaxHeadSlots ? up : kMaxHeadSlots);
 }
 
 // 256 bytes of device memory for a device-driven loop's control block.
@@ -288,13 +296,15 @@ struct medusa_graph {
     medusa::HBuf<unsigned long long> h_ctr_raw;
     // device-driven superstep loops: control blocks and captured superstep batches
     medusa::DBuf<medusa::CtlStorage> bfs_ctl, mbfs_ctl, sssp_ctl;
-    medusa::GraphCache bfs_graph, mbfs_graph;
-    medusa::GraphCache sssp_heads[medusa::kMaxHeadSlots / 4 + 1];  // by slot count / 4
+    medusa::GraphCache bfs_graph;
+    // by slot count / kHeadStep
+    medusa::GraphCache sssp_heads[medusa::kMaxHeadSlots / medusa::kHeadStep + 1];
+    medusa::GraphCache mbfs_heads[medusa::kMaxHeadSlots / medusa::kHeadStep + 1];
     // first replay of the BFS / MBFS loops: as many slots as the previous run on this handle
     // used, so a repeated traversal ends after one replay with no idle slots (BFS: one graph per
     // slot count, so runs of different lengths do not capture again)
-    medusa::GraphCache bfs_heads[medusa::kMaxHeadSlots + 1], mbfs_head;
-    uint32_t bfs_next_head = medusa::kNoHead, mbfs_last_steps = 0, sssp_last_slots = 0;
+    medusa::GraphCache bfs_heads[medusa::kMaxHeadSlots + 1];
+    uint32_t bfs_next_head = medusa::kNoHead, mbfs_last_slots = 0, sssp_last_slots = 0;
     // pinned: parameters of a BFS run and its control block afterwards; levels on their way to a
     // small host output
     medusa::HBuf<unsigned long long> h_bfs;
@@ -339,7 +349,6 @@ bool build_pr_bins(medusa_graph* g, bool required);
 uint32_t pr_send_tile_slots(const medusa_graph* g, uint32_t nblk);
 // Binned-combine workgroups that run at once on g's device.
 uint32_t pr_combine_slots(const medusa_graph* g);
-void build_pull_layout(medusa_graph* g);
 // 8-byte words of the pinned memory that BFS runs use (bfs.hip).
 size_t bfs_host_words();
 

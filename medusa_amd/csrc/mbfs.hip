@@ -5,27 +5,29 @@
 // (HowToBuild:13); the semantics here are those of k independent BFS runs
 // (Algorithm/UserOperators.h:17-36 per source), checked against exactly that.
 //
-// Superstep:
-//   push: active vertices (frontier mask != 0) OR their mask into next[v] of every
-//         out-neighbour that still lacks some of those bits (64-bit atomicOr); vertices
-//         up to `large` out-degree go through the wave-cooperative queue, hubs above it
-//         are split over whole workgroups (the threshold is autotunable);
-//   pull: every vertex not yet visited by all sources ORs the frontier masks of its
-//         in-neighbours, stopping early once every missing bit has been found; vertices are
-//         visited in in-degree order over ELL slabs of source ids (the pull layout), so the
-//         index loads are coalesced;
-//   update: new = next & ~visited; visited |= new; frontier = new; the level of the new bits goes
-//         into bit planes (plane p holds bit p of every (vertex, source) level); the two active
-//         queues and the counters are rebuilt with ballot + in-workgroup prefix scan;
-//   finish: once, after the last superstep: the planes as one level byte per (source, vertex).
+// Superstep, over vertices in the pull layout's internal order:
+//   push:   active vertices (frontier mask != 0) OR their mask into next[v] of every
+//           out-neighbour that still lacks some of those bits (64-bit atomicOr); vertices
+//           up to `large` out-degree go through the wave-cooperative queue, hubs above it
+//           are split over whole workgroups (the threshold is autotunable);
+//   update: after a push: new = next & ~visited, and the queues of the next push, with ballot
+//           + in-workgroup prefix scan;
+//   pull:   every vertex not yet visited by all sources ORs the frontier masks of its
+//           in-neighbours, stopping early once every missing bit has been found, and takes its
+//           own new bits in the same pass;
+//   queue:  after a pull, before a push: the queues from the frontier masks.
+// New bits: visited |= new; frontier = new (in the other of two frontier arrays); the level goes
+// into bit planes (plane p holds bit p of every (vertex, source) level).  After the last superstep the
+// finish turns the planes into one level byte per (source, vertex) in the original order.
 //
-// Drivers as for BFS: device-driven (the last workgroup of each update writes the next superstep
-// into a control block; batches of supersteps are captured as hipGraphs and replayed until done,
-// the first batch sized by the previous run on the handle, and each ends with the finish, which
-// returns at once unless the run is done) and host-driven (timing or tracing) over the same kernels.
+// Drivers as for BFS: device-driven (the last workgroup of each update or pull writes the
+// next superstep into a control block; batches of launches, each doing what the control block says,
+// are captured as hipGraphs and replayed until done, sized by the previous run on the handle, and
+// each ends with the finish, which returns at once unless the run is done) and host-driven (timing or tracing) over the same kernels.
 
 #include <algorithm>
-#include <cstring>
+#include <cstddef>
+#include <vector>
 
 #include "engine.h"
 #include "sched.h"
@@ -34,51 +36,204 @@ namespace medusa {
 
 constexpr uint32_t kMbfsLargeDefault = 1024;
 constexpr uint32_t kMbfsGridDefault = 2048;
-constexpr uint32_t kMbfsBatch = 8;
+constexpr uint32_t kMbfsBatch = 16;  // launches of a replay without a previous run
 constexpr uint32_t kMbfsSplit = 8;  // minimum workgroup items per hub
 
 constexpr uint32_t kMbfsProbeLines = 8;
 
-// Sums of an update, on lines of their own.
-enum { kMbfsActive, kMbfsActiveDeg, kMbfsNewBits, kMbfsReachedEdges, kMbfsLargeDeg, kMbfsSums };
+// Counters of a launch, spread over kMbfsSegs lines by workgroup: same-address atomics serialise.
+constexpr uint32_t kMbfsSegs = 32;
+// active vertices, their out-degrees, those of the hubs among them (above `large`), queue entries and
+// hubs (low and high word), in-edges examined, new (source, vertex) pairs, the pairs' out-degrees
+enum { kMbfsActive, kMbfsActiveDeg, kMbfsLargeDeg, kMbfsQueued, kMbfsProbes, kMbfsNewBits, kMbfsReachedEdges, kMbfsSums };
 struct MbfsLine {
-    alignas(128) unsigned long long v;
+    alignas(128) uint32_t v;
 };
 struct MbfsCounters {
-    MDS_COUNTER(uint32_t, n_small);   // active vertices with 1 <= outdeg <= large
-    MDS_COUNTER(uint32_t, n_large);   // active vertices with outdeg > large
-    MDS_COUNTER(uint32_t, ticket);    // workgroups of the update that are done
-    MbfsLine sum[kMbfsSums];
-    MbfsLine probes[kMbfsProbeLines];  // in-edges examined, by workgroup number
+    struct {
+        alignas(128) unsigned long long v[kMbfsSums];
+    } sum[kMbfsSegs];
+    MbfsLine queued[2][kMbfsSegs];  // queue entries per segment, by superstep parity
+    MbfsLine hubs[2];
+    MbfsLine sub[kMbfsSegs], top;   // tickets
 };
 
+enum : uint32_t { kMbfsPush, kMbfsUpdate, kMbfsPull, kMbfsQueue };
 struct MbfsCtl {
     int32_t step;
-    uint32_t pull, done, n_small, n_large, hub_wgs, mode, saturated;
-    uint32_t supersteps, push_steps, pull_steps, k;
+    uint32_t phase, pull, done, n_large, hub_wgs, mode, saturated;
+    uint32_t supersteps, push_steps, pull_steps, k, slots, pad;
     unsigned long long n, m, n_f, m_f, n_u, m_u, reached, reached_edges, kernel_bytes, alg_bytes, full;
     uint8_t* out;  // where the finish of a device-driven run writes the levels, or null
 };
 
 struct MbfsArgs {
-    const uint32_t *row_ptr, *col, *cptr, *csrc;
+    const uint32_t *col, *pos;
+    const uint2* out;        // first out-edge, out-degree
+    const uint8_t* indeg;
+    const uint64_t* base;
+    const uint4* hub;
+    const uint32_t* src;
     uint32_t *q_small, *q_large;
-    unsigned long long *visited, *frontier, *next;
-    const PrRun* runs;
-    const uint32_t *wg_run, *perm, *ell;
+    unsigned long long *visited, *next, *frontier[2];  // frontier of superstep t: [t % 2]
     MbfsCounters* ctr;
-    MbfsCtl* ctl;
+    MbfsCtl* ctl;  // two: a launch reads one and writes the other
     const float* policy;
     void* planes;  // kMbfsPlanes of n words each, of the width that holds k bits
-    uint32_t n, large, items, grid;
+    uint32_t n, large, nslices, nhubs, grid, span;
 };
 constexpr uint32_t kMbfsPlanes = 8;
+constexpr uint32_t kMbfsTile = 1024;  // vertices of a workgroup's round of an update or queue pass
+
+// Queue segment span for n vertices: kMbfsSegs segments cover [0, n) in whole tiles.
+static uint32_t mbfs_span(uint32_t n) {
+    const uint64_t tiles = ((uint64_t)n + kMbfsTile - 1) / kMbfsTile;
+    return (uint32_t)((tiles + kMbfsSegs - 1) / kMbfsSegs * kMbfsTile);
+}
+
+// ---- layout ---------------------------------------------------------------------------
+
+// One workgroup per window: its vertices by in-degree, hubs first.  The order of vertices of one
+// degree is whatever the LDS counters give: it changes no result.
+__global__ __launch_bounds__(1024) void k_pull_sort(uint32_t n, const uint32_t* __restrict__ cptr,
+                                                    const uint32_t* __restrict__ row_ptr, uint32_t* __restrict__ perm,
+                                                    uint32_t* __restrict__ pos, uint2* __restrict__ out,
+                                                    uint8_t* __restrict__ indeg, uint32_t* __restrict__ hub_count) {
+    __shared__ uint32_t cnt[kWave + 2], first[kWave + 2];
+    static_assert(kPullLaneMax == kWave, "one wave scans the degrees' counts");
+    const uint32_t t = threadIdx.x;
+    const uint64_t w0 = (uint64_t)blockIdx.x * kPullWindow;
+    if (t < kWave + 2) cnt[t] = 0;
+    __syncthreads();
+    uint32_t deg[4], key[4], at[4];
+#pragma unroll
+    for (uint32_t j = 0; j < 4; ++j) {
+        const uint64_t v = w0 + j * 1024 + t;
+        if (v >= n) continue;
+        deg[j] = cptr[v + 1] - cptr[v];
+        key[j] = deg[j] > kPullLaneMax ? 0u : 1u + kPullLaneMax - deg[j];
+        at[j] = atomicAdd(&cnt[key[j]], 1u);
+    }
+    __syncthreads();
+    if (t < kWave) {
+        const uint32_t c = cnt[t], incl = wave_incl_scan(c);
+        first[t] = incl - c;
+        if (t == kWave - 1) {
+            first[kWave] = incl;
+            first[kWave + 1] = incl + cnt[kWave];
+        }
+    }
+    __syncthreads();
+    if (t == 0 && cnt[0]) atomicAdd(hub_count, cnt[0]);
+#pragma unroll
+    for (uint32_t j = 0; j < 4; ++j) {
+        const uint64_t v = w0 + j * 1024 + t;
+        if (v >= n) continue;
+        const uint32_t p = (uint32_t)w0 + first[key[j]] + at[j];
+        perm[p] = (uint32_t)v;
+        pos[v] = p;
+        out[p] = uint2{row_ptr[v], row_ptr[v + 1] - row_ptr[v]};
+        indeg[p] = deg[j] > kPullLaneMax ? kPullHub : (uint8_t)deg[j];
+    }
+}
+
+// The columns of every slice and the in-edges of every hub; one wave per slice or hub.
+__global__ __launch_bounds__(256) void k_pull_fill(uint32_t n, uint32_t nslices, uint32_t nhubs,
+                                                   const uint32_t* __restrict__ cptr, const uint32_t* __restrict__ csrc,
+                                                   const uint32_t* __restrict__ perm, const uint32_t* __restrict__ pos,
+                                                   const uint8_t* __restrict__ indeg, const uint64_t* __restrict__ base,
+                                                   const uint4* __restrict__ hub, uint32_t* __restrict__ src) {
+    const uint32_t lane = threadIdx.x & (kWave - 1);
+    const uint64_t nw = (uint64_t)gridDim.x * 4, total = (uint64_t)nslices + nhubs;
+    for (uint64_t s = (uint64_t)blockIdx.x * 4 + threadIdx.x / kWave; s < total; s += nw) {  // uniform per wave
+        if (s >= nslices) {
+            const uint4 h = hub[s - nslices];
+            const uint32_t b = cptr[perm[h.x]];
+            uint32_t* to = src + (((uint64_t)h.w << 32) | h.z);
+            for (uint32_t k = lane; k < h.y; k += kWave) to[k] = pos[csrc[b + k]];
+            continue;
+        }
+        const uint64_t b = base[s], len = (base[s + 1] - b) / kWave, p = s * kWave + lane;
+        const uint32_t d = p < n && indeg[p] != kPullHub ? indeg[p] : 0u;
+        const uint32_t e = d ? cptr[perm[p]] : 0u;
+        for (uint64_t k = 0; k < len; ++k) src[b + k * kWave + lane] = k < d ? pos[csrc[e + k]] : 0u;
+    }
+}
+
+// Sorted and filled on the GPU (RMAT-20: 1.5 ms; on the host, with the sort over all vertices and an
+// upload of every slab, 130 ms); the host sums the slices' and hubs' lengths.
+static void build_pull_layout(medusa_graph* g) {
+    if (g->pull) return;
+    const uint32_t n = g->n;
+    hipStream_t s = g->stream;
+    auto L = std::make_unique<PullLayout>();
+    const uint32_t windows = (uint32_t)(((uint64_t)n + kPullWindow - 1) / kPullWindow);
+    L->nslices = (uint32_t)(((uint64_t)n + kWave - 1) / kWave);
+    L->pos.alloc(n);
+    L->out.alloc(n);
+    L->indeg.alloc(n);
+    DBuf<uint32_t> perm, count;
+    perm.alloc(n);
+    count.alloc(1);
+    const uint32_t zero = 0;
+    MDS_HIP(hipMemcpyAsync(count.p, &zero, 4, hipMemcpyHostToDevice, s));
+    hipLaunchKernelGGL(k_pull_sort, dim3(windows), dim3(1024), 0, s, n, g->cptr.p, g->row_ptr.p, perm.p, L->pos.p,
+                       L->out.p, L->indeg.p, count.p);
+    MDS_LAUNCHED();
+    std::vector<uint8_t> indeg(n);
+    std::vector<uint32_t> order;
+    MDS_HIP(hipMemcpyAsync(indeg.data(), L->indeg.p, n, hipMemcpyDeviceToHost, s));
+    MDS_HIP(hipMemcpyAsync(&L->nhubs, count.p, 4, hipMemcpyDeviceToHost, s));
+    MDS_HIP(hipStreamSynchronize(s));
+    if (L->nhubs) {
+        order.resize(n);
+        MDS_HIP(hipMemcpyAsync(order.data(), perm.p, (size_t)n * 4, hipMemcpyDeviceToHost, s));
+        MDS_HIP(hipStreamSynchronize(s));
+    }
+    // a slice is as long as its longest in-edge list that is not a hub's: in a window sorted by
+    // in-degree, its first one's
+    std::vector<uint64_t> base((size_t)L->nslices + 1);
+    uint64_t at = 0;
+    for (uint32_t i = 0; i < L->nslices; ++i) {
+        base[i] = at;
+        const uint64_t p1 = std::min<uint64_t>(n, (uint64_t)(i + 1) * kWave);
+        for (uint64_t p = (uint64_t)i * kWave; p < p1; ++p)
+            if (indeg[p] != kPullHub) {
+                at += (uint64_t)indeg[p] * kWave;
+                break;
+            }
+    }
+    base[L->nslices] = at;
+    std::vector<uint4> hub;
+    hub.reserve(L->nhubs);
+    if (L->nhubs)
+        for (uint32_t p = 0; p < n; ++p)
+            if (indeg[p] == kPullHub) {
+                const uint32_t v = order[p], d = g->h_cptr[v + 1] - g->h_cptr[v];
+                hub.push_back(uint4{p, d, (uint32_t)at, (uint32_t)(at >> 32)});
+                at += d;
+            }
+    MDS_CHECK(hub.size() == L->nhubs, MEDUSA_ERR_INTERNAL, "mbfs: hub count");
+    // longest first: a wave that starts one late would end the launch late
+    std::sort(hub.begin(), hub.end(), [](const uint4& a, const uint4& b) { return a.y != b.y ? a.y > b.y : a.x < b.x; });
+    L->base.upload(base.data(), base.size(), s);
+    if (L->nhubs) L->hub.upload(hub.data(), hub.size(), s);
+    L->src.alloc(std::max<uint64_t>(at, 1));
+    hipLaunchKernelGGL(k_pull_fill, dim3(grid_for((uint64_t)L->nslices + L->nhubs, 4, 8192)), dim3(256), 0, s, n,
+                       L->nslices, L->nhubs, g->cptr.p, g->csrc.p, (const uint32_t*)perm.p, (const uint32_t*)L->pos.p,
+                       (const uint8_t*)L->indeg.p, (const uint64_t*)L->base.p, (const uint4*)L->hub.p, L->src.p);
+    MDS_LAUNCHED();
+    MDS_HIP(hipStreamSynchronize(s));
+    g->pull = std::move(L);
+}
+
+// ---- start ----------------------------------------------------------------------------
 
 // Masks cleared, counters and control block set up.
 __global__ __launch_bounds__(256) void k_mbfs_fill(MbfsArgs a, unsigned long long m, uint32_t k, uint32_t mode,
                                                    uint8_t* out) {
     const uint64_t tid = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x, stride = (uint64_t)gridDim.x * blockDim.x;
-    // visited, frontier and next follow each other
+    // visited, next and frontier 0 follow each other; frontier 1 is written whole before it is read
     for (uint64_t i = tid; i < 3ull * a.n; i += stride) a.visited[i] = 0;
     if (blockIdx.x != 0) return;
     for (uint32_t i = threadIdx.x; i < sizeof(MbfsCounters) / 8; i += blockDim.x)
@@ -93,7 +248,7 @@ __global__ __launch_bounds__(256) void k_mbfs_fill(MbfsArgs a, unsigned long lon
         z.m_u = m * k;
         z.full = k == 64 ? ~0ull : ((1ull << k) - 1);
         z.out = out;
-        *a.ctl = z;
+        a.ctl[0] = z;
     }
 }
 
@@ -110,176 +265,354 @@ __host__ __device__ inline uint32_t mbfs_hub_wgs(uint32_t grid, uint32_t n_small
 
 // ---- superstep bodies ---------------------------------------------------------------
 
+struct MbfsPushLds {
+    uint32_t beg[4][kWave], off[4][kWave];
+    unsigned long long mask[4][kWave];
+    uint32_t pre[kMbfsSegs + 1];
+};
+
+__device__ __forceinline__ void mbfs_offer(const MbfsArgs& a, uint32_t e, unsigned long long mask) {
+    const uint32_t v = a.pos[a.col[e]];
+    const unsigned long long add = mask & ~a.visited[v];
+    if (add && (a.next[v] & add) != add) atomicOr(&a.next[v], add);
+}
+
 // Wave-cooperative push; wave w of the nwaves taking part holds queue entries
-// w, w + nwaves, ... one per lane.
-__device__ __forceinline__ void mbfs_push_small(const uint32_t* __restrict__ q, uint32_t qn,
-                                                const uint32_t* __restrict__ row_ptr, const uint32_t* __restrict__ col,
-                                                const unsigned long long* __restrict__ frontier,
-                                                const unsigned long long* __restrict__ visited,
-                                                unsigned long long* __restrict__ next, uint32_t wave0, uint32_t nwaves) {
-    __shared__ uint32_t s_beg[4][kWave], s_off[4][kWave];
-    __shared__ unsigned long long s_mask[4][kWave];
+// w, w + nwaves, ... one per lane.  Entries [pre[s], pre[s + 1]) of the queue lie in segment s.
+__device__ __forceinline__ void mbfs_push_small(const MbfsArgs& a, const MbfsLine* __restrict__ queued,
+                                                const unsigned long long* __restrict__ frontier, uint32_t wave0,
+                                                uint32_t nwaves, MbfsPushLds& L) {
     const uint32_t lane = threadIdx.x & (kWave - 1), wv = threadIdx.x / kWave;
+    if (wv == 0) {
+        const uint32_t incl = wave_incl_scan(lane < kMbfsSegs ? queued[lane].v : 0u);
+        if (lane < kMbfsSegs) L.pre[lane + 1] = incl;
+        if (lane == 0) L.pre[0] = 0;
+    }
+    __syncthreads();
+    const uint32_t qn = L.pre[kMbfsSegs];
     for (uint64_t r = 0; wave0 + r * kWave * nwaves < qn; ++r) {  // uniform across the wave
         const uint64_t i = wave0 + (r * kWave + lane) * nwaves;
-        uint32_t beg = 0, deg = 0;
+        uint2 edges{0, 0};
         unsigned long long fm = 0;
         if (i < qn) {
-            const uint32_t u = q[i];
-            beg = row_ptr[u];
-            deg = row_ptr[u + 1] - beg;
+            uint32_t sg = 0;
+#pragma unroll
+            for (uint32_t step = kMbfsSegs / 2; step; step >>= 1)
+                if (L.pre[sg + step] <= i) sg += step;
+            const uint32_t u = a.q_small[(size_t)sg * a.span + (uint32_t)(i - L.pre[sg])];
+            edges = a.out[u];
             fm = frontier[u];
         }
-        const uint32_t incl = wave_incl_scan(deg);
-        const uint32_t total = __shfl(incl, kWave - 1, kWave);
-        s_beg[wv][lane] = beg;
-        s_off[wv][lane] = incl - deg;
-        s_mask[wv][lane] = fm;
-        __builtin_amdgcn_wave_barrier();
+        const uint32_t incl = wave_incl_scan(edges.y);
+        const uint32_t total = __builtin_amdgcn_readlane(incl, kWave - 1);
+        L.beg[wv][lane] = edges.x;
+        L.off[wv][lane] = incl - edges.y;
+        L.mask[wv][lane] = fm;
+        wave_lds_fence();
         for (uint32_t e = lane; e < total; e += kWave) {
             uint32_t lo = 0;
 #pragma unroll
             for (uint32_t step = kWave / 2; step; step >>= 1)
-                if (s_off[wv][lo + step] <= e) lo += step;
-            const uint32_t v = col[s_beg[wv][lo] + (e - s_off[wv][lo])];
-            const unsigned long long add = s_mask[wv][lo] & ~visited[v];
-            if (add && (next[v] & add) != add) atomicOr(&next[v], add);
+                if (L.off[wv][lo + step] <= e) lo += step;
+            mbfs_offer(a, L.beg[wv][lo] + (e - L.off[wv][lo]), L.mask[wv][lo]);
         }
-        __builtin_amdgcn_wave_barrier();
+        wave_lds_fence();
     }
 }
 
 // Hubs: each queue vertex split into `split` edge ranges, one per workgroup item.
-__device__ __forceinline__ void mbfs_push_large(const uint32_t* __restrict__ q, uint32_t qn,
-                                                const uint32_t* __restrict__ row_ptr, const uint32_t* __restrict__ col,
-                                                const unsigned long long* __restrict__ frontier,
-                                                const unsigned long long* __restrict__ visited,
-                                                unsigned long long* __restrict__ next, uint32_t wg0, uint32_t nwg) {
+__device__ __forceinline__ void mbfs_push_large(const MbfsArgs& a, uint32_t qn,
+                                                const unsigned long long* __restrict__ frontier, uint32_t wg0,
+                                                uint32_t nwg) {
     uint32_t split = nwg / qn;
     split = split < kMbfsSplit ? kMbfsSplit : (split > 4096u ? 4096u : split);
     for (uint64_t w = wg0; w < (uint64_t)qn * split; w += nwg) {
-        const uint32_t u = q[w / split], part = (uint32_t)(w % split);
-        const uint32_t b = row_ptr[u], deg = row_ptr[u + 1] - b;
+        const uint32_t u = a.q_large[w / split], part = (uint32_t)(w % split);
+        const uint2 edges = a.out[u];
         const unsigned long long fm = frontier[u];
-        const uint32_t per = (deg + split - 1) / split;
-        const uint32_t lo = b + min(deg, part * per), hi = b + min(deg, (part + 1) * per);
-        for (uint32_t k = lo + threadIdx.x; k < hi; k += blockDim.x) {
-            const uint32_t v = col[k];
-            const unsigned long long add = fm & ~visited[v];
-            if (add && (next[v] & add) != add) atomicOr(&next[v], add);
+        const uint32_t per = (edges.y + split - 1) / split;
+        const uint32_t lo = edges.x + min(edges.y, part * per), hi = edges.x + min(edges.y, (part + 1) * per);
+        for (uint32_t k = lo + threadIdx.x; k < hi; k += blockDim.x) mbfs_offer(a, k, fm);
+    }
+}
+
+// A thread's share of a launch's sums.  Out-degrees and in-edges of distinct vertices add up to at
+// most m, below 2^32.
+struct MbfsAcc {
+    uint32_t active = 0, deg = 0, large_deg = 0, small = 0, large = 0, probes = 0;
+    unsigned long long bits = 0, edges = 0;
+    __device__ __forceinline__ void add(const MbfsArgs& a, unsigned long long nx, uint32_t d) {
+        const uint32_t b = (uint32_t)__popcll(nx);
+        active += 1;
+        deg += d;
+        bits += b;
+        edges += (unsigned long long)b * d;
+        if (d > a.large) {
+            large += 1;
+            large_deg += d;
+        } else if (d) {
+            small += 1;
         }
     }
+};
+
+// The new bits of vertex p (every p < n that the caller owns, with nx = 0 if none) at level lv.
+template <class T>
+__device__ __forceinline__ void mbfs_set_level(const MbfsArgs& a, uint32_t lv, uint32_t p, unsigned long long nx) {
+    T* plane = static_cast<T*>(a.planes) + p;
+    if (!(lv & (lv - 1))) {  // a plane's first use: every word written, none read
+        plane[(size_t)__builtin_ctz(lv) * a.n] = (T)nx;
+        return;
+    }
+    if (!nx) return;
+    for (uint32_t b = 0; b < kMbfsPlanes; ++b)  // uniform
+        if ((lv >> b) & 1u) plane[(size_t)b * a.n] |= (T)nx;
 }
 
 constexpr uint32_t kMbfsPullGroup = 4;  // in-edges a lane probes per round
 
-// Bottom-up over the pull layout: a vertex missing some sources ORs its in-neighbours'
-// frontier masks until every missing bit is found.  Work item w of the layout is 256
-// lane-vertices of one equal-in-degree run (their k-th sources are one coalesced ELL load;
-// kMbfsPullGroup in-edges per round, loads issued together, merged one by one with the same
-// early exit and probe count as a plain loop) or 4 wave-vertices of in-degree > 64 (the wave
-// scans 64 in-edges per step and ORs them by shuffles).  Workgroups stride over the items.
-// `probes` counts in-edges examined up to and including the last one needed.
-__device__ __forceinline__ void mbfs_pull_ell(unsigned long long full, const PrRun* __restrict__ runs,
-                                              const uint32_t* __restrict__ wg_run, uint32_t items,
-                                              const uint32_t* __restrict__ perm, const uint32_t* __restrict__ ell,
-                                              const uint32_t* __restrict__ cptr, const uint32_t* __restrict__ csrc,
-                                              const unsigned long long* __restrict__ frontier,
-                                              const unsigned long long* __restrict__ visited,
-                                              unsigned long long* __restrict__ next, MbfsCounters* __restrict__ ctr) {
-    const uint32_t lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
-    unsigned long long probes = 0;
-    for (uint32_t w = blockIdx.x; w < items; w += gridDim.x) {  // uniform per block
-        const PrRun R = runs[wg_run[w]];
-        const uint32_t local = w - R.wg_begin;
-        if (R.kind == kPrWave) {
-            const uint32_t p = R.begin + local * 4 + wave;
-            if (p >= R.begin + R.count) continue;  // uniform across the wave
-            const uint32_t v = perm[p];
-            const unsigned long long vis = visited[v];
-            if (vis == full) continue;
-            const uint32_t vb = cptr[v], ve = cptr[v + 1];
-            unsigned long long acc = 0;
-            for (uint32_t k0 = vb; k0 < ve; k0 += kWave) {
-                const uint32_t k = k0 + lane;
-                unsigned long long x = k < ve ? frontier[csrc[k]] : 0ull;
+__device__ __forceinline__ uint32_t wave_or(uint32_t x) {
+    x |= dpp_or_zero<0x111>(x);
+    x |= dpp_or_zero<0x112>(x);
+    x |= dpp_or_zero<0x114>(x);
+    x |= dpp_or_zero<0x118>(x);
+    x |= dpp_or_zero<0x142, 0xa>(x);
+    x |= dpp_or_zero<0x143, 0xc>(x);
+    return (uint32_t)__builtin_amdgcn_readlane((int)x, kWave - 1);
+}
+__device__ __forceinline__ unsigned long long wave_or(unsigned long long x) {
+    return ((unsigned long long)wave_or((uint32_t)(x >> 32)) << 32) | wave_or((uint32_t)x);
+}
+
+// Bottom-up: a vertex missing some sources ORs its in-neighbours' frontier masks until every missing
+// bit is found, then takes the new bits: masks, level and sums, in the same pass.  A wave takes a
+// slice (a vertex per lane; the k-th sources of 64 vertices are one load, kMbfsPullGroup in-edges per
+// round, loads issued together, merged one by one with the same early exit and probe count as a plain
+// loop) or a hub (64 in-edges per step, four steps' loads together).  Bound by the gather of
+// 8-byte masks: in RMAT-20's full sweeps (17 M in-edges, 64 sources, 142 us) 35 % of 17 M requests
+// miss the L2s, 770 MB of lines from the memory-side cache.  Eight in-edges per round, nontemporal
+// loads of the sources and half as many registers changed nothing or lost.  In the original order over
+// slabs sorted across all vertices the sweep took as long and an update of 20..24 us followed.  `probes` counts in-edges examined up to and including the last
+// one needed (a hub's in steps of 64).
+template <class T>
+__device__ __forceinline__ void mbfs_pull(const MbfsArgs& a, unsigned long long full, uint32_t lv,
+                                          const unsigned long long* __restrict__ frontier,
+                                          unsigned long long* __restrict__ nxt, MbfsAcc& acc) {
+    const uint32_t lane = threadIdx.x & (kWave - 1);
+    const uint32_t nw = gridDim.x * 4, w = blockIdx.x * 4 + threadIdx.x / kWave;
+    for (uint32_t h = w; h < a.nhubs; h += nw) {  // uniform across the wave
+        const uint4 H = a.hub[h];
+        const uint32_t p = H.x, deg = H.y;
+        const uint32_t* src = a.src + (((uint64_t)H.w << 32) | H.z);
+        const unsigned long long vis = a.visited[p];
+        unsigned long long found = 0;
+        uint32_t probes = 0;
+        bool all = vis == full;
+        for (uint32_t k0 = 0; k0 < deg && !all; k0 += 4 * kWave) {
+            uint32_t u[4];
+            unsigned long long f[4];
 #pragma unroll
-                for (int off = kWave / 2; off >= 1; off >>= 1) x |= __shfl_xor(x, off, kWave);
-                acc |= x;
-                if (lane == 0) probes += min(ve - k0, (uint32_t)kWave);
-                if ((acc | vis) == full) break;
+            for (uint32_t j = 0; j < 4; ++j) {
+                const uint32_t k = k0 + j * kWave + lane;
+                u[j] = k < deg ? src[k] : 0u;
             }
-            acc &= ~vis;
-            if (lane == 0 && acc) next[v] = acc;
-            continue;
+#pragma unroll
+            for (uint32_t j = 0; j < 4; ++j) f[j] = k0 + j * kWave + lane < deg ? frontier[u[j]] : 0ull;
+#pragma unroll
+            for (uint32_t j = 0; j < 4; ++j) {
+                if (all || k0 + j * kWave >= deg) continue;
+                found |= wave_or(f[j]);
+                probes += min(deg - k0 - j * kWave, (uint32_t)kWave);
+                all = (found | vis) == full;
+            }
         }
-        const uint32_t i = local * 256 + threadIdx.x;
-        if (i >= R.count) continue;
-        const uint32_t v = perm[R.begin + i];
-        const unsigned long long vis = visited[v];
-        if (vis == full) continue;
-        const uint32_t* col = ell + R.ell_base + i;
-        const uint32_t deg = R.deg, st = R.ell_stride;
-        unsigned long long acc = 0;
-        bool all = false;
+        const unsigned long long nx = found & ~vis;
+        if (lane == 0) {
+            acc.probes += probes;
+            nxt[p] = nx;
+            mbfs_set_level<T>(a, lv, p, nx);
+            if (nx) {
+                a.visited[p] = vis | nx;
+                acc.add(a, nx, a.out[p].y);
+            }
+        }
+    }
+    // slices are heavier towards a window's start: every second round is dealt the other way round
+    uint32_t r = 0;
+    for (uint64_t s0 = 0; s0 < a.nslices; s0 += nw, ++r) {
+        const uint64_t s = s0 + ((r & 1u) ? nw - 1 - w : w);
+        if (s >= a.nslices) continue;  // uniform across the wave
+        const uint32_t p = (uint32_t)(s * kWave) + lane;
+        const uint32_t ind = s * kWave + lane < a.n ? a.indeg[p] : kPullHub;
+        const bool mine = ind != kPullHub;  // hubs above
+        const unsigned long long vis = mine ? a.visited[p] : full;
+        const uint32_t deg = vis != full ? ind : 0u;
+        const uint32_t* src = a.src + a.base[s] + lane;
+        unsigned long long found = 0;
+        bool all = deg == 0;
+        uint32_t u[kMbfsPullGroup];
+#pragma unroll
+        for (uint32_t j = 0; j < kMbfsPullGroup; ++j) u[j] = j < deg ? src[j * kWave] : 0u;
         for (uint32_t k0 = 0; k0 < deg && !all; k0 += kMbfsPullGroup) {
-            uint32_t u[kMbfsPullGroup];
             unsigned long long f[kMbfsPullGroup];
 #pragma unroll
-            for (uint32_t j = 0; j < kMbfsPullGroup; ++j) u[j] = k0 + j < deg ? col[(size_t)(k0 + j) * st] : 0u;
-#pragma unroll
             for (uint32_t j = 0; j < kMbfsPullGroup; ++j) f[j] = k0 + j < deg ? frontier[u[j]] : 0ull;
+            // the next round's sources while the masks are on their way
+#pragma unroll
+            for (uint32_t j = 0; j < kMbfsPullGroup; ++j) {
+                const uint32_t k = k0 + kMbfsPullGroup + j;
+                u[j] = k < deg ? src[(size_t)k * kWave] : 0u;
+            }
 #pragma unroll
             for (uint32_t j = 0; j < kMbfsPullGroup; ++j) {
                 if (all || k0 + j >= deg) continue;
-                acc |= f[j];
-                ++probes;
-                all = (acc | vis) == full;
+                found |= f[j];
+                ++acc.probes;
+                all = (found | vis) == full;
             }
         }
-        acc &= ~vis;
-        if (acc) next[v] = acc;
-    }
-    // one atomic per workgroup (every wave of the block reaches this point)
-    __shared__ unsigned long long s_probe[4];
-    probes = wave_sum_u64(probes);
-    if (lane == 0) s_probe[threadIdx.x / kWave] = probes;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        const unsigned long long t = s_probe[0] + s_probe[1] + s_probe[2] + s_probe[3];
-        if (t) atomicAdd(&ctr->probes[blockIdx.x % kMbfsProbeLines].v, t);
+        if (mine) {
+            const unsigned long long nx = found & ~vis;
+            nxt[p] = nx;
+            mbfs_set_level<T>(a, lv, p, nx);
+            if (nx) {
+                a.visited[p] = vis | nx;
+                acc.add(a, nx, a.out[p].y);
+            }
+        }
     }
 }
 
-__global__ __launch_bounds__(256) void k_mbfs_expand(MbfsArgs a) {
-    const MbfsCtl* ctl = a.ctl;
-    if (ctl->done) return;
-    if (ctl->pull) {
-        mbfs_pull_ell(ctl->full, a.runs, a.wg_run, a.items, a.perm, a.ell, a.cptr, a.csrc, a.frontier, a.visited,
-                      a.next, a.ctr);
-        return;
+struct MbfsTileLds {
+    uint32_t sm[4], lg[4], base_sm, base_lg;
+};
+
+// The frontier that the next push reads, in tiles of kMbfsTile vertices: after a push (kUpdate) new =
+// next & ~visited with masks, level and sums, else the frontier as it is; its vertices with out-edges
+// appended to the queues.  Bound by its passes over the masks.
+template <class T, bool kUpdate>
+__device__ __forceinline__ void mbfs_tiles(const MbfsArgs& a, uint32_t lv, unsigned long long* __restrict__ nxt,
+                                           MbfsLine* __restrict__ queued, uint32_t* __restrict__ hubs, MbfsAcc& acc,
+                                           MbfsTileLds& L) {
+    const uint32_t n = a.n, lane = threadIdx.x & (kWave - 1), wv = threadIdx.x / kWave;
+    for (uint64_t base = (uint64_t)blockIdx.x * kMbfsTile; base < n; base += (uint64_t)gridDim.x * kMbfsTile) {
+        const uint64_t v0 = base + wv * 4 * kWave + lane;
+        unsigned long long nx[4];
+        uint32_t dg[4];
+        if constexpr (kUpdate) {
+            unsigned long long raw[4], vis[4];
+#pragma unroll
+            for (uint32_t c = 0; c < 4; ++c) raw[c] = v0 + c * kWave < n ? a.next[v0 + c * kWave] : 0ull;
+#pragma unroll
+            for (uint32_t c = 0; c < 4; ++c) vis[c] = raw[c] ? a.visited[v0 + c * kWave] : 0ull;
+#pragma unroll
+            for (uint32_t c = 0; c < 4; ++c) {
+                const uint64_t v = v0 + c * kWave;
+                nx[c] = raw[c] & ~vis[c];
+                if (raw[c]) a.next[v] = 0;
+                if (nx[c]) a.visited[v] = vis[c] | nx[c];
+                if (v < n) {
+                    nxt[v] = nx[c];
+                    mbfs_set_level<T>(a, lv, (uint32_t)v, nx[c]);
+                }
+            }
+        } else {
+#pragma unroll
+            for (uint32_t c = 0; c < 4; ++c) nx[c] = v0 + c * kWave < n ? nxt[v0 + c * kWave] : 0ull;
+        }
+#pragma unroll
+        for (uint32_t c = 0; c < 4; ++c) dg[c] = nx[c] ? a.out[v0 + c * kWave].y : 0u;
+        unsigned long long msm[4], mlg[4];
+        uint32_t csm = 0, clg = 0;
+#pragma unroll
+        for (uint32_t c = 0; c < 4; ++c) {
+            if (kUpdate && nx[c]) acc.add(a, nx[c], dg[c]);
+            msm[c] = __ballot(dg[c] > 0 && dg[c] <= a.large);
+            mlg[c] = __ballot(dg[c] > a.large);
+            csm += (uint32_t)__popcll(msm[c]);
+            clg += (uint32_t)__popcll(mlg[c]);
+        }
+        if (lane == 0) {
+            L.sm[wv] = csm;
+            L.lg[wv] = clg;
+        }
+        __syncthreads();
+        const uint32_t sg = (uint32_t)(base / a.span);
+        if (threadIdx.x == 0) {
+            const uint32_t tsm = L.sm[0] + L.sm[1] + L.sm[2] + L.sm[3], tlg = L.lg[0] + L.lg[1] + L.lg[2] + L.lg[3];
+            L.base_sm = tsm ? atomicAdd(&queued[sg].v, tsm) : 0u;
+            L.base_lg = tlg ? atomicAdd(hubs, tlg) : 0u;
+        }
+        __syncthreads();
+        uint32_t osm = L.base_sm, olg = L.base_lg;
+        for (uint32_t x = 0; x < wv; ++x) {
+            osm += L.sm[x];
+            olg += L.lg[x];
+        }
+        uint32_t* q = a.q_small + (size_t)sg * a.span;
+#pragma unroll
+        for (uint32_t c = 0; c < 4; ++c) {
+            const uint32_t v = (uint32_t)(v0 + c * kWave);
+            if ((msm[c] >> lane) & 1ull) q[osm + lanes_below(msm[c])] = v;
+            if ((mlg[c] >> lane) & 1ull) a.q_large[olg + lanes_below(mlg[c])] = v;
+            osm += (uint32_t)__popcll(msm[c]);
+            olg += (uint32_t)__popcll(mlg[c]);
+        }
+        __syncthreads();
     }
-    const uint32_t hub = ctl->hub_wgs;
-    if (blockIdx.x < hub) {
-        mbfs_push_large(a.q_large, ctl->n_large, a.row_ptr, a.col, a.frontier, a.visited, a.next, blockIdx.x, hub);
-        return;
+}
+
+// End of an update or pull: the workgroup's sums to its counter line and, with kDecide, its ticket
+// (two levels, so no address sees more than grid / kMbfsSegs atomics).  True in the first wave of
+// the workgroup that came last.
+template <bool kDecide>
+__device__ __forceinline__ bool mbfs_finish_launch(MbfsCounters* __restrict__ ctr, const MbfsAcc& acc) {
+    __shared__ unsigned long long s_sum[kMbfsSums];
+    const uint32_t lane = threadIdx.x & (kWave - 1);
+    if (threadIdx.x < kMbfsSums) s_sum[threadIdx.x] = 0;
+    __syncthreads();
+    auto total = [](uint32_t x) { return (uint32_t)__builtin_amdgcn_readlane((int)wave_incl_scan(x), kWave - 1); };
+    const uint32_t active = total(acc.active), probes = total(acc.probes);
+    if (active | probes) {  // uniform across the wave
+        const uint32_t deg = total(acc.deg), large_deg = total(acc.large_deg);
+        const uint32_t small = total(acc.small), large = total(acc.large);
+        const unsigned long long bits = wave_sum_u64(acc.bits), edges = wave_sum_u64(acc.edges);
+        if (lane == 0) {
+            atomicAdd(&s_sum[kMbfsActive], (unsigned long long)active);
+            atomicAdd(&s_sum[kMbfsActiveDeg], (unsigned long long)deg);
+            atomicAdd(&s_sum[kMbfsLargeDeg], (unsigned long long)large_deg);
+            atomicAdd(&s_sum[kMbfsQueued], ((unsigned long long)large << 32) | small);
+            atomicAdd(&s_sum[kMbfsProbes], (unsigned long long)probes);
+            atomicAdd(&s_sum[kMbfsNewBits], bits);
+            atomicAdd(&s_sum[kMbfsReachedEdges], edges);
+        }
     }
-    const uint32_t wg = blockIdx.x - hub, nwg = gridDim.x - hub;
-    mbfs_push_small(a.q_small, ctl->n_small, a.row_ptr, a.col, a.frontier, a.visited, a.next,
-                    wg * 4 + threadIdx.x / kWave, nwg * 4);
+    __syncthreads();
+    if (threadIdx.x >= kWave) return false;
+    const uint32_t sg = blockIdx.x % kMbfsSegs;
+    const unsigned long long sum = lane < kMbfsSums ? s_sum[lane] : 0ull;
+    if (sum) atomicAdd(&ctr->sum[sg].v[lane], sum);
+    if constexpr (!kDecide) return false;
+    // the workgroup's atomics (all by this wave or returned) have been performed before its ticket
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    uint32_t last = 0;
+    if (lane == 0) {
+        const uint32_t members = (gridDim.x - sg + kMbfsSegs - 1) / kMbfsSegs;  // workgroups of line sg
+        const uint32_t nsegs = gridDim.x < kMbfsSegs ? gridDim.x : kMbfsSegs;
+        if (atomicAdd(&ctr->sub[sg].v, 1u) == members - 1) last = atomicAdd(&ctr->top.v, 1u) == nsegs - 1;
+    }
+    return __builtin_amdgcn_readfirstlane((int)last) != 0;
 }
 
 // Direction of the next superstep, by one wave: fixed, learned, or the direction-optimising
 // heuristic.
-__device__ __forceinline__ bool mbfs_direction(const MbfsCtl& c, bool pull, const float* __restrict__ policy,
-                                               float* s_params) {
+__device__ __forceinline__ bool mbfs_direction(const MbfsCtl& c, const float* __restrict__ policy, float* s_params) {
     if (c.mode == 1) return false;
     if (c.mode == 2) return true;
-    const bool plain = !pull ? (double)c.m_f > (double)c.m_u / Sched::kAlphaMbfs
-                             : !((double)c.n_f < (double)c.n / Sched::kBeta);
+    const double alpha = Sched::kAlphaMbfs * c.k;
+    const bool plain = (double)c.m_f > (double)c.m_u / alpha;
     if (c.mode != 3 || !policy ||
-        !bfs_policy_consulted(pull, (double)c.n_f, (double)c.m_f, (double)c.m_u, (double)c.n, Sched::kAlphaMbfs,
-                              Sched::kBeta))
+        !bfs_policy_consulted(false, (double)c.n_f, (double)c.m_f, (double)c.m_u, (double)c.n, alpha, Sched::kBeta))
         return plain;
     const double rec[MEDUSA_TRACE_FIELDS] = {(double)c.step, (double)c.n_f, (double)c.m_f, (double)c.n_u,
                                              (double)c.m_u, (double)c.n, (double)c.m, 0.0, 0.0};
@@ -288,18 +621,23 @@ __device__ __forceinline__ bool mbfs_direction(const MbfsCtl& c, bool pull, cons
     return policy_pull(c_push, c_pull, plain);
 }
 
-// One wave, after every workgroup of an update (or the start, when `first`) has added its counters:
-// folds them into the control block, decides the next superstep and clears them.
-__device__ __forceinline__ void mbfs_decide(const MbfsArgs& a, bool first, float* s_params) {
+// One wave, after every workgroup of an update or pull (or the start, when `first`) has added its
+// counters: folds them into the control block, decides the next superstep and clears them.
+__device__ __forceinline__ void mbfs_decide(const MbfsArgs& a, bool first, uint32_t slot, float* s_params) {
     MbfsCounters* ctr = a.ctr;
     const uint32_t lane = threadIdx.x & (kWave - 1);
-    const uint32_t n_small = load_now(&ctr->n_small), n_large = load_now(&ctr->n_large);
-    unsigned long long sum[kMbfsSums];
+    unsigned long long line[kMbfsSums];
 #pragma unroll
-    for (int i = 0; i < kMbfsSums; ++i) sum[i] = load_now(&ctr->sum[i].v);
-    const unsigned long long probe = lane < kMbfsProbeLines ? load_now(&ctr->probes[lane].v) : 0ull;
-    MbfsCtl c = load_now_block(a.ctl);
-    const unsigned long long probes = wave_sum_u64(probe);
+    for (int i = 0; i < kMbfsSums; ++i) line[i] = lane < kMbfsSegs ? load_now(&ctr->sum[lane].v[i]) : 0ull;
+    MbfsCtl c = load_now_block(a.ctl + slot);
+    auto total = [](unsigned long long x) {
+        return (uint32_t)__builtin_amdgcn_readlane((int)wave_incl_scan((uint32_t)x), kWave - 1);
+    };
+    const uint32_t n_active = total(line[kMbfsActive]), active_deg = total(line[kMbfsActiveDeg]);
+    const uint32_t large_deg = total(line[kMbfsLargeDeg]), probes = total(line[kMbfsProbes]);
+    const uint32_t n_small = total(line[kMbfsQueued]), n_large = total(line[kMbfsQueued] >> 32);
+    const unsigned long long bits = wave_sum_u64(line[kMbfsNewBits]), edges = wave_sum_u64(line[kMbfsReachedEdges]);
+    const uint32_t par = (uint32_t)c.step & 1u;
     const unsigned long long n = c.n;
     if (!first) {
         // byte model of the superstep just finished: push = queue + offsets + mask per active
@@ -308,30 +646,37 @@ __device__ __forceinline__ void mbfs_decide(const MbfsArgs& a, bool first, float
         const unsigned long long kb = c.pull ? 4ull * (n + 1) + 8ull * n + 12ull * probes
                                              : 20ull * c.n_f + 20ull * c.m_f;
         c.kernel_bytes += kb;
-        c.alg_bytes += kb + 24ull * n + sum[kMbfsNewBits];
+        c.alg_bytes += kb + 24ull * n + bits;
         c.supersteps += 1;
         if (c.pull) c.pull_steps += 1; else c.push_steps += 1;
+        c.slots += c.pull ? 1u : 2u;
         c.step += 1;
     }
-    const unsigned long long n_active = sum[kMbfsActive];
     if (c.step >= 255 && n_active) c.saturated = 1;
-    c.reached += sum[kMbfsNewBits];
-    c.reached_edges += sum[kMbfsReachedEdges];
-    c.n_u -= sum[kMbfsNewBits];
-    c.m_u -= sum[kMbfsReachedEdges];
+    c.reached += bits;
+    c.reached_edges += edges;
+    c.n_u -= bits;
+    c.m_u -= edges;
     c.n_f = n_active;
-    c.m_f = sum[kMbfsActiveDeg];
-    c.n_small = n_small;
+    c.m_f = active_deg;
     c.n_large = n_large;
-    c.hub_wgs = mbfs_hub_wgs(a.grid, n_small, n_large, sum[kMbfsLargeDeg], c.m_f);
+    c.hub_wgs = mbfs_hub_wgs(a.grid, n_small, n_large, large_deg, active_deg);
     if (n_active == 0) c.done = 1;
-    c.pull = !c.done && mbfs_direction(c, first ? false : c.pull != 0, a.policy, s_params) ? 1u : 0u;
-    if (lane == 0) {
-        *a.ctl = c;
-        ctr->n_small = ctr->n_large = ctr->ticket = 0;
+    const bool queued = first || !c.pull;  // by the start or the update
+    c.pull = !c.done && mbfs_direction(c, a.policy, s_params) ? 1u : 0u;
+    c.phase = c.pull ? kMbfsPull : queued ? kMbfsPush : kMbfsQueue;
+    if (c.phase == kMbfsQueue && !c.done) c.slots += 1;
+    if (lane < kMbfsSegs) {
+#pragma unroll
+        for (int i = 0; i < kMbfsSums; ++i) ctr->sum[lane].v[i] = 0;
+        ctr->sub[lane].v = 0;
+        if (!first) ctr->queued[par][lane].v = 0;  // the queue of the superstep just finished
     }
-    if (lane < kMbfsSums) ctr->sum[lane].v = 0;
-    if (lane < kMbfsProbeLines) ctr->probes[lane].v = 0;
+    if (lane == 0) {
+        ctr->top.v = 0;
+        if (!first) ctr->hubs[par].v = 0;
+        a.ctl[first ? slot : slot ^ 1u] = c;
+    }
 }
 
 struct MbfsSources {
@@ -343,169 +688,74 @@ struct MbfsSources {
 __global__ __launch_bounds__(kWave) void k_mbfs_start(MbfsArgs a, MbfsSources src, uint32_t k, uint32_t decide) {
     __shared__ float s_params[kMlpWaveLds];
     const uint32_t lane = threadIdx.x;
-    const uint32_t v = lane < k ? src.v[lane] : 0xFFFFFFFFu;  // (vertices are below 2^32 - 1)
+    const uint32_t v = lane < k ? a.pos[src.v[lane]] : 0xFFFFFFFFu;  // (vertices are below 2^32 - 1)
     unsigned long long mask = 0;
     for (uint32_t j = 0; j < k; ++j)
-        if (v == (uint32_t)__builtin_amdgcn_readlane(v, j)) mask |= 1ull << j;
+        if (v == (uint32_t)__builtin_amdgcn_readlane((int)v, j)) mask |= 1ull << j;
     const bool one = lane < k && (uint32_t)__builtin_ctzll(mask) == lane;  // the first of its vertex
-    uint32_t deg = 0;
+    MbfsAcc acc;
     if (one) {
-        deg = a.row_ptr[v + 1] - a.row_ptr[v];
-        a.frontier[v] = mask;
+        const uint32_t deg = a.out[v].y;
+        a.frontier[0][v] = mask;
         a.visited[v] = mask;
+        acc.add(a, mask, deg);
     }
-    const bool large = deg > a.large, small = deg > 0 && !large;
-    const unsigned long long sm = __ballot(small), lm = __ballot(large);
-    if (small) a.q_small[lanes_below(sm)] = v;
-    if (large) a.q_large[lanes_below(lm)] = v;
-    const unsigned long long sum[kMbfsSums] = {(unsigned long long)__popcll(__ballot(one)), wave_sum_u64(deg), k,
-                                               wave_sum_u64((unsigned long long)__popcll(mask) * deg),
-                                               wave_sum_u64(large ? deg : 0u)};
+    const unsigned long long sm = __ballot(acc.small != 0), lm = __ballot(acc.large != 0);
+    if (acc.small) a.q_small[lanes_below(sm)] = v;  // segment 0
+    if (acc.large) a.q_large[lanes_below(lm)] = v;
     if (lane == 0) {
-        MbfsCounters* ctr = a.ctr;
-        __hip_atomic_store(&ctr->n_small, (uint32_t)__popcll(sm), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        __hip_atomic_store(&ctr->n_large, (uint32_t)__popcll(lm), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-#pragma unroll
-        for (int i = 0; i < kMbfsSums; ++i)
-            __hip_atomic_store(&ctr->sum[i].v, sum[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        a.ctr->queued[0][0].v = (uint32_t)__popcll(sm);
+        a.ctr->hubs[0].v = (uint32_t)__popcll(lm);
     }
+    mbfs_finish_launch<false>(a.ctr, acc);
     if (!decide) return;
-    __threadfence();
-    mbfs_decide(a, true, s_params);
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // its atomics have been performed
+    mbfs_decide(a, true, 0, s_params);
 }
 
-constexpr uint32_t kMbfsWg = 1024, kMbfsTile = 4 * kMbfsWg;  // vertices per workgroup tile (4 chunks per wave)
-
-// new = next & ~visited for every vertex: masks, level planes, the two active queues, counters.
-// kDecide: the last workgroup to add its counters decides the next superstep (one launch less per
-// superstep, 5 us).  Bound by its passes over next and frontier and the joins' plane words, and on
-// few vertices by the chain of atomics on each counter, hence workgroups of 1024 threads: 256 chains
-// of one add for 2^20 vertices.  Levels go into bit planes: as one byte store per joining (source,
-// vertex) with the wave's other lanes masked, this kernel took 36..46 us in the five supersteps of RMAT-20
-// with 64 sources that join most, and 20..24 with planes.
+// One launch of the superstep loop, doing what the control block says.
 template <class T, bool kDecide>
-__global__ __launch_bounds__(kMbfsWg) void k_mbfs_update(MbfsArgs a, int32_t level_fixed) {
-    constexpr uint32_t kWaves = kMbfsWg / kWave;
-    __shared__ uint32_t s_sm[kWaves], s_lg[kWaves], s_bsm[kWaves], s_blg[kWaves];
-    __shared__ unsigned long long s_sum[kMbfsSums];
-    __shared__ uint32_t s_last;
+__global__ __launch_bounds__(256, 8) void k_mbfs_super(MbfsArgs a, uint32_t slot) {
+    __shared__ MbfsPushLds s_push;
+    __shared__ MbfsTileLds s_tile;
     __shared__ float s_params[kDecide ? kMlpWaveLds : 4];
-    if (kDecide && a.ctl->done) return;
-    const int32_t level = kDecide ? a.ctl->step + 1 : level_fixed;
-    const uint32_t lv = level >= 255 ? 255u : (uint32_t)level;  // 255: saturated, reported as unreached
-    const uint32_t n = a.n, lane = threadIdx.x & (kWave - 1), wv = threadIdx.x / kWave;
-    T* planes = static_cast<T*>(a.planes);
-    if (threadIdx.x < kMbfsSums) s_sum[threadIdx.x] = 0;  // read behind the first tile's barriers
-    uint32_t cact = 0;
-    unsigned long long adeg = 0, bits = 0, redges = 0, dlg = 0;
-    for (uint64_t base = (uint64_t)blockIdx.x * kMbfsTile; base < n; base += (uint64_t)gridDim.x * kMbfsTile) {
-        const uint64_t v0 = base + wv * 4 * kWave + lane;
-        unsigned long long raw[4], fr[4], nx[4], vis[4];
-        uint32_t dg[4];
-#pragma unroll
-        for (uint32_t c = 0; c < 4; ++c) {
-            const uint64_t v = v0 + c * kWave;
-            raw[c] = v < n ? a.next[v] : 0ull;
-            fr[c] = v < n ? a.frontier[v] : 0ull;
-        }
-#pragma unroll
-        for (uint32_t c = 0; c < 4; ++c) vis[c] = raw[c] ? a.visited[v0 + c * kWave] : 0ull;
-#pragma unroll
-        for (uint32_t c = 0; c < 4; ++c) {
-            const uint64_t v = v0 + c * kWave;
-            nx[c] = raw[c] & ~vis[c];
-            dg[c] = nx[c] ? a.row_ptr[v + 1] - a.row_ptr[v] : 0u;
-        }
-#pragma unroll
-        for (uint32_t c = 0; c < 4; ++c) {
-            const uint64_t v = v0 + c * kWave;
-            if (raw[c]) a.next[v] = 0;
-            if (nx[c]) a.visited[v] = vis[c] | nx[c];
-            if (fr[c] != nx[c]) a.frontier[v] = nx[c];
-        }
-        for (uint32_t p = 0; p < kMbfsPlanes; ++p) {  // uniform
-            if (!((lv >> p) & 1u)) continue;
-            T* plane = planes + (size_t)p * n;
-            if (lv == 1u << p) {  // the plane's first use: every word written, none read
-#pragma unroll
-                for (uint32_t c = 0; c < 4; ++c)
-                    if (v0 + c * kWave < n) plane[v0 + c * kWave] = (T)nx[c];
-                continue;
-            }
-            T x[4];
-#pragma unroll
-            for (uint32_t c = 0; c < 4; ++c) x[c] = nx[c] ? plane[v0 + c * kWave] : (T)0;
-#pragma unroll
-            for (uint32_t c = 0; c < 4; ++c)
-                if (nx[c]) plane[v0 + c * kWave] = (T)(x[c] | (T)nx[c]);
-        }
-        unsigned long long msm[4], mlg[4];
-        uint32_t csm = 0, clg = 0;
-#pragma unroll
-        for (uint32_t c = 0; c < 4; ++c) {
-            const uint32_t deg = dg[c];
-            cact += (uint32_t)__popcll(__ballot(nx[c] != 0));
-            msm[c] = __ballot(deg > 0 && deg <= a.large);
-            mlg[c] = __ballot(deg > a.large);
-            csm += (uint32_t)__popcll(msm[c]);
-            clg += (uint32_t)__popcll(mlg[c]);
-            adeg += deg;
-            dlg += deg > a.large ? deg : 0u;
-            bits += __popcll(nx[c]);
-            redges += (unsigned long long)__popcll(nx[c]) * deg;
-        }
-        if (lane == 0) {
-            s_sm[wv] = csm;
-            s_lg[wv] = clg;
-        }
-        __syncthreads();
-        if (wv == 0) {
-            const uint32_t sm = lane < kWaves ? s_sm[lane] : 0u, lg = lane < kWaves ? s_lg[lane] : 0u;
-            const uint32_t ism = wave_incl_scan(sm), ilg = wave_incl_scan(lg);
-            uint32_t got = 0;
-            if (lane == kWave - 2 && ism) got = atomicAdd(&a.ctr->n_small, ism);
-            if (lane == kWave - 1 && ilg) got = atomicAdd(&a.ctr->n_large, ilg);
-            const uint32_t bsm = __builtin_amdgcn_readlane(got, kWave - 2), blg = __builtin_amdgcn_readlane(got, kWave - 1);
-            if (lane < kWaves) {
-                s_bsm[lane] = bsm + ism - sm;
-                s_blg[lane] = blg + ilg - lg;
-            }
-        }
-        __syncthreads();
-        uint32_t osm = s_bsm[wv], olg = s_blg[wv];
-#pragma unroll
-        for (uint32_t c = 0; c < 4; ++c) {
-            const uint32_t v = (uint32_t)(v0 + c * kWave);
-            if ((msm[c] >> lane) & 1ull) a.q_small[osm + lanes_below(msm[c])] = v;
-            if ((mlg[c] >> lane) & 1ull) a.q_large[olg + lanes_below(mlg[c])] = v;
-            osm += (uint32_t)__popcll(msm[c]);
-            olg += (uint32_t)__popcll(mlg[c]);
-        }
+    const MbfsCtl* ctl = a.ctl + slot;
+    // the control block with the phase that follows in the same superstep, for the next launch
+    auto pass_on = [&](uint32_t phase) {
+        if (!kDecide || blockIdx.x != 0 || threadIdx.x >= sizeof(MbfsCtl) / 4) return;
+        uint32_t x = reinterpret_cast<const uint32_t*>(ctl)[threadIdx.x];
+        if (threadIdx.x == offsetof(MbfsCtl, phase) / 4) x = phase;
+        reinterpret_cast<uint32_t*>(a.ctl + (slot ^ 1u))[threadIdx.x] = x;
+    };
+    const uint32_t phase = ctl->phase;
+    if (ctl->done) {
+        pass_on(phase);
+        return;
     }
-    if (cact) {  // uniform across the wave
-        adeg = wave_sum_u64(adeg);
-        bits = wave_sum_u64(bits);
-        redges = wave_sum_u64(redges);
-        dlg = wave_sum_u64(dlg);
-        if (lane == 0) {
-            atomicAdd(&s_sum[kMbfsActive], (unsigned long long)cact);
-            atomicAdd(&s_sum[kMbfsActiveDeg], adeg);
-            atomicAdd(&s_sum[kMbfsNewBits], bits);
-            atomicAdd(&s_sum[kMbfsReachedEdges], redges);
-            atomicAdd(&s_sum[kMbfsLargeDeg], dlg);
+    const uint32_t step = (uint32_t)ctl->step, par = step & 1u;
+    const uint32_t lv = step + 1 >= 255 ? 255u : step + 1;  // 255: saturated, reported as unreached
+    MbfsAcc acc;
+    if (phase == kMbfsPush) {
+        pass_on(kMbfsUpdate);
+        const uint32_t hub = ctl->hub_wgs;
+        if (blockIdx.x < hub) {
+            mbfs_push_large(a, ctl->n_large, a.frontier[par], blockIdx.x, hub);
+        } else {
+            const uint32_t wg = blockIdx.x - hub, nwg = gridDim.x - hub;
+            mbfs_push_small(a, a.ctr->queued[par], a.frontier[par], wg * 4 + threadIdx.x / kWave, nwg * 4, s_push);
         }
+        return;
     }
-    __syncthreads();
-    if (wv != 0) return;
-    const unsigned long long sum = lane < kMbfsSums ? s_sum[lane] : 0ull;
-    if (sum) atomicAdd(&a.ctr->sum[lane].v, sum);
-    if constexpr (kDecide) {
-        // the wave's atomics have been performed before its ticket is taken
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-        uint32_t t = 0;
-        if (lane == 0) t = atomicAdd(&a.ctr->ticket, 1u);
-        if ((uint32_t)__builtin_amdgcn_readfirstlane(t) == gridDim.x - 1) mbfs_decide(a, false, s_params);
+    if (phase == kMbfsQueue) {
+        pass_on(kMbfsPush);
+        mbfs_tiles<T, false>(a, lv, a.frontier[par], a.ctr->queued[par], &a.ctr->hubs[par].v, acc, s_tile);
+        return;
     }
+    if (phase == kMbfsPull)
+        mbfs_pull<T>(a, ctl->full, lv, a.frontier[par], a.frontier[par ^ 1u], acc);
+    else
+        mbfs_tiles<T, true>(a, lv, a.frontier[par ^ 1u], a.ctr->queued[par ^ 1u], &a.ctr->hubs[par ^ 1u].v, acc, s_tile);
+    if (mbfs_finish_launch<kDecide>(a.ctr, acc)) mbfs_decide(a, false, slot, s_params);
 }
 
 // Bit j, j + 4, .. j + 28 of four planes' words as the nibbles of a word.
@@ -519,11 +769,11 @@ __device__ __forceinline__ uint32_t mbfs_nibbles(uint32_t x0, uint32_t x1, uint3
 // A lane takes 4 vertices: the planes' words become nibbles, then bytes, 32 sources at a time, and 4
 // words of 4 sources each are transposed into 4 stores of 4 vertices each.  Bound by the stores: a
 // wave writes 256 contiguous bytes of a row at a time.  RMAT-20, 64 sources:
-// 25 us for 64 MiB of levels from 40 of planes and masks.
+// 30 us for 64 MiB of levels from 40 of planes and masks. 
 template <class T>
-__global__ __launch_bounds__(256) void k_mbfs_finish(MbfsArgs a, MbfsCtl* __restrict__ host, uint8_t* out, uint32_t row0,
+__global__ __launch_bounds__(1024) void k_mbfs_finish(MbfsArgs a, MbfsCtl* __restrict__ host, uint8_t* out, uint32_t row0,
                                                      uint32_t row1) {
-    const MbfsCtl* ctl = a.ctl;
+    const MbfsCtl* ctl = a.ctl;  // a batch has an even number of launches
     if (host) {
         if (blockIdx.x == 0 && threadIdx.x < sizeof(MbfsCtl) / 8)
             reinterpret_cast<unsigned long long*>(host)[threadIdx.x] =
@@ -543,12 +793,14 @@ __global__ __launch_bounds__(256) void k_mbfs_finish(MbfsArgs a, MbfsCtl* __rest
         const uint32_t cnt = n - v0 < 4 ? (uint32_t)(n - v0) : 4u;
         T x[kMbfsPlanes][4];
         unsigned long long vis[4];
+        uint32_t at[4];
+#pragma unroll
+        for (uint32_t i = 0; i < 4; ++i) at[i] = a.pos[i < cnt ? v0 + i : v0];
 #pragma unroll
         for (uint32_t i = 0; i < 4; ++i) {
-            vis[i] = i < cnt ? a.visited[v0 + i] : 0ull;
+            vis[i] = a.visited[at[i]];
 #pragma unroll
-            for (uint32_t p = 0; p < kMbfsPlanes; ++p)
-                x[p][i] = p < np && i < cnt ? planes[(size_t)p * n + v0 + i] : (T)0;
+            for (uint32_t p = 0; p < kMbfsPlanes; ++p) x[p][i] = p < np ? planes[(size_t)p * n + at[i]] : (T)0;
         }
 #pragma unroll
         for (uint32_t h = 0; h < (sizeof(T) == 8 ? 2u : 1u); ++h) {
@@ -593,17 +845,21 @@ __global__ __launch_bounds__(256) void k_mbfs_finish(MbfsArgs a, MbfsCtl* __rest
     }
 }
 
-// Host-driven superstep: the host's decision written into the control block.
-__global__ void k_mbfs_set_ctl(MbfsCtl* ctl, int32_t step, uint32_t pull, uint32_t n_small, uint32_t n_large,
-                               uint32_t hub_wgs) {
+// Host-driven launch: the host's decision written into the control block.
+__global__ void k_mbfs_set_ctl(MbfsCtl* ctl, int32_t step, uint32_t phase, uint32_t n_large, uint32_t hub_wgs) {
     ctl->step = step;
-    ctl->pull = pull;
-    ctl->n_small = n_small;
+    ctl->phase = phase;
     ctl->n_large = n_large;
     ctl->hub_wgs = hub_wgs;
 }
-__global__ void k_mbfs_zero(MbfsCounters* c) {
-    if (threadIdx.x < sizeof(MbfsCounters) / 8) reinterpret_cast<unsigned long long*>(c)[threadIdx.x] = 0;
+// Host-driven superstep of parity `par`: every counter cleared except its own queue's.
+__global__ __launch_bounds__(kWave) void k_mbfs_zero(MbfsCounters* c, uint32_t par) {
+    const uint32_t lane = threadIdx.x;
+    if (lane < kMbfsSegs) {
+        for (int i = 0; i < kMbfsSums; ++i) c->sum[lane].v[i] = 0;
+        c->queued[par ^ 1u][lane].v = 0;
+    }
+    if (lane == 0) c->hubs[par ^ 1u].v = 0;
 }
 
 static uint32_t mbfs_large(const medusa_graph* g, const medusa_opts& o) {
@@ -622,16 +878,19 @@ static void mbfs_run(medusa_graph* g, const uint32_t* srcs, uint32_t k, uint8_t*
     const uint32_t n = g->n;
     const uint64_t m = g->m;
     const uint32_t large = mbfs_large(g, o), grid = mbfs_grid(g, o);
-    g->q_small.ensure(n);
+    g->q_small.ensure((size_t)kMbfsSegs * mbfs_span(n));
     g->q_large.ensure(n);
     DBuf<unsigned long long>& masks = g->bitmap;
-    masks.ensure(3 * (size_t)n);
+    masks.ensure(4 * (size_t)n);
     DBuf<uint32_t>& planes = g->stamp;  // reused as the storage of the level planes
     planes.ensure((kMbfsPlanes * sizeof(T) * (size_t)n + 3) / 4);
-    MbfsCounters* C = dev_counters<MbfsCounters>(g);
+    // the two control blocks, then the counters
     static_assert(sizeof(MbfsCtl) <= sizeof(CtlStorage), "control block storage");
-    g->mbfs_ctl.ensure(1);
+    static_assert(sizeof(MbfsCtl) % 8 == 0 && sizeof(CtlStorage) % 128 == 0, "control block and counter alignment");
+    g->mbfs_ctl.ensure(2 + (sizeof(MbfsCounters) + sizeof(CtlStorage) - 1) / sizeof(CtlStorage));
     MbfsCtl* ctl = reinterpret_cast<MbfsCtl*>(g->mbfs_ctl.p);
+    MbfsCounters* C = reinterpret_cast<MbfsCounters*>(g->mbfs_ctl.p + 2);
+    g->h_ctr_raw.ensure((sizeof(MbfsCounters) + 7) / 8);
     MbfsCtl* host = reinterpret_cast<MbfsCtl*>(g->h_ctr_raw.p);
     hipStream_t s = g->stream;
     const bool host_driven = o.timing || o.trace;
@@ -645,51 +904,52 @@ static void mbfs_run(medusa_graph* g, const uint32_t* srcs, uint32_t k, uint8_t*
     build_pull_layout(g);
     const PullLayout& PL = *g->pull;
     MbfsArgs a{};
-    a.row_ptr = g->row_ptr.p;
     a.col = g->col.p;
-    a.cptr = g->cptr.p;
-    a.csrc = g->csrc.p;
+    a.pos = PL.pos.p;
+    a.out = PL.out.p;
+    a.indeg = PL.indeg.p;
+    a.base = PL.base.p;
+    a.hub = PL.hub.p;
+    a.src = PL.src.p;
     a.q_small = g->q_small.p;
     a.q_large = g->q_large.p;
     a.visited = masks.p;
-    a.frontier = masks.p + n;
-    a.next = masks.p + 2 * (size_t)n;
-    a.runs = PL.d_runs.p;
-    a.wg_run = PL.wg_run.p;
-    a.perm = PL.perm.p;
-    a.ell = PL.ell.p;
+    a.next = masks.p + n;
+    a.frontier[0] = masks.p + 2 * (size_t)n;
+    a.frontier[1] = masks.p + 3 * (size_t)n;
     a.ctr = C;
     a.ctl = ctl;
     a.policy = policy;
     a.planes = planes.p;
     a.n = n;
     a.large = large;
-    a.items = PL.total_wgs;
+    a.nslices = PL.nslices;
+    a.nhubs = PL.nhubs;
     a.grid = grid;
-    const dim3 update_grid(grid_for(n, kMbfsTile, 512)), finish_grid(grid_for(n, 1024, 8192));
+    a.span = mbfs_span(n);
+    // a workgroup per window of the layout, which fetches every line of it once, where that fills the
+    // 256 CUs (RMAT-20 30 us against 35 with quarters of windows), else quarters
+    const uint32_t finish_wg = n >= 256 * kPullWindow ? 1024 : 256;
+    const dim3 finish_grid(grid_for(n, 4 * finish_wg, 8192));
     const bool direct = kernels_can_write(g, out);  // else the rows are copied out at the end
 
-    auto expand = [&]() {
-        hipLaunchKernelGGL(k_mbfs_expand, dim3(grid), dim3(256), 0, s, a);
-        MDS_LAUNCHED();
-    };
-    // capture (once per buffers, launch shape, policy buffer and slot count) a batch of supersteps
-    auto captured = [&](GraphCache& gc, uint32_t slots) -> hipGraphExec_t {
+    // capture (once per buffers, launch shape, policy buffer and slot count) a batch of launches
+    auto captured = [&](uint32_t slots) -> hipGraphExec_t {
+        static_assert(kHeadStep % 2 == 0, "a batch starts and ends with the first control block");
+        GraphCache& gc = g->mbfs_heads[slots / kHeadStep];
         const uintptr_t key[8] = {(uintptr_t)masks.p,   (uintptr_t)policy,
                                   ((uintptr_t)grid << 32) | large,
                                   (uintptr_t)planes.p,  (uintptr_t)host,
                                   (uintptr_t)a.q_small, (uintptr_t)a.q_large,
-                                  ((uintptr_t)sizeof(T) << 32) | slots};
+                                  (uintptr_t)sizeof(T)};
         if (gc.exec && std::equal(key, key + 8, gc.key)) return gc.exec;
         gc.reset();
         MDS_HIP(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
         hipGraph_t graph = nullptr;
         try {
-            for (uint32_t b = 0; b < slots; ++b) {
-                expand();
-                hipLaunchKernelGGL((k_mbfs_update<T, true>), update_grid, dim3(kMbfsWg), 0, s, a, 0);
-            }
-            hipLaunchKernelGGL(k_mbfs_finish<T>, finish_grid, dim3(256), 0, s, a, host, (uint8_t*)nullptr, 0u, 0u);
+            for (uint32_t b = 0; b < slots; ++b)
+                hipLaunchKernelGGL((k_mbfs_super<T, true>), dim3(grid), dim3(256), 0, s, a, b & 1u);
+            hipLaunchKernelGGL(k_mbfs_finish<T>, finish_grid, dim3(finish_wg), 0, s, a, host, (uint8_t*)nullptr, 0u, 0u);
             MDS_LAUNCHED();
         } catch (...) {
             (void)hipStreamEndCapture(s, &graph);
@@ -703,9 +963,8 @@ static void mbfs_run(medusa_graph* g, const uint32_t* srcs, uint32_t k, uint8_t*
         std::copy(key, key + 8, gc.key);
         return gc.exec;
     };
-    const uint32_t head = head_slots(g->mbfs_last_steps, kMbfsBatch);
-    hipGraphExec_t head_exec = nullptr;
-    if (!host_driven) head_exec = captured(head == kMbfsBatch ? g->mbfs_graph : g->mbfs_head, head);
+    uint32_t slots = next_slots(g->mbfs_last_slots, 0, kMbfsBatch);
+    hipGraphExec_t exec = host_driven ? nullptr : captured(slots);
 
     MbfsSources sources{};
     std::copy(srcs, srcs + k, sources.v);
@@ -718,49 +977,65 @@ static void mbfs_run(medusa_graph* g, const uint32_t* srcs, uint32_t k, uint8_t*
 
     MbfsCtl h{};
     if (!host_driven) {
-        for (uint32_t batch = 0;; ++batch) {
-            MDS_HIP(hipGraphLaunch(batch == 0 ? head_exec : captured(g->mbfs_graph, kMbfsBatch), s));
+        for (uint64_t done = 0;; exec = captured(slots = next_slots(g->mbfs_last_slots, done, kMbfsBatch))) {
+            MDS_HIP(hipGraphLaunch(exec, s));
             MDS_HIP(hipEventRecord(g->ev_end, s));
             MDS_HIP(hipStreamSynchronize(s));
             if (host->done) break;
-            MDS_CHECK(batch < (n + kMbfsBatch) / kMbfsBatch + 2, MEDUSA_ERR_INTERNAL,
-                      "mbfs: superstep loop did not end");
+            done += slots;
+            MDS_CHECK(done < 3ull * n + 16ull * kMbfsBatch, MEDUSA_ERR_INTERNAL, "mbfs: superstep loop did not end");
         }
         h = *host;
-        g->mbfs_last_steps = h.supersteps;
+        g->mbfs_last_slots = h.slots;
     } else {
-        Sched sched(o, Sched::kMbfs);
+        Sched sched(o, Sched::kMbfs, k);
         const bool timing = o.timing != 0;
         if (timing) ensure_events(g, 2);
-        MbfsCounters c = read_counters<MbfsCounters>(g);
+        unsigned long long c[kMbfsSums];
+        auto read_sums = [&]() {  // waits for the stream
+            MDS_HIP(hipMemcpyAsync(g->h_ctr_raw.p, C, sizeof(MbfsCounters), hipMemcpyDeviceToHost, s));
+            MDS_HIP(hipStreamSynchronize(s));
+            const MbfsCounters* x = reinterpret_cast<const MbfsCounters*>(g->h_ctr_raw.p);
+            for (int i = 0; i < kMbfsSums; ++i) {
+                c[i] = 0;
+                for (uint32_t sg = 0; sg < kMbfsSegs; ++sg) c[i] += x->sum[sg].v[i];
+            }
+        };
+        auto launch = [&](uint32_t t, uint32_t phase) {
+            const uint32_t n_small = (uint32_t)c[kMbfsQueued], n_large = (uint32_t)(c[kMbfsQueued] >> 32);
+            hipLaunchKernelGGL(k_mbfs_set_ctl, dim3(1), dim3(1), 0, s, ctl, (int32_t)t, phase, n_large,
+                               mbfs_hub_wgs(grid, n_small, n_large, c[kMbfsLargeDeg], c[kMbfsActiveDeg]));
+            MDS_LAUNCHED();
+            hipLaunchKernelGGL((k_mbfs_super<T, false>), dim3(grid), dim3(256), 0, s, a, 0u);
+            MDS_LAUNCHED();
+        };
+        read_sums();
         Frontier f{};
         f.n = n;
         f.m = m;
-        h.n_u = (uint64_t)n * k - c.sum[kMbfsNewBits].v;
-        h.m_u = (uint64_t)m * k - c.sum[kMbfsReachedEdges].v;
-        h.reached = c.sum[kMbfsNewBits].v;
-        h.reached_edges = c.sum[kMbfsReachedEdges].v;
-        bool pull = false;
-        for (uint32_t t = 0; c.sum[kMbfsActive].v; ++t) {
+        h.n_u = (uint64_t)n * k - c[kMbfsNewBits];
+        h.m_u = (uint64_t)m * k - c[kMbfsReachedEdges];
+        h.reached = c[kMbfsNewBits];
+        h.reached_edges = c[kMbfsReachedEdges];
+        bool pull = false, queued = true;
+        for (uint32_t t = 0; c[kMbfsActive]; ++t) {
             f.step = t;
-            f.n_f = c.sum[kMbfsActive].v;
-            f.m_f = c.sum[kMbfsActiveDeg].v;
+            f.n_f = c[kMbfsActive];
+            f.m_f = c[kMbfsActiveDeg];
             f.n_u = h.n_u;
             f.m_u = h.m_u;
             if (o.direction == MEDUSA_DIR_PUSH) pull = false;
             else if (o.direction == MEDUSA_DIR_PULL) pull = true;
             else pull = sched.bfs_pull(f, pull);
-            hipLaunchKernelGGL(k_mbfs_set_ctl, dim3(1), dim3(1), 0, s, ctl, (int32_t)t, pull ? 1u : 0u, c.n_small,
-                               c.n_large, mbfs_hub_wgs(grid, c.n_small, c.n_large, c.sum[kMbfsLargeDeg].v, f.m_f));
+            hipLaunchKernelGGL(k_mbfs_zero, dim3(1), dim3(kWave), 0, s, C, t & 1u);
             MDS_LAUNCHED();
-            hipLaunchKernelGGL(k_mbfs_zero, dim3(1), dim3(sizeof(MbfsCounters) / 8), 0, s, C);
-            MDS_LAUNCHED();
+            if (!pull && !queued) launch(t, kMbfsQueue);
             if (timing) MDS_HIP(hipEventRecord(g->events[0], s));
-            expand();
+            launch(t, pull ? kMbfsPull : kMbfsPush);
+            if (!pull) launch(t, kMbfsUpdate);
             if (timing) MDS_HIP(hipEventRecord(g->events[1], s));
-            hipLaunchKernelGGL((k_mbfs_update<T, false>), update_grid, dim3(kMbfsWg), 0, s, a, (int32_t)(t + 1));
-            MDS_LAUNCHED();
-            c = read_counters<MbfsCounters>(g);
+            queued = !pull;
+            read_sums();
             double kms = 0;
             if (timing) {
                 float ms = 0;
@@ -769,26 +1044,23 @@ static void mbfs_run(medusa_graph* g, const uint32_t* srcs, uint32_t k, uint8_t*
                 st.kernel_ms += ms;
                 ++st.kernel_launches;
             }
-            uint64_t probes = 0;
-            for (const MbfsLine& l : c.probes) probes += l.v;
-            const uint64_t kb = pull ? 4ull * (n + 1) + 8ull * n + 12ull * probes : 20ull * f.n_f + 20ull * f.m_f;
-            const uint64_t new_bits = c.sum[kMbfsNewBits].v;
+            const uint64_t kb = pull ? 4ull * (n + 1) + 8ull * n + 12ull * c[kMbfsProbes] : 20ull * f.n_f + 20ull * f.m_f;
             h.kernel_bytes += kb;
-            h.alg_bytes += kb + 24ull * n + new_bits;
+            h.alg_bytes += kb + 24ull * n + c[kMbfsNewBits];
             if (pull) ++h.pull_steps; else ++h.push_steps;
             sched.record(g, f, pull ? 1.0 : 0.0, kms);
             ++h.supersteps;
-            if (t + 1 >= 255 && new_bits) h.saturated = 1;
-            h.reached += new_bits;
-            h.reached_edges += c.sum[kMbfsReachedEdges].v;
-            h.n_u -= new_bits;
-            h.m_u -= c.sum[kMbfsReachedEdges].v;
+            if (t + 1 >= 255 && c[kMbfsNewBits]) h.saturated = 1;
+            h.reached += c[kMbfsNewBits];
+            h.reached_edges += c[kMbfsReachedEdges];
+            h.n_u -= c[kMbfsNewBits];
+            h.m_u -= c[kMbfsReachedEdges];
         }
-        // the last update's level, for the finish
-        hipLaunchKernelGGL(k_mbfs_set_ctl, dim3(1), dim3(1), 0, s, ctl, (int32_t)h.supersteps, 0u, 0u, 0u, 0u);
+        // the last level, for the finish
+        hipLaunchKernelGGL(k_mbfs_set_ctl, dim3(1), dim3(1), 0, s, ctl, (int32_t)h.supersteps, 0u, 0u, 0u);
         MDS_LAUNCHED();
         if (direct) {
-            hipLaunchKernelGGL(k_mbfs_finish<T>, finish_grid, dim3(256), 0, s, a, (MbfsCtl*)nullptr, out, 0u, k);
+            hipLaunchKernelGGL(k_mbfs_finish<T>, finish_grid, dim3(finish_wg), 0, s, a, (MbfsCtl*)nullptr, out, 0u, k);
             MDS_LAUNCHED();
         }
         MDS_HIP(hipEventRecord(g->ev_end, s));
@@ -812,7 +1084,7 @@ static void mbfs_run(medusa_graph* g, const uint32_t* srcs, uint32_t k, uint8_t*
     for (uint32_t r = 0; r < k; r += rows) {
         const uint32_t r1 = std::min(k, r + rows);
         uint8_t* buf = reinterpret_cast<uint8_t*>(g->mbfs_rows.p);
-        hipLaunchKernelGGL(k_mbfs_finish<T>, finish_grid, dim3(256), 0, s, a, (MbfsCtl*)nullptr, buf, r, r1);
+        hipLaunchKernelGGL(k_mbfs_finish<T>, finish_grid, dim3(finish_wg), 0, s, a, (MbfsCtl*)nullptr, buf, r, r1);
         MDS_LAUNCHED();
         copy_out(g, out + (size_t)r * n, buf, (size_t)(r1 - r) * n);
     }

@@ -150,7 +150,7 @@ struct Frontier {
 
 // BFS and MBFS consult the learned direction policy only near the heuristic's switching
 // point, where its decision ratio (alpha * m_f / m_u while pushing, beta * n_f / n while
-// pulling) lies within a factor kPolicyBand of 1; farther out the heuristic's choice is taken
+// pulling; the mask engine has only the first) lies within a factor kPolicyBand of 1; farther out the heuristic's choice is taken
 // without evaluating the network, which saves its cost on most supersteps.
 constexpr double kPolicyBand = 8.0;
 __host__ __device__ inline bool bfs_policy_consulted(bool cur_pull, double n_f, double m_f, double m_u, double n,
@@ -168,27 +168,30 @@ struct Sched {
     // frontier's out-edges exceed the unvisited out-edges / alpha, push again once the frontier
     // falls below n / beta.  The paper uses alpha = 14.  Set from per-superstep push and pull
     // times measured on Erdos-Renyi, RMAT, Chung-Lu and lattice graphs: alpha = 3 for the
-    // single-source engine, whose pull costs relatively more on this GPU, and alpha = 100 for
-    // the 64-source mask engine, whose pull (over coalesced ELL slabs, reading nearly every
-    // in-edge) beats the push much earlier.
-    static constexpr double kAlphaBfs = 3.0, kAlphaMbfs = 100.0, kBeta = 24.0;
+    // single-source engine, whose pull costs relatively more on this GPU.  The mask engine counts
+    // the unvisited out-edges once per source that misses the vertex, so its alpha is per source,
+    // and it takes the cheaper side of the same line in every superstep: its pull leaves out
+    // visited vertices 64 at a time, so late pulls stay cheap.  RMAT-20 (push with update against
+    // pull): 137 us and 138 at 0.130 m out-edges, 4 sources; 146 and 152 at 0.086, 64 sources; 27 and
+    // 17 at 0.0009 with 0.2 % unvisited.  Chung-Lu, 2.4 M vertices, 64 sources: 82 and 66 at 0.068;
+    // 58 and 60 at 0.013.
+    static constexpr double kAlphaBfs = 3.0, kAlphaMbfs = 10.0, kBeta = 24.0;
     const medusa_opts& o;
     Algo algo;
-    Sched(const medusa_opts& opts, Algo a) : o(opts), algo(a) {}
+    double alpha;
+    Sched(const medusa_opts& opts, Algo a, uint32_t sources = 1)
+        : o(opts), algo(a), alpha(a == kMbfs ? kAlphaMbfs * sources : kAlphaBfs) {}
 
-    // Plain engine: switch to pull when the frontier's out-edges exceed the
-    // unvisited out-edges / alpha; back to push when the frontier shrinks below n / beta.
     bool heuristic_pull(const Frontier& f, bool cur_pull) const {
-        const double alpha = algo == kMbfs ? kAlphaMbfs : kAlphaBfs;
-        if (!cur_pull) return (double)f.m_f > (double)f.m_u / alpha;
+        if (!cur_pull || algo == kMbfs) return (double)f.m_f > (double)f.m_u / alpha;
         return !((double)f.n_f < (double)f.n / kBeta);
     }
     // Direction for the next superstep: the learned policy's cheaper action when one is
     // given (and of the right kind), else the heuristic.
     bool bfs_pull(const Frontier& f, bool cur_pull) const {
         if (!o.policy || policy_kind(o.policy) != MEDUSA_POLICY_DIRECTION) return heuristic_pull(f, cur_pull);
-        if (!bfs_policy_consulted(cur_pull, (double)f.n_f, (double)f.m_f, (double)f.m_u, (double)f.n,
-                                  algo == kMbfs ? kAlphaMbfs : kAlphaBfs, kBeta))
+        if (!bfs_policy_consulted(cur_pull && algo != kMbfs, (double)f.n_f, (double)f.m_f, (double)f.m_u, (double)f.n,
+                                  alpha, kBeta))
             return heuristic_pull(f, cur_pull);
         double rec[MEDUSA_TRACE_FIELDS];
         to_record(f, cur_pull ? 1.0 : 0.0, 0.0, rec);

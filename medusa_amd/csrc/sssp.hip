@@ -759,7 +759,6 @@ __global__ __launch_bounds__(256) void k_sssp_split(const uint32_t* __restrict__
 // kSsspBatch slots are captured once as a hipGraph and replayed until done.
 
 constexpr uint32_t kSsspBatch = 32;
-constexpr uint32_t kSsspStep = 4;  // granularity of a replay's slots: one captured graph per multiple
 // Workgroups of a work launch: about the resident count (5 per CU at this LDS size) without local
 // rounds, so every tile is in flight at once (RMAT-20 at width 250: 1.51 ms against 1.79 with
 // 2048; ER 2^20/2^24: 1.15 against 1.36); twice that with local rounds, whose short queues spread
@@ -1296,7 +1295,7 @@ static void sssp_run_device(medusa_graph* g, uint32_t src, uint32_t* out, const 
     };
     // `slots` work launches and the closing kernel, captured once per slot count
     auto captured = [&](uint32_t slots) -> hipGraphExec_t {
-        GraphCache& gc = g->sssp_heads[slots / kSsspStep];
+        GraphCache& gc = g->sssp_heads[slots / kHeadStep];
         // the marks buffer is 256-byte aligned, so its low bits can carry the kernel variant
         const uintptr_t key[7] = {(uintptr_t)g->dist.p, (uintptr_t)g->near_q.p, (uintptr_t)g->q_aux.p,
                                   (uintptr_t)g->stamp.p, (uintptr_t)marks | (rec ? 2u : local_cfg ? 1u : 0u),
@@ -1324,13 +1323,7 @@ static void sssp_run_device(medusa_graph* g, uint32_t src, uint32_t* out, const 
         std::copy(key, key + 7, gc.key);
         return gc.exec;
     };
-    // slots of the next replay: what the previous run on the handle still took from here, in steps of
-    // kSsspStep; a batch where there is no previous run or this one is longer
-    auto next_slots = [&](uint64_t done) {
-        const uint64_t left = g->sssp_last_slots > done ? g->sssp_last_slots - done : kSsspBatch;
-        return (uint32_t)std::min<uint64_t>(kMaxHeadSlots, (left + kSsspStep - 1) / kSsspStep * kSsspStep);
-    };
-    uint32_t slots = next_slots(0);
+    uint32_t slots = next_slots(g->sssp_last_slots, 0, kSsspBatch);
     hipGraphExec_t exec = captured(slots);
     const bool direct = kernels_can_write(g, out);
 
@@ -1340,7 +1333,7 @@ static void sssp_run_device(medusa_graph* g, uint32_t src, uint32_t* out, const 
     MDS_LAUNCHED();
     // every replay either relaxes a non-empty queue or raises the threshold
     const uint64_t max_slots = 4ull * n + 1024ull * kSsspBatch;
-    for (uint64_t done = 0;; exec = captured(slots = next_slots(done))) {
+    for (uint64_t done = 0;; exec = captured(slots = next_slots(g->sssp_last_slots, done, kSsspBatch))) {
         MDS_HIP(hipGraphLaunch(exec, s));
         MDS_HIP(hipStreamSynchronize(s));
         MDS_CHECK(!host->ctl.lost, MEDUSA_ERR_INTERNAL, "sssp: near queue overflow");

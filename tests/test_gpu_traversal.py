@@ -284,6 +284,32 @@ def test_mbfs_level_planes(oracle, n, k):
         assert G.mbfs(srcs)[1].reserved[0] == int(saturated)
 
 
+@pytest.mark.parametrize("n", [70, 4096, 9000])
+def test_mbfs_hubs_and_slices(oracle, n):
+    """In-degrees on both sides of the 64 of a lane and of the 256 of a hub's round, in windows of
+    mixed degrees and vertices without in-edges, pulled by two workgroups (many rounds of slices and
+    hubs each) and by the default; pull to push and back by the heuristic."""
+    rng = np.random.default_rng(n)
+    src = [rng.integers(0, n, 2 * n)]
+    dst = [rng.integers(0, n // 2, 2 * n)]
+    for d in (63, 64, 65, 255, 256, 257, 1000):
+        v = rng.integers(0, n, 12)
+        src.append(rng.integers(0, n, 12 * d))
+        dst.append(np.repeat(v, d))
+    rp, col, _ = csr_from_edges(n, np.stack([np.concatenate(src), np.concatenate(dst)], 1))
+    with md.Graph(rp, col) as G:
+        for k in (1, 5, 64):
+            srcs = rng.integers(0, n, k).astype(np.uint32)
+            want = oracle.mbfs(rp, col, srcs)
+            for d in _dirs():
+                for grid in (2, 0):
+                    out, st = G.mbfs(srcs, direction=d, grid=grid, large_degree=8)
+                    assert np.array_equal(out, want), (k, d, grid)
+                    host = G.mbfs(srcs, direction=d, grid=grid, large_degree=8, timing=1)[1]
+                    assert (st.supersteps, st.push_steps, st.pull_steps, st.edges_traversed) == (
+                        host.supersteps, host.push_steps, host.pull_steps, host.edges_traversed)
+
+
 def test_mbfs_rows_in_pieces():
     """A host output of more bytes than the row buffer holds: no vertex but the sources is reached."""
     n, k = 5_000_001, 64
