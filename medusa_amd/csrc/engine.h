@@ -218,6 +218,7 @@ struct PullLayout {
     DBuf<uint64_t> base;      // per slice: first column (length: up to the next slice's base / 64)
     DBuf<uint4> hub;          // vertex, in-degree, first in-edge (low, high word)
     DBuf<uint32_t> src;       // slices' columns, then the hubs' in-edges
+    DBuf<uint32_t> dst;       // targets of the out-edges
 };
 constexpr uint8_t kPullHub = 255;
 

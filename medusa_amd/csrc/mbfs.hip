@@ -67,8 +67,14 @@ struct MbfsCtl {
     uint8_t* out;  // where the finish of a device-driven run writes the levels, or null
 };
 
+// What a device-driven run leaves in pinned memory.
+struct MbfsHost {
+    MbfsCtl ctl;
+    unsigned long long t_begin, t_end;
+};
+
 struct MbfsArgs {
-    const uint32_t *col, *pos;
+    const uint32_t *dst, *pos;
     const uint2* out;        // first out-edge, out-degree
     const uint8_t* indeg;
     const uint64_t* base;
@@ -160,6 +166,12 @@ __global__ __launch_bounds__(256) void k_pull_fill(uint32_t n, uint32_t nslices,
     }
 }
 
+__global__ void k_pull_dst(uint64_t m, const uint32_t* __restrict__ col, const uint32_t* __restrict__ pos,
+                           uint32_t* __restrict__ dst) {
+    const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
+    for (uint64_t e = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x; e < m; e += stride) dst[e] = pos[col[e]];
+}
+
 // Sorted and filled on the GPU (RMAT-20: 1.5 ms; on the host, with the sort over all vertices and an
 // upload of every slab, 130 ms); the host sums the slices' and hubs' lengths.
 static void build_pull_layout(medusa_graph* g) {
@@ -223,6 +235,10 @@ static void build_pull_layout(medusa_graph* g) {
                        L->nslices, L->nhubs, g->cptr.p, g->csrc.p, (const uint32_t*)perm.p, (const uint32_t*)L->pos.p,
                        (const uint8_t*)L->indeg.p, (const uint64_t*)L->base.p, (const uint4*)L->hub.p, L->src.p);
     MDS_LAUNCHED();
+    L->dst.alloc(std::max<uint64_t>(g->m, 1));
+    hipLaunchKernelGGL(k_pull_dst, dim3(grid_for(g->m, 1024, 8192)), dim3(256), 0, s, g->m, g->col.p,
+                       (const uint32_t*)L->pos.p, L->dst.p);
+    MDS_LAUNCHED();
     MDS_HIP(hipStreamSynchronize(s));
     g->pull = std::move(L);
 }
@@ -231,7 +247,7 @@ static void build_pull_layout(medusa_graph* g) {
 
 // Masks cleared, counters and control block set up.
 __global__ __launch_bounds__(256) void k_mbfs_fill(MbfsArgs a, unsigned long long m, uint32_t k, uint32_t mode,
-                                                   uint8_t* out) {
+                                                   uint8_t* out, MbfsHost* host) {
     const uint64_t tid = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x, stride = (uint64_t)gridDim.x * blockDim.x;
     // visited, next and frontier 0 follow each other; frontier 1 is written whole before it is read
     for (uint64_t i = tid; i < 3ull * a.n; i += stride) a.visited[i] = 0;
@@ -239,6 +255,7 @@ __global__ __launch_bounds__(256) void k_mbfs_fill(MbfsArgs a, unsigned long lon
     for (uint32_t i = threadIdx.x; i < sizeof(MbfsCounters) / 8; i += blockDim.x)
         reinterpret_cast<unsigned long long*>(a.ctr)[i] = 0;
     if (threadIdx.x == 0) {
+        host->t_begin = (unsigned long long)wall_clock64();
         MbfsCtl z{};
         z.mode = mode;
         z.n = a.n;
@@ -272,7 +289,7 @@ struct MbfsPushLds {
 };
 
 __device__ __forceinline__ void mbfs_offer(const MbfsArgs& a, uint32_t e, unsigned long long mask) {
-    const uint32_t v = a.pos[a.col[e]];
+    const uint32_t v = a.dst[e];
     const unsigned long long add = mask & ~a.visited[v];
     if (add && (a.next[v] & add) != add) atomicOr(&a.next[v], add);
 }
@@ -610,7 +627,7 @@ __device__ __forceinline__ bool mbfs_direction(const MbfsCtl& c, const float* __
     if (c.mode == 1) return false;
     if (c.mode == 2) return true;
     const double alpha = Sched::kAlphaMbfs * c.k;
-    const bool plain = (double)c.m_f > (double)c.m_u / alpha;
+    const bool plain = c.m <= Sched::kMbfsPullEdges || (double)c.m_f > (double)c.m_u / alpha;
     if (c.mode != 3 || !policy ||
         !bfs_policy_consulted(false, (double)c.n_f, (double)c.m_f, (double)c.m_u, (double)c.n, alpha, Sched::kBeta))
         return plain;
@@ -771,13 +788,16 @@ __device__ __forceinline__ uint32_t mbfs_nibbles(uint32_t x0, uint32_t x1, uint3
 // wave writes 256 contiguous bytes of a row at a time.  RMAT-20, 64 sources:
 // 30 us for 64 MiB of levels from 40 of planes and masks. 
 template <class T>
-__global__ __launch_bounds__(1024) void k_mbfs_finish(MbfsArgs a, MbfsCtl* __restrict__ host, uint8_t* out, uint32_t row0,
+__global__ __launch_bounds__(1024) void k_mbfs_finish(MbfsArgs a, MbfsHost* __restrict__ host, uint8_t* out, uint32_t row0,
                                                      uint32_t row1) {
     const MbfsCtl* ctl = a.ctl;  // a batch has an even number of launches
     if (host) {
-        if (blockIdx.x == 0 && threadIdx.x < sizeof(MbfsCtl) / 8)
-            reinterpret_cast<unsigned long long*>(host)[threadIdx.x] =
-                reinterpret_cast<const unsigned long long*>(ctl)[threadIdx.x];
+        if (blockIdx.x == 0) {
+            if (threadIdx.x < sizeof(MbfsCtl) / 8)
+                reinterpret_cast<unsigned long long*>(&host->ctl)[threadIdx.x] =
+                    reinterpret_cast<const unsigned long long*>(ctl)[threadIdx.x];
+            if (threadIdx.x == 0) host->t_end = (unsigned long long)wall_clock64();
+        }
         if (!ctl->done || !ctl->out) return;
         out = ctl->out;
         row0 = 0;
@@ -891,7 +911,7 @@ static void mbfs_run(medusa_graph* g, const uint32_t* srcs, uint32_t k, uint8_t*
     MbfsCtl* ctl = reinterpret_cast<MbfsCtl*>(g->mbfs_ctl.p);
     MbfsCounters* C = reinterpret_cast<MbfsCounters*>(g->mbfs_ctl.p + 2);
     g->h_ctr_raw.ensure((sizeof(MbfsCounters) + 7) / 8);
-    MbfsCtl* host = reinterpret_cast<MbfsCtl*>(g->h_ctr_raw.p);
+    MbfsHost* host = reinterpret_cast<MbfsHost*>(g->h_ctr_raw.p);  // (or the host-driven loop's counters)
     hipStream_t s = g->stream;
     const bool host_driven = o.timing || o.trace;
     uint32_t mode = 0;
@@ -904,7 +924,7 @@ static void mbfs_run(medusa_graph* g, const uint32_t* srcs, uint32_t k, uint8_t*
     build_pull_layout(g);
     const PullLayout& PL = *g->pull;
     MbfsArgs a{};
-    a.col = g->col.p;
+    a.dst = PL.dst.p;
     a.pos = PL.pos.p;
     a.out = PL.out.p;
     a.indeg = PL.indeg.p;
@@ -968,9 +988,9 @@ static void mbfs_run(medusa_graph* g, const uint32_t* srcs, uint32_t k, uint8_t*
 
     MbfsSources sources{};
     std::copy(srcs, srcs + k, sources.v);
-    MDS_HIP(hipEventRecord(g->ev_begin, s));
+    if (host_driven) MDS_HIP(hipEventRecord(g->ev_begin, s));
     hipLaunchKernelGGL(k_mbfs_fill, dim3(grid_for(3ull * n, 256, 4096)), dim3(256), 0, s, a, (unsigned long long)m, k,
-                       mode, direct ? out : nullptr);
+                       mode, direct ? out : nullptr, host);
     MDS_LAUNCHED();
     hipLaunchKernelGGL(k_mbfs_start, dim3(1), dim3(kWave), 0, s, a, sources, k, host_driven ? 0u : 1u);
     MDS_LAUNCHED();
@@ -979,14 +999,14 @@ static void mbfs_run(medusa_graph* g, const uint32_t* srcs, uint32_t k, uint8_t*
     if (!host_driven) {
         for (uint64_t done = 0;; exec = captured(slots = next_slots(g->mbfs_last_slots, done, kMbfsBatch))) {
             MDS_HIP(hipGraphLaunch(exec, s));
-            MDS_HIP(hipEventRecord(g->ev_end, s));
             MDS_HIP(hipStreamSynchronize(s));
-            if (host->done) break;
+            if (host->ctl.done) break;
             done += slots;
             MDS_CHECK(done < 3ull * n + 16ull * kMbfsBatch, MEDUSA_ERR_INTERNAL, "mbfs: superstep loop did not end");
         }
-        h = *host;
+        h = host->ctl;
         g->mbfs_last_slots = h.slots;
+        st.device_ms = (double)(host->t_end - host->t_begin) / (double)g->wall_khz;
     } else {
         Sched sched(o, Sched::kMbfs, k);
         const bool timing = o.timing != 0;
@@ -1060,15 +1080,15 @@ static void mbfs_run(medusa_graph* g, const uint32_t* srcs, uint32_t k, uint8_t*
         hipLaunchKernelGGL(k_mbfs_set_ctl, dim3(1), dim3(1), 0, s, ctl, (int32_t)h.supersteps, 0u, 0u, 0u);
         MDS_LAUNCHED();
         if (direct) {
-            hipLaunchKernelGGL(k_mbfs_finish<T>, finish_grid, dim3(finish_wg), 0, s, a, (MbfsCtl*)nullptr, out, 0u, k);
+            hipLaunchKernelGGL(k_mbfs_finish<T>, finish_grid, dim3(finish_wg), 0, s, a, (MbfsHost*)nullptr, out, 0u, k);
             MDS_LAUNCHED();
         }
         MDS_HIP(hipEventRecord(g->ev_end, s));
         MDS_HIP(hipStreamSynchronize(s));
+        float ms = 0;
+        MDS_HIP(hipEventElapsedTime(&ms, g->ev_begin, g->ev_end));
+        st.device_ms = ms;
     }
-    float ms = 0;
-    MDS_HIP(hipEventElapsedTime(&ms, g->ev_begin, g->ev_end));
-    st.device_ms = ms;
     st.supersteps = h.supersteps;
     st.push_steps = h.push_steps;
     st.pull_steps = h.pull_steps;
@@ -1084,7 +1104,7 @@ static void mbfs_run(medusa_graph* g, const uint32_t* srcs, uint32_t k, uint8_t*
     for (uint32_t r = 0; r < k; r += rows) {
         const uint32_t r1 = std::min(k, r + rows);
         uint8_t* buf = reinterpret_cast<uint8_t*>(g->mbfs_rows.p);
-        hipLaunchKernelGGL(k_mbfs_finish<T>, finish_grid, dim3(finish_wg), 0, s, a, (MbfsCtl*)nullptr, buf, r, r1);
+        hipLaunchKernelGGL(k_mbfs_finish<T>, finish_grid, dim3(finish_wg), 0, s, a, (MbfsHost*)nullptr, buf, r, r1);
         MDS_LAUNCHED();
         copy_out(g, out + (size_t)r * n, buf, (size_t)(r1 - r) * n);
     }

@@ -172,9 +172,12 @@ struct Sched {
     // the unvisited out-edges once per source that misses the vertex, so its alpha is per source,
     // and it takes the cheaper side of the same line in every superstep: its pull leaves out
     // visited vertices 64 at a time, so late pulls stay cheap.  RMAT-20 (push with update against
-    // pull): 137 us and 138 at 0.130 m out-edges, 4 sources; 146 and 152 at 0.086, 64 sources; 27 and
-    // 17 at 0.0009 with 0.2 % unvisited.  Chung-Lu, 2.4 M vertices, 64 sources: 82 and 66 at 0.068;
-    // 58 and 60 at 0.013.
+    // pull): 119 us and 137 at 0.130 m out-edges, 4 sources; 132 and 151 at 0.086, 64 sources; 25 and
+    // 17 at 0.0009 with 0.2 % unvisited.  Erdos-Renyi, 2^20 vertices: 223 and 162 at 0.227.  Chung-Lu,
+    // 2.4 M vertices, 64 sources: 67 and 66 at 0.068; 50 and 61 at 0.013.  Up to kMbfsPullEdges edges
+    // it always pulls: a sweep is one launch, a push and its update are two (Erdos-Renyi, 65536
+    // vertices and 2^19 edges: 15 us and 19 to 25 from the first superstep on).
+    static constexpr uint64_t kMbfsPullEdges = 1ull << 19;
     static constexpr double kAlphaBfs = 3.0, kAlphaMbfs = 10.0, kBeta = 24.0;
     const medusa_opts& o;
     Algo algo;
@@ -183,7 +186,8 @@ struct Sched {
         : o(opts), algo(a), alpha(a == kMbfs ? kAlphaMbfs * sources : kAlphaBfs) {}
 
     bool heuristic_pull(const Frontier& f, bool cur_pull) const {
-        if (!cur_pull || algo == kMbfs) return (double)f.m_f > (double)f.m_u / alpha;
+        if (algo == kMbfs) return f.m <= kMbfsPullEdges || (double)f.m_f > (double)f.m_u / alpha;
+        if (!cur_pull) return (double)f.m_f > (double)f.m_u / alpha;
         return !((double)f.n_f < (double)f.n / kBeta);
     }
     // Direction for the next superstep: the learned policy's cheaper action when one is
