@@ -168,7 +168,7 @@ struct BfsArgs {
     BfsCtl* ctl;
     const float* policy;  // learned direction policy (device parameters) or null
     uint32_t n, nwords, large, grid, span;
-    unsigned long long exact_edges;  // frontier out-edges up to which a push claims exactly
+    unsigned long long m, exact_edges;  // frontier out-edges up to which a push claims exactly
 };
 
 // Segment span for n vertices: kBfsSlots segments cover [0, n) in whole compaction rounds.
@@ -206,83 +206,133 @@ __device__ __forceinline__ unsigned long long bfs_pack(uint32_t lo, uint32_t hi)
     return (unsigned long long)lo | ((unsigned long long)hi << 32);
 }
 
-// LDS of a workgroup's queue appends.
-struct BfsAppendLds {
-    uint32_t cnt[4];
-    unsigned long long deg[4];
-    uint32_t base;
-};
-
 constexpr uint32_t kRoundChunks = kBfsRound / 256;  // 64-vertex chunks per wave per workgroup round
 
-// One workgroup round's joins (every thread calls it; the round covers kBfsRound consecutive
-// vertices from `blk`, wave w holding chunks w * kRoundChunks + k, and all of them lie in one
-// queue segment): jm[k] is this wave's join mask of its chunk k.  The joined vertices are
-// appended to the next queue's segment with one atomic, whose packed increment also counts
-// them and their out-degrees; joined hubs (out-degree above `large`) also go to the next hub
-// queue (one atomic per wave that has any; hubs are few) and their degrees into `hacc`.
-__device__ __forceinline__ void bfs_append_round(const BfsArgs& a, const unsigned long long* jm, uint64_t blk,
-                                                 uint32_t* __restrict__ q_next, BfsLine* __restrict__ seg_next,
-                                                 uint32_t* __restrict__ hub_next, unsigned long long& hacc,
-                                                 BfsAppendLds& L) {
-    const uint32_t lane = threadIdx.x & (kWave - 1), wv = threadIdx.x / kWave;
-    const uint32_t sg = (uint32_t)(blk / a.span);
-    const uint32_t v0 = (uint32_t)blk + wv * kRoundChunks * kWave + lane;  // this lane's vertex in chunk 0
-    uint32_t deg[kRoundChunks], dsum = 0, cnt = 0;
-#pragma unroll
-    for (uint32_t k = 0; k < kRoundChunks; ++k) {
-        const uint32_t v = v0 + k * kWave;
-        deg[k] = (jm[k] >> lane) & 1ull ? a.row_ptr[v + 1] - a.row_ptr[v] : 0u;
+// Joined vertices that a wave holds in LDS before it appends them to the next queue: an append is a
+// chain of three round trips to memory (place, offsets, store), which a wave's rounds share, without a
+// barrier.  Compactions of the 2.4 M-vertex Chung-Lu graph, two to three rounds a wave: 16..24 us with an
+// append of the workgroup per round, 13 now.
+constexpr uint32_t kJoinCap = 1024, kJoinRound = 256;  // entries; most of them added per round
+struct BfsJoinLds {
+    unsigned long long words[4][kJoinCap / kWave];  // of a pull: next-bitmap words of the listed vertices
+    uint32_t v[4][kJoinCap];
+};
+struct BfsJoins {
+    uint32_t* list;  // the wave's, kJoinCap entries
+    uint32_t n = 0;  // uniform
+    // Every lane calls it: lanes with `joined` add v.
+    __device__ __forceinline__ void put(bool joined, uint32_t v) {
+        const unsigned long long m = __ballot(joined);
+        if (joined) list[n + lanes_below(m)] = v;
+        n += (uint32_t)__popcll(m);
     }
-    unsigned long long hm[kRoundChunks], hany = 0;
-    uint32_t hcnt = 0;
+};
+
+// Where a wave's joins go: a segment of the next queue and the hub queue.
+struct BfsSink {
+    uint32_t* q_next;
+    BfsLine* seg_next;
+    uint32_t* hub_next;
+};
+
+// The wave's held joins, at their place in the next queue; hubs (out-degree above `large`) also go to
+// the next hub queue (one atomic per 64 vertices that have any; hubs are few) and their degrees into
+// `hacc`.  `place` is called once, behind the first offsets' loads.  Returns the joins' out-degrees
+// (of distinct vertices: below 2^32), in every lane.
+template <class Place>
+__device__ __forceinline__ uint32_t bfs_flush_list(const BfsArgs& a, const BfsJoins& J, const BfsSink& o, Place place,
+                                                   unsigned long long& hacc) {
+    const uint32_t lane = threadIdx.x & (kWave - 1);
+    uint32_t* q = nullptr;
+    uint32_t dsum = 0;
+    constexpr uint32_t kN = 4;
+    for (uint32_t i0 = 0; i0 == 0 || i0 < J.n; i0 += kWave * kN) {
+        uint32_t v[kN], b[kN], e[kN];
 #pragma unroll
-    for (uint32_t k = 0; k < kRoundChunks; ++k) {
-        dsum += deg[k];
-        cnt += (uint32_t)__popcll(jm[k]);
-        hm[k] = __ballot(deg[k] > a.large);  // deg is 0 unless the lane's vertex joined
-        hany |= hm[k];
-        hcnt += (uint32_t)__popcll(hm[k]);
-    }
-    if (hany) {
-        uint32_t hb = 0;
-        if (lane == 0) hb = atomicAdd(&a.ctr->n_hub, hcnt);
-        hb = __shfl(hb, 0, kWave);
-#pragma unroll
-        for (uint32_t k = 0; k < kRoundChunks; ++k) {
-            if ((hm[k] >> lane) & 1ull) {
-                hub_next[hb + lanes_below(hm[k])] = v0 + k * kWave;
-                hacc += deg[k];
+        for (uint32_t j = 0; j < kN; ++j) {
+            const uint32_t i = i0 + j * kWave + lane;
+            v[j] = i < J.n ? J.list[i] : 0xFFFFFFFFu;
+            b[j] = e[j] = 0;
+            if (i < J.n) {
+                b[j] = a.row_ptr[v[j]];
+                e[j] = a.row_ptr[v[j] + 1];
             }
-            hb += (uint32_t)__popcll(hm[k]);
+        }
+        if (i0 == 0) q = place();
+#pragma unroll
+        for (uint32_t j = 0; j < kN; ++j) {
+            const uint32_t i = i0 + j * kWave + lane, deg = e[j] - b[j];
+            if (i < J.n) q[i] = v[j];
+            dsum += deg;
+            const unsigned long long hm = __ballot(deg > a.large);
+            if (hm) {
+                uint32_t hb = 0;
+                if (lane == 0) hb = atomicAdd(&a.ctr->n_hub, (uint32_t)__popcll(hm));
+                hb = __builtin_amdgcn_readfirstlane(hb);
+                if (deg > a.large) {
+                    o.hub_next[hb + lanes_below(hm)] = v[j];
+                    hacc += deg;
+                }
+            }
         }
     }
-    const unsigned long long dtot = wave_sum_u64(dsum);
-    if (lane == 0) {
-        L.cnt[wv] = cnt;
-        L.deg[wv] = dtot;
+    return __builtin_amdgcn_readlane(wave_incl_scan(dsum), kWave - 1);
+}
+
+// One wave's held joins appended to segment sg of the next queue: one atomic for their place and
+// number, one for their out-degrees, both performed on return.
+__device__ __forceinline__ void bfs_flush_wave(const BfsArgs& a, BfsJoins& J, const BfsSink& o, uint32_t sg,
+                                               unsigned long long& hacc) {
+    if (!J.n) return;  // uniform across the wave
+    const bool first = (threadIdx.x & (kWave - 1)) == 0;
+    wave_lds_fence();
+    uint32_t base = 0;
+    if (first) base = (uint32_t)atomicAdd(&o.seg_next[sg].v, bfs_pack(J.n, 0));
+    const uint32_t dsum = bfs_flush_list(
+        a, J, o, [&] { return o.q_next + (size_t)sg * a.span + __builtin_amdgcn_readfirstlane(base); }, hacc);
+    if (first) atomicAdd(&o.seg_next[sg].v, bfs_pack(0, dsum));
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    J.n = 0;
+    wave_lds_fence();
+}
+
+// The same for every wave of the workgroup at once (every thread calls it, all with the same sg), with
+// one pair of atomics: at the end of a superstep all waves append, and 4096 pairs on kBfsSlots
+// addresses took 1.5 us more than 1024.
+__device__ __forceinline__ void bfs_flush(const BfsArgs& a, BfsJoins& J, const BfsSink& o, uint32_t sg,
+                                          unsigned long long& hacc) {
+    __shared__ uint32_t s_n[4], s_base, s_deg[4];
+    const uint32_t lane = threadIdx.x & (kWave - 1), wv = threadIdx.x / kWave;
+    if (lane == 0) s_n[wv] = J.n;
+    __syncthreads();
+    const uint32_t n = s_n[0] + s_n[1] + s_n[2] + s_n[3];
+    if (!n) {  // uniform
+        __syncthreads();  // s_n is written again by the next call
+        return;
     }
+    if (threadIdx.x == 0) s_base = (uint32_t)atomicAdd(&o.seg_next[sg].v, bfs_pack(n, 0));
+    const uint32_t dsum = bfs_flush_list(
+        a, J, o,
+        [&] {
+            __syncthreads();
+            uint32_t at = s_base;
+            for (uint32_t w = 0; w < wv; ++w) at += s_n[w];
+            return o.q_next + (size_t)sg * a.span + at;
+        },
+        hacc);
+    if (lane == 0) s_deg[wv] = dsum;
     __syncthreads();
     if (threadIdx.x == 0) {
-        const uint32_t c = L.cnt[0] + L.cnt[1] + L.cnt[2] + L.cnt[3];
-        const unsigned long long d = L.deg[0] + L.deg[1] + L.deg[2] + L.deg[3];
-        L.base = c ? (uint32_t)atomicAdd(&seg_next[sg].v, bfs_pack(c, (uint32_t)d)) : 0u;
+        atomicAdd(&o.seg_next[sg].v, bfs_pack(0, s_deg[0] + s_deg[1] + s_deg[2] + s_deg[3]));
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     }
-    __syncthreads();
-    uint32_t off = L.base;
-    for (uint32_t w = 0; w < wv; ++w) off += L.cnt[w];
-#pragma unroll
-    for (uint32_t k = 0; k < kRoundChunks; ++k) {
-        if ((jm[k] >> lane) & 1ull) q_next[(size_t)sg * a.span + off + lanes_below(jm[k])] = v0 + k * kWave;
-        off += (uint32_t)__popcll(jm[k]);
-    }
-    __syncthreads();  // L is reused by the next round
+    J.n = 0;
 }
 
 // End of a counting kernel: the workgroup's hub degrees and probes go into its slot (one
 // atomic), then, with kDecide, it draws a ticket; returns true (to every thread) in the last
 // workgroup to finish.  Tickets are drawn only after the counter atomics have returned (the
-// asm makes the increment depend on their results), and every append of the block returned
+// asm makes the increment depend on their results), and every wave waited for its appends
 // before a barrier above, so when the last ticket is drawn every workgroup's counts have been
 // performed at the device's coherence point.  Device-scope atomics and atomic loads are
 // coherent across the XCDs' L2 caches without a fence (a device-scope release fence would
@@ -345,87 +395,48 @@ __device__ __forceinline__ uint32_t bfs_queue_at(const BfsArgs& a, const uint32_
     return q[(size_t)s * a.span + (i - pre[s])];
 }
 
-// Output of an exact-claim push: its winners go to the workgroup's segment of the next queue, the
-// next bitmap and the hub queue.
-struct BfsExactOut {
-    unsigned long long* nxt;
-    uint32_t* q_next;   // the workgroup's segment
-    BfsLine* seg_next;  // its counter
-    uint32_t* hub_next;
-};
-
-// A push claim of v for level `next`; a vertex whose visited bit is set is skipped (the bitmap
-// is small enough to stay in L2, the level array is not).  Plain: `level[v] = next`, a plain
-// store; every writer stores the same value, so the race is benign (as in the reference) and
-// the compaction after the push finds the vertices that joined.  Exact: a compare-and-swap
-// from -1 picks one winner per vertex, which sets its visited bit and is recorded at once
-// (bfs_record_round).
-template <bool kExact>
-__device__ __forceinline__ bool bfs_claim(const BfsArgs& a, uint32_t v, int32_t next) {
-    const unsigned long long bit = 1ull << (v & 63);
-    if (a.visited[v >> 6] & bit) return false;
-    if constexpr (!kExact) {
-        a.level[v] = next;
-        return false;
-    } else {
-        if (atomicCAS(&a.level[v], -1, next) != -1) return false;
-        atomicOr(&a.visited[v >> 6], bit);
-        return true;
-    }
-}
-
 constexpr uint32_t kPushUnroll = 4;  // out-edges per lane per round of the push, loads issued together
 
-// Winners of a round of an exact-claim push (the calling wave is converged; won[j] / v[j] for
-// the round's kPushUnroll edges of this lane): one packed atomic per wave appends them to the
-// workgroup's segment of the next queue and counts them with their out-degrees; each sets its bit in the
-// next bitmap; hubs also go to the next hub queue.
-__device__ __forceinline__ void bfs_record_round(const BfsArgs& a, const BfsExactOut& o, const bool* won,
-                                                 const uint32_t* v, unsigned long long& hacc) {
-    unsigned long long wm[kPushUnroll], any = 0;
+// Claims of a round's targets v[j] (0xFFFFFFFF: none) for level `next`; a vertex whose visited bit is
+// set is skipped (the bitmap is small enough to stay in L2, the level array is not).  Plain: `level[v]
+// = next`, a plain store; every writer stores the same value, so the race is benign (as in the
+// reference) and the compaction after the push finds the vertices that joined.
+__device__ __forceinline__ void bfs_claim_plain(const BfsArgs& a, const uint32_t (&v)[kPushUnroll], int32_t next) {
+#pragma unroll
+    for (uint32_t j = 0; j < kPushUnroll; ++j)
+        if (v[j] != 0xFFFFFFFFu && !(a.visited[v[j] >> 6] & (1ull << (v[j] & 63)))) a.level[v[j]] = next;
+}
+
+// Exact: whoever sets the visited bit wins the vertex, stores its level, sets its bit in the next
+// bitmap and holds it for the next queue's segment `own`.  The calling wave is converged.  A wave with
+// many out-edges goes through this chain of dependent accesses once per round, so the round's loads
+// and atomics are issued together (a compare-and-swap on the level one after the other, then the
+// bit: 34..36 us for 46 K and 62 K out-edges of that graph, 20 now).
+struct BfsExact {
+    unsigned long long* nxt;
+    BfsSink sink;
+    uint32_t own;
+    BfsJoins J;
+};
+__device__ __forceinline__ void bfs_claim_exact(const BfsArgs& a, BfsExact& x, const uint32_t (&v)[kPushUnroll],
+                                                int32_t next, unsigned long long& hacc) {
+    unsigned long long seen[kPushUnroll];
+#pragma unroll
+    for (uint32_t j = 0; j < kPushUnroll; ++j) seen[j] = v[j] != 0xFFFFFFFFu ? a.visited[v[j] >> 6] : ~0ull;
+#pragma unroll
+    for (uint32_t j = 0; j < kPushUnroll; ++j)
+        if (!((seen[j] >> (v[j] & 63)) & 1ull)) seen[j] = atomicOr(&a.visited[v[j] >> 6], 1ull << (v[j] & 63));
 #pragma unroll
     for (uint32_t j = 0; j < kPushUnroll; ++j) {
-        wm[j] = __ballot(won[j]);
-        any |= wm[j];
-    }
-    if (!any) return;
-    const uint32_t lane = threadIdx.x & (kWave - 1);
-    uint32_t deg[kPushUnroll], dsum = 0, cnt = 0;
-#pragma unroll
-    for (uint32_t j = 0; j < kPushUnroll; ++j) deg[j] = won[j] ? a.row_ptr[v[j] + 1] - a.row_ptr[v[j]] : 0u;
-#pragma unroll
-    for (uint32_t j = 0; j < kPushUnroll; ++j) {
-        if (won[j]) atomicOr(&o.nxt[v[j] >> 6], 1ull << (v[j] & 63));
-        dsum += deg[j];
-        cnt += (uint32_t)__popcll(wm[j]);
-    }
-    const unsigned long long dtot = wave_sum_u64(dsum);
-    uint32_t base = 0;
-    if (lane == 0) base = (uint32_t)atomicAdd(&o.seg_next->v, bfs_pack(cnt, (uint32_t)dtot));
-    base = __shfl(base, 0, kWave);
-    unsigned long long hm[kPushUnroll], hany = 0;
-    uint32_t hcnt = 0;
-#pragma unroll
-    for (uint32_t j = 0; j < kPushUnroll; ++j) {
-        if (won[j]) o.q_next[base + lanes_below(wm[j])] = v[j];
-        base += (uint32_t)__popcll(wm[j]);
-        hm[j] = __ballot(won[j] && deg[j] > a.large);
-        hany |= hm[j];
-        hcnt += (uint32_t)__popcll(hm[j]);
-    }
-    if (hany) {
-        uint32_t hb = 0;
-        if (lane == 0) hb = atomicAdd(&a.ctr->n_hub, hcnt);
-        hb = __shfl(hb, 0, kWave);
-#pragma unroll
-        for (uint32_t j = 0; j < kPushUnroll; ++j) {
-            if ((hm[j] >> lane) & 1ull) {
-                o.hub_next[hb + lanes_below(hm[j])] = v[j];
-                hacc += deg[j];
-            }
-            hb += (uint32_t)__popcll(hm[j]);
+        const bool won = !((seen[j] >> (v[j] & 63)) & 1ull);
+        if (won) {
+            a.level[v[j]] = next;
+            atomicOr(&x.nxt[v[j] >> 6], 1ull << (v[j] & 63));
         }
+        x.J.put(won, v[j]);
     }
+    static_assert(kJoinRound >= kWave * kPushUnroll, "a round's winners");
+    if (x.J.n > kJoinCap - kJoinRound) bfs_flush_wave(a, x.J, x.sink, x.own, hacc);
 }
 
 // Wave-cooperative push over the frontier queue (hubs and vertices without out-edges are
@@ -437,7 +448,7 @@ __device__ __forceinline__ void bfs_record_round(const BfsArgs& a, const BfsExac
 template <bool kExact>
 __device__ __forceinline__ void push_queue(const BfsArgs& a, const uint32_t* __restrict__ q, const uint32_t* pre,
                                            int32_t next, uint32_t wave0, uint32_t nwaves, uint32_t (*s_beg)[kWave],
-                                           uint32_t (*s_off)[kWave], const BfsExactOut& o, unsigned long long& hacc) {
+                                           uint32_t (*s_off)[kWave], BfsExact& x, unsigned long long& hacc) {
     const uint32_t lane = threadIdx.x & (kWave - 1), wv = threadIdx.x / kWave;
     const uint32_t qn = pre[kBfsSlots];
     for (uint64_t r = 0; wave0 + r * kWave * nwaves < qn; ++r) {  // uniform across the wave
@@ -469,11 +480,8 @@ __device__ __forceinline__ void push_queue(const BfsArgs& a, const uint32_t* __r
                     v[j] = a.col[s_beg[wv][lo] + (e - s_off[wv][lo])];
                 }
             }
-            bool won[kPushUnroll];
-#pragma unroll
-            for (uint32_t j = 0; j < kPushUnroll; ++j)
-                won[j] = v[j] != 0xFFFFFFFFu && bfs_claim<kExact>(a, v[j], next);
-            if constexpr (kExact) bfs_record_round(a, o, won, v, hacc);
+            if constexpr (kExact) bfs_claim_exact(a, x, v, next, hacc);
+            else bfs_claim_plain(a, v, next);
         }
         __builtin_amdgcn_wave_barrier();
     }
@@ -485,7 +493,7 @@ __device__ __forceinline__ void push_queue(const BfsArgs& a, const uint32_t* __r
 // one high-degree vertex still spreads over many waves.
 __device__ __forceinline__ void push_tiny(const BfsArgs& a, const uint32_t* __restrict__ q, const uint32_t* pre,
                                           int32_t next, uint32_t (*s_beg)[kWave], uint32_t (*s_off)[kWave],
-                                          const BfsExactOut& o, unsigned long long& hacc) {
+                                          BfsExact& x, unsigned long long& hacc) {
     const uint32_t lane = threadIdx.x & (kWave - 1), wv = threadIdx.x / kWave;
     const uint32_t qn = pre[kBfsSlots];
     const uint64_t e_begin = ((uint64_t)blockIdx.x * (blockDim.x / kWave) + wv) * kWave * kPushUnroll;
@@ -514,17 +522,14 @@ __device__ __forceinline__ void push_tiny(const BfsArgs& a, const uint32_t* __re
             v[j] = a.col[s_beg[wv][lo] + ((uint32_t)e - s_off[wv][lo])];
         }
     }
-    bool won[kPushUnroll];
-#pragma unroll
-    for (uint32_t j = 0; j < kPushUnroll; ++j) won[j] = v[j] != 0xFFFFFFFFu && bfs_claim<true>(a, v[j], next);
-    bfs_record_round(a, o, won, v, hacc);
+    bfs_claim_exact(a, x, v, next, hacc);
 }
 
 // Hubs: each vertex of the hub queue is split into `split` contiguous edge ranges, one per
 // workgroup item; the `nwg` workgroups taking part stride over the items.
 template <bool kExact>
 __device__ __forceinline__ void push_hubs(const BfsArgs& a, const uint32_t* __restrict__ q, uint32_t qn, int32_t next,
-                                          uint32_t wg0, uint32_t nwg, const BfsExactOut& o,
+                                          uint32_t wg0, uint32_t nwg, BfsExact& x,
                                           unsigned long long& hacc) {
     const uint32_t lane = threadIdx.x & (kWave - 1);
     uint32_t split = nwg / qn;
@@ -537,16 +542,13 @@ __device__ __forceinline__ void push_hubs(const BfsArgs& a, const uint32_t* __re
         for (uint32_t k0 = lo + (threadIdx.x - lane) * kPushUnroll; k0 < hi;
              k0 += blockDim.x * kPushUnroll) {  // uniform per wave
             uint32_t v[kPushUnroll];
-            bool won[kPushUnroll];
 #pragma unroll
             for (uint32_t j = 0; j < kPushUnroll; ++j) {
                 const uint32_t k = k0 + j * kWave + lane;
                 v[j] = k < hi ? a.col[k] : 0xFFFFFFFFu;
             }
-#pragma unroll
-            for (uint32_t j = 0; j < kPushUnroll; ++j)
-                won[j] = v[j] != 0xFFFFFFFFu && bfs_claim<kExact>(a, v[j], next);
-            if constexpr (kExact) bfs_record_round(a, o, won, v, hacc);
+            if constexpr (kExact) bfs_claim_exact(a, x, v, next, hacc);
+            else bfs_claim_plain(a, v, next);
         }
     }
 }
@@ -554,42 +556,61 @@ __device__ __forceinline__ void push_hubs(const BfsArgs& a, const uint32_t* __re
 constexpr uint32_t kPullLane = 32;  // in-degree up to which one lane scans a vertex alone
 constexpr uint32_t kPullGroup = 4;  // in-edges a lane probes per round
 
-// Bottom-up over this wave's kRoundChunks chunks of 64 consecutive vertices from `base` (one vertex
-// of each chunk per lane; the wave is converged): an unvisited vertex (visited bitmap) joins if any
-// in-neighbour is in the frontier bitmap.  The chunks go through the chain of dependent loads
-// (visited word, in-offsets, sources, bitmap words) together, so a round of the workgroup costs one
-// such chain and not one per chunk (2.4 M-vertex Chung-Lu graph, pulls of 1.2 M to 0.5 M unvisited
-// vertices: 37 .. 31 us -> 34 .. 26).  A lane scans a vertex of in-degree <= kPullLane
-// alone, kPullGroup in-edges of every chunk per round; above that the whole wave scans it 64
-// in-edges at a time and stops at the first hit (ballot), so one high in-degree vertex does not
-// hold its wave for hundreds of sequential probes.  jm[k] receives chunk k's join mask, which is
-// also written as the chunk's word of the next bitmap.  `probes` counts in-edges examined up to and
-// including the first hit in either case.
-__device__ __forceinline__ void pull_chunks(const BfsArgs& a, const unsigned long long* __restrict__ cur,
-                                            unsigned long long* __restrict__ nxt, uint64_t base, int32_t next,
-                                            const unsigned long long (&vis)[kRoundChunks],
-                                            const uint32_t (&b)[kRoundChunks], const uint32_t (&e)[kRoundChunks],
-                                            unsigned long long (&jm)[kRoundChunks], unsigned long long& probes) {
+// Segment of the next queue for the joins of a round of kBfsRound vertices from `blk`: the rounds are
+// dealt over the segments, so none gets more than its span, and with a multiple of kBfsSlots
+// workgroups all rounds of one have the same segment.
+__device__ __forceinline__ uint32_t bfs_round_segment(uint64_t blk) { return (uint32_t)(blk / kBfsRound) % kBfsSlots; }
+
+// A wave's round (join masks of its kRoundChunks chunks from vertex v0) held, and the held ones
+// appended when the list is full or the next round has another segment.
+__device__ __forceinline__ void bfs_join_round(const BfsArgs& a, BfsJoins& J, const BfsSink& o,
+                                               const unsigned long long (&jm)[kRoundChunks], uint64_t v0, uint64_t blk,
+                                               unsigned long long& hacc) {
     const uint32_t lane = threadIdx.x & (kWave - 1);
-    const uint64_t word0 = base / kWave;
-    unsigned long long joined[kRoundChunks];
-    unsigned long long big[kRoundChunks];
+    static_assert(kJoinRound >= kWave * kRoundChunks, "a round's joins");
+#pragma unroll
+    for (uint32_t k = 0; k < kRoundChunks; ++k) J.put((jm[k] >> lane) & 1ull, (uint32_t)(v0 + k * kWave) + lane);
+    if (gridDim.x % kBfsSlots || J.n > kJoinCap - kJoinRound) bfs_flush_wave(a, J, o, bfs_round_segment(blk), hacc);
+}
+
+constexpr uint32_t kPullWords = kJoinCap / kWave;          // visited words a wave takes at a time
+constexpr uint32_t kPullRounds = kPullWords / kRoundChunks;  // in rounds
+
+// Bottom-up probe of one vertex per lane and j (in-edges [b, e), none if b == e): joined[j] where a source
+// is in the frontier bitmap.  A lane scans a vertex of in-degree <= kPullLane alone, kPullGroup in-edges
+// of every j per round; above that the whole wave scans it 64 in-edges at a time and stops at the
+// first hit (ballot), so one high in-degree vertex does not hold its wave for hundreds of sequential
+// probes.  `probes` counts in-edges examined up to and including the first hit in either case.
+__device__ __forceinline__ void pull_probe(const BfsArgs& a, const unsigned long long* __restrict__ cur,
+                                           const uint32_t (&b)[kRoundChunks], const uint32_t (&e)[kRoundChunks],
+                                           bool (&joined)[kRoundChunks], unsigned long long& probes) {
+    typedef uint32_t Sources __attribute__((ext_vector_type(kPullGroup), aligned(4)));
+    const uint32_t lane = threadIdx.x & (kWave - 1);
     uint32_t sb[kRoundChunks], se[kRoundChunks];
     bool more = false;
 #pragma unroll
     for (uint32_t k = 0; k < kRoundChunks; ++k) {
-        big[k] = __ballot(e[k] - b[k] > kPullLane);
-        joined[k] = 0;
+        joined[k] = false;
         sb[k] = b[k];
         se[k] = e[k] - b[k] > kPullLane ? b[k] : e[k];
         more |= sb[k] < se[k];
     }
     while (__ballot(more)) {  // uniform across the wave
-        uint32_t u[kRoundChunks][kPullGroup];
+        // a group is one load where the array goes on that far (4-byte aligned; entries past se unused)
+        Sources u[kRoundChunks];
 #pragma unroll
-        for (uint32_t k = 0; k < kRoundChunks; ++k)
+        for (uint32_t k = 0; k < kRoundChunks; ++k) {
+            u[k] = Sources{0, 0, 0, 0};
+            if (sb[k] < se[k]) {
+                if (sb[k] + kPullGroup <= a.m) {
+                    u[k] = *reinterpret_cast<const Sources*>(a.csrc + sb[k]);
+                } else {
 #pragma unroll
-            for (uint32_t j = 0; j < kPullGroup; ++j) u[k][j] = sb[k] + j < se[k] ? a.csrc[sb[k] + j] : 0u;
+                    for (uint32_t j = 0; j < kPullGroup; ++j)
+                        if (sb[k] + j < se[k]) u[k][j] = a.csrc[sb[k] + j];
+                }
+            }
+        }
         unsigned long long word[kRoundChunks][kPullGroup];
 #pragma unroll
         for (uint32_t k = 0; k < kRoundChunks; ++k)
@@ -605,8 +626,7 @@ __device__ __forceinline__ void pull_chunks(const BfsArgs& a, const unsigned lon
             const uint32_t left = min(se[k] - sb[k], kPullGroup);
             if (hit < kPullGroup) {
                 probes += hit + 1;
-                a.level[base + k * kWave + lane] = next;
-                joined[k] = 1;
+                joined[k] = true;
                 sb[k] = se[k];
             } else {
                 probes += left;
@@ -617,8 +637,7 @@ __device__ __forceinline__ void pull_chunks(const BfsArgs& a, const unsigned lon
     }
 #pragma unroll
     for (uint32_t k = 0; k < kRoundChunks; ++k) {
-        jm[k] = __ballot(joined[k] != 0);
-        for (unsigned long long bm = big[k]; bm; bm &= bm - 1) {
+        for (unsigned long long bm = __ballot(e[k] - b[k] > kPullLane); bm; bm &= bm - 1) {
             const uint32_t owner = __builtin_ctzll(bm);
             const uint32_t vb = __shfl(b[k], owner, kWave), ve = __shfl(e[k], owner, kWave);
             for (uint32_t k0 = vb; k0 < ve; k0 += kWave) {
@@ -629,64 +648,83 @@ __device__ __forceinline__ void pull_chunks(const BfsArgs& a, const unsigned lon
                     hit = (cur[u >> 6] >> (u & 63)) & 1ull;
                 }
                 const unsigned long long hm = __ballot(hit);
-                if (hm) {
-                    if (lane == 0) {
-                        probes += __builtin_ctzll(hm) + 1;
-                        a.level[base + k * kWave + owner] = next;
-                    }
-                    jm[k] |= 1ull << owner;
-                    break;
+                if (lane == owner) {
+                    probes += hm ? (uint32_t)__builtin_ctzll(hm) + 1 : min(ve - k0, (uint32_t)kWave);
+                    joined[k] = joined[k] || hm;
                 }
-                if (lane == 0) probes += min(ve - k0, (uint32_t)kWave);
+                if (hm) break;
             }
-        }
-        if (lane == 0 && word0 + k < a.nwords) {
-            nxt[word0 + k] = jm[k];
-            a.visited[word0 + k] = vis[k] | jm[k];  // the wave owns this word in a pull
         }
     }
 }
 
-// Pull superstep: workgroup rounds of kBfsRound consecutive vertices, wave w taking chunks
-// w * kRoundChunks + k; each wave writes its chunks' words of the next bitmap whole and the
-// round's joins are appended to the next queue, so the pull needs no compaction.
+// Pull superstep: workgroup rounds of kBfsRound consecutive vertices, of which each wave owns
+// kRoundChunks visited words.  A wave lists the unvisited vertices of kPullRounds rounds, which then
+// fill its lanes however few of each word they are, and probes kRoundChunks of them per lane at a time;
+// the joins replace them at the front of the list and go to the next queue together, and every owned
+// word of the next and visited bitmaps is written whole, so the pull needs no compaction.  Bound by
+// the chain of dependent loads (visited word, in-offsets, sources, bitmap words), which a pass over
+// the list goes through once.  Chung-Lu, 2.4 M vertices, pulls of 1.3 M to 0.5 M unvisited vertices:
+// 34..26 us with a lane per vertex of the round, 25..20 now.
 __device__ __forceinline__ void pull_all(const BfsArgs& a, const unsigned long long* __restrict__ cur,
-                                         unsigned long long* __restrict__ nxt, uint32_t* __restrict__ q_next,
-                                         BfsLine* __restrict__ seg_next, uint32_t* __restrict__ hub_next, int32_t next,
-                                         unsigned long long& hacc, unsigned long long& probes, BfsAppendLds& L) {
-    const uint32_t lane = threadIdx.x & (kWave - 1), wv = threadIdx.x / kWave;
-    const uint64_t step = (uint64_t)gridDim.x * kBfsRound;
-    const uint64_t first = (uint64_t)blockIdx.x * kBfsRound + (uint64_t)wv * kRoundChunks * kWave;
-    // the visited words of 64 / kRoundChunks rounds, one per lane, in one load: lane r * kRoundChunks
-    // + k holds round r's chunk k
-    constexpr uint32_t kAhead = kWave / kRoundChunks;
-    uint64_t blk = (uint64_t)blockIdx.x * kBfsRound;
-    for (uint64_t r0 = 0; blk < a.n; r0 += kAhead) {
-        const uint64_t w = (first + (r0 + lane / kRoundChunks) * step) / kWave + lane % kRoundChunks;
-        const unsigned long long mine = w < a.nwords ? a.visited[w] : ~0ull;
-        unsigned long long vis[kRoundChunks];
-        uint32_t b[kRoundChunks], e[kRoundChunks];  // in-edges of the lane's unvisited vertices
-        auto offsets = [&](uint32_t r) {
-            const uint64_t base = first + (r0 + r) * step;
+                                         unsigned long long* __restrict__ nxt, const BfsSink& o, int32_t next,
+                                         unsigned long long& hacc, unsigned long long& probes, BfsJoins J,
+                                         unsigned long long* words) {
+    const uint32_t lane = threadIdx.x & (kWave - 1), wv = threadIdx.x / kWave, grid = gridDim.x;
+    // all rounds of a pass over the list have the same segment
+    const uint32_t rounds = grid % kBfsSlots ? 1u : kPullRounds;
+    for (uint64_t round0 = blockIdx.x; round0 * kBfsRound < a.n; round0 += (uint64_t)rounds * grid) {
+        // lane l owns word l % kRoundChunks of the wave's part of round l / kRoundChunks
+        const uint64_t w = (round0 + (uint64_t)(lane / kRoundChunks) * grid) * (kBfsRound / kWave) + wv * kRoundChunks +
+                           lane % kRoundChunks;
+        const bool owner = lane < rounds * kRoundChunks && w < a.nwords;
+        const unsigned long long vis = owner ? a.visited[w] : 0ull;
+        unsigned long long open = owner ? ~vis : 0ull;
+        if (owner && (w + 1) * kWave > a.n) open &= (1ull << (a.n % kWave)) - 1;
+        uint32_t cand = 0;
+        const uint32_t owned = (uint32_t)__popcll(__ballot(owner));  // lanes 0, 1, .. (a round may end short)
+        for (uint32_t i = 0; i < owned; ++i) {
+            const unsigned long long m = bfs_pack(__builtin_amdgcn_readlane((uint32_t)open, i),
+                                                  __builtin_amdgcn_readlane((uint32_t)(open >> 32), i));
+            const uint32_t v = (uint32_t)__builtin_amdgcn_readlane((uint32_t)w, i) * kWave + lane;
+            if ((m >> lane) & 1ull) J.list[cand + lanes_below(m)] = v;
+            cand += (uint32_t)__popcll(m);
+        }
+        if (lane < kPullWords) words[lane] = 0;
+        wave_lds_fence();
+        for (uint32_t i0 = 0; i0 < cand; i0 += kWave * kRoundChunks) {
+            uint32_t v[kRoundChunks], b[kRoundChunks], e[kRoundChunks];
+            bool joined[kRoundChunks];
 #pragma unroll
             for (uint32_t k = 0; k < kRoundChunks; ++k) {
-                vis[k] = bfs_pack(__builtin_amdgcn_readlane((uint32_t)mine, r * kRoundChunks + k),
-                                  __builtin_amdgcn_readlane((uint32_t)(mine >> 32), r * kRoundChunks + k));
-                const uint64_t v = base + k * kWave + lane;
+                const uint32_t i = i0 + k * kWave + lane;
+                v[k] = i < cand ? J.list[i] : 0u;
                 b[k] = e[k] = 0;
-                if (v < a.n && !((vis[k] >> lane) & 1ull)) {
-                    b[k] = a.cptr[v];
-                    e[k] = a.cptr[v + 1];
+                if (i < cand) {
+                    b[k] = a.cptr[v[k]];
+                    e[k] = a.cptr[v[k] + 1];
                 }
             }
-        };
-        offsets(0);
-        for (uint32_t r = 0; r < kAhead && blk < a.n; ++r, blk += step) {
-            unsigned long long jm[kRoundChunks];
-            pull_chunks(a, cur, nxt, first + (r0 + r) * step, next, vis, b, e, jm, probes);
-            if (r + 1 < kAhead) offsets(r + 1);  // in flight while this round's joins are appended
-            bfs_append_round(a, jm, blk, q_next, seg_next, hub_next, hacc, L);
+            wave_lds_fence();
+            pull_probe(a, cur, b, e, joined, probes);
+#pragma unroll
+            for (uint32_t k = 0; k < kRoundChunks; ++k) {
+                if (joined[k]) {
+                    a.level[v[k]] = next;
+                    const uint32_t d = v[k] / kBfsRound - (uint32_t)round0;  // 0, grid, 2 grid or 3 grid
+                    const uint32_t r = (d >= grid) + (d >= 2 * grid) + (d >= 3 * grid);
+                    atomicOr(&words[r * kRoundChunks + v[k] / kWave % kRoundChunks], 1ull << (v[k] % kWave));
+                }
+                J.put(joined[k], v[k]);  // behind the entries read so far
+            }
         }
+        wave_lds_fence();
+        if (owner) {
+            const unsigned long long m = words[lane];
+            nxt[w] = m;
+            a.visited[w] = vis | m;  // the wave owns this word in a pull
+        }
+        bfs_flush(a, J, o, bfs_round_segment(round0 * kBfsRound), hacc);
     }
 }
 
@@ -1234,11 +1272,10 @@ __global__ __launch_bounds__(64) void k_zero_counters(BfsCounters* c, uint32_t p
 // kBfsRound consecutive vertices (wave w the chunks w * kRoundChunks + k), whose level loads are
 // issued together.
 __device__ __forceinline__ void compact_level(const BfsArgs& a, int32_t next, unsigned long long* __restrict__ nxt,
-                                              uint32_t* __restrict__ q_next, BfsLine* __restrict__ seg_next,
-                                              uint32_t* __restrict__ hub_next, unsigned long long& hacc,
-                                              BfsAppendLds& L) {
+                                              const BfsSink& o, unsigned long long& hacc, BfsJoins J) {
     const uint32_t lane = threadIdx.x & (kWave - 1), wv = threadIdx.x / kWave;
-    for (uint64_t blk = (uint64_t)blockIdx.x * kBfsRound; blk < a.n; blk += (uint64_t)gridDim.x * kBfsRound) {
+    uint64_t blk = (uint64_t)blockIdx.x * kBfsRound;
+    for (; blk < a.n; blk += (uint64_t)gridDim.x * kBfsRound) {
         const uint64_t c0 = blk / kWave + wv * kRoundChunks;  // first chunk of this wave
         int32_t lv[kRoundChunks];
 #pragma unroll
@@ -1256,8 +1293,9 @@ __device__ __forceinline__ void compact_level(const BfsArgs& a, int32_t next, un
                 a.visited[c0 + k] = vm;
             }
         }
-        bfs_append_round(a, jm, blk, q_next, seg_next, hub_next, hacc, L);
+        bfs_join_round(a, J, o, jm, c0 * kWave, blk, hacc);
     }
+    bfs_flush(a, J, o, bfs_round_segment(blk), hacc);
 }
 
 // One launch of the superstep loop, doing what the control block says:
@@ -1276,7 +1314,12 @@ template <bool kDecide>
 __global__ __launch_bounds__(256) void k_bfs_super(BfsArgs a, uint32_t slot) {
     __shared__ uint32_t s_beg[4][kWave], s_off[4][kWave];
     __shared__ uint32_t s_pre[kBfsSlots + 1];
-    __shared__ BfsAppendLds s_app;
+    // the joins of the whole grid's supersteps, or the solo supersteps' frontier
+    union Work {
+        BfsJoinLds joins;
+        BfsSoloLds<256> solo;
+    };
+    __shared__ alignas(16) unsigned char s_work[kDecide ? sizeof(Work) : sizeof(BfsJoinLds)];
     __shared__ BfsCtl s_c;
     __shared__ float s_params[kDecide ? kMlpWaveLds : 4];
     const BfsCtl* ctl = a.ctl + slot;
@@ -1296,12 +1339,11 @@ __global__ __launch_bounds__(256) void k_bfs_super(BfsArgs a, uint32_t slot) {
     const int32_t step = ctl->step, next = step + 1;
     const uint32_t par = (uint32_t)step & 1u, t3 = ctl->rot;
     unsigned long long* nxt = a.bm[t3 == 2 ? 0 : t3 + 1];
-    uint32_t* q_next = a.q[par ^ 1u];
-    BfsLine* seg_next = a.ctr->seg[par ^ 1u];
-    uint32_t* hub_next = a.hub[par ^ 1u];
+    const BfsSink sink{a.q[par ^ 1u], a.ctr->seg[par ^ 1u], a.hub[par ^ 1u]};
+    const BfsJoins joins{reinterpret_cast<BfsJoinLds*>(s_work)->v[threadIdx.x / kWave]};
     unsigned long long hacc = 0;
     if (ctl->pending) {
-        compact_level(a, next, nxt, q_next, seg_next, hub_next, hacc, s_app);
+        compact_level(a, next, nxt, sink, hacc, joins);
         if (bfs_finish<kDecide>(a.ctr, hacc)) bfs_decide(a, slot, &s_c, s_params);
         return;
     }
@@ -1310,17 +1352,17 @@ __global__ __launch_bounds__(256) void k_bfs_super(BfsArgs a, uint32_t slot) {
     for (uint64_t w = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; w < a.nwords; w += stride) clr[w] = 0;
     if (ctl->pull) {
         unsigned long long probes = 0;
-        pull_all(a, a.bm[t3], nxt, q_next, seg_next, hub_next, next, hacc, probes, s_app);
+        pull_all(a, a.bm[t3], nxt, sink, next, hacc, probes, joins,
+                 reinterpret_cast<BfsJoinLds*>(s_work)->words[threadIdx.x / kWave]);
         if (bfs_finish<kDecide>(a.ctr, hacc + (probes << 32))) bfs_decide(a, slot, &s_c, s_params);
         return;
     }
-    const uint32_t own = blockIdx.x % kBfsSlots;
-    const BfsExactOut o{nxt, q_next + (size_t)own * a.span, seg_next + own, hub_next};
+    BfsExact x{nxt, sink, blockIdx.x % kBfsSlots, joins};
     const uint32_t hub = ctl->hub_wgs, small = ctl->small;
     if constexpr (kDecide) {
         if (small == 3) {
             if (blockIdx.x != 0) return;  // (each cleared its share of the bitmap above)
-            __shared__ BfsSoloLds<256> L;
+            BfsSoloLds<256>& L = *reinterpret_cast<BfsSoloLds<256>*>(s_work);
             bfs_queue_prefix(a.ctr->seg[par], s_pre);
             const uint32_t qn = s_pre[kBfsSlots];
             for (uint32_t i = threadIdx.x; i < qn; i += 256) {
@@ -1343,20 +1385,21 @@ __global__ __launch_bounds__(256) void k_bfs_super(BfsArgs a, uint32_t slot) {
     if (!small) pass_on(1);
     if (small == 2) {
         bfs_queue_prefix(a.ctr->seg[par], s_pre);
-        push_tiny(a, a.q[par], s_pre, next, s_beg, s_off, o, hacc);
+        push_tiny(a, a.q[par], s_pre, next, s_beg, s_off, x, hacc);
     } else if (blockIdx.x < hub) {
         if (small)
-            push_hubs<true>(a, a.hub[par], ctl->n_large, next, blockIdx.x, hub, o, hacc);
+            push_hubs<true>(a, a.hub[par], ctl->n_large, next, blockIdx.x, hub, x, hacc);
         else
-            push_hubs<false>(a, a.hub[par], ctl->n_large, next, blockIdx.x, hub, o, hacc);
+            push_hubs<false>(a, a.hub[par], ctl->n_large, next, blockIdx.x, hub, x, hacc);
     } else {
         bfs_queue_prefix(a.ctr->seg[par], s_pre);
         const uint32_t wg = blockIdx.x - hub, nwg = gridDim.x - hub, w0 = wg * 4 + threadIdx.x / kWave;
         if (small)
-            push_queue<true>(a, a.q[par], s_pre, next, w0, nwg * 4, s_beg, s_off, o, hacc);
+            push_queue<true>(a, a.q[par], s_pre, next, w0, nwg * 4, s_beg, s_off, x, hacc);
         else
-            push_queue<false>(a, a.q[par], s_pre, next, w0, nwg * 4, s_beg, s_off, o, hacc);
+            push_queue<false>(a, a.q[par], s_pre, next, w0, nwg * 4, s_beg, s_off, x, hacc);
     }
+    if (small) bfs_flush(a, x.J, x.sink, x.own, hacc);
     if (small && bfs_finish<kDecide>(a.ctr, hacc)) bfs_decide(a, slot, &s_c, s_params);
 }
 
@@ -1430,6 +1473,7 @@ static BfsArgs bfs_args(medusa_graph* g, const BfsBufs& B, uint32_t large, uint3
     a.large = large;
     a.grid = grid;
     a.span = bfs_span(g->n);
+    a.m = g->m;
     a.exact_edges = bfs_exact_edges(g->n);
     return a;
 }

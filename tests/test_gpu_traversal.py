@@ -124,6 +124,28 @@ def test_bfs_frontiers_of_one_workgroup(oracle, n, width, fan):
             assert np.array_equal(G.bfs_multi(np.resize(sources, k))[0], want), k
 
 
+@pytest.mark.parametrize("n", [32 * 1024 + 1, 140_000, 262_144])
+@pytest.mark.parametrize("fan", [700, 60_000])
+def test_bfs_held_joins(oracle, n, fan):
+    """Waves with several rounds of vertices (one segment for all of a workgroup's at 32 and 64
+    workgroups, one each at 33): a source whose targets all join at once, so a wave's list of joins
+    fills up and is appended in the middle, then a random graph that leaves some vertices to pulls of
+    sparsely unvisited words; hubs among the joins."""
+    rng = np.random.default_rng(n + fan)
+    first = rng.permutation(np.arange(1, n))[:min(fan, n - 1)]
+    dense = np.arange(1, min(fan, n - 1) + 1)
+    src = np.concatenate([np.zeros(len(first), np.int64), np.full(len(dense), first[0]), rng.integers(0, n, 2 * n)])
+    dst = np.concatenate([first, dense, rng.integers(0, n, 2 * n)])
+    rp, col, _ = csr_from_edges(n, np.stack([src, dst], 1))
+    want = oracle.bfs_queue(rp, col, 0)
+    with md.Graph(rp, col) as G:
+        for d in _dirs():
+            for grid in (2, 32, 33, 64, 0):
+                got, st = G.bfs(0, direction=d, grid=grid, large_degree=6)
+                assert np.array_equal(got, want), (d, grid)
+                assert st.reached == (want >= 0).sum(), (d, grid)
+
+
 def test_bfs_edge_cases(oracle):
     with md.Graph(np.array([0, 0], np.uint32), np.array([], np.uint32)) as G:
         lv, st = G.bfs(0)
