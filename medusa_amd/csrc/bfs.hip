@@ -93,7 +93,7 @@ struct BfsHost {
     uint32_t count, mode;
     uint32_t src[kBfsHostSources];
 };
-size_t bfs_host_words() { return (sizeof(BfsHost) + 7) / 8; }
+static_assert(sizeof(BfsHost) <= kHostWords * 8, "pinned memory of a handle");
 
 // Workgroups of a push expansion given to the hub queue: in proportion to its share of
 // the frontier's out-edges, at least one for each non-empty queue.
@@ -1517,7 +1517,7 @@ static void bfs_run_device(medusa_graph* g, const BfsBufs& B, uint32_t nsrc, con
     const uint32_t mode = bfs_mode(o);
     const float* policy = mode == 3 ? policy_device_params(o.policy) : nullptr;
     const BfsArgs a = bfs_args(g, B, large, grid, policy);
-    BfsHost* host = reinterpret_cast<BfsHost*>(g->h_bfs.p);
+    BfsHost* host = host_counters<BfsHost>(g);
 
     // where the closing kernel puts the levels: the output itself, or pinned memory for a small host
     // output; larger host outputs are copied afterwards
@@ -1605,7 +1605,7 @@ struct BfsSums {
     unsigned long long deg_sum = 0, deg_large = 0, probes = 0;
 };
 static BfsSums read_bfs_counters(medusa_graph* g, const BfsCounters* ctr, uint32_t par_next) {
-    g->h_ctr_raw.ensure((sizeof(BfsCounters) + 7) / 8);
+    static_assert(sizeof(BfsCounters) <= kHostWords * 8, "pinned memory of a handle");
     MDS_HIP(hipMemcpyAsync(g->h_ctr_raw.p, ctr, sizeof(BfsCounters), hipMemcpyDeviceToHost, g->stream));
     MDS_HIP(hipStreamSynchronize(g->stream));
     BfsCounters h;

@@ -291,8 +291,8 @@ struct medusa_graph {
     medusa::DBuf<unsigned long long> sssp_phases;  // SSSP device-loop phase marks (trace on)
     medusa::DBuf<uint32_t> mbfs_rows;  // MBFS: level rows on their way to a host output
     medusa::DBuf<uint4> sssp_rec;  // SSSP vertex records (local rounds without hubs), 64 bytes each
-    // per-superstep counters (device) and their pinned host mirror; each engine
-    // views the 256 bytes as its own counter struct
+    // per-superstep counters (device) and kHostWords of pinned memory: each engine views them as its
+    // own counter struct, or as what its device-driven run leaves for the host
     medusa::DBuf<unsigned long long> ctr_raw;
     medusa::HBuf<unsigned long long> h_ctr_raw;
     // device-driven superstep loops: control blocks and captured superstep batches
@@ -306,11 +306,8 @@ struct medusa_graph {
     // slot count, so runs of different lengths do not capture again)
     medusa::GraphCache bfs_heads[medusa::kMaxHeadSlots + 1];
     uint32_t bfs_next_head = medusa::kNoHead, mbfs_last_slots = 0, sssp_last_slots = 0;
-    // pinned: parameters of a BFS run and its control block afterwards; levels on their way to a
-    // small host output
-    medusa::HBuf<unsigned long long> h_bfs;
+    // pinned: levels on their way to a small host output
     medusa::HBuf<int32_t> h_levels;
-    medusa::HBuf<unsigned long long> h_sssp;  // pinned: control block and sums of an SSSP run
     int wall_khz = 0;  // rate of the device's wall clock
     std::unique_ptr<medusa::PrLayout> pr;
     std::unique_ptr<medusa::PullLayout> pull;  // built on the first MBFS run
@@ -350,10 +347,9 @@ bool build_pr_bins(medusa_graph* g, bool required);
 uint32_t pr_send_tile_slots(const medusa_graph* g, uint32_t nblk);
 // Binned-combine workgroups that run at once on g's device.
 uint32_t pr_combine_slots(const medusa_graph* g);
-// 8-byte words of the pinned memory that BFS runs use (bfs.hip).
-size_t bfs_host_words();
 
 constexpr size_t kCounterWords = 256;  // 2 KiB
+constexpr size_t kHostWords = 4096;    // 32 KiB
 template <class T>
 T* dev_counters(medusa_graph* g) {
     static_assert(sizeof(T) <= kCounterWords * 8, "counter struct too large");

@@ -335,8 +335,7 @@ extern "C" int medusa_graph_create(uint32_t n, uint64_t m, const uint32_t* row_p
             g->cw.upload(g->h_cw.data(), m, s);
         }
         g->ctr_raw.alloc(kCounterWords);
-        g->h_ctr_raw.ensure(kCounterWords);
-        g->h_bfs.ensure(bfs_host_words());
+        g->h_ctr_raw.ensure(kHostWords);
         MDS_HIP(hipDeviceGetAttribute(&g->wall_khz, hipDeviceAttributeWallClockRate, g->device));
         MDS_CHECK(g->wall_khz > 0, MEDUSA_ERR_HIP, "graph_create: no wall clock rate");
         MDS_HIP(hipStreamSynchronize(s));

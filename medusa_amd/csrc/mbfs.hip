@@ -910,8 +910,8 @@ static void mbfs_run(medusa_graph* g, const uint32_t* srcs, uint32_t k, uint8_t*
     g->mbfs_ctl.ensure(2 + (sizeof(MbfsCounters) + sizeof(CtlStorage) - 1) / sizeof(CtlStorage));
     MbfsCtl* ctl = reinterpret_cast<MbfsCtl*>(g->mbfs_ctl.p);
     MbfsCounters* C = reinterpret_cast<MbfsCounters*>(g->mbfs_ctl.p + 2);
-    g->h_ctr_raw.ensure((sizeof(MbfsCounters) + 7) / 8);
-    MbfsHost* host = reinterpret_cast<MbfsHost*>(g->h_ctr_raw.p);  // (or the host-driven loop's counters)
+    static_assert(sizeof(MbfsCounters) <= kHostWords * 8, "pinned memory of a handle");
+    MbfsHost* host = host_counters<MbfsHost>(g);  // (or the host-driven loop's counters)
     hipStream_t s = g->stream;
     const bool host_driven = o.timing || o.trace;
     uint32_t mode = 0;

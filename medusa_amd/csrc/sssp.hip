@@ -1288,7 +1288,7 @@ static void sssp_run_device(medusa_graph* g, uint32_t src, uint32_t* out, const 
     unsigned long long* marks = g->sssp_phases.p;
     const uint32_t local_cfg = sssp_local_cfg(g, o);
     const uint4* rec = sssp_records(g, o);
-    SsspHost* host = reinterpret_cast<SsspHost*>(g->h_sssp.p);
+    SsspHost* host = host_counters<SsspHost>(g);
     auto close = [&]() {
         hipLaunchKernelGGL(k_sssp_close, dim3(grid_for(n, 1024, kSsspCloseGrid)), dim3(1024), 0, s, (const SsspCtl*)ctl,
                            host, n, (const uint32_t*)g->dist.p, g->row_ptr.p, (uint32_t*)nullptr);
@@ -1491,7 +1491,7 @@ static void sssp_run_host(medusa_graph* g, uint32_t src, uint32_t* out, const me
     st.reserved[1] = phase;
     MDS_HIP(hipEventRecord(g->ev_end, s));
     hipLaunchKernelGGL(k_sssp_close, dim3(grid_for(n, 1024, kSsspCloseGrid)), dim3(1024), 0, s, (const SsspCtl*)nullptr,
-                       reinterpret_cast<SsspHost*>(g->h_sssp.p), n, (const uint32_t*)g->dist.p, g->row_ptr.p,
+                       host_counters<SsspHost>(g), n, (const uint32_t*)g->dist.p, g->row_ptr.p,
                        (uint32_t*)nullptr);
     MDS_LAUNCHED();
     MDS_HIP(hipStreamSynchronize(s));
@@ -1525,14 +1525,14 @@ extern "C" int medusa_sssp(medusa_graph* g, uint32_t source, uint32_t* dist, con
         g->near_q.ensure(2 * near_capacity(n, g->m));  // near queues A and B ((vertex, slice) entries)
         g->sssp_phases.ensure(3ull * kMaxPhaseMarks);     // phase marks of a traced device-driven run
         g->q_aux.ensure(2 * far_cap);                   // far queues A and B
-        g->h_sssp.ensure((sizeof(SsspHost) + 7) / 8);
+        static_assert(sizeof(SsspHost) <= kHostWords * 8, "pinned memory of a handle");
         medusa_stats st{};
         // timing: host-driven, every relaxation launch timed; otherwise device-driven (traced
         // by phase marks when trace is on)
         if (o.timing) sssp_run_host(g, source, dist, o, st);
         else sssp_run_device(g, source, dist, o, st);
         if (o.trace) sssp_trace_settled(g);
-        const SsspHost* h = reinterpret_cast<const SsspHost*>(g->h_sssp.p);
+        const SsspHost* h = host_counters<SsspHost>(g);
         const uint32_t wgs = grid_for(n, 1024, kSsspCloseGrid);
         st.edges_traversed = std::accumulate(h->edges, h->edges + wgs, 0ull);
         st.reached = (uint32_t)std::accumulate(h->reached, h->reached + wgs, 0ull);
