@@ -1201,7 +1201,13 @@ static size_t sssp_far_cap(const medusa_graph* g, const medusa_opts& o) {
 
 // Mean weight (sampled) and the default bucket width, a multiple of it: 8x with local rounds,
 // which absorb the extra hops of a wider bucket (1400x1400 lattice, 32 rounds: 8.0 ms at 8x,
-// 8.6 ms at 6x, 11.5 ms at 3x), else 2x.
+// 8.6 ms at 6x, 11.5 ms at 3x).  Without them 2x up to kWideEdges edges, where a superstep costs its
+// launch and a wider bucket has fewer (RMAT-16, 8 edges a vertex: 35, 30 and 28
+// supersteps, 497, 463 and 439 us at 1x, 1.5x and 2x); on larger graphs the edges relaxed more than once cost
+// more than the supersteps: 1x on graphs with hubs, whose wide buckets relax them again and again
+// (RMAT-20: 1.79, 1.95 and 2.06 ms, 3.2, 3.9 and 4.2 relaxations per edge), 1.5x on the others
+// (Erdos-Renyi, 2^20 vertices, 8 edges a vertex: 1.07, 0.98 and 1.02 ms; 16: 1.18, 1.17 and 1.26).
+constexpr uint64_t kWideEdges = 1ull << 22;
 static void sssp_widths(medusa_graph* g, const medusa_opts& o, uint32_t& wmean, uint32_t& dflt) {
     if (!g->w_mean) {  // once per graph: 4096 cache misses, 60 us on 64 MiB of weights
         uint64_t wsum = 0, wcnt = 0;
@@ -1211,8 +1217,8 @@ static void sssp_widths(medusa_graph* g, const medusa_opts& o, uint32_t& wmean, 
         g->w_mean = (uint32_t)std::max<uint64_t>(1, wcnt ? wsum / wcnt : 1);
     }
     wmean = g->w_mean;
-    const uint64_t mult = sssp_local_cfg(g, o) ? 8 : 2;
-    dflt = (uint32_t)std::min<uint64_t>(0xFFFFFFFEull, mult * wmean);
+    const uint64_t halves = sssp_local_cfg(g, o) ? 16 : g->m < kWideEdges ? 4 : g->max_outdeg > kSlice ? 2 : 3;
+    dflt = (uint32_t)std::min<uint64_t>(0xFFFFFFFEull, std::max<uint64_t>(1, halves * wmean / 2));
 }
 
 // Field 4 of every phase record: the vertices the phase settled, i.e. those whose final
