@@ -223,12 +223,13 @@ __device__ __forceinline__ float pr_base_value(float D, float d, uint32_t n_g) {
     return fmaf(d, D / (float)n_g, tele);
 }
 
-// A single graph with at most this many dangling vertices (one block): every wave of the pull or
-// push superstep sums them itself (16 loads a lane) instead of a launch of one workgroup doing it
-// before.  RMAT-16 (547 dangling), pull: 10.8 -> 9.2 us per superstep.  The
-// limit is one round of the sum's loads; each further round would add about as much to every wave
-// as the launch costs.
-constexpr uint32_t kOwnBaseVertices = 1024;
+// A single graph with at most this many dangling vertices (one block) can have every wave of the
+// pull or push superstep sum them itself, 16 loads a lane and round, instead of a launch of one workgroup
+// doing it before.  The launch costs 5 us, a round about 1.3 us for every 2048 workgroups, which
+// run at once: own_base where that is at most kOwnBaseRounds.  Pull superstep with the launch and
+// without: RMAT-14 (1781 dangling) 7.5 and 5.9 us, RMAT-16, 8 edges a vertex (2593) 8.9 and 7.5, RMAT-17
+// (1263) 13.9 and 12.5, RMAT-18 (3034) 26.5 and 26.7, RMAT-19, 24 edges a vertex (2539) 62 and 75.
+constexpr uint32_t kOwnBaseVertices = 4096, kOwnBaseRounds = 4;
 
 // One superstep for every vertex.  kFromMsg: values come from the message
 // array in slot order (push variant) instead of contrib[src] (pull variant).  kOwnBase: every
@@ -842,9 +843,10 @@ __global__ __launch_bounds__(256) void k_pr_finish(uint32_t n, const uint32_t* _
 constexpr uint32_t kFoldBlocks = 64;
 
 // In-edges up to which the default variant is the pull, when its superstep is one launch
-// (kOwnBaseVertices); us per superstep, pull against binned: R-MAT 12 (66 K arcs) 4.7 and 8.0,
-// 14 (262 K) 5.2 and 8.3, 15 (524 K) 5.6 and 9.1, 16 (1.05 M) 7.5 and 10.9, 17 (2.1 M) 14.0 and
-// 18.0, 18 (4.2 M) 27.5 and 25.6.  From here to about 3 M in-edges the pull is still the faster,
+// (own_base); us per superstep, pull against binned: R-MAT 12 (66 K arcs) 4.7 and 8.0,
+// 14 (262 K) 5.2 and 8.3, 15 (524 K) 5.6 and 9.1, 16 (1.05 M) 7.3 and 10.9, 17 (2.1 M) 12.5 and
+// 17.7, 18 (4.2 M) 26.7 and 24.4; 14 with 65 K arcs (1781 dangling) 5.9 and 7.9; Chung-Lu, 4200
+// vertices (2490 dangling) 6.1 and 7.2.  From here to about 3 M in-edges the pull is still the faster,
 // but what decides there (dangling share, in-degree spread) is what the variant policy learns,
 // and its measured gain is defined against the fixed binned variant.
 constexpr uint64_t kPullDefaultEdges = 1u << 19;
@@ -863,7 +865,8 @@ static void pr_run(medusa_graph* g, float damping, uint32_t steps, float* out, c
               MEDUSA_ERR_ARG, "pagerank: unknown variant %d", o.variant);
     // the engine's default: the pull on small graphs, else the binned exchange wherever its layout
     // can be planned
-    const bool own_base = L.parts.size() == 1 && nd <= kOwnBaseVertices;
+    const bool own_base = L.parts.size() == 1 && nd <= kOwnBaseVertices &&
+                          ((nd + 1023) / 1024) * ((L.total_wgs + 2047) / 2048) <= kOwnBaseRounds;
     const int dflt = o.variant != MEDUSA_PR_DEFAULT             ? o.variant
                      : own_base && m <= kPullDefaultEdges       ? MEDUSA_PR_PULL
                      : build_pr_bins(g, /*required=*/false)     ? MEDUSA_PR_BINNED
@@ -932,12 +935,16 @@ static void pr_run(medusa_graph* g, float damping, uint32_t steps, float* out, c
     MDS_LAUNCHED();
 
     const bool timing = o.timing != 0 || o.trace != 0;
-    // per superstep: [3t] superstep start, [3t+1] main kernel start, [3t+2] main kernel end
+    // per superstep: [3t] superstep start, [3t+1] main kernel start where launches come before it (an
+    // event between two others takes 3 us, half of a small graph's superstep), [3t+2] main kernel end
     if (timing) ensure_events(g, 3 * (size_t)steps);
     g->trace.clear();
     float* rk[2] = {L.rank.p, L.rank_prev.p};
     float* ct[2] = {L.contrib0.p, L.contrib1.p};
 
+    auto launches_before = [&](uint32_t t) {
+        return var[t] != MEDUSA_PR_BINNED && (!own_base || var[t] == MEDUSA_PR_PUSH);
+    };
     auto enqueue_steps = [&](bool with_events) {
         for (uint32_t t = 0; t < steps; ++t) {
             const float* r_in = rk[t & 1];
@@ -950,7 +957,6 @@ static void pr_run(medusa_graph* g, float damping, uint32_t steps, float* out, c
                 // send: the contributions of r_t as messages, and the dangling block pairs of r_t;
                 // combine: r_{t+1} (and c_{t+1} when the next superstep runs another variant)
                 const uint32_t dwg = (nblk + kSendWaves - 1) / kSendWaves;
-                if (with_events) MDS_HIP(hipEventRecord(g->events[3 * t + 1], s));
                 if (dwg + Bn->ntiles) {  // none when nothing dangles and every in-edge goes to a hub
                     hipLaunchKernelGGL(k_pr_send, dim3(Bn->ntiles + dwg), dim3(kSendThreads), 0, s,
                                        (const PrTile*)Bn->tiles.p, Bn->ntiles, (const uint16_t*)Bn->srcloc.p, r_in,
@@ -984,7 +990,7 @@ static void pr_run(medusa_graph* g, float damping, uint32_t steps, float* out, c
                                    L.oslot.p, c_in, L.msg.p);
                 MDS_LAUNCHED();
             }
-            if (with_events) MDS_HIP(hipEventRecord(g->events[3 * t + 1], s));
+            if (with_events && launches_before(t)) MDS_HIP(hipEventRecord(g->events[3 * t + 1], s));
             auto kern = step_push ? (own_base ? k_pr_main<true, true> : k_pr_main<true, false>)
                                   : (own_base ? k_pr_main<false, true> : k_pr_main<false, false>);
             hipLaunchKernelGGL(kern, dim3(L.total_wgs), dim3(256), 0, s, (const PrRun*)L.d_runs.p,
@@ -1058,7 +1064,7 @@ static void pr_run(medusa_graph* g, float damping, uint32_t steps, float* out, c
         else if (var[t] == MEDUSA_PR_PULL) ++st.pull_steps;
         if (timing) {
             float k_ms = 0, s_ms = 0;
-            MDS_HIP(hipEventElapsedTime(&k_ms, g->events[3 * t + 1], g->events[3 * t + 2]));
+            MDS_HIP(hipEventElapsedTime(&k_ms, g->events[3 * t + (launches_before(t) ? 1 : 0)], g->events[3 * t + 2]));
             MDS_HIP(hipEventElapsedTime(&s_ms, g->events[3 * t], g->events[3 * t + 2]));
             st.kernel_ms += k_ms;
             if (o.trace) {

@@ -115,9 +115,9 @@ def test_pagerank_binned_shapes(oracle):
                     assert np.array_equal(_bits(r), _bits(want)), (len(rp) - 1, steps, use_graph)
 
 
-@pytest.mark.parametrize("dangling", [0, 1, 63, 1024, 1025])
+@pytest.mark.parametrize("dangling", [0, 1, 63, 1024, 1025, 4096, 4097])
 def test_own_base_and_default_variant(oracle, dangling):
-    """Pull and push supersteps that sum up to 1024 dangling vertices themselves, the launch above
+    """Pull and push supersteps that sum up to 4096 dangling vertices themselves, the launch above
     that, and the default variant on either side of both limits; bits equal throughout."""
     rng = np.random.default_rng(7 + dangling)
     core = 3000
@@ -130,7 +130,7 @@ def test_own_base_and_default_variant(oracle, dangling):
             for v in (md.PR_PULL, md.PR_PUSH, md.PR_BINNED, md.PR_DEFAULT):
                 r, st = G.pagerank(0.85, 4, variant=v)
                 assert np.array_equal(_bits(r), _bits(want)), (m, v)
-            assert st.pull_steps == (4 if dangling <= 1024 and m <= 1 << 19 else 0)
+            assert st.pull_steps == (4 if dangling <= 4096 and m <= 1 << 19 else 0)
 
 
 @pytest.mark.parametrize("deg", [1, 8, 9, 16, 17, 32, 33, 64, 65, 127, 192, 4096])
