@@ -12,15 +12,14 @@
 // packed batch of disjoint graphs with one source per graph gives every graph's own BFS
 // levels in one run.  Here a superstep is ONE kernel that only touches the frontier and
 // builds the next one as it goes:
-//   frontier: a bitmap (one bit per vertex, three buffers in rotation) plus a queue of its
-//          hubs (out-degree above `large`);
-//   push:  waves take bitmap words and share the out-edges of a word's frontier vertices
-//          through an in-wave prefix scan; hubs are split over whole workgroups; a target is
-//          claimed by the lane whose 64-bit atomic OR first sets its bit in the next bitmap,
-//          so each joining vertex is counted exactly once;
-//   pull:  every unvisited vertex scans its in-edges for a parent in the frontier bitmap and
-//          stops at the first hit; each wave owns 64 consecutive vertices and writes their
-//          word of the next bitmap whole (ballot), no atomics;
+//   frontier: a queue in segments plus a queue of its hubs (out-degree above `large`), and which
+//          vertices have been visited as a bitmap;
+//   push:  waves take queue entries and share their out-edges through an in-wave prefix scan;
+//          hubs are split over whole workgroups; a target is claimed by the lane whose 64-bit
+//          atomic OR first sets its visited bit, so each joining vertex is counted exactly once
+//          (large frontiers store levels instead, and a compaction finds who joined);
+//   pull:  every unvisited vertex scans its in-edges for a visited vertex and stops at the first
+//          hit; each wave owns some words of the next bitmap and writes them whole, no atomics;
 //   counters: joined vertices, their out-degrees, hub degrees and probed in-edges, summed
 //          per workgroup into two packed 64-bit atomics; joined hubs are appended to the next
 //          hub queue (one atomic per wave that has any);
@@ -77,7 +76,7 @@ struct BfsCtl {
     uint32_t pending;   // a push with plain claims has run and its compaction has not
     uint32_t small;     // push with exact (atomic) claims: the frontier's out-edges fit one queue segment
     uint32_t slots;     // kernel launches the loop has used (a push with plain claims takes two)
-    uint32_t rot;       // which bitmap holds the frontier; the next one is built in bm[(rot + 1) % 3]
+    uint32_t vsel;      // which visited bitmap is current
     unsigned long long n, m, n_f, m_f, n_u, m_u, reached, reached_edges, kernel_bytes, alg_bytes;
     int32_t* out;              // where the closing kernel copies the levels (null: nowhere)
     unsigned long long t_begin;  // wall clock at the reset
@@ -109,7 +108,7 @@ __host__ __device__ inline uint32_t bfs_hub_wgs(uint32_t grid, uint32_t n_small,
 
 // Host-driven superstep: the host's decision written into the control block.
 __global__ void k_bfs_set_ctl(BfsCtl* ctl, int32_t step, uint32_t pull, uint32_t small, uint32_t n_small,
-                              uint32_t n_large, uint32_t hub_wgs) {
+                              uint32_t n_large, uint32_t hub_wgs, uint32_t vsel) {
     ctl->step = step;
     ctl->pull = pull;
     ctl->small = small;
@@ -118,7 +117,7 @@ __global__ void k_bfs_set_ctl(BfsCtl* ctl, int32_t step, uint32_t pull, uint32_t
     ctl->n_large = n_large;
     ctl->hub_wgs = hub_wgs;
     ctl->pending = 0;
-    ctl->rot = (uint32_t)step % 3u;
+    ctl->vsel = vsel;
     BfsCtl c = *ctl;  // for the compaction, if one follows
     c.pending = 1;
     ctl[1] = c;
@@ -152,18 +151,20 @@ struct BfsCounters {
 };
 
 // Buffers and shape of a BFS run, passed by value to every superstep kernel.  Superstep t
-// reads the frontier as bitmap bm[rot] (pull), queue q[t % 2] (push) and hub queue
-// hub[t % 2], builds the next frontier's in bm[(rot + 1) % 3], q[(t + 1) % 2] and
-// hub[(t + 1) % 2], and clears bm[(rot + 2) % 3] for superstep t + 1 (an exact-claim push sets
-// bits in its next bitmap).  The control block's rot advances by one with every superstep of the
-// whole grid and with every run of solo supersteps.
+// reads the frontier as queue q[t % 2] (push) and hub queue hub[t % 2] and builds the next
+// frontier's in q[(t + 1) % 2] and hub[(t + 1) % 2].  A pull needs no frontier bitmap: all
+// out-neighbours of the earlier frontiers have been visited, so a visited in-neighbour of an
+// unvisited vertex is in the frontier.  It reads one visited bitmap and writes the other, which is
+// then the current one; pushes change the current one in place.  (Three frontier bitmaps in
+// rotation took a second atomic from every exact claim and a pass that cleared one in every
+// superstep; a run's kernels with them and without: RMAT-20 154 and 151 us, Erdos-Renyi with 65536
+// vertices 69 and 67, Chung-Lu with 2.4 M 477 and 470.)
 struct BfsArgs {
     const uint32_t *row_ptr, *col, *cptr, *csrc;
     int32_t* level;
     uint32_t* q[2];    // segmented queues, kBfsSlots * span entries each
     uint32_t* hub[2];  // hub queues, n entries each
-    unsigned long long* bm[3];
-    unsigned long long* visited;  // one bit per vertex that has a level (n / 8 bytes, stays in L2)
+    unsigned long long* vis[2];  // one bit per vertex that has a level (n / 8 bytes, stays in L2)
     BfsCounters* ctr;
     BfsCtl* ctl;
     const float* policy;  // learned direction policy (device parameters) or null
@@ -214,7 +215,7 @@ constexpr uint32_t kRoundChunks = kBfsRound / 256;  // 64-vertex chunks per wave
 // append of the workgroup per round, 13 now.
 constexpr uint32_t kJoinCap = 1024, kJoinRound = 256;  // entries; most of them added per round
 struct BfsJoinLds {
-    unsigned long long words[4][kJoinCap / kWave];  // of a pull: next-bitmap words of the listed vertices
+    unsigned long long words[4][kJoinCap / kWave];  // of a pull: joins among the listed vertices of a word
     uint32_t v[4][kJoinCap];
 };
 struct BfsJoins {
@@ -401,19 +402,19 @@ constexpr uint32_t kPushUnroll = 4;  // out-edges per lane per round of the push
 // set is skipped (the bitmap is small enough to stay in L2, the level array is not).  Plain: `level[v]
 // = next`, a plain store; every writer stores the same value, so the race is benign (as in the
 // reference) and the compaction after the push finds the vertices that joined.
-__device__ __forceinline__ void bfs_claim_plain(const BfsArgs& a, const uint32_t (&v)[kPushUnroll], int32_t next) {
+__device__ __forceinline__ void bfs_claim_plain(const BfsArgs& a, const unsigned long long* __restrict__ visited,
+                                                const uint32_t (&v)[kPushUnroll], int32_t next) {
 #pragma unroll
     for (uint32_t j = 0; j < kPushUnroll; ++j)
-        if (v[j] != 0xFFFFFFFFu && !(a.visited[v[j] >> 6] & (1ull << (v[j] & 63)))) a.level[v[j]] = next;
+        if (v[j] != 0xFFFFFFFFu && !(visited[v[j] >> 6] & (1ull << (v[j] & 63)))) a.level[v[j]] = next;
 }
 
-// Exact: whoever sets the visited bit wins the vertex, stores its level, sets its bit in the next
-// bitmap and holds it for the next queue's segment `own`.  The calling wave is converged.  A wave with
+// Exact: whoever sets the visited bit wins the vertex, stores its level and holds it for the next queue's segment `own`.  The calling wave is converged.  A wave with
 // many out-edges goes through this chain of dependent accesses once per round, so the round's loads
 // and atomics are issued together (a compare-and-swap on the level one after the other, then the
 // bit: 34..36 us for 46 K and 62 K out-edges of that graph, 20 now).
 struct BfsExact {
-    unsigned long long* nxt;
+    unsigned long long* visited;
     BfsSink sink;
     uint32_t own;
     BfsJoins J;
@@ -422,17 +423,14 @@ __device__ __forceinline__ void bfs_claim_exact(const BfsArgs& a, BfsExact& x, c
                                                 int32_t next, unsigned long long& hacc) {
     unsigned long long seen[kPushUnroll];
 #pragma unroll
-    for (uint32_t j = 0; j < kPushUnroll; ++j) seen[j] = v[j] != 0xFFFFFFFFu ? a.visited[v[j] >> 6] : ~0ull;
+    for (uint32_t j = 0; j < kPushUnroll; ++j) seen[j] = v[j] != 0xFFFFFFFFu ? x.visited[v[j] >> 6] : ~0ull;
 #pragma unroll
     for (uint32_t j = 0; j < kPushUnroll; ++j)
-        if (!((seen[j] >> (v[j] & 63)) & 1ull)) seen[j] = atomicOr(&a.visited[v[j] >> 6], 1ull << (v[j] & 63));
+        if (!((seen[j] >> (v[j] & 63)) & 1ull)) seen[j] = atomicOr(&x.visited[v[j] >> 6], 1ull << (v[j] & 63));
 #pragma unroll
     for (uint32_t j = 0; j < kPushUnroll; ++j) {
         const bool won = !((seen[j] >> (v[j] & 63)) & 1ull);
-        if (won) {
-            a.level[v[j]] = next;
-            atomicOr(&x.nxt[v[j] >> 6], 1ull << (v[j] & 63));
-        }
+        if (won) a.level[v[j]] = next;
         x.J.put(won, v[j]);
     }
     static_assert(kJoinRound >= kWave * kPushUnroll, "a round's winners");
@@ -481,7 +479,7 @@ __device__ __forceinline__ void push_queue(const BfsArgs& a, const uint32_t* __r
                 }
             }
             if constexpr (kExact) bfs_claim_exact(a, x, v, next, hacc);
-            else bfs_claim_plain(a, v, next);
+            else bfs_claim_plain(a, x.visited, v, next);
         }
         __builtin_amdgcn_wave_barrier();
     }
@@ -548,7 +546,7 @@ __device__ __forceinline__ void push_hubs(const BfsArgs& a, const uint32_t* __re
                 v[j] = k < hi ? a.col[k] : 0xFFFFFFFFu;
             }
             if constexpr (kExact) bfs_claim_exact(a, x, v, next, hacc);
-            else bfs_claim_plain(a, v, next);
+            else bfs_claim_plain(a, x.visited, v, next);
         }
     }
 }
@@ -577,7 +575,7 @@ constexpr uint32_t kPullWords = kJoinCap / kWave;          // visited words a wa
 constexpr uint32_t kPullRounds = kPullWords / kRoundChunks;  // in rounds
 
 // Bottom-up probe of one vertex per lane and j (in-edges [b, e), none if b == e): joined[j] where a source
-// is in the frontier bitmap.  A lane scans a vertex of in-degree <= kPullLane alone, kPullGroup in-edges
+// is visited.  A lane scans a vertex of in-degree <= kPullLane alone, kPullGroup in-edges
 // of every j per round; above that the whole wave scans it 64 in-edges at a time and stops at the
 // first hit (ballot), so one high in-degree vertex does not hold its wave for hundreds of sequential
 // probes.  `probes` counts in-edges examined up to and including the first hit in either case.
@@ -662,7 +660,7 @@ __device__ __forceinline__ void pull_probe(const BfsArgs& a, const unsigned long
 // kRoundChunks visited words.  A wave lists the unvisited vertices of kPullRounds rounds, which then
 // fill its lanes however few of each word they are, and probes kRoundChunks of them per lane at a time;
 // the joins replace them at the front of the list and go to the next queue together, and every owned
-// word of the next and visited bitmaps is written whole, so the pull needs no compaction.  Bound by
+// word of the next visited bitmap is written whole, so the pull needs no compaction.  Bound by
 // the chain of dependent loads (visited word, in-offsets, sources, bitmap words), which a pass over
 // the list goes through once.  Chung-Lu, 2.4 M vertices, pulls of 1.3 M to 0.5 M unvisited vertices:
 // 34..26 us with a lane per vertex of the round, 25..20 now.
@@ -678,7 +676,7 @@ __device__ __forceinline__ void pull_all(const BfsArgs& a, const unsigned long l
         const uint64_t w = (round0 + (uint64_t)(lane / kRoundChunks) * grid) * (kBfsRound / kWave) + wv * kRoundChunks +
                            lane % kRoundChunks;
         const bool owner = lane < rounds * kRoundChunks && w < a.nwords;
-        const unsigned long long vis = owner ? a.visited[w] : 0ull;
+        const unsigned long long vis = owner ? cur[w] : 0ull;
         unsigned long long open = owner ? ~vis : 0ull;
         if (owner && (w + 1) * kWave > a.n) open &= (1ull << (a.n % kWave)) - 1;
         uint32_t cand = 0;
@@ -719,11 +717,7 @@ __device__ __forceinline__ void pull_all(const BfsArgs& a, const unsigned long l
             }
         }
         wave_lds_fence();
-        if (owner) {
-            const unsigned long long m = words[lane];
-            nxt[w] = m;
-            a.visited[w] = vis | m;  // the wave owns this word in a pull
-        }
+        if (owner) nxt[w] = vis | words[lane];
         bfs_flush(a, J, o, bfs_round_segment(round0 * kBfsRound), hacc);
     }
 }
@@ -769,18 +763,17 @@ struct BfsCounts {
 // The counts of the superstep just finished folded into the control block; true if another follows.
 __device__ __forceinline__ bool bfs_fold(const BfsArgs& a, BfsCtl& c, const BfsCounts& k) {
     const uint32_t n = a.n, n_new = k.n_new;
-    // bytes of the superstep just finished (every expansion clears one bitmap: 8 per word):
-    // push = queue entry and out-offsets per frontier vertex (12) + target id and visited bit
-    // per out-edge (8); exact claims then add compare-and-swap (4), two bit ORs (16),
-    // out-offsets (8) and queue entry (4) per join, plain claims the store per join (4) and the compaction's level
-    // pass (4n), next and visited bitmaps (16 per word), out-offsets and queue entry per join
-    // (12); pull = visited word per 64 vertices and in-offsets of unvisited vertices (8) +
-    // source id and bitmap word per probed in-edge (8) + next and visited bitmaps (16 per
-    // word) + level, out-offsets and queue entry per join (16)
+    // bytes of the superstep just finished: push = queue entry and out-offsets per frontier vertex
+    // (12) + target id and visited bit per out-edge (8); exact claims then add the bit OR (8), level
+    // (4), out-offsets (8) and queue entry (4) per join, plain claims the store per join (4) and the
+    // compaction's level pass (4n), visited bitmap (8 per word), out-offsets and queue entry per
+    // join (12); pull = visited word per 64 vertices, read and written (16), and in-offsets of
+    // unvisited vertices (8) + source id and bitmap word per probed in-edge (8) + level, out-offsets
+    // and queue entry per join (16)
     const unsigned long long kb =
-        c.pull    ? 8ull * c.n_u + 8ull * k.probes + 32ull * a.nwords + 16ull * n_new
-        : c.small ? 12ull * c.n_f + 8ull * c.m_f + 8ull * a.nwords + 32ull * n_new
-                  : 12ull * c.n_f + 8ull * c.m_f + 4ull * n + 24ull * a.nwords + 16ull * n_new;
+        c.pull    ? 8ull * c.n_u + 8ull * k.probes + 16ull * a.nwords + 16ull * n_new
+        : c.small ? 12ull * c.n_f + 8ull * c.m_f + 24ull * n_new
+                  : 12ull * c.n_f + 8ull * c.m_f + 4ull * n + 8ull * a.nwords + 16ull * n_new;
     c.kernel_bytes += kb;
     c.alg_bytes += kb;
     c.slots += k.slots;
@@ -855,7 +848,7 @@ __device__ __forceinline__ void bfs_decide(const BfsArgs& a, uint32_t slot, BfsC
         const uint32_t n_hub = load_now(&ctr->n_hub);
         const BfsCounts k{(uint32_t)joined, n_hub, joined >> 32, (uint32_t)work, work >> 32,
                           c.pending ? 2u : 1u};
-        c.rot = c.rot == 2 ? 0 : c.rot + 1;
+        c.vsel ^= c.pull;  // a pull wrote the other bitmap
         c.pending = 0;
         more = bfs_fold(a, c, k);
         if (more) {
@@ -920,7 +913,7 @@ __device__ __forceinline__ void solo_reset(BfsSoloLds<kThreads>& L) {
 // bitmap is L.vis (a small graph's few lines of global memory would take one atomic at a time:
 // 33 K out-edges of 4096 vertices 80 us instead of 49).
 template <bool kLdsVis, uint32_t kThreads, uint32_t kN>
-__device__ __forceinline__ void solo_claim(const BfsArgs& a, BfsSoloLds<kThreads>& L, const uint32_t (&v)[kN],
+__device__ __forceinline__ void solo_claim(const BfsArgs& a, unsigned long long* visited, BfsSoloLds<kThreads>& L, const uint32_t (&v)[kN],
                                            int32_t level) {
     unsigned long long old[kN];
     uint32_t b[kN], e[kN];
@@ -931,7 +924,7 @@ __device__ __forceinline__ void solo_claim(const BfsArgs& a, BfsSoloLds<kThreads
         if (v[j] != 0xFFFFFFFFu) {
             b[j] = a.row_ptr[v[j]];
             e[j] = a.row_ptr[v[j] + 1];
-            old[j] = __hip_atomic_fetch_or(kLdsVis ? &L.vis[v[j] >> 6] : &a.visited[v[j] >> 6], 1ull << (v[j] & 63),
+            old[j] = __hip_atomic_fetch_or(kLdsVis ? &L.vis[v[j] >> 6] : &visited[v[j] >> 6], 1ull << (v[j] & 63),
                                            __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
         }
     }
@@ -979,7 +972,8 @@ __device__ __forceinline__ void solo_claim(const BfsArgs& a, BfsSoloLds<kThreads
 // ones after it while they fit; c (the same in every thread) follows.  Ends with c.done, or with the
 // first frontier that does not fit in L and no direction chosen for it.  Every thread calls it.
 template <bool kLdsVis, uint32_t kThreads>
-__device__ __forceinline__ void bfs_solo(const BfsArgs& a, BfsSoloLds<kThreads>& L, BfsCtl& c) {
+__device__ __forceinline__ void bfs_solo(const BfsArgs& a, unsigned long long* visited, BfsSoloLds<kThreads>& L,
+                                         BfsCtl& c) {
     constexpr uint32_t kCap = BfsSoloLds<kThreads>::kCap, kPer = kPushUnroll;
     const uint32_t t = threadIdx.x, lane = t & (kWave - 1), wv = t / kWave;
     for (;;) {
@@ -1030,7 +1024,7 @@ __device__ __forceinline__ void bfs_solo(const BfsArgs& a, BfsSoloLds<kThreads>&
             }
 #pragma unroll
             for (uint32_t j = 0; j < kPushUnroll; ++j) v[j] = first + j < total ? a.col[x[j]] : 0xFFFFFFFFu;
-            solo_claim<kLdsVis>(a, L, v, c.step + 1);
+            solo_claim<kLdsVis>(a, visited, L, v, c.step + 1);
         }
         __syncthreads();
         if (!bfs_fold(a, c, BfsCounts{L.n, L.n_hub, L.deg_sum, L.deg_large, 0, 0})) return;
@@ -1039,7 +1033,7 @@ __device__ __forceinline__ void bfs_solo(const BfsArgs& a, BfsSoloLds<kThreads>&
     }
 }
 
-// The frontier in L handed to the next launch, in bm[c.rot] (all zero), queue step % 2 (segment 0,
+// The frontier in L handed to the next launch, in queue step % 2 (segment 0,
 // which may run on over the others' space), its hub queue and its counters; the control block goes
 // to *ctl.  (Counters other than the queues' are zero: nobody adds to them in this launch.)
 template <uint32_t kThreads>
@@ -1048,7 +1042,6 @@ __device__ __forceinline__ void solo_publish(const BfsArgs& a, BfsSoloLds<kThrea
     const uint32_t t = threadIdx.x, par = (uint32_t)c.step & 1u;
     if (!c.done) {
         const uint32_t n = L.n;
-        unsigned long long* bm = a.bm[c.rot];
         if (t < kBfsSlots) {
             a.ctr->seg[par][t].v = t == 0 ? bfs_pack(n, (uint32_t)L.deg_sum) : 0ull;
             a.ctr->seg[par ^ 1u][t].v = 0;
@@ -1059,7 +1052,6 @@ __device__ __forceinline__ void solo_publish(const BfsArgs& a, BfsSoloLds<kThrea
         for (uint32_t i = t; i < n; i += kThreads) {
             const uint32_t v = L.v[i];
             a.q[par][i] = v;
-            __hip_atomic_fetch_or(&bm[v >> 6], 1ull << (v & 63), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
             if (L.deg[i] > a.large) a.hub[par][atomicAdd(&L.n_hub, 1u)] = v;
         }
     }
@@ -1141,18 +1133,18 @@ __global__ __launch_bounds__(1024) void k_bfs_start(BfsArgs a, const BfsHost* __
     for (uint32_t i0 = 0; i0 < count; i0 += 1024) {
         if (i0) src = i0 + t < count ? param(&host->src[i0 + t]) : 0u;
         const uint32_t v[1] = {i0 + t < count ? src : 0xFFFFFFFFu};
-        solo_claim<false>(a, L, v, 0);
+        solo_claim<false>(a, a.vis[0], L, v, 0);
     }
     __syncthreads();
     BfsCtl c = bfs_first(a, BfsCounts{L.n, L.n_hub, L.deg_sum, L.deg_large, 0, 0}, m, mode, out);
     if (c.mode != 2 && bfs_solo_fits(kSoloStart, c.n, c.n_f, c.m_f)) {
         bfs_set_direction(a, c, false, true);
         if (a.n <= BfsSoloLds<1024>::kCap) {
-            if (t < a.nwords) L.vis[t] = a.visited[t];  // behind the barrier above
-            bfs_solo<true>(a, L, c);
-            if (t < a.nwords) a.visited[t] = L.vis[t];
+            if (t < a.nwords) L.vis[t] = a.vis[0][t];  // behind the barrier above
+            bfs_solo<true>(a, a.vis[0], L, c);
+            if (t < a.nwords) a.vis[0][t] = L.vis[t];
         } else {
-            bfs_solo<false>(a, L, c);
+            bfs_solo<false>(a, a.vis[0], L, c);
         }
     }
     if (!c.done) {
@@ -1163,7 +1155,7 @@ __global__ __launch_bounds__(1024) void k_bfs_start(BfsArgs a, const BfsHost* __
         __syncthreads();
         bfs_set_direction(a, c, s_pull != 0, false);
     }
-    solo_publish(a, L, c, a.ctl);  // into bitmap 0, which the reset cleared
+    solo_publish(a, L, c, a.ctl);
 }
 
 // End of a batch of slots: the control block to the host, and the levels to their destination when
@@ -1193,8 +1185,8 @@ __global__ __launch_bounds__(256) void k_bfs_close(BfsArgs a, BfsHost* __restric
     for (; i < a.n; i += stride) out[i] = a.level[i];
 }
 
-// Level reset, counters, bitmaps 0 and 1 and the visited bitmap cleared; with `single` < n that
-// vertex is placed at level 0, in bitmap 0 and in queue 0 with its counters (the host-driven loop;
+// Level reset, counters and the visited bitmap cleared; with `single` < n that
+// vertex is placed at level 0, in the bitmap and in queue 0 with its counters (the host-driven loop;
 // otherwise k_bfs_start or k_bfs_mark places the sources).
 __global__ __launch_bounds__(256) void k_bfs_seed(BfsArgs a, uint32_t single) {
     const uint32_t n = a.n;
@@ -1203,10 +1195,8 @@ __global__ __launch_bounds__(256) void k_bfs_seed(BfsArgs a, uint32_t single) {
     const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
     for (uint64_t v = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; v < n; v += stride)
         a.level[v] = v == single ? 0 : -1;
-    for (uint64_t w = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; w < a.nwords; w += stride) {
-        a.bm[0][w] = a.visited[w] = one && w == single / kWave ? 1ull << (single & 63) : 0ull;
-        a.bm[1][w] = 0;  // superstep 0's next bitmap (superstep 0 clears bitmap 2 itself)
-    }
+    for (uint64_t w = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; w < a.nwords; w += stride)
+        a.vis[0][w] = one && w == single / kWave ? 1ull << (single & 63) : 0ull;
     if (blockIdx.x != 0) return;
     bfs_clear_counters(a.ctr, 0);
     bfs_clear_counters(a.ctr, 1);
@@ -1223,7 +1213,7 @@ __global__ __launch_bounds__(256) void k_bfs_seed(BfsArgs a, uint32_t single) {
     }
 }
 
-// Several sources: each is placed at level 0, in bitmap 0 and in queue 0; a vertex given more
+// Several sources: each is placed at level 0, in the bitmap and in queue 0; a vertex given more
 // than once is counted once (the lane that sets its bit).  One queue atomic per source.
 __global__ __launch_bounds__(256) void k_bfs_mark(BfsArgs a, const uint32_t* __restrict__ src, uint32_t count) {
     const uint32_t lane = threadIdx.x & (kWave - 1);
@@ -1236,8 +1226,7 @@ __global__ __launch_bounds__(256) void k_bfs_mark(BfsArgs a, const uint32_t* __r
         if (i < count) {
             v = src[i];
             const unsigned long long bit = 1ull << (v & 63);
-            won = !(atomicOr(&a.bm[0][v >> 6], bit) & bit);
-            if (won) atomicOr(&a.visited[v >> 6], bit);
+            won = !(atomicOr(&a.vis[0][v >> 6], bit) & bit);
         }
         if (won) {
             a.level[v] = 0;
@@ -1267,12 +1256,11 @@ __global__ __launch_bounds__(64) void k_zero_counters(BfsCounters* c, uint32_t p
 }
 
 // After a push with plain claims: the next frontier = {v : level[v] == step + 1}, as its
-// bitmap (one ballot per 64 vertices), queue, hub queue and counters, and the visited bitmap
-// rebuilt from the levels, in workgroup rounds of
+// queue, hub queue and counters, and the visited bitmap (one ballot per 64 vertices) rebuilt from the levels, in workgroup rounds of
 // kBfsRound consecutive vertices (wave w the chunks w * kRoundChunks + k), whose level loads are
 // issued together.
-__device__ __forceinline__ void compact_level(const BfsArgs& a, int32_t next, unsigned long long* __restrict__ nxt,
-                                              const BfsSink& o, unsigned long long& hacc, BfsJoins J) {
+__device__ __forceinline__ void compact_level(const BfsArgs& a, unsigned long long* visited, int32_t next, const BfsSink& o,
+                                              unsigned long long& hacc, BfsJoins J) {
     const uint32_t lane = threadIdx.x & (kWave - 1), wv = threadIdx.x / kWave;
     uint64_t blk = (uint64_t)blockIdx.x * kBfsRound;
     for (; blk < a.n; blk += (uint64_t)gridDim.x * kBfsRound) {
@@ -1288,10 +1276,7 @@ __device__ __forceinline__ void compact_level(const BfsArgs& a, int32_t next, un
         for (uint32_t k = 0; k < kRoundChunks; ++k) {
             jm[k] = __ballot(lv[k] == next);
             const unsigned long long vm = __ballot(lv[k] >= 0);
-            if (lane == 0 && c0 + k < a.nwords) {
-                nxt[c0 + k] = jm[k];
-                a.visited[c0 + k] = vm;
-            }
+            if (lane == 0 && c0 + k < a.nwords) visited[c0 + k] = vm;
         }
         bfs_join_round(a, J, o, jm, c0 * kWave, blk, hacc);
     }
@@ -1300,7 +1285,7 @@ __device__ __forceinline__ void compact_level(const BfsArgs& a, int32_t next, un
 
 // One launch of the superstep loop, doing what the control block says:
 //   pending: the compaction after a push with plain claims;
-//   pull:    every unvisited vertex; the next frontier's bitmap, queue, hub queue and
+//   pull:    every unvisited vertex; the next frontier's queue, hub queue, visited bitmap and
 //            counters come out of the same pass;
 //   small:   3: workgroup 0 runs this superstep and the ones after it solo; else push with exact
 //            claims (the frontier's out-edges fit one queue segment); the
@@ -1337,31 +1322,28 @@ __global__ __launch_bounds__(256) void k_bfs_super(BfsArgs a, uint32_t slot) {
         return;
     }
     const int32_t step = ctl->step, next = step + 1;
-    const uint32_t par = (uint32_t)step & 1u, t3 = ctl->rot;
-    unsigned long long* nxt = a.bm[t3 == 2 ? 0 : t3 + 1];
+    const uint32_t par = (uint32_t)step & 1u, vsel = ctl->vsel;
+    unsigned long long *visited = vsel ? a.vis[1] : a.vis[0], *other = vsel ? a.vis[0] : a.vis[1];
     const BfsSink sink{a.q[par ^ 1u], a.ctr->seg[par ^ 1u], a.hub[par ^ 1u]};
     const BfsJoins joins{reinterpret_cast<BfsJoinLds*>(s_work)->v[threadIdx.x / kWave]};
     unsigned long long hacc = 0;
     if (ctl->pending) {
-        compact_level(a, next, nxt, sink, hacc, joins);
+        compact_level(a, visited, next, sink, hacc, joins);
         if (bfs_finish<kDecide>(a.ctr, hacc)) bfs_decide(a, slot, &s_c, s_params);
         return;
     }
-    unsigned long long* clr = a.bm[t3 == 0 ? 2 : t3 - 1];
-    const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
-    for (uint64_t w = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; w < a.nwords; w += stride) clr[w] = 0;
     if (ctl->pull) {
         unsigned long long probes = 0;
-        pull_all(a, a.bm[t3], nxt, sink, next, hacc, probes, joins,
+        pull_all(a, visited, other, sink, next, hacc, probes, joins,
                  reinterpret_cast<BfsJoinLds*>(s_work)->words[threadIdx.x / kWave]);
         if (bfs_finish<kDecide>(a.ctr, hacc + (probes << 32))) bfs_decide(a, slot, &s_c, s_params);
         return;
     }
-    BfsExact x{nxt, sink, blockIdx.x % kBfsSlots, joins};
+    BfsExact x{visited, sink, blockIdx.x % kBfsSlots, joins};
     const uint32_t hub = ctl->hub_wgs, small = ctl->small;
     if constexpr (kDecide) {
         if (small == 3) {
-            if (blockIdx.x != 0) return;  // (each cleared its share of the bitmap above)
+            if (blockIdx.x != 0) return;
             BfsSoloLds<256>& L = *reinterpret_cast<BfsSoloLds<256>*>(s_work);
             bfs_queue_prefix(a.ctr->seg[par], s_pre);
             const uint32_t qn = s_pre[kBfsSlots];
@@ -1374,9 +1356,10 @@ __global__ __launch_bounds__(256) void k_bfs_super(BfsArgs a, uint32_t slot) {
             if (threadIdx.x == 0) L.n = qn;
             BfsCtl c = *ctl;
             __syncthreads();
-            bfs_solo<false>(a, L, c);
+            bfs_solo<false>(a, visited, L, c);
             c.slots += 1;
-            c.rot = t3 == 2 ? 0 : t3 + 1;  // cleared by the launch before this one
+            c.out = ctl->out;  // again, rather than kept (on the stack) through the supersteps
+            c.t_begin = ctl->t_begin;
             if (!c.done) bfs_set_direction(a, c, c.mode != 1 && bfs_heuristic(c, false), false);
             solo_publish(a, L, c, a.ctl + (slot ^ 1u));
             return;
@@ -1425,8 +1408,7 @@ struct BfsBufs {
     int32_t* level;
     uint32_t* q[2];                 // frontier queues, kBfsSlots * bfs_span(n) entries each
     uint32_t* hub[2];               // hub queues, n entries each
-    unsigned long long* bm[3];      // frontier bitmaps, (n + 63) / 64 words each
-    unsigned long long* visited;    // visited bitmap, (n + 63) / 64 words
+    unsigned long long* vis[2];     // visited bitmaps, (n + 63) / 64 words each
     const uint32_t* sources;        // several sources (device), or null
     BfsCtl* ctl;
     BfsCounters* ctr;
@@ -1442,8 +1424,7 @@ static BfsBufs handle_bufs(medusa_graph* g) {
     return {g->level.p,
             {g->q_small.p, g->q_small.p + qcap},
             {g->q_large.p, g->q_large.p + g->n},
-            {g->bitmap.p, g->bitmap.p + nwords, g->bitmap.p + 2 * nwords},
-            g->bitmap.p + 3 * nwords,
+            {g->bitmap.p, g->bitmap.p + nwords},
             g->q_aux.p,
             reinterpret_cast<BfsCtl*>(g->bfs_ctl.p),
             reinterpret_cast<BfsCounters*>(g->bfs_ctl.p + 2)};
@@ -1463,8 +1444,8 @@ static BfsArgs bfs_args(medusa_graph* g, const BfsBufs& B, uint32_t large, uint3
     a.q[1] = B.q[1];
     a.hub[0] = B.hub[0];
     a.hub[1] = B.hub[1];
-    for (int i = 0; i < 3; ++i) a.bm[i] = B.bm[i];
-    a.visited = B.visited;
+    a.vis[0] = B.vis[0];
+    a.vis[1] = B.vis[1];
     a.ctr = B.ctr;
     a.ctl = B.ctl;
     a.policy = policy;
@@ -1479,7 +1460,7 @@ static BfsArgs bfs_args(medusa_graph* g, const BfsBufs& B, uint32_t large, uint3
 }
 
 // Seeding of the host-driven loop, and of a device-driven run of more sources than the starting
-// kernel takes: every source at level 0 and in bitmap 0 (one source by value, several from
+// kernel takes: every source at level 0 and in the bitmap (one source by value, several from
 // B.sources), the first queue, hub queue and counters.
 static void bfs_seed(medusa_graph* g, const BfsBufs& B, const BfsArgs& a, uint32_t nsrc, uint32_t single) {
     hipStream_t s = g->stream;
@@ -1498,10 +1479,9 @@ static void bfs_enqueue_slot(medusa_graph* g, const BfsArgs& a, uint32_t parity)
     hipLaunchKernelGGL(k_bfs_super<true>, dim3(a.grid), dim3(256), 0, g->stream, a, parity);
 }
 
-// Bytes of the seeding: the level reset (4 per vertex), bitmaps 0 and 1 and the visited bitmap
-// (24 per word) and the sources (16 each: id, level, bit OR).
+// Bytes of the seeding: the level reset (4 per vertex), the visited bitmap (8 per word) and the sources (16 each: id, level, bit OR).
 static uint64_t bfs_seed_bytes(uint32_t n, uint32_t nwords, uint32_t nsrc) {
-    return 4ull * n + 24ull * nwords + 16ull * nsrc;
+    return 4ull * n + 8ull * nwords + 16ull * nsrc;
 }
 
 // Device-driven run: reset, start, superstep slots and close, then batches of slots and a close until
@@ -1539,7 +1519,7 @@ static void bfs_run_device(medusa_graph* g, const BfsBufs& B, uint32_t nsrc, con
     // capture (once per graph, threshold, policy buffer and slot count) a run's kernels
     auto captured = [&](GraphCache& gc, bool start, uint32_t slots) -> hipGraphExec_t {
         const uintptr_t key[6] = {(uintptr_t)B.level, (uintptr_t)B.hub[0], (uintptr_t)policy,
-                                  ((uintptr_t)grid << 32) | large, (uintptr_t)B.bm[0], (uintptr_t)B.q[0]};
+                                  ((uintptr_t)grid << 32) | large, (uintptr_t)B.vis[0], (uintptr_t)B.q[0]};
         if (gc.exec && std::equal(key, key + 6, gc.key)) return gc.exec;
         gc.reset();
         MDS_HIP(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
@@ -1652,6 +1632,7 @@ static void bfs_run_host(medusa_graph* g, uint32_t nsrc, uint32_t single, int32_
     f.m_u = m - f.m_f;
     uint64_t reached_edges = f.m_f, reached = f.n_f, bytes = bfs_seed_bytes(n, nwords, nsrc);
     bool pull = false;
+    uint32_t vsel = 0;
     uint32_t solo_cap = nsrc <= kBfsHostSources ? kSoloStart : kSoloSlot;
     Sched sched(o, Sched::kBfs);
     if (timing) ensure_events(g, 2);
@@ -1666,7 +1647,7 @@ static void bfs_run_host(medusa_graph* g, uint32_t nsrc, uint32_t single, int32_
         const uint32_t hub = bfs_hub_wgs(grid, n_small, c.n_hub, c.deg_large, c.deg_sum);
         const uint32_t small = bfs_small(pull, f.n_f, f.m_f, a.exact_edges);
         hipLaunchKernelGGL(k_bfs_set_ctl, dim3(1), dim3(1), 0, s, B.ctl, (int32_t)t, pull ? 1u : 0u, small, n_small,
-                           c.n_hub, hub);
+                           c.n_hub, hub, vsel);
         MDS_LAUNCHED();
         hipLaunchKernelGGL(k_zero_counters, dim3(1), dim3(kWave), 0, s, a.ctr, (t & 1u) ^ 1u);
         MDS_LAUNCHED();
@@ -1690,13 +1671,14 @@ static void bfs_run_host(medusa_graph* g, uint32_t nsrc, uint32_t single, int32_
         // the byte model of the device-driven loop's decision
         uint64_t kb;
         if (pull) {
-            kb = 8ull * f.n_u + 8ull * c.probes + 32ull * nwords + 16ull * c.n_new;
+            kb = 8ull * f.n_u + 8ull * c.probes + 16ull * nwords + 16ull * c.n_new;
             ++st.pull_steps;
+            vsel ^= 1u;
         } else if (small) {
-            kb = 12ull * f.n_f + 8ull * f.m_f + 8ull * nwords + 32ull * c.n_new;
+            kb = 12ull * f.n_f + 8ull * f.m_f + 24ull * c.n_new;
             ++st.push_steps;
         } else {
-            kb = 12ull * f.n_f + 8ull * f.m_f + 4ull * n + 24ull * nwords + 16ull * c.n_new;
+            kb = 12ull * f.n_f + 8ull * f.m_f + 4ull * n + 8ull * nwords + 16ull * c.n_new;
             ++st.push_steps;
         }
         st.kernel_bytes += kb;
@@ -1738,7 +1720,7 @@ static void bfs_entry(medusa_graph* g, const uint32_t* sources, uint32_t count, 
     g->q_small.ensure(2 * bfs_queue_cap(n));
     g->q_large.ensure(2 * (size_t)n);
     g->q_aux.ensure(std::max(n, count));
-    g->bitmap.ensure(4 * (((size_t)n + 63) / 64));
+    g->bitmap.ensure(2 * (((size_t)n + 63) / 64));
     if (count > (o.timing || o.trace ? 1u : kBfsHostSources))
         MDS_HIP(hipMemcpyAsync(g->q_aux.p, sources, (size_t)count * 4, hipMemcpyHostToDevice, g->stream));
     medusa_stats st{};
@@ -1749,8 +1731,8 @@ static void bfs_entry(medusa_graph* g, const uint32_t* sources, uint32_t count, 
 
 // ---- BFS with no device allocation ------------------------------------------------
 // Work buffers of medusa_bfs_noalloc: two frontier queues and two hub queues of
-// kNoAllocMaxVertices entries each, three frontier bitmaps and the visited bitmap, the control
-// block and the counters, in one array per GPU that lives as long as the process.  Host code
+// kNoAllocMaxVertices entries each, two visited bitmaps, the control
+// blocks and the counters, in one array per GPU that lives as long as the process.  Host code
 // must not pass `scratch` itself to a kernel (in host code the name is a stand-in, not a device
 // address): the device address is looked up once per device with hipGetSymbolAddress and kept
 // in s_scratch.
@@ -1759,7 +1741,7 @@ constexpr size_t kNoAllocQueueBytes = (size_t)kNoAllocMaxVertices * 4;
 constexpr size_t kNoAllocBitmapBytes = (size_t)kNoAllocMaxVertices / 8;
 static_assert((size_t)kBfsSlots * bfs_span(kNoAllocMaxVertices) == kNoAllocMaxVertices,
               "the segmented queue of the largest graph fills kNoAllocMaxVertices entries exactly");
-constexpr size_t kNoAllocBytes = 4 * kNoAllocQueueBytes + 4 * kNoAllocBitmapBytes + kBfsCtlUnits * sizeof(CtlStorage);
+constexpr size_t kNoAllocBytes = 4 * kNoAllocQueueBytes + 2 * kNoAllocBitmapBytes + kBfsCtlUnits * sizeof(CtlStorage);
 static_assert(kNoAllocMaxVertices % 2048 == 0, "queue and bitmap regions stay 256-byte aligned");
 static __device__ __align__(256) unsigned char scratch[kNoAllocBytes];
 
@@ -1801,10 +1783,9 @@ static void bfs_noalloc(medusa_graph* g, uint32_t source, int32_t* levels, medus
         B.q[i] = reinterpret_cast<uint32_t*>(base + i * kNoAllocQueueBytes);
         B.hub[i] = reinterpret_cast<uint32_t*>(base + (2 + i) * kNoAllocQueueBytes);
     }
-    for (int i = 0; i < 3; ++i)
-        B.bm[i] = reinterpret_cast<unsigned long long*>(base + 4 * kNoAllocQueueBytes + i * kNoAllocBitmapBytes);
-    B.visited = reinterpret_cast<unsigned long long*>(base + 4 * kNoAllocQueueBytes + 3 * kNoAllocBitmapBytes);
-    CtlStorage* ctl = reinterpret_cast<CtlStorage*>(base + 4 * kNoAllocQueueBytes + 4 * kNoAllocBitmapBytes);
+    for (int i = 0; i < 2; ++i)
+        B.vis[i] = reinterpret_cast<unsigned long long*>(base + 4 * kNoAllocQueueBytes + i * kNoAllocBitmapBytes);
+    CtlStorage* ctl = reinterpret_cast<CtlStorage*>(base + 4 * kNoAllocQueueBytes + 2 * kNoAllocBitmapBytes);
     B.ctl = reinterpret_cast<BfsCtl*>(ctl);
     B.ctr = reinterpret_cast<BfsCounters*>(ctl + 2);
     B.sources = nullptr;  // one source: not used
