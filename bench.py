@@ -324,7 +324,7 @@ def _roofline(stats, kernel, traffic=None):
 
 
 BFS_KERNEL = "k_bfs_super (superstep: pull, exact-claim push, or plain push + compaction)"
-MBFS_KERNEL = "k_mbfs_expand + k_mbfs_update (mask superstep: push or pull expansion, then the level update)"
+MBFS_KERNEL = "k_mbfs_super (mask superstep: pull, or push and update)"
 
 
 def _emit(a, metric_cfg, value, ms_per_step, roofline, cpu, extra):

@@ -52,7 +52,7 @@ extern "C" {
 #define MEDUSA_DIR_PULL 2  /* bottom-up over CSC every superstep */
 
 /* PageRank kernel variant (opts.variant); all variants give bit-identical ranks. */
-#define MEDUSA_PR_DEFAULT 0 /* the engine's choice: MEDUSA_PR_PULL on a small graph (at most 2^19 arcs and 1024
+#define MEDUSA_PR_DEFAULT 0 /* the engine's choice: MEDUSA_PR_PULL on a small graph (at most 2^19 arcs and 4096
                                vertices without out-edges) or one whose binned layout cannot be planned,
                                else MEDUSA_PR_BINNED */
 #define MEDUSA_PR_PUSH 1   /* scatter into per-in-edge message slots, then combine (reference style) */
@@ -85,7 +85,8 @@ typedef struct medusa_opts {
 /* Per-run statistics.  Reference: printf of wall time / steps (Algorithm/main.cu:316,355,
  * SSSP/main.cu:391-392, MPG/main.cu:173). */
 typedef struct medusa_stats {
-    double   device_ms;        /* hipEvent time of the superstep loop on HBM-resident data */
+    double   device_ms;        /* GPU time of the run on HBM-resident data: by the device's clock from its first
+                                  kernel to its last (BFS, SSSP, MBFS), by hipEvents (PageRank, timed runs) */
     double   kernel_ms;        /* summed duration of the dominant kernel's launches (opts.timing) */
     uint64_t kernel_launches;  /* launches of the dominant kernel */
     uint64_t kernel_bytes;     /* algorithmic bytes moved by those launches (byte model) */
