@@ -258,7 +258,6 @@ inline uint32_t next_slots(uint64_t last, uint64_t done, uint32_t batch) {
 struct CtlStorage {
     unsigned long long w[32];
 };
-using BfsCtlStorage = CtlStorage;
 
 }  // namespace medusa
 

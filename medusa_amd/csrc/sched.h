@@ -98,15 +98,6 @@ __host__ __device__ inline void variant_row(const double* r, double action, floa
 }
 
 #if defined(__HIPCC__)
-// LDS working set of a policy evaluation inside a decide kernel (up to 12 candidate rows).
-struct MlpShared {
-    float P[kMlpParams];
-    float x[12 * MEDUSA_POLICY_INPUTS];
-    float a1[12 * kMlpH];
-    float a2[12 * kMlpH];
-    float out[12];
-};
-
 // direction_log in FP32 with the hardware logarithm: within about 2e-6 of it, far below any
 // decision margin, and a few instructions instead of an FP64 logarithm's long dependent chain.
 __device__ inline float direction_log_f32(const double* r, int i) {
