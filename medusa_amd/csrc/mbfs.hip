@@ -89,6 +89,7 @@ struct MbfsArgs {
     uint32_t n, large, nslices, nhubs, grid, span;
 };
 constexpr uint32_t kMbfsPlanes = 8;
+constexpr uint32_t kMbfsSplitRows = 1u << 17;  // vertices below which the finish deals rows over workgroups
 constexpr uint32_t kMbfsTile = 1024;  // vertices of a workgroup's round of an update or queue pass
 
 // Queue segment span for n vertices: kMbfsSegs segments cover [0, n) in whole tiles.
@@ -792,7 +793,7 @@ __global__ __launch_bounds__(1024) void k_mbfs_finish(MbfsArgs a, MbfsHost* __re
                                                      uint32_t row1) {
     const MbfsCtl* ctl = a.ctl;  // a batch has an even number of launches
     if (host) {
-        if (blockIdx.x == 0) {
+        if (blockIdx.x == 0 && blockIdx.y == 0) {
             if (threadIdx.x < sizeof(MbfsCtl) / 8)
                 reinterpret_cast<unsigned long long*>(&host->ctl)[threadIdx.x] =
                     reinterpret_cast<const unsigned long long*>(ctl)[threadIdx.x];
@@ -827,6 +828,7 @@ __global__ __launch_bounds__(1024) void k_mbfs_finish(MbfsArgs a, MbfsHost* __re
             auto word = [h](unsigned long long w) { return (uint32_t)(w >> (32 * h)); };
 #pragma unroll
             for (uint32_t j = 0; j < 4; ++j) {
+                if (gridDim.y > 1 && blockIdx.y != 4 * h + j) continue;
                 uint32_t lo[4], hi[4];  // nibbles of sources 32h + j + 4i
 #pragma unroll
                 for (uint32_t i = 0; i < 4; ++i) {
@@ -950,7 +952,9 @@ static void mbfs_run(medusa_graph* g, const uint32_t* srcs, uint32_t k, uint8_t*
     // a workgroup per window of the layout, which fetches every line of it once, where that fills the
     // 256 CUs (RMAT-20 30 us against 35 with quarters of windows), else quarters
     const uint32_t finish_wg = n >= 256 * kPullWindow ? 1024 : 256;
-    const dim3 finish_grid(grid_for(n, 4 * finish_wg, 8192));
+    // on few vertices the rows are dealt over workgroups too: a workgroup with all 64 of them is a chain
+    // of 256 stores a lane (25 K vertices, 46 sources: 11.9 us, 7.3 dealt out)
+    const dim3 finish_grid(grid_for(n, 4 * finish_wg, 8192), n < kMbfsSplitRows ? 4 * ((sizeof(T) + 3) / 4) : 1);
     const bool direct = kernels_can_write(g, out);  // else the rows are copied out at the end
 
     // capture (once per buffers, launch shape, policy buffer and slot count) a batch of launches
