@@ -600,7 +600,7 @@ __device__ __forceinline__ void pull_probe(const BfsArgs& a, const unsigned long
         for (uint32_t k = 0; k < kRoundChunks; ++k) {
             u[k] = Sources{0, 0, 0, 0};
             if (sb[k] < se[k]) {
-                if (sb[k] + kPullGroup <= a.m) {
+                if ((unsigned long long)sb[k] + kPullGroup <= a.m) {
                     u[k] = *reinterpret_cast<const Sources*>(a.csrc + sb[k]);
                 } else {
 #pragma unroll
