@@ -1485,8 +1485,9 @@ static uint64_t bfs_seed_bytes(uint32_t n, uint32_t nwords, uint32_t nsrc) {
 }
 
 // Device-driven run: reset, start, superstep slots and close, then batches of slots and a close until
-// the control block says done.  capture: each sequence is captured once as a hipGraph and replayed;
-// without it (medusa_bfs_noalloc, which may not allocate) the same kernels are launched one by one.
+// the control block says done.  capture: each sequence is captured once as a hipGraph and replayed
+// (but for a handle's first, see below); without it (medusa_bfs_noalloc, which may not allocate) the
+// same kernels are launched one by one.
 static void bfs_run_device(medusa_graph* g, const BfsBufs& B, uint32_t nsrc, const uint32_t* sources, int32_t* out,
                            const medusa_opts& o, medusa_stats& st, bool capture = true) {
     const uint32_t n = g->n;
@@ -1539,9 +1540,14 @@ static void bfs_run_device(medusa_graph* g, const BfsBufs& B, uint32_t nsrc, con
         std::copy(key, key + 6, gc.key);
         return gc.exec;
     };
-    const uint32_t head = g->bfs_next_head == kNoHead ? kBfsBatch : g->bfs_next_head;
+    // a handle's first run launches its first sequence: what it would capture has a slot count that the
+    // next run, which knows how many it takes, rarely wants again (first run on ER with 80 K vertices
+    // 280 us with the capture, 149 without; with 8.7 K 210 and 124; RMAT-20 704 and 678)
+    const bool known = g->bfs_next_head != kNoHead;
+    const uint32_t head = known ? g->bfs_next_head : kBfsBatch;
     hipGraphExec_t exec = nullptr;
-    if (capture) exec = by_start ? captured(g->bfs_heads[head], true, head) : captured(g->bfs_graph, false, kBfsBatch);
+    if (capture && !by_start) exec = captured(g->bfs_graph, false, kBfsBatch);
+    else if (capture && known) exec = captured(g->bfs_heads[head], true, head);
 
     host->out = target;
     host->count = nsrc;
@@ -1555,12 +1561,9 @@ static void bfs_run_device(medusa_graph* g, const BfsBufs& B, uint32_t nsrc, con
         MDS_LAUNCHED();
     }
     for (uint32_t batch = 0;; ++batch) {
-        if (capture) {
-            if (batch > 0) exec = captured(g->bfs_graph, false, kBfsBatch);
-            MDS_HIP(hipGraphLaunch(exec, s));
-        } else {
-            launch(by_start && batch == 0, kBfsBatch);
-        }
+        if (capture && batch > 0) exec = captured(g->bfs_graph, false, kBfsBatch);
+        if (exec) MDS_HIP(hipGraphLaunch(exec, s));
+        else launch(by_start && batch == 0, kBfsBatch);
         MDS_HIP(hipStreamSynchronize(s));
         if (host->ctl.done) break;
         MDS_CHECK(batch < (2ull * n + 2) / kBfsBatch + 2, MEDUSA_ERR_INTERNAL, "bfs: superstep loop did not end");

@@ -377,6 +377,28 @@ def test_mbfs_rmat20_config(oracle, mbfs_policy):
             assert st.edges_traversed == reached
 
 
+@pytest.mark.parametrize("layers", [0, 5, 7, 8, 9, 17, 40])
+def test_bfs_first_run_of_a_handle(oracle, layers):
+    """The first run of a handle launches its kernels one by one and may need replays after them: wide
+    layers of vertices, too many edges for one workgroup, whose count is around the eight slots of a
+    first sequence; later runs on the handle are shorter, equal and longer."""
+    wide = 6000
+    n = 1 + layers * wide
+    at = np.arange(wide)
+    edges = [np.stack([np.zeros(wide, np.int64), 1 + at], 1)] if layers else [np.zeros((0, 2), np.int64)]
+    for k in range(1, layers):
+        for step in (0, 1, 77, 2500):
+            edges.append(np.stack([1 + (k - 1) * wide + at, 1 + k * wide + (at + step) % wide], 1))
+    rp, col, _ = csr_from_edges(n, np.concatenate(edges))
+    for first, d in ((0, md.DIR_AUTO), (0, md.DIR_PUSH), (1 + (layers // 2) * wide if layers > 1 else 0, md.DIR_AUTO)):
+        with md.Graph(rp, col) as G:
+            for s in (first, 0, n - 1, 0, first):
+                got, st = G.bfs(s, direction=d)
+                want = oracle.bfs_queue(rp, col, s)
+                assert np.array_equal(got, want), (first, s)
+                assert st.reached == int((want >= 0).sum()), (first, s)
+
+
 @pytest.mark.parametrize("n", [1, 1023, 1025, 9000])
 def test_sssp_runs_of_different_lengths(oracle, n):
     """Runs on one handle whose slot counts differ by more than a replay (a path of `n` vertices
