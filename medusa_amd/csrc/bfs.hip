@@ -857,8 +857,9 @@ __device__ __forceinline__ void bfs_decide(const BfsArgs& a, uint32_t slot, BfsC
                 pull = true;
             } else if (c.mode != 1 && !solo) {
                 ask = bfs_asks(a, c, c.pull != 0);
-                // the heuristic's choice stands unless the policy predicts a clear gain
-                pull = plain = bfs_heuristic(c, c.pull != 0);
+                pull = bfs_heuristic(c, c.pull != 0);
+                // between the margins the heuristic's choice stands, and with a policy a pull goes on
+                plain = pull || c.pull != 0;
                 if (ask) bfs_record(c, rec);
             }
         }
