@@ -486,9 +486,10 @@ __device__ __forceinline__ void push_queue(const BfsArgs& a, const uint32_t* __r
 }
 
 // Exact-claim push of a frontier of at most 64 vertices (hubs included): every wave reads the
-// whole frontier and its out-degree prefix, and wave w of the grid takes out-edges
-// [w * 64 * kPushUnroll, (w + 1) * 64 * kPushUnroll) of their concatenation, so a frontier of
-// one high-degree vertex still spreads over many waves.
+// whole frontier and its out-degree prefix, and the grid's waves take the out-edges of their
+// concatenation 64 * kPushUnroll at a time, wave w the w-th share and every (waves of the grid)-th
+// after it, so a frontier of one high-degree vertex still spreads over many waves.  (One share a
+// wave covers the default grid's frontiers up to 2^25 vertices, and fewer out-edges on a smaller grid.)
 __device__ __forceinline__ void push_tiny(const BfsArgs& a, const uint32_t* __restrict__ q, const uint32_t* pre,
                                           int32_t next, uint32_t (*s_beg)[kWave], uint32_t (*s_off)[kWave],
                                           BfsExact& x, unsigned long long& hacc) {
@@ -507,20 +508,22 @@ __device__ __forceinline__ void push_tiny(const BfsArgs& a, const uint32_t* __re
     s_beg[wv][lane] = beg;
     s_off[wv][lane] = incl - deg;
     __builtin_amdgcn_wave_barrier();
-    uint32_t v[kPushUnroll];
+    for (uint64_t e0 = e_begin; e0 < total; e0 += (uint64_t)gridDim.x * blockDim.x * kPushUnroll) {
+        uint32_t v[kPushUnroll];
 #pragma unroll
-    for (uint32_t j = 0; j < kPushUnroll; ++j) {
-        const uint64_t e = e_begin + j * kWave + lane;
-        v[j] = 0xFFFFFFFFu;
-        if (e < total) {
-            uint32_t lo = 0;
+        for (uint32_t j = 0; j < kPushUnroll; ++j) {
+            const uint64_t e = e0 + j * kWave + lane;
+            v[j] = 0xFFFFFFFFu;
+            if (e < total) {
+                uint32_t lo = 0;
 #pragma unroll
-            for (uint32_t step = kWave / 2; step; step >>= 1)
-                if (s_off[wv][lo + step] <= e) lo += step;
-            v[j] = a.col[s_beg[wv][lo] + ((uint32_t)e - s_off[wv][lo])];
+                for (uint32_t step = kWave / 2; step; step >>= 1)
+                    if (s_off[wv][lo + step] <= e) lo += step;
+                v[j] = a.col[s_beg[wv][lo] + ((uint32_t)e - s_off[wv][lo])];
+            }
         }
+        bfs_claim_exact(a, x, v, next, hacc);
     }
-    bfs_claim_exact(a, x, v, next, hacc);
 }
 
 // Hubs: each vertex of the hub queue is split into `split` contiguous edge ranges, one per

@@ -146,6 +146,30 @@ def test_bfs_held_joins(oracle, n, fan):
                 assert st.reached == (want >= 0).sum(), (d, grid)
 
 
+@pytest.mark.parametrize("parents", [1, 3, 64])
+@pytest.mark.parametrize("total", [4097, 8192])
+def test_bfs_few_vertices_with_many_out_edges(oracle, parents, total):
+    """A frontier of at most 64 vertices with more out-edges than two or seven workgroups take at once
+    (1024 each), up to a queue segment's 8192: every out-edge counts on every grid, in both drivers."""
+    n = 262_144  # segments of 8192
+    rng = np.random.default_rng(parents + total)
+    ids = rng.permutation(np.arange(1, n))
+    par, kids = ids[:parents], ids[parents:parents + total]
+    src = [np.zeros(parents, np.int64), par[np.arange(total) * parents // total], rng.integers(1, n, 2 * n)]
+    dst = [par, kids, rng.integers(1, n, 2 * n)]
+    keep = ~np.isin(src[2], par)  # the parents' only out-edges are those to their children
+    src[2], dst[2] = src[2][keep], dst[2][keep]
+    rp, col, _ = csr_from_edges(n, np.stack([np.concatenate(src), np.concatenate(dst)], 1))
+    want = oracle.bfs_queue(rp, col, 0)
+    with md.Graph(rp, col) as G:
+        for grid in (2, 7, 0):
+            for d in (md.DIR_AUTO, md.DIR_PUSH):
+                for timing in (0, 1):
+                    lv, st = G.bfs(0, direction=d, grid=grid, timing=timing)
+                    assert np.array_equal(lv, want), (grid, d, timing)
+                    assert st.reached == (want >= 0).sum(), (grid, d, timing)
+
+
 def test_bfs_edge_cases(oracle):
     with md.Graph(np.array([0, 0], np.uint32), np.array([], np.uint32)) as G:
         lv, st = G.bfs(0)
