@@ -1506,7 +1506,7 @@ static void bfs_run_device(medusa_graph* g, const BfsBufs& B, uint32_t nsrc, con
 
     // where the closing kernel puts the levels: the output itself, or pinned memory for a small host
     // output; larger host outputs are copied afterwards
-    const bool in_place = out == B.level, direct = !in_place && kernels_can_write(g, out);
+    const bool in_place = out == B.level, direct = !in_place && kernels_can_write(g, out, (size_t)n * 4);
     const bool staged = !in_place && !direct && (size_t)n * 4 <= kBfsStageBytes && !is_device_memory(out);
     if (staged) g->h_levels.ensure(n);
     int32_t* target = direct ? out : staged ? g->h_levels.p : nullptr;

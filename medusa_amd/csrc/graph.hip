@@ -62,16 +62,34 @@ bool is_device_memory(const void* p) {
     return e == hipSuccess && attr.type == hipMemoryTypeDevice;
 }
 
-bool kernels_can_write(const medusa_graph* g, const void* p) {
+// Bytes from device pointer `p` to the end of its allocation; 0 where HIP does not know.
+static size_t allocation_left(const void* p) {
+    hipDeviceptr_t base = nullptr;
+    size_t size = 0;
+    const hipError_t e = hipMemGetAddressRange(&base, &size, const_cast<void*>(p));
+    (void)hipGetLastError();
+    const size_t at = (size_t)(static_cast<const char*>(p) - static_cast<const char*>(base));
+    return e == hipSuccess && at <= size ? size - at : 0;
+}
+
+bool kernels_can_write(const medusa_graph* g, const void* p, size_t bytes) {
     hipPointerAttribute_t attr{};
     const hipError_t e = hipPointerGetAttributes(&attr, p);
     (void)hipGetLastError();
     return e == hipSuccess && attr.type == hipMemoryTypeDevice && attr.device == g->device &&
-           reinterpret_cast<uintptr_t>(p) % 4 == 0;
+           reinterpret_cast<uintptr_t>(p) % 4 == 0 && allocation_left(p) >= bytes;
+}
+
+void check_device_output(const void* p, size_t bytes) {
+    if (!is_device_memory(p)) return;
+    const size_t left = allocation_left(p);
+    MDS_CHECK(left == 0 || left >= bytes, MEDUSA_ERR_HIP, "output of %zu bytes in device memory that ends after %zu",
+              bytes, left);
 }
 
 void copy_out(medusa_graph* g, void* dst, const void* src, size_t bytes) {
     if (!bytes) return;
+    check_device_output(dst, bytes);
     const bool dev = is_device_memory(dst);
     MDS_HIP(hipMemcpyAsync(dst, src, bytes, dev ? hipMemcpyDeviceToDevice : hipMemcpyDeviceToHost, g->stream));
     MDS_HIP(hipStreamSynchronize(g->stream));

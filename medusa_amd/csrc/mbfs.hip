@@ -955,7 +955,7 @@ static void mbfs_run(medusa_graph* g, const uint32_t* srcs, uint32_t k, uint8_t*
     // on few vertices the rows are dealt over workgroups too: a workgroup with all 64 of them is a chain
     // of 256 stores a lane (25 K vertices, 46 sources: 11.9 us, 7.3 dealt out)
     const dim3 finish_grid(grid_for(n, 4 * finish_wg, 8192), n < kMbfsSplitRows ? 4 * ((sizeof(T) + 3) / 4) : 1);
-    const bool direct = kernels_can_write(g, out);  // else the rows are copied out at the end
+    const bool direct = kernels_can_write(g, out, (size_t)k * n);  // else the rows are copied out at the end
 
     // capture (once per buffers, launch shape, policy buffer and slot count) a batch of launches
     auto captured = [&](uint32_t slots) -> hipGraphExec_t {
@@ -1102,6 +1102,7 @@ static void mbfs_run(medusa_graph* g, const uint32_t* srcs, uint32_t k, uint8_t*
     st.reached = (uint32_t)std::min<uint64_t>(h.reached, 0xFFFFFFFFull);
     st.reserved[0] = h.saturated;
     if (direct) return;
+    check_device_output(out, (size_t)k * n);  // before the first row is written
     // as many rows at a time as the row buffer holds
     const uint32_t rows = (uint32_t)std::min<uint64_t>(k, std::max<uint64_t>(1, kMbfsRowBytes / n));
     g->mbfs_rows.ensure(((size_t)rows * n + 3) / 4);

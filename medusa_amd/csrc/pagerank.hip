@@ -905,7 +905,7 @@ static void pr_run(medusa_graph* g, float damping, uint32_t steps, float* out, c
     if (push) L.msg.ensure(m);
     hipStream_t s = g->stream;
     // an output the kernels can write is written by the last one itself
-    const bool direct = kernels_can_write(g, out);
+    const bool direct = kernels_can_write(g, out, (size_t)n * 4);
     if (!direct) L.unperm.ensure(n);
     const bool send_folds = !fold && pr_send_folds(L);
 

@@ -1331,7 +1331,7 @@ static void sssp_run_device(medusa_graph* g, uint32_t src, uint32_t* out, const 
     };
     uint32_t slots = next_slots(g->sssp_last_slots, 0, kSsspBatch);
     hipGraphExec_t exec = captured(slots);
-    const bool direct = kernels_can_write(g, out);
+    const bool direct = kernels_can_write(g, out, (size_t)n * 4);
 
     hipLaunchKernelGGL(k_sssp_start, dim3(grid_for(n, 256, 4096)), dim3(256), 0, s, n, g->dist.p, g->stamp.p, src,
                        src_slices, near0, ctl, ctr, (unsigned long long)m, thr0, d0, local_cfg, o.trace ? 1u : 0u, marks,

@@ -57,3 +57,63 @@ def test_device_arrays_match_oracle_csc_small(oracle):
 def test_device_arrays_match_oracle_csc_rmat20(oracle):
     rp, col = wl.rmat_graph()
     _check(oracle, rp, col)
+
+
+class _DeviceArray:
+    """An allocation of `nbytes` of device memory, every byte 7."""
+
+    def __init__(self, nbytes):
+        L = md.lib()
+        L.hipMalloc.argtypes, L.hipMalloc.restype = [ctypes.POINTER(ctypes.c_void_p), ctypes.c_size_t], ctypes.c_int
+        L.hipFree.argtypes, L.hipFree.restype = [ctypes.c_void_p], ctypes.c_int
+        L.hipMemset.argtypes, L.hipMemset.restype = [ctypes.c_void_p, ctypes.c_int, ctypes.c_size_t], ctypes.c_int
+        p = ctypes.c_void_p()
+        assert L.hipMalloc(ctypes.byref(p), nbytes) == 0
+        self.base, self.nbytes = p.value, nbytes
+        self.clear()
+
+    def clear(self):
+        assert md.lib().hipMemset(self.base, 7, self.nbytes) == 0
+        assert md.lib().hipDeviceSynchronize() == 0
+
+    def at(self, offset):
+        class Out:
+            data_ptr = lambda _: self.base + offset  # noqa: E731
+        return Out()
+
+    def bytes(self):
+        return _d2h(self.base, self.nbytes // 4).view(np.uint8)
+
+    def free(self):
+        assert md.lib().hipFree(self.base) == 0
+
+
+@pytest.mark.parametrize("short", [4, 4096])
+def test_device_output_past_its_allocation_is_refused(oracle, short):
+    """A device output whose allocation ends before the result does is an error of every entry point,
+    host- and device-driven, and nothing is written; one that ends where the result does is filled."""
+    n, k = 40_000, 9
+    rng = np.random.default_rng(short)
+    rp, col, _ = csr_from_edges(n, rng.integers(0, n, (4 * n, 2)))
+    w = rng.integers(1, 1001, len(col)).astype(np.uint32)
+    srcs = rng.integers(0, n, k).astype(np.uint32)
+    calls = [(4 * n, lambda G, o: G.bfs(0, out=o), lambda: oracle.bfs_queue(rp, col, 0)),
+             (4 * n, lambda G, o: G.bfs(0, out=o, timing=1), lambda: oracle.bfs_queue(rp, col, 0)),
+             (4 * n, lambda G, o: G.sssp(0, out=o), lambda: oracle.sssp_dijkstra(rp, col, w, 0)),
+             (4 * n, lambda G, o: G.sssp(0, out=o, timing=1), lambda: oracle.sssp_dijkstra(rp, col, w, 0)),
+             (4 * n, lambda G, o: G.pagerank(0.85, 3, out=o), lambda: oracle.pagerank_f32(rp, col, 0.85, 3)),
+             (k * n, lambda G, o: G.mbfs(srcs, out=o), lambda: oracle.mbfs(rp, col, srcs)),
+             (k * n, lambda G, o: G.mbfs(srcs, out=o, timing=1), lambda: oracle.mbfs(rp, col, srcs))]
+    with md.Graph(rp, col, w) as G:
+        for i, (need, call, want) in enumerate(calls):
+            print(f"[case] call {i}", flush=True)
+            A = _DeviceArray(need + 256)
+            call(G, A.at(256))
+            got = A.bytes()
+            assert (got[:256] == 7).all() and np.array_equal(got[256:], np.ascontiguousarray(want()).view(np.uint8).ravel())
+            A.clear()
+            with pytest.raises(md.MedusaError) as e:
+                call(G, A.at(256 + short))
+            assert e.value.code == -2  # MEDUSA_ERR_HIP
+            assert (A.bytes() == 7).all(), i
+            A.free()
