@@ -463,13 +463,13 @@ __device__ __forceinline__ void push_queue(const BfsArgs& a, const uint32_t* __r
         s_beg[wv][lane] = beg;
         s_off[wv][lane] = incl - deg;
         __builtin_amdgcn_wave_barrier();
-        for (uint32_t e0 = 0; e0 < total; e0 += kWave * kPushUnroll) {  // uniform across the wave
+        for (uint32_t e0 = 0; e0 < total; e0 = advance_to(e0, kWave * kPushUnroll, total)) {  // uniform across the wave
             uint32_t v[kPushUnroll];
 #pragma unroll
             for (uint32_t j = 0; j < kPushUnroll; ++j) {
                 const uint32_t e = e0 + j * kWave + lane;
                 v[j] = 0xFFFFFFFFu;
-                if (e < total) {
+                if (lies_before(e0, j * kWave + lane, total)) {
                     // owner = last lane whose exclusive offset is <= e (it has deg > 0)
                     uint32_t lo = 0;
 #pragma unroll
@@ -538,15 +538,15 @@ __device__ __forceinline__ void push_hubs(const BfsArgs& a, const uint32_t* __re
     for (uint64_t w = wg0; w < (uint64_t)qn * split; w += nwg) {
         const uint32_t u = q[w / split], part = (uint32_t)(w % split);
         const uint32_t b = a.row_ptr[u], deg = a.row_ptr[u + 1] - b;
-        const uint32_t per = (deg + split - 1) / split;
-        const uint32_t lo = b + min(deg, part * per), hi = b + min(deg, (part + 1) * per);
-        for (uint32_t k0 = lo + (threadIdx.x - lane) * kPushUnroll; k0 < hi;
+        const EdgePart E = edge_part(b, deg, part, split);
+        const uint32_t cnt = E.hi - E.lo;  // a sixteenth of an edge array at most
+        for (uint32_t k0 = (threadIdx.x - lane) * kPushUnroll; k0 < cnt;
              k0 += blockDim.x * kPushUnroll) {  // uniform per wave
             uint32_t v[kPushUnroll];
 #pragma unroll
             for (uint32_t j = 0; j < kPushUnroll; ++j) {
                 const uint32_t k = k0 + j * kWave + lane;
-                v[j] = k < hi ? a.col[k] : 0xFFFFFFFFu;
+                v[j] = k < cnt ? a.col[E.lo + k] : 0xFFFFFFFFu;
             }
             if constexpr (kExact) bfs_claim_exact(a, x, v, next, hacc);
             else bfs_claim_plain(a, x.visited, v, next);
@@ -608,7 +608,7 @@ __device__ __forceinline__ void pull_probe(const BfsArgs& a, const unsigned long
                 } else {
 #pragma unroll
                     for (uint32_t j = 0; j < kPullGroup; ++j)
-                        if (sb[k] + j < se[k]) u[k][j] = a.csrc[sb[k] + j];
+                        if (lies_before(sb[k], j, se[k])) u[k][j] = a.csrc[sb[k] + j];
                 }
             }
         }
@@ -616,7 +616,8 @@ __device__ __forceinline__ void pull_probe(const BfsArgs& a, const unsigned long
 #pragma unroll
         for (uint32_t k = 0; k < kRoundChunks; ++k)
 #pragma unroll
-            for (uint32_t j = 0; j < kPullGroup; ++j) word[k][j] = sb[k] + j < se[k] ? cur[u[k][j] >> 6] : 0ull;
+            for (uint32_t j = 0; j < kPullGroup; ++j)
+                word[k][j] = lies_before(sb[k], j, se[k]) ? cur[u[k][j] >> 6] : 0ull;
         more = false;
 #pragma unroll
         for (uint32_t k = 0; k < kRoundChunks; ++k) {
@@ -641,11 +642,10 @@ __device__ __forceinline__ void pull_probe(const BfsArgs& a, const unsigned long
         for (unsigned long long bm = __ballot(e[k] - b[k] > kPullLane); bm; bm &= bm - 1) {
             const uint32_t owner = __builtin_ctzll(bm);
             const uint32_t vb = __shfl(b[k], owner, kWave), ve = __shfl(e[k], owner, kWave);
-            for (uint32_t k0 = vb; k0 < ve; k0 += kWave) {
-                const uint32_t i = k0 + lane;
+            for (uint32_t k0 = vb; k0 < ve; k0 = advance_to(k0, kWave, ve)) {
                 bool hit = false;
-                if (i < ve) {
-                    const uint32_t u = a.csrc[i];
+                if (lies_before(k0, lane, ve)) {
+                    const uint32_t u = a.csrc[k0 + lane];
                     hit = (cur[u >> 6] >> (u & 63)) & 1ull;
                 }
                 const unsigned long long hm = __ballot(hit);

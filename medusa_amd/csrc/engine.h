@@ -15,6 +15,7 @@
 #include <vector>
 
 #include "common.h"
+#include "edge_range.h"
 #include "pr_bins.h"
 
 namespace medusa {

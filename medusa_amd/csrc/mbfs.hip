@@ -157,7 +157,7 @@ __global__ __launch_bounds__(256) void k_pull_fill(uint32_t n, uint32_t nslices,
             const uint4 h = hub[s - nslices];
             const uint32_t b = cptr[perm[h.x]];
             uint32_t* to = src + (((uint64_t)h.w << 32) | h.z);
-            for (uint32_t k = lane; k < h.y; k += kWave) to[k] = pos[csrc[b + k]];
+            for (uint32_t k = lane; k < h.y; k = advance_to(k, kWave, h.y)) to[k] = pos[csrc[b + k]];
             continue;
         }
         const uint64_t b = base[s], len = (base[s + 1] - b) / kWave, p = s * kWave + lane;
@@ -327,7 +327,9 @@ __device__ __forceinline__ void mbfs_push_small(const MbfsArgs& a, const MbfsLin
         L.off[wv][lane] = incl - edges.y;
         L.mask[wv][lane] = fm;
         wave_lds_fence();
-        for (uint32_t e = lane; e < total; e += kWave) {
+        for (uint32_t e0 = 0; e0 < total; e0 = advance_to(e0, kWave, total)) {  // uniform across the wave
+            if (!lies_before(e0, lane, total)) continue;
+            const uint32_t e = e0 + lane;
             uint32_t lo = 0;
 #pragma unroll
             for (uint32_t step = kWave / 2; step; step >>= 1)
@@ -348,9 +350,9 @@ __device__ __forceinline__ void mbfs_push_large(const MbfsArgs& a, uint32_t qn,
         const uint32_t u = a.q_large[w / split], part = (uint32_t)(w % split);
         const uint2 edges = a.out[u];
         const unsigned long long fm = frontier[u];
-        const uint32_t per = (edges.y + split - 1) / split;
-        const uint32_t lo = edges.x + min(edges.y, part * per), hi = edges.x + min(edges.y, (part + 1) * per);
-        for (uint32_t k = lo + threadIdx.x; k < hi; k += blockDim.x) mbfs_offer(a, k, fm);
+        const EdgePart E = edge_part(edges.x, edges.y, part, split);
+        const uint32_t cnt = E.hi - E.lo;  // an eighth of an edge array at most
+        for (uint32_t k = threadIdx.x; k < cnt; k += blockDim.x) mbfs_offer(a, E.lo + k, fm);
     }
 }
 
@@ -426,19 +428,19 @@ __device__ __forceinline__ void mbfs_pull(const MbfsArgs& a, unsigned long long 
         unsigned long long found = 0;
         uint32_t probes = 0;
         bool all = vis == full;
-        for (uint32_t k0 = 0; k0 < deg && !all; k0 += 4 * kWave) {
+        for (uint32_t k0 = 0; k0 < deg && !all; k0 = advance_to(k0, 4 * kWave, deg)) {
             uint32_t u[4];
             unsigned long long f[4];
 #pragma unroll
             for (uint32_t j = 0; j < 4; ++j) {
-                const uint32_t k = k0 + j * kWave + lane;
-                u[j] = k < deg ? src[k] : 0u;
+                const uint32_t off = j * kWave + lane;
+                u[j] = lies_before(k0, off, deg) ? src[k0 + off] : 0u;
             }
 #pragma unroll
-            for (uint32_t j = 0; j < 4; ++j) f[j] = k0 + j * kWave + lane < deg ? frontier[u[j]] : 0ull;
+            for (uint32_t j = 0; j < 4; ++j) f[j] = lies_before(k0, j * kWave + lane, deg) ? frontier[u[j]] : 0ull;
 #pragma unroll
             for (uint32_t j = 0; j < 4; ++j) {
-                if (all || k0 + j * kWave >= deg) continue;
+                if (all || !lies_before(k0, j * kWave, deg)) continue;
                 found |= wave_or(f[j]);
                 probes += min(deg - k0 - j * kWave, (uint32_t)kWave);
                 all = (found | vis) == full;

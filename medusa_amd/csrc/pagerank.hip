@@ -95,7 +95,7 @@ template <class Load>
 __device__ __forceinline__ float wave_segment_sum(uint32_t len, Load load) {
     const uint32_t lane = threadIdx.x & (kWave - 1);
     float as = 0.f, ac = 0.f;
-    for (uint32_t b0 = 0; b0 < len; b0 += kBlock) {
+    for (uint32_t b0 = 0; b0 < len; b0 = advance_to(b0, kBlock, len)) {
         const uint32_t lim = min(len - b0, kBlock);
         float s = 0.f, c = 0.f;
         for (uint32_t r0 = 0; r0 * kWave < lim; r0 += 16) {
@@ -814,7 +814,7 @@ __global__ void k_pr_scatter(uint32_t n, const uint32_t* __restrict__ optr, cons
         const uint32_t b = optr[p], e = optr[p + 1];
         if (b == e) continue;
         const float x = contrib[p];
-        for (uint32_t k = b + lane; k < e; k += kWave) msg[oslot[k]] = x;
+        for (uint32_t k = advance_to(b, lane, e); k < e; k = advance_to(k, kWave, e)) msg[oslot[k]] = x;
     }
 }
 
