@@ -30,8 +30,9 @@
 // wave does this on its own (wave rounds, below).
 
 #include <algorithm>
-#include <numeric>
 #include <chrono>
+#include <numeric>
+#include <type_traits>
 
 #include "engine.h"
 #include "sched.h"
@@ -47,7 +48,6 @@ struct SsspCounters {
 };
 
 constexpr uint32_t kSlice = 128;       // out-edges per near-queue entry
-constexpr uint32_t kStage = 2048;      // LDS staging entries per queue per workgroup
 constexpr uint32_t kStageSlices = 4;   // a vertex with more slices goes straight to HBM
 
 __host__ __device__ inline uint32_t slices_of(uint32_t deg) { return deg <= kSlice ? 1u : (deg + kSlice - 1) / kSlice; }
@@ -85,11 +85,17 @@ __global__ void k_sssp_zero(SsspCounters* c, uint32_t keep_far) {
 // flush, instead of one atomic per wave per 64 edges on a single counter (which serialises
 // on that address).
 
-struct Stage {
-    unsigned long long near[kStage];
-    uint32_t far[kStage];
+// kSlices: slices of a vertex that a stage of a workgroup of kThreads takes.
+template <uint32_t kThreads, uint32_t kSlices>
+struct StageOf {
+    static constexpr uint32_t kWidth = kThreads;
+    static constexpr uint32_t kMost = kThreads * kSlices;  // near entries of one round
+    static constexpr uint32_t kRoom = 2 * kMost;           // entries per queue
+    unsigned long long near[kRoom];
+    uint32_t far[kRoom];
     uint32_t n_near, n_far, base_near, base_far, flush;
 };
+using Stage = StageOf<256, kStageSlices>;
 
 // Where a kernel's appends go.
 struct Sinks {
@@ -102,7 +108,8 @@ struct Sinks {
     const uint32_t* row_ptr;
 };
 
-__device__ __forceinline__ void stage_init(Stage& st) {
+template <class St>
+__device__ __forceinline__ void stage_init(St& st) {
     if (threadIdx.x == 0) {
         st.n_near = 0;
         st.n_far = 0;
@@ -112,12 +119,13 @@ __device__ __forceinline__ void stage_init(Stage& st) {
 
 // One thread's appends: v (out-degree deg) to the near queue (as its slices) and/or to the
 // far queue.
-__device__ __forceinline__ void stage_put(Stage& st, const Sinks& k, bool to_near, bool to_far, uint32_t v,
-                                          uint32_t deg, unsigned long long& ndeg) {
+template <uint32_t kThreads, uint32_t kSlices>
+__device__ __forceinline__ void stage_put(StageOf<kThreads, kSlices>& st, const Sinks& k, bool to_near, bool to_far,
+                                          uint32_t v, uint32_t deg, unsigned long long& ndeg) {
     if (to_near) {
         ndeg += deg;
         const uint32_t cnt = slices_of(deg);
-        if (cnt > kStageSlices) {
+        if (cnt > kSlices) {
             const uint32_t base = atomicAdd(k.near_cnt, cnt);
             for (uint32_t j = 0; j < cnt; ++j)
                 if (base + j < k.near_cap) k.near[base + j] = ((unsigned long long)j << 32) | v;
@@ -132,11 +140,12 @@ __device__ __forceinline__ void stage_put(Stage& st, const Sinks& k, bool to_nea
 // Called by every thread of the block after each round of stage_put (at most one call per
 // thread per round): copies the staged entries to HBM when another round could overflow
 // the stage, or whenever anything is staged if `last`.
-__device__ __forceinline__ void stage_flush(Stage& st, const Sinks& k, bool last) {
+template <class St>
+__device__ __forceinline__ void stage_flush(St& st, const Sinks& k, bool last) {
     __syncthreads();
     if (threadIdx.x == 0) {
         const uint32_t nn = st.n_near, nf = st.n_far;
-        const bool go = last ? (nn | nf) != 0 : (nn > kStage - 256 * kStageSlices || nf > kStage - 256);
+        const bool go = last ? (nn | nf) != 0 : (nn > St::kRoom - St::kMost || nf > St::kRoom - St::kWidth);
         st.flush = go ? 1u : 0u;
         if (go) {
             st.base_near = nn ? atomicAdd(k.near_cnt, nn) : 0u;
@@ -158,7 +167,8 @@ __device__ __forceinline__ void stage_flush(Stage& st, const Sinks& k, bool last
     __syncthreads();
 }
 
-// Exclusive prefix sum over the 256 threads of the block; `total` = the block's sum.
+// Exclusive prefix sum over the kThreads threads of the block; `total` = the block's sum.
+template <uint32_t kThreads>
 __device__ __forceinline__ uint32_t block_excl_scan(uint32_t x, uint32_t* s_wave, uint32_t& total) {
     const uint32_t lane = threadIdx.x & (kWave - 1), wv = threadIdx.x / kWave;
     const uint32_t incl = wave_incl_scan(x);
@@ -166,7 +176,9 @@ __device__ __forceinline__ uint32_t block_excl_scan(uint32_t x, uint32_t* s_wave
     __syncthreads();
     uint32_t off = 0;
     for (uint32_t w = 0; w < wv; ++w) off += s_wave[w];
-    total = s_wave[0] + s_wave[1] + s_wave[2] + s_wave[3];
+    total = 0;
+#pragma unroll
+    for (uint32_t w = 0; w < kThreads / kWave; ++w) total += s_wave[w];
     return off + incl - x;
 }
 
@@ -186,7 +198,7 @@ struct LocalList {
     uint32_t n[2];
 };
 
-// Relaxes one tile of at most 256 entries with the whole block: thread t brings the edge
+// Relaxes one tile of at most kThreads entries with the whole block: thread t brings the edge
 // range [beg, beg + deg) of its entry and the entry's distance du.  The block shares the
 // out-edges through a prefix scan of the degrees and every thread binary-searches the
 // owner of its edge.  A lowered vertex below the threshold goes to side `side` of the local
@@ -197,28 +209,29 @@ struct LocalList {
 // offsets together with its distance whenever the offer is below the threshold, so a
 // lowered vertex costs one round trip fewer (worth it on sparse graphs, where rounds are
 // latency-bound; on dense ones most offers lose and the extra reads cost bandwidth).
-template <bool kSpec>
+template <bool kSpec, uint32_t kThreads, uint32_t kSlices>
 __device__ __forceinline__ uint32_t relax_tile(uint32_t beg, uint32_t deg, uint32_t du,
                                                const uint32_t* __restrict__ col, const uint32_t* __restrict__ w,
                                                uint32_t* dist, uint32_t* __restrict__ stamp, uint32_t epoch,
-                                               uint32_t thr, Stage& st, const Sinks& k, unsigned long long& ndeg,
-                                               LocalList* loc, uint32_t side, uint32_t& fmin) {
-    __shared__ uint32_t s_beg[256], s_off[256], s_du[256], s_wave[4];
+                                               uint32_t thr, StageOf<kThreads, kSlices>& st, const Sinks& k,
+                                               unsigned long long& ndeg, LocalList* loc, uint32_t side,
+                                               uint32_t& fmin) {
+    __shared__ uint32_t s_beg[kThreads], s_off[kThreads], s_du[kThreads], s_wave[kThreads / kWave];
     const uint32_t t = threadIdx.x;
     uint32_t total;
-    const uint32_t excl = block_excl_scan(deg, s_wave, total);
+    const uint32_t excl = block_excl_scan<kThreads>(deg, s_wave, total);
     s_beg[t] = beg;
     s_off[t] = excl;
     s_du[t] = du;
     __syncthreads();
-    for (uint32_t e0 = 0; e0 < total; e0 += 256) {  // uniform per block
+    for (uint32_t e0 = 0; e0 < total; e0 += kThreads) {  // uniform per block
         const uint32_t e = e0 + t;
         bool to_near = false, to_far = false;
         uint32_t v = 0, vdeg = 0;
         if (e < total) {
             uint32_t lo = 0;
 #pragma unroll
-            for (uint32_t step = 128; step; step >>= 1)
+            for (uint32_t step = kThreads / 2; step; step >>= 1)
                 if (s_off[lo + step] <= e) lo += step;
             const uint32_t x = s_beg[lo] + (e - s_off[lo]);
             v = col[x];
@@ -308,32 +321,33 @@ __device__ __forceinline__ unsigned long long local_rounds(LocalList* loc, uint3
     return relax;
 }
 
-// Entries per workgroup tile: 256, or fewer when the queue is short, so that every workgroup
+// Entries per workgroup tile: one per thread, or fewer when the queue is short, so that every workgroup
 // of the grid gets a tile (a queue of 1000 entries, hub slices of 128 out-edges among them,
 // would otherwise give its edges to 4 workgroups).  With local rounds each workgroup then
 // continues from the vertices its own tile lowered, so a short queue also spreads those
 // rounds over the whole grid.
+template <uint32_t kThreads>
 __device__ __forceinline__ uint32_t relax_tile_entries(uint32_t qn) {
     const uint32_t per = (uint32_t)(((uint64_t)qn + gridDim.x - 1) / gridDim.x);
-    return per < 1u ? 1u : (per > 256u ? 256u : per);
+    return per < 1u ? 1u : (per > kThreads ? kThreads : per);
 }
 
 // Relaxes near entries q[0, qn) with the whole block: workgroup b takes the T entries of
 // chunks b, b + grid, ... (T = relax_tile_entries).  With a local list and rounds > 0, the
 // block then runs up to `rounds` further tiles over the vertices it lowered itself.  Returns
 // (in every thread) the edges relaxed by this block.  kSpec as for relax_tile.
-template <bool kSpec>
+template <bool kSpec, class St>
 __device__ __forceinline__ unsigned long long relax_block(const unsigned long long* __restrict__ q, uint32_t qn,
                                                           const uint32_t* __restrict__ col,
                                                           const uint32_t* __restrict__ w, uint32_t* dist,
                                                           uint32_t* __restrict__ stamp, uint32_t epoch, uint32_t thr,
-                                                          Stage& st, const Sinks& k, unsigned long long& ndeg,
+                                                          St& st, const Sinks& k, unsigned long long& ndeg,
                                                           LocalList* loc = nullptr, uint32_t rounds = 0) {
     const uint32_t t = threadIdx.x;
     if (!loc) rounds = 0;
     unsigned long long relax = 0;
     uint32_t fmin = 0xFFFFFFFFu;  // not needed after a relaxation superstep
-    const uint32_t T = relax_tile_entries(qn);
+    const uint32_t T = relax_tile_entries<St::kWidth>(qn);
     for (uint32_t chunk = blockIdx.x; (uint64_t)chunk * T < qn; chunk += gridDim.x) {  // uniform per block
         const uint64_t i = (uint64_t)chunk * T + t;
         uint32_t beg = 0, deg = 0, du = 0;
@@ -348,7 +362,9 @@ __device__ __forceinline__ unsigned long long relax_block(const unsigned long lo
         relax += relax_tile<kSpec>(beg, deg, du, col, w, dist, stamp, epoch, thr, st, k, ndeg, loc,
                                    rounds ? 0u : 2u, fmin);
     }
-    if (rounds) relax += local_rounds<kSpec>(loc, rounds, col, w, dist, stamp, epoch, thr, st, k, ndeg, fmin);
+    if constexpr (std::is_same_v<St, Stage>) {
+        if (rounds) relax += local_rounds<kSpec>(loc, rounds, col, w, dist, stamp, epoch, thr, st, k, ndeg, fmin);
+    }
     return relax;
 }
 
@@ -358,12 +374,13 @@ __device__ __forceinline__ unsigned long long relax_block(const unsigned long lo
 // Returns the smallest kept far distance of this thread.  With a local list, a vertex moved
 // to the near side (one slice) goes to side 0 of the list instead, for the block to relax in
 // the same launch; the stamp still marks it moved, so duplicates in the far queue move once.
+template <class St>
 __device__ __forceinline__ uint32_t split_block(const uint32_t* __restrict__ far_in, uint32_t nin, bool rescan,
                                                 const uint32_t* __restrict__ dist, uint32_t* __restrict__ stamp,
-                                                uint32_t epoch, uint32_t old_thr, uint32_t thr, Stage& st,
+                                                uint32_t epoch, uint32_t old_thr, uint32_t thr, St& st,
                                                 const Sinks& k, unsigned long long& ndeg, LocalList* loc = nullptr) {
     uint32_t fmin = 0xFFFFFFFFu;
-    for (uint32_t i0 = blockIdx.x * 256; i0 < nin; i0 += gridDim.x * 256) {  // uniform per block
+    for (uint32_t i0 = blockIdx.x * St::kWidth; i0 < nin; i0 += gridDim.x * St::kWidth) {  // uniform per block
         const uint32_t i = i0 + threadIdx.x;
         bool to_near = false, keep = false;
         uint32_t v = 0, vdeg = 0;
@@ -420,6 +437,16 @@ __device__ __forceinline__ uint32_t wave_min_u32(uint32_t x) {
 // graphs of mean out-degree 2 and 4 (262 K vertices) 0.47 -> 0.23 and 0.77 -> 0.46 ms.  With hubs
 // the rings of a few waves hold the frontier and the others idle (2.4 M-vertex Chung-Lu graph,
 // out-degrees up to 100 K: 1.3 ms against 0.75 in the block-wide tiles), hence the rule.
+//
+// They run up to kWaveQueue entries.  Wider frontiers are bound by the rate of random accesses, and
+// there the rounds relax vertices at distances that fall again, with an atomicMin for every offer and
+// an append to the near queue for every 64: such a superstep is a block-wide tile without rounds, as on
+// denser graphs.  Uniform random graphs of mean out-degree 4, without the bound, with it, and with the
+// block-wide rounds everywhere: 2^22 vertices 3.93, 2.02 and 2.47 ms, 2^24 13.2, 5.7 and 6.5; with 8 rounds
+// asked for on mean out-degree 8 (2^20) 6.03, 1.68 and 2.72.  Bounds of 32768 and 65536 are level with this one
+// there, but in the 1400^2 lattice without buckets, whose frontier is that wide, they take 31 and 24 ms
+// instead of 8.8 (without any bound 8.8).  The other side of it: 3000^2 without buckets 77 ms unbounded, 159
+// bounded, 146 with the block-wide rounds; with buckets (9.4 ms) it does not get there.
 constexpr uint32_t kRecEdges = 7;
 constexpr uint32_t kRecWords = 4;        // uint4 per record: {out-degree, row_ptr, (target, weight) x 7}
 constexpr uint32_t kRing = 512;          // offers per wave
@@ -430,6 +457,7 @@ constexpr uint32_t kWide = 4;            // out-edges per lane in flight of vert
 constexpr uint32_t kWaveThreads = 1024;  // few workgroups, so few atomics on the queue counters
 constexpr uint32_t kBlockWaves = kWaveThreads / kWave;
 constexpr uint32_t kSsspGridWave = 256;  // a workgroup per CU (LDS)
+constexpr uint32_t kWaveQueue = 131072;  // near (split: far) entries up to which the wave rounds run
 static_assert(kRing >= kWave * kRecEdges && kRing >= kWave * kWide && kRing >= kKeep && (kRing & (kRing - 1)) == 0,
               "a tile's offers fit");
 
@@ -1025,13 +1053,17 @@ __global__ __launch_bounds__(256) void k_sssp_work(SsspCtl* ctl,
     if (sssp_last_block(ctr, dep, relax) && threadIdx.x == 0) sssp_decide(ctl, ctr, relax, far_cap, near_cap, marks);
 }
 
-// The same slot with wave rounds.
+// The same slot with wave rounds, up to kWaveQueue entries; block-wide above.
 __global__ __launch_bounds__(kWaveThreads) void k_sssp_work_wave(
     SsspCtl* ctl, unsigned long long* __restrict__ near0, unsigned long long* __restrict__ near1, uint32_t near_cap,
     uint32_t* __restrict__ far0, uint32_t* __restrict__ far1, uint32_t far_cap, const uint32_t* __restrict__ row_ptr,
     const uint32_t* __restrict__ col, const uint32_t* __restrict__ w, const uint4* __restrict__ rec, uint32_t* dist,
     uint32_t* __restrict__ stamp, SsspDevCounters* __restrict__ ctr, unsigned long long* __restrict__ marks) {
-    __shared__ WaveLds lds;
+    // one slice per vertex: no hubs
+    using WideStage = StageOf<kWaveThreads, 1>;
+    __shared__ alignas(16) unsigned char s_lds[sizeof(WaveLds) > sizeof(WideStage) ? sizeof(WaveLds) : sizeof(WideStage)];
+    WaveLds& lds = *reinterpret_cast<WaveLds*>(s_lds);
+    WideStage& st = *reinterpret_cast<WideStage*>(s_lds);
     const SsspCtl c = *ctl;
     // every field this kernel reads, loaded in one round trip
     keep_here(c.done);
@@ -1049,6 +1081,7 @@ __global__ __launch_bounds__(kWaveThreads) void k_sssp_work_wave(
     if (c.done) return;  // uniform: no workgroup takes a ticket
     unsigned long long relax = 0;
     unsigned long long dep = 0;  // thread 0's last counter atomic result
+    unsigned long long ndeg = 0;
     uint32_t fmin;
     if (c.split_pending) {
         // the moved vertices are relaxed at once; what that lowers is stamped with the next epoch, so
@@ -1056,16 +1089,36 @@ __global__ __launch_bounds__(kWaveThreads) void k_sssp_work_wave(
         const Sinks k{c.near_sel ? near1 : near0, &ctr->n_near, near_cap, c.far_sel ? far0 : far1,
                       &ctr->far_out, far_cap, row_ptr};
         const uint32_t rescan = c.overflow != 0;
-        const WaveIn in{rec, col, w, dist, stamp, c.epoch + 1, c.thr, c.local_cfg, nullptr, c.far_sel ? far1 : far0,
-                        rescan ? (uint32_t)c.n : c.n_far, rescan, c.epoch, c.old_thr};
-        wave_superstep<true>(in, lds, k, relax, fmin);
-        if (threadIdx.x == 0 && fmin != 0xFFFFFFFFu) dep += atomicMin(&ctr->far_min, fmin);
+        const uint32_t nin = rescan ? (uint32_t)c.n : c.n_far;
+        if (nin > kWaveQueue) {
+            stage_init(st);
+            fmin = split_block(c.far_sel ? far1 : far0, nin, rescan != 0, dist, stamp, c.epoch, c.old_thr, c.thr, st, k,
+                               ndeg);
+            stage_flush(st, k, true);  // thread 0 stored its atomics' results in LDS
+            fmin = wave_min_u32(fmin);
+            if ((threadIdx.x & (kWave - 1)) == 0 && fmin != 0xFFFFFFFFu) {
+                const uint32_t r = atomicMin(&ctr->far_min, fmin);
+                asm volatile("" ::"v"(r));  // wait for it before the barrier in sssp_last_block
+            }
+        } else {
+            const WaveIn in{rec, col, w, dist, stamp, c.epoch + 1, c.thr, c.local_cfg, nullptr,
+                            c.far_sel ? far1 : far0, nin, rescan, c.epoch, c.old_thr};
+            wave_superstep<true>(in, lds, k, relax, fmin);
+            if (threadIdx.x == 0 && fmin != 0xFFFFFFFFu) dep += atomicMin(&ctr->far_min, fmin);
+        }
     } else {
         const Sinks k{c.near_sel ? near0 : near1, &ctr->n_near, near_cap, c.far_sel ? far1 : far0, &ctr->n_far,
                       far_cap, row_ptr};
-        const WaveIn in{rec, col, w, dist, stamp, c.epoch, c.thr, c.local_cfg, c.near_sel ? near1 : near0, nullptr,
-                        c.n_near, 0, 0, 0};
-        wave_superstep<false>(in, lds, k, relax, fmin);
+        if (c.n_near > kWaveQueue) {
+            stage_init(st);
+            relax = relax_block<false>(c.near_sel ? near1 : near0, c.n_near, col, w, dist, stamp, c.epoch, c.thr, st, k,
+                                       ndeg);
+            stage_flush(st, k, true);  // thread 0 stored its atomics' results in LDS
+        } else {
+            const WaveIn in{rec, col, w, dist, stamp, c.epoch, c.thr, c.local_cfg, c.near_sel ? near1 : near0, nullptr,
+                            c.n_near, 0, 0, 0};
+            wave_superstep<false>(in, lds, k, relax, fmin);
+        }
     }
     if (sssp_last_block(ctr, dep, relax) && threadIdx.x == 0) sssp_decide(ctl, ctr, relax, far_cap, near_cap, marks);
 }
@@ -1458,7 +1511,7 @@ static void sssp_run_host(medusa_graph* g, uint32_t src, uint32_t* out, const me
         if (timing) MDS_HIP(hipEventRecord(g->events[0], s));  // brackets the relaxation launch alone
         // 256 entries per workgroup chunk; the far queue keeps growing at far_a[n_far..)
         const uint32_t rounds = n_near <= kLocalQueue ? local_cfg : 0u;
-        if (rec)
+        if (rec && n_near <= kWaveQueue)
             hipLaunchKernelGGL(k_sssp_relax_wave, dim3(kSsspGridWave), dim3(kWaveThreads), 0, s, near_cur, n_near,
                                g->row_ptr.p, g->col.p, g->w.p, rec, g->dist.p, g->stamp.p, epoch, thr, near_nxt,
                                (uint32_t)near_cap, far_a, (uint32_t)far_cap, C, local_cfg);
