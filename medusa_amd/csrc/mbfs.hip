@@ -62,7 +62,7 @@ enum : uint32_t { kMbfsPush, kMbfsUpdate, kMbfsPull, kMbfsQueue };
 struct MbfsCtl {
     int32_t step;
     uint32_t phase, pull, done, n_large, hub_wgs, mode, saturated;
-    uint32_t supersteps, push_steps, pull_steps, k, slots, pad;
+    uint32_t supersteps, push_steps, pull_steps, k, slots, n_small;
     unsigned long long n, m, n_f, m_f, n_u, m_u, reached, reached_edges, kernel_bytes, alg_bytes, full;
     uint8_t* out;  // where the finish of a device-driven run writes the levels, or null
 };
@@ -376,17 +376,57 @@ struct MbfsAcc {
     }
 };
 
-// The new bits of vertex p (every p < n that the caller owns, with nx = 0 if none) at level lv.
-template <class T>
-__device__ __forceinline__ void mbfs_set_level(const MbfsArgs& a, uint32_t lv, uint32_t p, unsigned long long nx) {
-    T* plane = static_cast<T*>(a.planes) + p;
-    if (!(lv & (lv - 1))) {  // a plane's first use: every word written, none read
-        plane[(size_t)__builtin_ctz(lv) * a.n] = (T)nx;
-        return;
+// What the planes hold for a level: the level, with 128 and 255 exchanged, so the levels past 254
+// (saturated, reported as unreached), which a long graph has one of in every superstep, take one plane
+// each and not all eight; and, above the code's eight bits, the plane that is used for the first time plus 1.
+constexpr uint32_t kMbfsSaturated = 255;
+__device__ __forceinline__ uint32_t mbfs_code(uint32_t level) {
+    const uint32_t code = level >= kMbfsSaturated ? 128u : level == 128 ? 255u : level;
+    const uint32_t first = level <= 128 && !(level & (level - 1)) ? (uint32_t)__builtin_ctz(level) + 1 : 0u;
+    return code | first << 8;
+}
+
+// The new bits of a lane's kN vertices v0, v0 + 64, .. (nx = 0 past the last vertex and where the caller
+// has none of its own: `mine`) at the level of `code`.  In a plane's first use every word is written and
+// none read.  The others' words are read and written a plane at a time, its kN loads together: vertex by
+// vertex these were up to 32 dependent accesses of a superstep.  700 x 700 lattice, 1262 supersteps of 8
+// sources: 25.8 ms so, 25.4 a plane at a time, 21.1 with the codes for the saturated levels (and with the
+// workgroups that find nothing to do leaving at once); two planes at a time are level, all eight at a time
+// spill (29.2).
+template <class T, uint32_t kN>
+__device__ __forceinline__ void mbfs_set_levels(const MbfsArgs& a, uint32_t code, uint64_t v0,
+                                                const unsigned long long (&nx)[kN], const bool (&mine)[kN]) {
+    T* const planes = static_cast<T*>(a.planes) + v0;
+    uint32_t bits = code & 0xFF;
+    if (code >> 8) {
+        const uint32_t p = (code >> 8) - 1;
+        T* plane = planes + (size_t)p * a.n;
+#pragma unroll
+        for (uint32_t c = 0; c < kN; ++c)
+            if (mine[c]) plane[c * kWave] = (T)nx[c];
+        bits &= ~(1u << p);
     }
-    if (!nx) return;
-    for (uint32_t b = 0; b < kMbfsPlanes; ++b)  // uniform
-        if ((lv >> b) & 1u) plane[(size_t)b * a.n] |= (T)nx;
+    unsigned long long any = 0;
+#pragma unroll
+    for (uint32_t c = 0; c < kN; ++c) any |= nx[c];
+    if (!any) return;
+#pragma unroll 1
+    for (; bits; bits &= bits - 1) {  // uniform
+        T* plane = planes + (size_t)__builtin_ctz(bits) * a.n;
+        T old[kN];
+#pragma unroll
+        for (uint32_t c = 0; c < kN; ++c)
+            if (nx[c]) old[c] = plane[c * kWave];
+#pragma unroll
+        for (uint32_t c = 0; c < kN; ++c)
+            if (nx[c]) plane[c * kWave] = old[c] | (T)nx[c];
+    }
+}
+template <class T>
+__device__ __forceinline__ void mbfs_set_level(const MbfsArgs& a, uint32_t code, uint32_t p, unsigned long long nx) {
+    const unsigned long long one[1] = {nx};
+    const bool mine[1] = {true};
+    mbfs_set_levels<T, 1>(a, code, p, one, mine);
 }
 
 constexpr uint32_t kMbfsPullGroup = 4;  // in-edges a lane probes per round
@@ -531,11 +571,12 @@ __device__ __forceinline__ void mbfs_tiles(const MbfsArgs& a, uint32_t lv, unsig
                 nx[c] = raw[c] & ~vis[c];
                 if (raw[c]) a.next[v] = 0;
                 if (nx[c]) a.visited[v] = vis[c] | nx[c];
-                if (v < n) {
-                    nxt[v] = nx[c];
-                    mbfs_set_level<T>(a, lv, (uint32_t)v, nx[c]);
-                }
+                if (v < n) nxt[v] = nx[c];
             }
+            bool mine[4];
+#pragma unroll
+            for (uint32_t c = 0; c < 4; ++c) mine[c] = v0 + c * kWave < n;
+            mbfs_set_levels<T, 4>(a, lv, v0, nx, mine);
         } else {
 #pragma unroll
             for (uint32_t c = 0; c < 4; ++c) nx[c] = v0 + c * kWave < n ? nxt[v0 + c * kWave] : 0ull;
@@ -582,11 +623,11 @@ __device__ __forceinline__ void mbfs_tiles(const MbfsArgs& a, uint32_t lv, unsig
     }
 }
 
-// End of an update or pull: the workgroup's sums to its counter line and, with kDecide, its ticket
-// (two levels, so no address sees more than grid / kMbfsSegs atomics).  True in the first wave of
-// the workgroup that came last.
+// End of an update or pull: the workgroup's sums to its counter line and, with kDecide, its ticket of
+// `wgs` that have work (two levels, so no address sees more than wgs / kMbfsSegs atomics).  True in the
+// first wave of the workgroup that came last.
 template <bool kDecide>
-__device__ __forceinline__ bool mbfs_finish_launch(MbfsCounters* __restrict__ ctr, const MbfsAcc& acc) {
+__device__ __forceinline__ bool mbfs_finish_launch(MbfsCounters* __restrict__ ctr, const MbfsAcc& acc, uint32_t wgs) {
     __shared__ unsigned long long s_sum[kMbfsSums];
     const uint32_t lane = threadIdx.x & (kWave - 1);
     if (threadIdx.x < kMbfsSums) s_sum[threadIdx.x] = 0;
@@ -617,8 +658,8 @@ __device__ __forceinline__ bool mbfs_finish_launch(MbfsCounters* __restrict__ ct
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     uint32_t last = 0;
     if (lane == 0) {
-        const uint32_t members = (gridDim.x - sg + kMbfsSegs - 1) / kMbfsSegs;  // workgroups of line sg
-        const uint32_t nsegs = gridDim.x < kMbfsSegs ? gridDim.x : kMbfsSegs;
+        const uint32_t members = (wgs - sg + kMbfsSegs - 1) / kMbfsSegs;  // workgroups of line sg
+        const uint32_t nsegs = wgs < kMbfsSegs ? wgs : kMbfsSegs;
         if (atomicAdd(&ctr->sub[sg].v, 1u) == members - 1) last = atomicAdd(&ctr->top.v, 1u) == nsegs - 1;
     }
     return __builtin_amdgcn_readfirstlane((int)last) != 0;
@@ -679,6 +720,7 @@ __device__ __forceinline__ void mbfs_decide(const MbfsArgs& a, bool first, uint3
     c.m_u -= edges;
     c.n_f = n_active;
     c.m_f = active_deg;
+    c.n_small = n_small;
     c.n_large = n_large;
     c.hub_wgs = mbfs_hub_wgs(a.grid, n_small, n_large, large_deg, active_deg);
     if (n_active == 0) c.done = 1;
@@ -727,7 +769,7 @@ __global__ __launch_bounds__(kWave) void k_mbfs_start(MbfsArgs a, MbfsSources sr
         a.ctr->queued[0][0].v = (uint32_t)__popcll(sm);
         a.ctr->hubs[0].v = (uint32_t)__popcll(lm);
     }
-    mbfs_finish_launch<false>(a.ctr, acc);
+    mbfs_finish_launch<false>(a.ctr, acc, 1);
     if (!decide) return;
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // its atomics have been performed
     mbfs_decide(a, true, 0, s_params);
@@ -753,7 +795,7 @@ __global__ __launch_bounds__(256, 8) void k_mbfs_super(MbfsArgs a, uint32_t slot
         return;
     }
     const uint32_t step = (uint32_t)ctl->step, par = step & 1u;
-    const uint32_t lv = step + 1 >= 255 ? 255u : step + 1;  // 255: saturated, reported as unreached
+    const uint32_t lv = mbfs_code(step + 1);
     MbfsAcc acc;
     if (phase == kMbfsPush) {
         pass_on(kMbfsUpdate);
@@ -762,6 +804,7 @@ __global__ __launch_bounds__(256, 8) void k_mbfs_super(MbfsArgs a, uint32_t slot
             mbfs_push_large(a, ctl->n_large, a.frontier[par], blockIdx.x, hub);
         } else {
             const uint32_t wg = blockIdx.x - hub, nwg = gridDim.x - hub;
+            if (wg * 4 >= ctl->n_small) return;  // no entry for its waves
             mbfs_push_small(a, a.ctr->queued[par], a.frontier[par], wg * 4 + threadIdx.x / kWave, nwg * 4, s_push);
         }
         return;
@@ -771,11 +814,16 @@ __global__ __launch_bounds__(256, 8) void k_mbfs_super(MbfsArgs a, uint32_t slot
         mbfs_tiles<T, false>(a, lv, a.frontier[par], a.ctr->queued[par], &a.ctr->hubs[par].v, acc, s_tile);
         return;
     }
+    // workgroups without a slice, hub or tile leave at once, without a ticket (RMAT-18 pushed from one source
+    // 254 us before, 248 now; 25 K vertices, 16 sources 478 and 470)
+    const uint32_t items = phase == kMbfsPull ? (max(a.nslices, a.nhubs) + 3) / 4 : (a.n - 1) / kMbfsTile + 1;
+    const uint32_t wgs = min(gridDim.x, items);
+    if (blockIdx.x >= wgs) return;
     if (phase == kMbfsPull)
         mbfs_pull<T>(a, ctl->full, lv, a.frontier[par], a.frontier[par ^ 1u], acc);
     else
         mbfs_tiles<T, true>(a, lv, a.frontier[par ^ 1u], a.ctr->queued[par ^ 1u], &a.ctr->hubs[par ^ 1u].v, acc, s_tile);
-    if (mbfs_finish_launch<kDecide>(a.ctr, acc)) mbfs_decide(a, false, slot, s_params);
+    if (mbfs_finish_launch<kDecide>(a.ctr, acc, wgs)) mbfs_decide(a, false, slot, s_params);
 }
 
 // Bit j, j + 4, .. j + 28 of four planes' words as the nibbles of a word.
@@ -820,10 +868,26 @@ __global__ __launch_bounds__(1024) void k_mbfs_finish(MbfsArgs a, MbfsHost* __re
 #pragma unroll
         for (uint32_t i = 0; i < 4; ++i) at[i] = a.pos[i < cnt ? v0 + i : v0];
 #pragma unroll
-        for (uint32_t i = 0; i < 4; ++i) {
-            vis[i] = a.visited[at[i]];
+        for (uint32_t i = 0; i < 4; ++i) vis[i] = a.visited[at[i]];
+        // a vertex that no source reaches has no level to read
 #pragma unroll
-            for (uint32_t p = 0; p < kMbfsPlanes; ++p) x[p][i] = p < np ? planes[(size_t)p * n + at[i]] : (T)0;
+        for (uint32_t i = 0; i < 4; ++i)
+#pragma unroll
+            for (uint32_t p = 0; p < kMbfsPlanes; ++p)
+                x[p][i] = p < np && vis[i] ? planes[(size_t)p * n + at[i]] : (T)0;
+        if (np == kMbfsPlanes) {  // uniform: codes back to levels (mbfs_code)
+#pragma unroll
+            for (uint32_t i = 0; i < 4; ++i) {
+                T some = 0, every = (T)~(T)0;
+#pragma unroll
+                for (uint32_t p = 0; p < kMbfsPlanes - 1; ++p) {
+                    some |= x[p][i];
+                    every &= x[p][i];
+                }
+                const T saturated = x[kMbfsPlanes - 1][i] & (T)~some, l128 = x[kMbfsPlanes - 1][i] & every;
+#pragma unroll
+                for (uint32_t p = 0; p < kMbfsPlanes - 1; ++p) x[p][i] = (T)((x[p][i] & (T)~l128) | saturated);
+            }
         }
 #pragma unroll
         for (uint32_t h = 0; h < (sizeof(T) == 8 ? 2u : 1u); ++h) {
@@ -870,9 +934,11 @@ __global__ __launch_bounds__(1024) void k_mbfs_finish(MbfsArgs a, MbfsHost* __re
 }
 
 // Host-driven launch: the host's decision written into the control block.
-__global__ void k_mbfs_set_ctl(MbfsCtl* ctl, int32_t step, uint32_t phase, uint32_t n_large, uint32_t hub_wgs) {
+__global__ void k_mbfs_set_ctl(MbfsCtl* ctl, int32_t step, uint32_t phase, uint32_t n_small, uint32_t n_large,
+                               uint32_t hub_wgs) {
     ctl->step = step;
     ctl->phase = phase;
+    ctl->n_small = n_small;
     ctl->n_large = n_large;
     ctl->hub_wgs = hub_wgs;
 }
@@ -1029,7 +1095,7 @@ static void mbfs_run(medusa_graph* g, const uint32_t* srcs, uint32_t k, uint8_t*
         };
         auto launch = [&](uint32_t t, uint32_t phase) {
             const uint32_t n_small = (uint32_t)c[kMbfsQueued], n_large = (uint32_t)(c[kMbfsQueued] >> 32);
-            hipLaunchKernelGGL(k_mbfs_set_ctl, dim3(1), dim3(1), 0, s, ctl, (int32_t)t, phase, n_large,
+            hipLaunchKernelGGL(k_mbfs_set_ctl, dim3(1), dim3(1), 0, s, ctl, (int32_t)t, phase, n_small, n_large,
                                mbfs_hub_wgs(grid, n_small, n_large, c[kMbfsLargeDeg], c[kMbfsActiveDeg]));
             MDS_LAUNCHED();
             hipLaunchKernelGGL((k_mbfs_super<T, false>), dim3(grid), dim3(256), 0, s, a, 0u);
@@ -1083,7 +1149,7 @@ static void mbfs_run(medusa_graph* g, const uint32_t* srcs, uint32_t k, uint8_t*
             h.m_u -= c[kMbfsReachedEdges];
         }
         // the last level, for the finish
-        hipLaunchKernelGGL(k_mbfs_set_ctl, dim3(1), dim3(1), 0, s, ctl, (int32_t)h.supersteps, 0u, 0u, 0u);
+        hipLaunchKernelGGL(k_mbfs_set_ctl, dim3(1), dim3(1), 0, s, ctl, (int32_t)h.supersteps, 0u, 0u, 0u, 0u);
         MDS_LAUNCHED();
         if (direct) {
             hipLaunchKernelGGL(k_mbfs_finish<T>, finish_grid, dim3(finish_wg), 0, s, a, (MbfsHost*)nullptr, out, 0u, k);
