@@ -85,8 +85,10 @@ typedef struct medusa_opts {
 /* Per-run statistics.  Reference: printf of wall time / steps (Algorithm/main.cu:316,355,
  * SSSP/main.cu:391-392, MPG/main.cu:173). */
 typedef struct medusa_stats {
-    double   device_ms;        /* GPU time of the run on HBM-resident data: by the device's clock from its first
-                                  kernel to its last (BFS, SSSP, MBFS), by hipEvents (PageRank, timed runs) */
+    double   device_ms;        /* GPU time of the run on HBM-resident data, from its first kernel to the end of its
+                                  last superstep (MBFS: of the making of the level bytes), without copying or
+                                  reordering the result into the output: by the device's clock (BFS, SSSP, MBFS),
+                                  by hipEvents (PageRank, timed runs) */
     double   kernel_ms;        /* summed duration of the dominant kernel's launches (opts.timing) */
     uint64_t kernel_launches;  /* launches of the dominant kernel */
     uint64_t kernel_bytes;     /* algorithmic bytes moved by those launches (byte model) */

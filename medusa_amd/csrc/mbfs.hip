@@ -68,9 +68,11 @@ struct MbfsCtl {
 };
 
 // What a device-driven run leaves in pinned memory.
+constexpr uint32_t kMbfsEnds = 1024;
 struct MbfsHost {
     MbfsCtl ctl;
-    unsigned long long t_begin, t_end;
+    unsigned long long t_begin, t_end;   // wall clock before the first kernel and after the last superstep
+    unsigned long long made[kMbfsEnds];  // and when workgroups of the finish had stored their levels
 };
 
 struct MbfsArgs {
@@ -931,6 +933,11 @@ __global__ __launch_bounds__(1024) void k_mbfs_finish(MbfsArgs a, MbfsHost* __re
             }
         }
     }
+    if (!host) return;
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    if (threadIdx.x == 0)
+        host->made[(blockIdx.y * gridDim.x + blockIdx.x) % kMbfsEnds] = (unsigned long long)wall_clock64();
 }
 
 // Host-driven launch: the host's decision written into the control block.
@@ -1078,7 +1085,10 @@ static void mbfs_run(medusa_graph* g, const uint32_t* srcs, uint32_t k, uint8_t*
         }
         h = host->ctl;
         g->mbfs_last_slots = h.slots;
-        st.device_ms = (double)(host->t_end - host->t_begin) / (double)g->wall_khz;
+        unsigned long long t_end = host->t_end;
+        const uint32_t ends = std::min(finish_grid.x * finish_grid.y, kMbfsEnds);
+        if (direct) t_end = std::max(t_end, *std::max_element(host->made, host->made + ends));
+        st.device_ms = (double)(t_end - host->t_begin) / (double)g->wall_khz;
     } else {
         Sched sched(o, Sched::kMbfs, k);
         const bool timing = o.timing != 0;
@@ -1177,9 +1187,14 @@ static void mbfs_run(medusa_graph* g, const uint32_t* srcs, uint32_t k, uint8_t*
     for (uint32_t r = 0; r < k; r += rows) {
         const uint32_t r1 = std::min(k, r + rows);
         uint8_t* buf = reinterpret_cast<uint8_t*>(g->mbfs_rows.p);
+        MDS_HIP(hipEventRecord(g->ev_begin, s));
         hipLaunchKernelGGL(k_mbfs_finish<T>, finish_grid, dim3(finish_wg), 0, s, a, (MbfsHost*)nullptr, buf, r, r1);
         MDS_LAUNCHED();
-        copy_out(g, out + (size_t)r * n, buf, (size_t)(r1 - r) * n);
+        MDS_HIP(hipEventRecord(g->ev_end, s));
+        copy_out(g, out + (size_t)r * n, buf, (size_t)(r1 - r) * n);  // waits for the stream
+        float ms = 0;
+        MDS_HIP(hipEventElapsedTime(&ms, g->ev_begin, g->ev_end));
+        st.device_ms += ms;
     }
 }
 

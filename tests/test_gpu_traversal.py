@@ -356,6 +356,23 @@ def test_mbfs_hubs_and_slices(oracle, n):
                         host.supersteps, host.push_steps, host.pull_steps, host.edges_traversed)
 
 
+@pytest.mark.parametrize("where", ["device", "host"])
+def test_mbfs_device_time_covers_the_levels(where):
+    """device_ms covers the making of the level bytes: without edges, 64 sources differ from 33 by 31 rows
+    of levels alone (the masks and planes are as wide), and the GPU cannot write those faster than its
+    memory-side cache takes them (17.2 TB/s)."""
+    torch = pytest.importorskip("torch")
+    n = 1 << 24
+    ms = {}
+    with md.Graph(np.zeros(n + 1, np.uint32), np.zeros(0, np.uint32)) as G:
+        for k in (33, 64):
+            out = torch.empty((k, n), dtype=torch.uint8, device="cuda") if where == "device" else np.empty((k, n), np.uint8)
+            srcs = np.arange(k, dtype=np.uint32)
+            ms[k] = min(G.mbfs(srcs, out=out)[1].device_ms for _ in range(5))
+    print(f"[mbfs levels {where}] 33 sources {ms[33]:.4f} ms, 64 sources {ms[64]:.4f} ms", flush=True)
+    assert ms[64] - ms[33] >= 31 * n / 17.2e12 * 1e3
+
+
 def test_mbfs_rows_in_pieces():
     """A host output of more bytes than the row buffer holds: no vertex but the sources is reached."""
     n, k = 5_000_001, 64
