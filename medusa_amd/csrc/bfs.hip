@@ -1368,7 +1368,14 @@ __global__ __launch_bounds__(256) void k_bfs_super(BfsArgs a, uint32_t slot) {
             c.slots += 1;
             c.out = ctl->out;  // again, rather than kept (on the stack) through the supersteps
             c.t_begin = ctl->t_begin;
-            if (!c.done) bfs_set_direction(a, c, c.mode != 1 && bfs_heuristic(c, false), false);
+            if (!c.done) {
+                if (threadIdx.x < kWave) {
+                    const bool pull = bfs_next_pull(a, c, s_params);
+                    if (threadIdx.x == 0) s_pre[0] = pull ? 1u : 0u;
+                }
+                __syncthreads();
+                bfs_set_direction(a, c, s_pre[0] != 0, false);
+            }
             solo_publish(a, L, c, a.ctl + (slot ^ 1u));
             return;
         }

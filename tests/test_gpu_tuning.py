@@ -78,6 +78,37 @@ def test_any_policy_keeps_results_exact(oracle, skewed, seed):
         assert np.array_equal(G.mbfs(srcs, policy=pol, trace=1)[0], want)
 
 
+def test_policy_asked_after_thin_supersteps(oracle):
+    """A frontier that one workgroup has taken through thin supersteps and that grows again (a chain, then
+    a vertex with 3000 out-edges, where the heuristic pushes and a policy is consulted): the device-driven
+    loop asks the policy for that superstep as the host-driven one does."""
+    a, d, e = 6000, 3000, 10_000
+    A = 1 + np.arange(a)
+    chain = 1 + a + np.arange(5)
+    D = 1 + a + 5 + np.arange(d)
+    E = 1 + a + 5 + d + np.arange(e)
+    rng = np.random.default_rng(3)
+    edges = [np.stack([np.zeros(a, np.int64), A], 1), np.stack([A, np.full(a, chain[0])], 1),
+             np.stack([chain[:-1], chain[1:]], 1), np.stack([np.full(d, chain[-1]), D], 1),
+             np.stack([np.repeat(D, 4), rng.choice(E, 4 * d)], 1)]
+    n = 1 + a + 5 + d + e
+    rp, col, _ = csr_from_edges(n, np.concatenate(edges))
+    want = oracle.bfs_queue(rp, col, 0)
+    at = 6  # the level of the chain's last vertex
+    pulls = []
+    with md.Graph(rp, col) as G:
+        for seed in range(1, 9):
+            pol = md.Policy(md.POLICY_DIRECTION, seed=seed)
+            lv, dev = G.bfs(0, policy=pol)
+            assert np.array_equal(lv, want), seed
+            lv, host = G.bfs(0, policy=pol, timing=1, trace=1)
+            assert np.array_equal(lv, want), seed
+            pulls.append(int(G.trace()[at, 7]))
+            assert (dev.push_steps, dev.pull_steps) == (host.push_steps, host.pull_steps), seed
+    print(f"[policy] directions at the chain's end: {pulls}", flush=True)
+    assert 0 < sum(pulls) < len(pulls)
+
+
 def test_mbfs_saturated_levels(oracle):
     """A path longer than 255: levels saturate at 0xFF and the flag is raised."""
     n = 300
