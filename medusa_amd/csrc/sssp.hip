@@ -1230,16 +1230,19 @@ static uint32_t sssp_local_cfg(const medusa_graph* g, const medusa_opts& o) {
 static const uint4* sssp_records(medusa_graph* g, const medusa_opts& o) {
     if (!sssp_local_cfg(g, o) || g->max_outdeg > kSlice) return nullptr;
     if (!g->sssp_rec.p) {
+        DBuf<uint4> rec;  // the handle's once it is written: a failed launch leaves none behind
         try {
-            g->sssp_rec.alloc((size_t)g->n * kRecWords);
+            rec.alloc((size_t)g->n * kRecWords);
         } catch (const Error& e) {
             if (e.code != MEDUSA_ERR_NOMEM) throw;
             (void)hipGetLastError();
             return nullptr;
         }
         hipLaunchKernelGGL(k_sssp_records, dim3(grid_for(g->n, 256, 8192)), dim3(256), 0, g->stream, g->n, g->row_ptr.p,
-                           g->col.p, g->w.p, g->sssp_rec.p);
+                           g->col.p, g->w.p, rec.p);
         MDS_LAUNCHED();
+        std::swap(rec.p, g->sssp_rec.p);
+        std::swap(rec.n, g->sssp_rec.n);
     }
     return g->sssp_rec.p;
 }
