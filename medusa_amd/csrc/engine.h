@@ -298,9 +298,10 @@ struct medusa_graph {
     // device-driven superstep loops: control blocks and captured superstep batches
     medusa::DBuf<medusa::CtlStorage> bfs_ctl, mbfs_ctl, sssp_ctl;
     medusa::GraphCache bfs_graph;
-    // by slot count / kHeadStep
+    // by slot count / kHeadStep; MBFS by the width of its level planes too (8, 16, 32 or 64 bits), so calls
+    // with different numbers of sources do not capture again
     medusa::GraphCache sssp_heads[medusa::kMaxHeadSlots / medusa::kHeadStep + 1];
-    medusa::GraphCache mbfs_heads[medusa::kMaxHeadSlots / medusa::kHeadStep + 1];
+    medusa::GraphCache mbfs_heads[4][medusa::kMaxHeadSlots / medusa::kHeadStep + 1];
     // first replay of the BFS / MBFS loops: as many slots as the previous run on this handle
     // used, so a repeated traversal ends after one replay with no idle slots (BFS: one graph per
     // slot count, so runs of different lengths do not capture again)

@@ -1035,13 +1035,12 @@ static void mbfs_run(medusa_graph* g, const uint32_t* srcs, uint32_t k, uint8_t*
     // capture (once per buffers, launch shape, policy buffer and slot count) a batch of launches
     auto captured = [&](uint32_t slots) -> hipGraphExec_t {
         static_assert(kHeadStep % 2 == 0, "a batch starts and ends with the first control block");
-        GraphCache& gc = g->mbfs_heads[slots / kHeadStep];
-        const uintptr_t key[8] = {(uintptr_t)masks.p,   (uintptr_t)policy,
+        GraphCache& gc = g->mbfs_heads[__builtin_ctz(sizeof(T))][slots / kHeadStep];
+        const uintptr_t key[7] = {(uintptr_t)masks.p,   (uintptr_t)policy,
                                   ((uintptr_t)grid << 32) | large,
                                   (uintptr_t)planes.p,  (uintptr_t)host,
-                                  (uintptr_t)a.q_small, (uintptr_t)a.q_large,
-                                  (uintptr_t)sizeof(T)};
-        if (gc.exec && std::equal(key, key + 8, gc.key)) return gc.exec;
+                                  (uintptr_t)a.q_small, (uintptr_t)a.q_large};
+        if (gc.exec && std::equal(key, key + 7, gc.key)) return gc.exec;
         gc.reset();
         MDS_HIP(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
         hipGraph_t graph = nullptr;
@@ -1059,7 +1058,7 @@ static void mbfs_run(medusa_graph* g, const uint32_t* srcs, uint32_t k, uint8_t*
         if (e == hipSuccess) e = hipGraphInstantiate(&gc.exec, graph, nullptr, nullptr, 0);
         if (graph) (void)hipGraphDestroy(graph);
         MDS_HIP(e);
-        std::copy(key, key + 8, gc.key);
+        std::copy(key, key + 7, gc.key);
         return gc.exec;
     };
     uint32_t slots = next_slots(g->mbfs_last_slots, 0, kMbfsBatch);

@@ -356,6 +356,17 @@ def test_mbfs_hubs_and_slices(oracle, n):
                         host.supersteps, host.push_steps, host.pull_steps, host.edges_traversed)
 
 
+def test_mbfs_widths_in_turn_on_one_handle(oracle):
+    """Calls of every plane width in turn on one handle, each width's captured supersteps used again after
+    the others, with a width's buffers growing in between."""
+    rp, col = wl.rmat_graph(scale=13, edge_factor=8, seed=3)
+    rng = np.random.default_rng(5)
+    with md.Graph(rp, col) as G:
+        for k in (3, 12, 3, 30, 12, 64, 3, 30, 8, 16, 64, 12):
+            srcs = rng.integers(0, len(rp) - 1, k).astype(np.uint32)
+            assert np.array_equal(G.mbfs(srcs)[0], oracle.mbfs(rp, col, srcs)), k
+
+
 @pytest.mark.parametrize("where", ["device", "host"])
 def test_mbfs_device_time_covers_the_levels(where):
     """device_ms covers the making of the level bytes: without edges, 64 sources differ from 33 by 31 rows
