@@ -432,6 +432,8 @@ __device__ __forceinline__ void mbfs_set_level(const MbfsArgs& a, uint32_t code,
 }
 
 constexpr uint32_t kMbfsPullGroup = 4;  // in-edges a lane probes per round
+constexpr uint32_t kMbfsPullGrid = 512;
+__device__ __forceinline__ uint32_t mbfs_pull_wgs(const MbfsArgs& a) { return max(a.grid, kMbfsPullGrid); }
 
 __device__ __forceinline__ uint32_t wave_or(uint32_t x) {
     x |= dpp_or_zero<0x111>(x);
@@ -461,7 +463,7 @@ __device__ __forceinline__ void mbfs_pull(const MbfsArgs& a, unsigned long long 
                                           const unsigned long long* __restrict__ frontier,
                                           unsigned long long* __restrict__ nxt, MbfsAcc& acc) {
     const uint32_t lane = threadIdx.x & (kWave - 1);
-    const uint32_t nw = gridDim.x * 4, w = blockIdx.x * 4 + threadIdx.x / kWave;
+    const uint32_t nw = mbfs_pull_wgs(a) * 4, w = blockIdx.x * 4 + threadIdx.x / kWave;
     for (uint32_t h = w; h < a.nhubs; h += nw) {  // uniform across the wave
         const uint4 H = a.hub[h];
         const uint32_t p = H.x, deg = H.y;
@@ -777,7 +779,11 @@ __global__ __launch_bounds__(kWave) void k_mbfs_start(MbfsArgs a, MbfsSources sr
     mbfs_decide(a, true, 0, s_params);
 }
 
-// One launch of the superstep loop, doing what the control block says.
+// One launch of the superstep loop, doing what the control block says.  Pushes take the first a.grid
+// workgroups, pulls at least kMbfsPullGrid and the other passes over the vertices all of them: a caller's
+// small grid is for the expansion of a frontier.  64 sources, 64 workgroups asked for: Chung-Lu with 600 K
+// vertices 2.52 ms where every pass had only those, 0.94 now; RMAT-18 1.03 and 0.34.  (Pulls of RMAT-18 are
+// faster on 512 workgroups than on all 2048, 344 and 400 us a run; Erdos-Renyi's slower, 583 and 567.)
 template <class T, bool kDecide>
 __global__ __launch_bounds__(256, 8) void k_mbfs_super(MbfsArgs a, uint32_t slot) {
     __shared__ MbfsPushLds s_push;
@@ -802,10 +808,11 @@ __global__ __launch_bounds__(256, 8) void k_mbfs_super(MbfsArgs a, uint32_t slot
     if (phase == kMbfsPush) {
         pass_on(kMbfsUpdate);
         const uint32_t hub = ctl->hub_wgs;
+        if (blockIdx.x >= a.grid) return;
         if (blockIdx.x < hub) {
             mbfs_push_large(a, ctl->n_large, a.frontier[par], blockIdx.x, hub);
         } else {
-            const uint32_t wg = blockIdx.x - hub, nwg = gridDim.x - hub;
+            const uint32_t wg = blockIdx.x - hub, nwg = a.grid - hub;
             if (wg * 4 >= ctl->n_small) return;  // no entry for its waves
             mbfs_push_small(a, a.ctr->queued[par], a.frontier[par], wg * 4 + threadIdx.x / kWave, nwg * 4, s_push);
         }
@@ -818,8 +825,8 @@ __global__ __launch_bounds__(256, 8) void k_mbfs_super(MbfsArgs a, uint32_t slot
     }
     // workgroups without a slice, hub or tile leave at once, without a ticket (RMAT-18 pushed from one source
     // 254 us before, 248 now; 25 K vertices, 16 sources 478 and 470)
-    const uint32_t items = phase == kMbfsPull ? (max(a.nslices, a.nhubs) + 3) / 4 : (a.n - 1) / kMbfsTile + 1;
-    const uint32_t wgs = min(gridDim.x, items);
+    const uint32_t wgs = phase == kMbfsPull ? min(mbfs_pull_wgs(a), (max(a.nslices, a.nhubs) + 3) / 4)
+                                            : min(gridDim.x, (a.n - 1) / kMbfsTile + 1);
     if (blockIdx.x >= wgs) return;
     if (phase == kMbfsPull)
         mbfs_pull<T>(a, ctl->full, lv, a.frontier[par], a.frontier[par ^ 1u], acc);
@@ -974,7 +981,7 @@ static void mbfs_run(medusa_graph* g, const uint32_t* srcs, uint32_t k, uint8_t*
                      medusa_stats& st) {
     const uint32_t n = g->n;
     const uint64_t m = g->m;
-    const uint32_t large = mbfs_large(g, o), grid = mbfs_grid(g, o);
+    const uint32_t large = mbfs_large(g, o), grid = mbfs_grid(g, o), wgs = std::max(grid, kMbfsGridDefault);
     g->q_small.ensure((size_t)kMbfsSegs * mbfs_span(n));
     g->q_large.ensure(n);
     DBuf<unsigned long long>& masks = g->bitmap;
@@ -1046,7 +1053,7 @@ static void mbfs_run(medusa_graph* g, const uint32_t* srcs, uint32_t k, uint8_t*
         hipGraph_t graph = nullptr;
         try {
             for (uint32_t b = 0; b < slots; ++b)
-                hipLaunchKernelGGL((k_mbfs_super<T, true>), dim3(grid), dim3(256), 0, s, a, b & 1u);
+                hipLaunchKernelGGL((k_mbfs_super<T, true>), dim3(wgs), dim3(256), 0, s, a, b & 1u);
             hipLaunchKernelGGL(k_mbfs_finish<T>, finish_grid, dim3(finish_wg), 0, s, a, host, (uint8_t*)nullptr, 0u, 0u);
             MDS_LAUNCHED();
         } catch (...) {
@@ -1107,7 +1114,7 @@ static void mbfs_run(medusa_graph* g, const uint32_t* srcs, uint32_t k, uint8_t*
             hipLaunchKernelGGL(k_mbfs_set_ctl, dim3(1), dim3(1), 0, s, ctl, (int32_t)t, phase, n_small, n_large,
                                mbfs_hub_wgs(grid, n_small, n_large, c[kMbfsLargeDeg], c[kMbfsActiveDeg]));
             MDS_LAUNCHED();
-            hipLaunchKernelGGL((k_mbfs_super<T, false>), dim3(grid), dim3(256), 0, s, a, 0u);
+            hipLaunchKernelGGL((k_mbfs_super<T, false>), dim3(wgs), dim3(256), 0, s, a, 0u);
             MDS_LAUNCHED();
         };
         read_sums();
