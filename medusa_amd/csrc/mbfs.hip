@@ -947,18 +947,24 @@ __global__ __launch_bounds__(1024) void k_mbfs_finish(MbfsArgs a, MbfsHost* __re
         host->made[(blockIdx.y * gridDim.x + blockIdx.x) % kMbfsEnds] = (unsigned long long)wall_clock64();
 }
 
-// Host-driven launch: the host's decision written into the control block.
-__global__ void k_mbfs_set_ctl(MbfsCtl* ctl, int32_t step, uint32_t phase, uint32_t n_small, uint32_t n_large,
-                               uint32_t hub_wgs) {
-    ctl->step = step;
-    ctl->phase = phase;
-    ctl->n_small = n_small;
-    ctl->n_large = n_large;
-    ctl->hub_wgs = hub_wgs;
-}
-// Host-driven superstep of parity `par`: every counter cleared except its own queue's.
-__global__ __launch_bounds__(kWave) void k_mbfs_zero(MbfsCounters* c, uint32_t par) {
-    const uint32_t lane = threadIdx.x;
+// Host-driven launch: the host's decision written into the control block, and into the second one for the
+// update that follows a push.  `first` of a superstep: every counter cleared except its own queue's
+// (parity step % 2).
+__global__ __launch_bounds__(kWave) void k_mbfs_set_ctl(MbfsCtl* ctl, MbfsCounters* c, uint32_t first, int32_t step,
+                                                        uint32_t phase, uint32_t n_small, uint32_t n_large,
+                                                        uint32_t hub_wgs) {
+    const uint32_t lane = threadIdx.x, par = (uint32_t)step & 1u;
+    if (lane == 0) {
+        ctl->step = step;
+        ctl->phase = phase;
+        ctl->n_small = n_small;
+        ctl->n_large = n_large;
+        ctl->hub_wgs = hub_wgs;
+        MbfsCtl c1 = *ctl;
+        c1.phase = kMbfsUpdate;
+        ctl[1] = c1;
+    }
+    if (!first) return;
     if (lane < kMbfsSegs) {
         for (int i = 0; i < kMbfsSums; ++i) c->sum[lane].v[i] = 0;
         c->queued[par ^ 1u][lane].v = 0;
@@ -1101,7 +1107,7 @@ static void mbfs_run(medusa_graph* g, const uint32_t* srcs, uint32_t k, uint8_t*
         if (timing) ensure_events(g, 2);
         unsigned long long c[kMbfsSums];
         auto read_sums = [&]() {  // waits for the stream
-            MDS_HIP(hipMemcpyAsync(g->h_ctr_raw.p, C, sizeof(MbfsCounters), hipMemcpyDeviceToHost, s));
+            MDS_HIP(hipMemcpyAsync(g->h_ctr_raw.p, C, sizeof(C->sum), hipMemcpyDeviceToHost, s));
             MDS_HIP(hipStreamSynchronize(s));
             const MbfsCounters* x = reinterpret_cast<const MbfsCounters*>(g->h_ctr_raw.p);
             for (int i = 0; i < kMbfsSums; ++i) {
@@ -1109,12 +1115,17 @@ static void mbfs_run(medusa_graph* g, const uint32_t* srcs, uint32_t k, uint8_t*
                 for (uint32_t sg = 0; sg < kMbfsSegs; ++sg) c[i] += x->sum[sg].v[i];
             }
         };
-        auto launch = [&](uint32_t t, uint32_t phase) {
+        bool first = true;  // launch of a superstep
+        auto decide = [&](uint32_t t, uint32_t phase) {
             const uint32_t n_small = (uint32_t)c[kMbfsQueued], n_large = (uint32_t)(c[kMbfsQueued] >> 32);
-            hipLaunchKernelGGL(k_mbfs_set_ctl, dim3(1), dim3(1), 0, s, ctl, (int32_t)t, phase, n_small, n_large,
+            hipLaunchKernelGGL(k_mbfs_set_ctl, dim3(1), dim3(kWave), 0, s, ctl, C, first ? 1u : 0u, (int32_t)t, phase,
+                               n_small, n_large,
                                mbfs_hub_wgs(grid, n_small, n_large, c[kMbfsLargeDeg], c[kMbfsActiveDeg]));
             MDS_LAUNCHED();
-            hipLaunchKernelGGL((k_mbfs_super<T, false>), dim3(wgs), dim3(256), 0, s, a, 0u);
+            first = false;
+        };
+        auto launch = [&](uint32_t slot) {
+            hipLaunchKernelGGL((k_mbfs_super<T, false>), dim3(wgs), dim3(256), 0, s, a, slot);
             MDS_LAUNCHED();
         };
         read_sums();
@@ -1135,12 +1146,15 @@ static void mbfs_run(medusa_graph* g, const uint32_t* srcs, uint32_t k, uint8_t*
             if (o.direction == MEDUSA_DIR_PUSH) pull = false;
             else if (o.direction == MEDUSA_DIR_PULL) pull = true;
             else pull = sched.bfs_pull(f, pull);
-            hipLaunchKernelGGL(k_mbfs_zero, dim3(1), dim3(kWave), 0, s, C, t & 1u);
-            MDS_LAUNCHED();
-            if (!pull && !queued) launch(t, kMbfsQueue);
+            first = true;
+            if (!pull && !queued) {
+                decide(t, kMbfsQueue);
+                launch(0);
+            }
+            decide(t, pull ? kMbfsPull : kMbfsPush);
             if (timing) MDS_HIP(hipEventRecord(g->events[0], s));
-            launch(t, pull ? kMbfsPull : kMbfsPush);
-            if (!pull) launch(t, kMbfsUpdate);
+            launch(0);
+            if (!pull) launch(1);  // the update
             if (timing) MDS_HIP(hipEventRecord(g->events[1], s));
             queued = !pull;
             read_sums();
@@ -1165,7 +1179,7 @@ static void mbfs_run(medusa_graph* g, const uint32_t* srcs, uint32_t k, uint8_t*
             h.m_u -= c[kMbfsReachedEdges];
         }
         // the last level, for the finish
-        hipLaunchKernelGGL(k_mbfs_set_ctl, dim3(1), dim3(1), 0, s, ctl, (int32_t)h.supersteps, 0u, 0u, 0u, 0u);
+        hipLaunchKernelGGL(k_mbfs_set_ctl, dim3(1), dim3(kWave), 0, s, ctl, C, 0u, (int32_t)h.supersteps, 0u, 0u, 0u, 0u);
         MDS_LAUNCHED();
         if (direct) {
             hipLaunchKernelGGL(k_mbfs_finish<T>, finish_grid, dim3(finish_wg), 0, s, a, (MbfsHost*)nullptr, out, 0u, k);
