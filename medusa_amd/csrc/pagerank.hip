@@ -814,7 +814,11 @@ __global__ void k_pr_scatter(uint32_t n, const uint32_t* __restrict__ optr, cons
         const uint32_t b = optr[p], e = optr[p + 1];
         if (b == e) continue;
         const float x = contrib[p];
-        for (uint32_t k = advance_to(b, lane, e); k < e; k = advance_to(k, kWave, e)) msg[oslot[k]] = x;
+        if (!lies_before(b, lane, e)) continue;
+        for (uint32_t k = b + lane;; k += kWave) {
+            msg[oslot[k]] = x;
+            if (!lies_before(k, kWave, e)) break;
+        }
     }
 }
 
