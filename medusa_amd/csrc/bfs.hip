@@ -50,17 +50,16 @@
 
 namespace medusa {
 
-// Out-degree above which a frontier vertex is split over workgroups.  Below it one wave walks the
-// whole list, 256 out-edges at a time, and the superstep waits for the longest: BFS of the
-// 2.4 M-vertex Chung-Lu graph takes 588 us at 2048, 514 at 1280, 461 at 1024, 424 at 512; RMAT-20
-// has no such vertex.  Further down the heuristic's pushes on that graph come out level with its
-// pulls, and the learned direction, which gains 5 % over the heuristic at 1280 (490 us), gains
-// 1..4 % at 1024 and loses 2 % to its own evaluation at 512; the autotuner finds the lower
-// thresholds for a caller's graph.
-constexpr uint32_t kLargeDefault = 1280;
+// kBfsLargeDefault, the out-degree above which a frontier vertex is split over workgroups.  Below it one
+// wave walks the whole list, 256 out-edges at a time, and the superstep waits for the longest.  us a run
+// at thresholds of 384, 512, 768, 1024, 1280 and 2048: Chung-Lu with 2.4 M vertices (out-degrees up to 39914)
+// 340, 345, 361, 378, 398 and 445; 8 M 711, 703, 719, 740, 764 and 830; 600 K 183, 185, 189, 193, 196
+// and 207; RMAT-20 (up to 598) 268 at 384 and 155 from 512 on; RMAT-22 (up to 866) 491, 484 and 339..334 from
+// 768 on.  So 768 or 1024 would be faster for the heuristic: it stays at 1280 for the learned direction,
+// whose gain over it on the 2.4 M-vertex graph is 6.3..6.9 % at 1280, 2.6..3.2 % at 1024 and none at 768 (six
+// trainings), where it has to be 2 %.  The autotuner finds the lower thresholds for a caller's graph.
 constexpr uint32_t kLargeSplit = 16;  // workgroups per hub in the large-vertex push
 constexpr uint32_t kBfsBatch = 8;     // supersteps per captured graph
-constexpr uint32_t kExpandGrid = 1024;
 
 // Control block of the device-driven loop.  There are two: launch k of a batch reads block k % 2
 // and leaves the next launch's in the other, so a workgroup that starts late never sees what an
@@ -1404,10 +1403,10 @@ __global__ __launch_bounds__(256) void k_bfs_super(BfsArgs a, uint32_t slot) {
 // Degree threshold of the hub queue and workgroups of the expansion: the caller's value,
 // else the handle's autotuned one, else the default.
 static uint32_t bfs_large(const medusa_graph* g, const medusa_opts& o) {
-    return o.large_degree ? o.large_degree : (g->tuned.bfs_large ? g->tuned.bfs_large : kLargeDefault);
+    return o.large_degree ? o.large_degree : (g->tuned.bfs_large ? g->tuned.bfs_large : kBfsLargeDefault);
 }
 static uint32_t bfs_grid(const medusa_graph* g, const medusa_opts& o) {
-    return o.grid ? o.grid : (g->tuned.bfs_grid ? g->tuned.bfs_grid : kExpandGrid);
+    return o.grid ? o.grid : (g->tuned.bfs_grid ? g->tuned.bfs_grid : kBfsGridDefault);
 }
 
 static uint32_t bfs_mode(const medusa_opts& o) {

@@ -115,15 +115,11 @@ __device__ __forceinline__ T load_now_block(const T* p) {
 }
 #endif
 
-// Frontier counters written by the compaction kernels, read back each superstep.
-struct FrontierCounters {
-    MDS_COUNTER(uint32_t, n_small);              // frontier vertices with 1 <= outdeg <= large (wave queue)
-    MDS_COUNTER(uint32_t, n_large);              // frontier vertices with outdeg > large (workgroup queue)
-    MDS_COUNTER(uint32_t, n_new);                // vertices that joined the frontier (any outdeg)
-    MDS_COUNTER(unsigned long long, deg_sum);    // sum of their out-degrees
-    MDS_COUNTER(unsigned long long, probes);     // in-edges examined by a pull superstep
-    MDS_COUNTER(unsigned long long, deg_large);  // out-degree sum of the workgroup (hub) queue
-};
+// Launch shapes of the frontier engines where neither the caller nor the autotuner gives one: the
+// out-degree above which a vertex goes to the hub queue (the reasons stand in bfs.hip) and the
+// workgroups of an expansion.
+constexpr uint32_t kBfsLargeDefault = 1280, kBfsGridDefault = 1024;
+constexpr uint32_t kMbfsLargeDefault = 1024, kMbfsGridDefault = 2048;
 
 // One contiguous run of PageRank vertices handled with the same lane mapping.
 struct PrRun {
@@ -333,8 +329,6 @@ bool kernels_can_write(const medusa_graph* g, const void* p, size_t bytes);
 void check_device_output(const void* p, size_t bytes);
 // Copies `bytes` from device pointer `src` to `dst`, which may be host or device memory.
 void copy_out(medusa_graph* g, void* dst, const void* src, size_t bytes);
-// Sums pairwise (start, stop) event intervals [0, pairs) in milliseconds.
-double sum_event_pairs(medusa_graph* g, size_t pairs);
 // Number of workgroups for a grid-stride launch over `items` with `per_wg` items each.
 inline uint32_t grid_for(uint64_t items, uint32_t per_wg, uint32_t cap = 8192) {
     uint64_t g = (items + per_wg - 1) / per_wg;

@@ -45,16 +45,6 @@ void ensure_events(medusa_graph* g, size_t count) {
     }
 }
 
-double sum_event_pairs(medusa_graph* g, size_t pairs) {
-    double ms = 0;
-    for (size_t i = 0; i < pairs; ++i) {
-        float t = 0;
-        MDS_HIP(hipEventElapsedTime(&t, g->events[2 * i], g->events[2 * i + 1]));
-        ms += t;
-    }
-    return ms;
-}
-
 bool is_device_memory(const void* p) {
     hipPointerAttribute_t attr{};
     const hipError_t e = hipPointerGetAttributes(&attr, p);

@@ -34,12 +34,8 @@
 
 namespace medusa {
 
-constexpr uint32_t kMbfsLargeDefault = 1024;
-constexpr uint32_t kMbfsGridDefault = 2048;
 constexpr uint32_t kMbfsBatch = 16;  // launches of a replay without a previous run
 constexpr uint32_t kMbfsSplit = 8;  // minimum workgroup items per hub
-
-constexpr uint32_t kMbfsProbeLines = 8;
 
 // Counters of a launch, spread over kMbfsSegs lines by workgroup: same-address atomics serialise.
 constexpr uint32_t kMbfsSegs = 32;

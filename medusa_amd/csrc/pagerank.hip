@@ -430,21 +430,8 @@ __global__ __launch_bounds__(256) void k_pr_dangle_base(const float* __restrict_
     __shared__ float s_s[kSmallBlocks], s_c[kSmallBlocks];
     const uint32_t lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
     for (uint32_t b = wave; b < nblk; b += 4) {
-        const PrBlock B = blocks[b];
-        const float* x = rank + B.begin;
-        float s = 0.f, c = 0.f;
-        for (uint32_t r0 = 0; r0 * kWave < B.len; r0 += 16) {
-            float v[16];
-#pragma unroll
-            for (uint32_t j = 0; j < 16; ++j) {
-                const uint32_t k = lane + (r0 + j) * kWave;
-                v[j] = k < B.len ? x[k] : 0.f;
-            }
-#pragma unroll
-            for (uint32_t j = 0; j < 16; ++j)
-                if (lane + (r0 + j) * kWave < B.len) kahan_add(s, c, v[j]);
-        }
-        wave_tree(s, c);
+        float s, c;
+        dangle_block_sum(rank, blocks[b], s, c);
         if (lane == 0) {
             s_s[b] = s;
             s_c[b] = c;
@@ -463,9 +450,7 @@ __global__ __launch_bounds__(256) void k_pr_dangle_base(const float* __restrict_
                 kahan_combine(as, ac, s_s[P.first_block + i], s_c[P.first_block + i]);
             }
         }
-        const float D = as - ac;
-        const float tele = (float)((1.0 - (double)d) / (double)P.n);
-        base_out[g] = fmaf(d, D / (float)P.n, tele);
+        base_out[g] = pr_base_value(as - ac, d, P.n);
     }
 }
 

@@ -59,8 +59,8 @@ extern "C" int medusa_autotune(medusa_graph* g, uint32_t algo, const uint32_t* s
             }
             return best;
         };
-        // the engines' defaults
-        const uint32_t dl = algo == MEDUSA_TUNE_BFS ? 1280u : 1024u, dg = algo == MEDUSA_TUNE_BFS ? 1024u : 2048u;
+        const uint32_t dl = algo == MEDUSA_TUNE_BFS ? kBfsLargeDefault : kMbfsLargeDefault;
+        const uint32_t dg = algo == MEDUSA_TUNE_BFS ? kBfsGridDefault : kMbfsGridDefault;
         medusa_tuning t{};
         t.default_ms = run(dl, dg);
         t.best_ms = t.default_ms;
