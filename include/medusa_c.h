@@ -52,9 +52,10 @@ extern "C" {
 #define MEDUSA_DIR_PULL 2  /* bottom-up over CSC every superstep */
 
 /* PageRank kernel variant (opts.variant); all variants give bit-identical ranks. */
-#define MEDUSA_PR_DEFAULT 0 /* the engine's choice: MEDUSA_PR_PULL on a small graph (at most 2^19 arcs and 4096
-                               vertices without out-edges) or one whose binned layout cannot be planned,
-                               else MEDUSA_PR_BINNED */
+#define MEDUSA_PR_DEFAULT 0 /* the engine's choice: MEDUSA_PR_PULL on one (not packed) graph of at most 2^19 arcs
+                               whose superstep is one launch (at most 4096 vertices without out-edges, fewer
+                               of them the more workgroups the pull has), or where no binned layout can be
+                               planned; else MEDUSA_PR_BINNED */
 #define MEDUSA_PR_PUSH 1   /* scatter into per-in-edge message slots, then combine (reference style) */
 #define MEDUSA_PR_BINNED 2 /* message array blocked by source chunk and destination bin: streaming
                               writes of one message per out-edge, then a combine from LDS per bin */
@@ -157,7 +158,7 @@ int medusa_bfs_multi(medusa_graph* g, const uint32_t* sources, uint32_t count, i
  * callers that cannot allocate device memory (code under HIP graph capture, tight serving
  * loops, harnesses that forbid hipMalloc).  levels[n] must be device memory of the graph's
  * GPU; the run writes it in place (the same levels as medusa_bfs, heuristic direction).  The
- * frontier queues, bitmap and control block live in one statically sized device array per
+ * frontier queues, bitmaps and control blocks live in one statically sized device array per
  * GPU, held until the process ends, so n may not exceed MEDUSA_NOALLOC_MAX_VERTICES
  * (MEDUSA_ERR_ARG otherwise).  Every call on a GPU shares that array: calls that overlap on one
  * GPU (from several threads or handles) race and must be serialised by the caller.  The graph

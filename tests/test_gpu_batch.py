@@ -139,6 +139,27 @@ def test_binned_dangling_bases(oracle, dangling):
             assert np.array_equal(_bits(r[begin[k]:begin[k + 1]]), _bits(want)), k
 
 
+def test_default_variant_of_small_packed_batches(oracle):
+    """The default variant of a small packed batch is the binned exchange, of the same graphs alone the
+    pull, unless their vertices (workgroups of the pull, each with the whole dangling sum) are many; the
+    ranks' bits are the oracle's throughout."""
+    ring = np.stack([np.arange(500), (np.arange(500) + 1) % 500], 1)
+    many = 526_000  # 523,000 edges and 3000 vertices without out-edges, but more than 2048 workgroups
+    sparse = np.stack([np.arange(523_000), np.arange(523_000) + 1], 1)
+    small = [csr_from_edges(500, ring)[:2], csr_from_edges(300, ring[:250] % 300)[:2]]
+    with md.Graph.packed(small) as G:
+        begin = G.batch()
+        r, st = G.pagerank(0.85, 4)
+        assert st.pull_steps == 0 and st.push_steps == 0
+        for k, (rp, col) in enumerate(small):
+            assert np.array_equal(_bits(r[begin[k]:begin[k + 1]]), _bits(oracle.pagerank_f32(rp, col, 0.85, 4))), k
+    for (rp, col), pulls in ((small[0], 4), (small[1], 4), (csr_from_edges(many, sparse)[:2], 0)):
+        with md.Graph(rp, col) as G:
+            r, st = G.pagerank(0.85, 4)
+            assert st.pull_steps == pulls, len(rp)
+            assert np.array_equal(_bits(r), _bits(oracle.pagerank_f32(rp, col, 0.85, 4))), len(rp)
+
+
 def test_set_batch_back_to_plain_graph(oracle):
     graphs = _mixed_batch()[:6]
     rp, col, _, begin = md.pack_graphs(graphs)
