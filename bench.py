@@ -296,8 +296,8 @@ def _ab(fa, fb, reps=AB_REPS):
     sequential timing of one form after the other (with policy training between them) does
     not.  The first run of a pair is not timed because a handle sizes a run's first replay by
     the slots its previous run used: right after the other form, a run that needs more slots
-    pays a second replay and host round trip.  device_ms is the library's own event span of the
-    whole run on its stream."""
+    pays a second replay and host round trip.  device_ms is the library's own time of the run on
+    the GPU, from its first kernel to its last superstep (MBFS: to the levels made)."""
     ta, tb = [], []
     for _ in range(reps):
         fa()

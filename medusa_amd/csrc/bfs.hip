@@ -38,7 +38,8 @@
 //     reads the run's parameters from pinned host memory, a number of superstep slots (as many as
 //     the previous run on the handle used) and a closing kernel that copies the levels out and
 //     the control block to pinned memory; the host launches it and waits once, and replays
-//     batches of kBfsBatch slots if the control block does not say done;
+//     batches of kBfsBatch slots if the control block does not say done (a handle's first run
+//     launches the same kernels one by one);
 //   host-driven (timing or trace requested): the host reads the counters after every
 //     superstep, times it with hipEvents and logs the trace record.
 
@@ -125,9 +126,9 @@ __global__ void k_bfs_set_ctl(BfsCtl* ctl, int32_t step, uint32_t pull, uint32_t
 // Counters of one superstep.  Atomics on one address serialise (about 10 ns each on this
 // GPU), so they are spread over kBfsSlots addresses, each on its own 128-byte line:
 //   seg[p][s]: the frontier of parity p (superstep t's frontier has parity t % 2) is a queue
-//     in kBfsSlots segments by vertex range (segment s holds vertices [s * span, (s + 1) *
-//     span)); its counter packs the vertices appended (low half, also the append offset) and
-//     the sum of their out-degrees (high half);
+//     in kBfsSlots segments of `span` entries, filled by rounds of vertices (bfs_round_segment)
+//     or by workgroups (exact claims); its counter packs the vertices appended (low half, also
+//     the append offset) and the sum of their out-degrees (high half);
 //   work[s]: workgroup b adds the out-degree sum of the hubs it found (low half) and the
 //     in-edges it probed (high half) into slot b % kBfsSlots;
 //   sub / top: two levels of tickets that find the last workgroup of a superstep.
@@ -190,7 +191,7 @@ __host__ __device__ inline bool bfs_solo_fits(uint32_t cap, unsigned long long n
     return n_f <= cap && (m_f <= cap || (n <= cap && m_f <= (unsigned long long)kSoloRounds * cap));
 }
 
-// A push claims exactly (compare-and-swap, no compaction) when the frontier has at most
+// A push claims exactly (an atomic OR of the visited bit, no compaction) when the frontier has at most
 // `exact_edges` out-edges: 1, or 2 when it also has at most 64 vertices (every wave then reads
 // all of them and takes an equal share of their out-edges).  Workgroup b appends its winners to
 // segment b mod kBfsSlots of the next queue whatever their ids: exact_edges is at most a
@@ -408,10 +409,11 @@ __device__ __forceinline__ void bfs_claim_plain(const BfsArgs& a, const unsigned
         if (v[j] != 0xFFFFFFFFu && !(visited[v[j] >> 6] & (1ull << (v[j] & 63)))) a.level[v[j]] = next;
 }
 
-// Exact: whoever sets the visited bit wins the vertex, stores its level and holds it for the next queue's segment `own`.  The calling wave is converged.  A wave with
-// many out-edges goes through this chain of dependent accesses once per round, so the round's loads
-// and atomics are issued together (a compare-and-swap on the level one after the other, then the
-// bit: 34..36 us for 46 K and 62 K out-edges of that graph, 20 now).
+// Exact: whoever sets the visited bit wins the vertex, stores its level and holds it for the next
+// queue's segment `own`.  The calling wave is converged.  A wave with many out-edges goes through this
+// chain of dependent accesses once per round, so the round's loads and atomics are issued together (a
+// compare-and-swap on the level one after the other, then the bit: 34..36 us for 46 K and 62 K out-edges
+// of that graph, 20 now).
 struct BfsExact {
     unsigned long long* visited;
     BfsSink sink;
@@ -920,8 +922,8 @@ __device__ __forceinline__ void solo_reset(BfsSoloLds<kThreads>& L) {
 // bitmap is L.vis (a small graph's few lines of global memory would take one atomic at a time:
 // 33 K out-edges of 4096 vertices 80 us instead of 49).
 template <bool kLdsVis, uint32_t kThreads, uint32_t kN>
-__device__ __forceinline__ void solo_claim(const BfsArgs& a, unsigned long long* visited, BfsSoloLds<kThreads>& L, const uint32_t (&v)[kN],
-                                           int32_t level) {
+__device__ __forceinline__ void solo_claim(const BfsArgs& a, unsigned long long* visited, BfsSoloLds<kThreads>& L,
+                                           const uint32_t (&v)[kN], int32_t level) {
     unsigned long long old[kN];
     uint32_t b[kN], e[kN];
 #pragma unroll
@@ -1102,7 +1104,8 @@ __device__ __forceinline__ bool bfs_next_pull(const BfsArgs& a, const BfsCtl& c,
 
 // First decision after k_bfs_mark placed the sources; one workgroup.  The work slots, tickets and
 // hub count are cleared (queue 0's counters stay: superstep 0 reads them).
-__global__ __launch_bounds__(kWave) void k_bfs_first_decide(BfsArgs a, unsigned long long m, uint32_t mode, int32_t* out) {
+__global__ __launch_bounds__(kWave) void k_bfs_first_decide(BfsArgs a, unsigned long long m, uint32_t mode,
+                                                            int32_t* out) {
     __shared__ float s_params[kMlpWaveLds];
     BfsCounters* ctr = a.ctr;
     unsigned long long joined, work;
@@ -1263,11 +1266,11 @@ __global__ __launch_bounds__(64) void k_zero_counters(BfsCounters* c, uint32_t p
 }
 
 // After a push with plain claims: the next frontier = {v : level[v] == step + 1}, as its
-// queue, hub queue and counters, and the visited bitmap (one ballot per 64 vertices) rebuilt from the levels, in workgroup rounds of
-// kBfsRound consecutive vertices (wave w the chunks w * kRoundChunks + k), whose level loads are
-// issued together.
-__device__ __forceinline__ void compact_level(const BfsArgs& a, unsigned long long* visited, int32_t next, const BfsSink& o,
-                                              unsigned long long& hacc, BfsJoins J) {
+// queue, hub queue and counters, and the visited bitmap (one ballot per 64 vertices) rebuilt from the
+// levels, in workgroup rounds of kBfsRound consecutive vertices (wave w the chunks w * kRoundChunks + k),
+// whose level loads are issued together.
+__device__ __forceinline__ void compact_level(const BfsArgs& a, unsigned long long* visited, int32_t next,
+                                              const BfsSink& o, unsigned long long& hacc, BfsJoins J) {
     const uint32_t lane = threadIdx.x & (kWave - 1), wv = threadIdx.x / kWave;
     uint64_t blk = (uint64_t)blockIdx.x * kBfsRound;
     for (; blk < a.n; blk += (uint64_t)gridDim.x * kBfsRound) {
@@ -1299,9 +1302,9 @@ __device__ __forceinline__ void compact_level(const BfsArgs& a, unsigned long lo
 //            winners are recorded as they are claimed; with at most 64 frontier vertices every
 //            wave takes an equal share of their out-edges (hubs included);
 //   else:    push with plain claims; it leaves `pending` set, so the next launch compacts.
-// The first hub_wgs workgroups of a push take the hub queue, the rest the frontier queue.  Every
-// expansion clears the bitmap that superstep + 1 builds.  With kDecide the last workgroup to
-// finish a counting phase decides the next superstep; otherwise the host reads the counters.
+// The first hub_wgs workgroups of a push take the hub queue, the rest the frontier queue.  With
+// kDecide the last workgroup to finish a counting phase decides the next superstep; otherwise the host
+// reads the counters.
 template <bool kDecide>
 __global__ __launch_bounds__(256) void k_bfs_super(BfsArgs a, uint32_t slot) {
     __shared__ uint32_t s_beg[4][kWave], s_off[4][kWave];
@@ -1493,7 +1496,8 @@ static void bfs_enqueue_slot(medusa_graph* g, const BfsArgs& a, uint32_t parity)
     hipLaunchKernelGGL(k_bfs_super<true>, dim3(a.grid), dim3(256), 0, g->stream, a, parity);
 }
 
-// Bytes of the seeding: the level reset (4 per vertex), the visited bitmap (8 per word) and the sources (16 each: id, level, bit OR).
+// Bytes of the seeding: the level reset (4 per vertex), the visited bitmap (8 per word) and the sources
+// (16 each: id, level, bit OR).
 static uint64_t bfs_seed_bytes(uint32_t n, uint32_t nwords, uint32_t nsrc) {
     return 4ull * n + 8ull * nwords + 16ull * nsrc;
 }

@@ -23,7 +23,8 @@
 // Drivers as for BFS: device-driven (the last workgroup of each update or pull writes the
 // next superstep into a control block; batches of launches, each doing what the control block says,
 // are captured as hipGraphs and replayed until done, sized by the previous run on the handle, and
-// each ends with the finish, which returns at once unless the run is done) and host-driven (timing or tracing) over the same kernels.
+// each ends with the finish, which returns at once unless the run is done) and host-driven (timing or
+// tracing) over the same kernels.
 
 #include <algorithm>
 #include <cstddef>
@@ -41,7 +42,10 @@ constexpr uint32_t kMbfsSplit = 8;  // minimum workgroup items per hub
 constexpr uint32_t kMbfsSegs = 32;
 // active vertices, their out-degrees, those of the hubs among them (above `large`), queue entries and
 // hubs (low and high word), in-edges examined, new (source, vertex) pairs, the pairs' out-degrees
-enum { kMbfsActive, kMbfsActiveDeg, kMbfsLargeDeg, kMbfsQueued, kMbfsProbes, kMbfsNewBits, kMbfsReachedEdges, kMbfsSums };
+enum {
+    kMbfsActive, kMbfsActiveDeg, kMbfsLargeDeg, kMbfsQueued, kMbfsProbes, kMbfsNewBits, kMbfsReachedEdges,
+    kMbfsSums
+};
 struct MbfsLine {
     alignas(128) uint32_t v;
 };
@@ -226,7 +230,8 @@ static void build_pull_layout(medusa_graph* g) {
             }
     MDS_CHECK(hub.size() == L->nhubs, MEDUSA_ERR_INTERNAL, "mbfs: hub count");
     // longest first: a wave that starts one late would end the launch late
-    std::sort(hub.begin(), hub.end(), [](const uint4& a, const uint4& b) { return a.y != b.y ? a.y > b.y : a.x < b.x; });
+    std::sort(hub.begin(), hub.end(),
+              [](const uint4& a, const uint4& b) { return a.y != b.y ? a.y > b.y : a.x < b.x; });
     L->base.upload(base.data(), base.size(), s);
     if (L->nhubs) L->hub.upload(hub.data(), hub.size(), s);
     L->src.alloc(std::max<uint64_t>(at, 1));
@@ -452,8 +457,8 @@ __device__ __forceinline__ unsigned long long wave_or(unsigned long long x) {
 // 8-byte masks: in RMAT-20's full sweeps (17 M in-edges, 64 sources, 142 us) 35 % of 17 M requests
 // miss the L2s, 770 MB of lines from the memory-side cache.  Eight in-edges per round, nontemporal
 // loads of the sources and half as many registers changed nothing or lost.  In the original order over
-// slabs sorted across all vertices the sweep took as long and an update of 20..24 us followed.  `probes` counts in-edges examined up to and including the last
-// one needed (a hub's in steps of 64).
+// slabs sorted across all vertices the sweep took as long and an update of 20..24 us followed.
+// `probes` counts in-edges examined up to and including the last one needed (a hub's in steps of 64).
 template <class T>
 __device__ __forceinline__ void mbfs_pull(const MbfsArgs& a, unsigned long long full, uint32_t lv,
                                           const unsigned long long* __restrict__ frontier,
@@ -827,7 +832,8 @@ __global__ __launch_bounds__(256, 8) void k_mbfs_super(MbfsArgs a, uint32_t slot
     if (phase == kMbfsPull)
         mbfs_pull<T>(a, ctl->full, lv, a.frontier[par], a.frontier[par ^ 1u], acc);
     else
-        mbfs_tiles<T, true>(a, lv, a.frontier[par ^ 1u], a.ctr->queued[par ^ 1u], &a.ctr->hubs[par ^ 1u].v, acc, s_tile);
+        mbfs_tiles<T, true>(a, lv, a.frontier[par ^ 1u], a.ctr->queued[par ^ 1u], &a.ctr->hubs[par ^ 1u].v, acc,
+                            s_tile);
     if (mbfs_finish_launch<kDecide>(a.ctr, acc, wgs)) mbfs_decide(a, false, slot, s_params);
 }
 
@@ -841,11 +847,11 @@ __device__ __forceinline__ uint32_t mbfs_nibbles(uint32_t x0, uint32_t x1, uint3
 // vertex: rows [row0, row1) at `out` (by the control block of a finished run: every row, at ctl->out).
 // A lane takes 4 vertices: the planes' words become nibbles, then bytes, 32 sources at a time, and 4
 // words of 4 sources each are transposed into 4 stores of 4 vertices each.  Bound by the stores: a
-// wave writes 256 contiguous bytes of a row at a time.  RMAT-20, 64 sources:
-// 30 us for 64 MiB of levels from 40 of planes and masks. 
+// wave writes 256 contiguous bytes of a row at a time.  RMAT-20, 64 sources: 30 us for 64 MiB of levels
+// from 40 of planes and masks.
 template <class T>
-__global__ __launch_bounds__(1024) void k_mbfs_finish(MbfsArgs a, MbfsHost* __restrict__ host, uint8_t* out, uint32_t row0,
-                                                     uint32_t row1) {
+__global__ __launch_bounds__(1024) void k_mbfs_finish(MbfsArgs a, MbfsHost* __restrict__ host, uint8_t* out,
+                                                      uint32_t row0, uint32_t row1) {
     const MbfsCtl* ctl = a.ctl;  // a batch has an even number of launches
     if (host) {
         if (blockIdx.x == 0 && blockIdx.y == 0) {
@@ -1056,7 +1062,8 @@ static void mbfs_run(medusa_graph* g, const uint32_t* srcs, uint32_t k, uint8_t*
         try {
             for (uint32_t b = 0; b < slots; ++b)
                 hipLaunchKernelGGL((k_mbfs_super<T, true>), dim3(wgs), dim3(256), 0, s, a, b & 1u);
-            hipLaunchKernelGGL(k_mbfs_finish<T>, finish_grid, dim3(finish_wg), 0, s, a, host, (uint8_t*)nullptr, 0u, 0u);
+            hipLaunchKernelGGL(k_mbfs_finish<T>, finish_grid, dim3(finish_wg), 0, s, a, host, (uint8_t*)nullptr, 0u,
+                               0u);
             MDS_LAUNCHED();
         } catch (...) {
             (void)hipStreamEndCapture(s, &graph);
@@ -1162,7 +1169,8 @@ static void mbfs_run(medusa_graph* g, const uint32_t* srcs, uint32_t k, uint8_t*
                 st.kernel_ms += ms;
                 ++st.kernel_launches;
             }
-            const uint64_t kb = pull ? 4ull * (n + 1) + 8ull * n + 12ull * c[kMbfsProbes] : 20ull * f.n_f + 20ull * f.m_f;
+            const uint64_t kb = pull ? 4ull * (n + 1) + 8ull * n + 12ull * c[kMbfsProbes]
+                                     : 20ull * f.n_f + 20ull * f.m_f;
             h.kernel_bytes += kb;
             h.alg_bytes += kb + 24ull * n + c[kMbfsNewBits];
             if (pull) ++h.pull_steps; else ++h.push_steps;
@@ -1175,7 +1183,8 @@ static void mbfs_run(medusa_graph* g, const uint32_t* srcs, uint32_t k, uint8_t*
             h.m_u -= c[kMbfsReachedEdges];
         }
         // the last level, for the finish
-        hipLaunchKernelGGL(k_mbfs_set_ctl, dim3(1), dim3(kWave), 0, s, ctl, C, 0u, (int32_t)h.supersteps, 0u, 0u, 0u, 0u);
+        hipLaunchKernelGGL(k_mbfs_set_ctl, dim3(1), dim3(kWave), 0, s, ctl, C, 0u, (int32_t)h.supersteps, 0u, 0u, 0u,
+                           0u);
         MDS_LAUNCHED();
         if (direct) {
             hipLaunchKernelGGL(k_mbfs_finish<T>, finish_grid, dim3(finish_wg), 0, s, a, (MbfsHost*)nullptr, out, 0u, k);

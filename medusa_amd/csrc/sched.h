@@ -141,8 +141,8 @@ struct Frontier {
 
 // BFS and MBFS consult the learned direction policy only near the heuristic's switching
 // point, where its decision ratio (alpha * m_f / m_u while pushing, beta * n_f / n while
-// pulling; the mask engine has only the first) lies within a factor kPolicyBand of 1; farther out the heuristic's choice is taken
-// without evaluating the network, which saves its cost on most supersteps.
+// pulling; the mask engine has only the first) lies within a factor kPolicyBand of 1; farther out the
+// heuristic's choice is taken without evaluating the network, which saves its cost on most supersteps.
 constexpr double kPolicyBand = 8.0;
 __host__ __device__ inline bool bfs_policy_consulted(bool cur_pull, double n_f, double m_f, double m_u, double n,
                                                      double alpha, double beta) {
@@ -185,7 +185,10 @@ struct Sched {
     // given (and of the right kind), else the heuristic.  Where the predictions lie within the margin
     // BFS goes on pulling: trained networks put the last pull of the 2.4 M-vertex Chung-Lu graph (13.7
     // us, 22.2 as a push) 0.1 to 0.5 log2 units ahead, and below the margin it was pushed (gain over the
-    // heuristic 1.015 to 1.085 in 54 trainings; going on 1.039 to 1.085 in 36).
+    // heuristic 1.015 to 1.085 in 54 trainings; going on 1.039 to 1.085 in 36).  16 trained networks with
+    // and without that on RMAT-21 and 22, Chung-Lu with 600 K and 8 M vertices and Erdos-Renyi with 1 and
+    // 4 M: the same directions but for one network on each of three graphs, whose runs it makes 1 to 3 %
+    // shorter.
     bool bfs_pull(const Frontier& f, bool cur_pull) const {
         if (!o.policy || policy_kind(o.policy) != MEDUSA_POLICY_DIRECTION) return heuristic_pull(f, cur_pull);
         if (!bfs_policy_consulted(cur_pull && algo != kMbfs, (double)f.n_f, (double)f.m_f, (double)f.m_u, (double)f.n,

@@ -784,7 +784,8 @@ __global__ __launch_bounds__(256) void k_sssp_split(const uint32_t* __restrict__
 //           raises the threshold by the run's bucket width (default, fixed, or chosen by the
 //           learned policy before the run) and marks a split pending; after a split, an empty
 //           bucket raises the threshold past the smallest far distance.
-// kSsspBatch slots are captured once as a hipGraph and replayed until done.
+// Slots, as many as the previous run on the handle took (kSsspBatch without one), are captured as a hipGraph
+// with the closing kernel and replayed until done.
 
 constexpr uint32_t kSsspBatch = 32;
 // Workgroups of a work launch: about the resident count (5 per CU at this LDS size) without local
@@ -1061,7 +1062,8 @@ __global__ __launch_bounds__(kWaveThreads) void k_sssp_work_wave(
     uint32_t* __restrict__ stamp, SsspDevCounters* __restrict__ ctr, unsigned long long* __restrict__ marks) {
     // one slice per vertex: no hubs
     using WideStage = StageOf<kWaveThreads, 1>;
-    __shared__ alignas(16) unsigned char s_lds[sizeof(WaveLds) > sizeof(WideStage) ? sizeof(WaveLds) : sizeof(WideStage)];
+    constexpr size_t kLdsBytes = sizeof(WaveLds) > sizeof(WideStage) ? sizeof(WaveLds) : sizeof(WideStage);
+    __shared__ alignas(16) unsigned char s_lds[kLdsBytes];
     WaveLds& lds = *reinterpret_cast<WaveLds*>(s_lds);
     WideStage& st = *reinterpret_cast<WideStage*>(s_lds);
     const SsspCtl c = *ctl;
@@ -1258,11 +1260,14 @@ static size_t sssp_far_cap(const medusa_graph* g, const medusa_opts& o) {
 // Mean weight (sampled) and the default bucket width, a multiple of it: 8x with local rounds,
 // which absorb the extra hops of a wider bucket (1400x1400 lattice, 32 rounds: 8.0 ms at 8x,
 // 8.6 ms at 6x, 11.5 ms at 3x).  Without them 2x up to kWideEdges edges, where a superstep costs its
-// launch and a wider bucket has fewer (RMAT-16, 8 edges a vertex: 35, 30 and 28
-// supersteps, 497, 463 and 439 us at 1x, 1.5x and 2x); on larger graphs the edges relaxed more than once cost
-// more than the supersteps: 1x on graphs with hubs, whose wide buckets relax them again and again
-// (RMAT-20: 1.79, 1.95 and 2.06 ms, 3.2, 3.9 and 4.2 relaxations per edge), 1.5x on the others
-// (Erdos-Renyi, 2^20 vertices, 8 edges a vertex: 1.07, 0.98 and 1.02 ms; 16: 1.18, 1.17 and 1.26).
+// launch and a wider bucket has fewer (RMAT-16, 8 edges a vertex: 624, 505, 469, 457 and 403 us at 0.5x,
+// 1x, 1.5x, 2x and 4x; RMAT-18, 8: 894, 760, 722, 732 and 699); on larger graphs the edges relaxed more than
+// once cost more than the supersteps: 1x on graphs with hubs, whose wide buckets relax them again and again,
+// 1.5x on the others.  At 0.5x, 0.75x, 1x, 1.5x and 2x: RMAT-20 1.43, 1.67, 1.89, 2.02 and 2.15 ms (1.5,
+// 2.6, 3.3, 4.0 and 4.4 relaxations per edge), with 8 edges a vertex 1.40, 1.18, 1.15, 1.27 and 1.30, RMAT-22
+// with 8 2.75, 2.49, 2.77, 3.43 and 3.92; Erdos-Renyi, 2^20 vertices, 8 edges a vertex 1.38, 1.19, 1.08, 0.98
+// and 1.01, 16 1.22, 1.21, 1.15, 1.23 and 1.20.  (The denser the graph, the narrower the best width; 0.5x
+// on RMAT-20 is what the learned width finds.)
 constexpr uint64_t kWideEdges = 1ull << 22;
 static void sssp_widths(medusa_graph* g, const medusa_opts& o, uint32_t& wmean, uint32_t& dflt) {
     if (!g->w_mean) {  // once per graph: 4096 cache misses, 60 us on 64 MiB of weights
