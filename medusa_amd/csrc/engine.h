@@ -323,10 +323,12 @@ void ensure_events(medusa_graph* g, size_t count);
 bool is_device_memory(const void* p);
 // Whether g's kernels may write `bytes` as 4-byte values at `p`: device memory of g's own GPU,
 // aligned, all of it in the allocation that p points into.  Other destinations (host, managed,
-// another GPU) are copied to; a copy is refused where the allocation ends too early.
+// another GPU, or over several mappings of one address range) are copied to; a copy is refused where
+// the allocation ends too early.
 bool kernels_can_write(const medusa_graph* g, const void* p, size_t bytes);
-// Fails where `p` is device memory whose allocation ends before `bytes`.
-void check_device_output(const void* p, size_t bytes);
+// Fails where `p` is device memory whose allocation ends before `bytes`.  An address range mapped in
+// pieces (hipMemMap) passes: the copy goes over all of them.
+void check_device_output(const medusa_graph* g, const void* p, size_t bytes);
 // Copies `bytes` from device pointer `src` to `dst`, which may be host or device memory.
 void copy_out(medusa_graph* g, void* dst, const void* src, size_t bytes);
 // Number of workgroups for a grid-stride launch over `items` with `per_wg` items each.

@@ -70,16 +70,27 @@ bool kernels_can_write(const medusa_graph* g, const void* p, size_t bytes) {
            reinterpret_cast<uintptr_t>(p) % 4 == 0 && allocation_left(p) >= bytes;
 }
 
-void check_device_output(const void* p, size_t bytes) {
+// Whether `p` lies in an address range of hipMemMap's, of which HIP names one mapping at a time.
+static bool is_mapped_range(const medusa_graph* g, const void* p) {
+    unsigned long long flags = 0;
+    hipMemLocation where{};
+    where.type = hipMemLocationTypeDevice;
+    where.id = g->device;
+    const hipError_t e = hipMemGetAccess(&flags, &where, const_cast<void*>(p));
+    (void)hipGetLastError();
+    return e == hipSuccess;
+}
+
+void check_device_output(const medusa_graph* g, const void* p, size_t bytes) {
     if (!is_device_memory(p)) return;
     const size_t left = allocation_left(p);
-    MDS_CHECK(left == 0 || left >= bytes, MEDUSA_ERR_HIP, "output of %zu bytes in device memory that ends after %zu",
+    MDS_CHECK(left == 0 || left >= bytes || is_mapped_range(g, p), MEDUSA_ERR_HIP, "output of %zu bytes in device memory that ends after %zu",
               bytes, left);
 }
 
 void copy_out(medusa_graph* g, void* dst, const void* src, size_t bytes) {
     if (!bytes) return;
-    check_device_output(dst, bytes);
+    check_device_output(g, dst, bytes);
     const bool dev = is_device_memory(dst);
     MDS_HIP(hipMemcpyAsync(dst, src, bytes, dev ? hipMemcpyDeviceToDevice : hipMemcpyDeviceToHost, g->stream));
     MDS_HIP(hipStreamSynchronize(g->stream));

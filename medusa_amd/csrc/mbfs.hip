@@ -1205,7 +1205,7 @@ static void mbfs_run(medusa_graph* g, const uint32_t* srcs, uint32_t k, uint8_t*
     st.reached = (uint32_t)std::min<uint64_t>(h.reached, 0xFFFFFFFFull);
     st.reserved[0] = h.saturated;
     if (direct) return;
-    check_device_output(out, (size_t)k * n);  // before the first row is written
+    check_device_output(g, out, (size_t)k * n);  // before the first row is written
     // as many rows at a time as the row buffer holds
     const uint32_t rows = (uint32_t)std::min<uint64_t>(k, std::max<uint64_t>(1, kMbfsRowBytes / n));
     g->mbfs_rows.ensure(((size_t)rows * n + 3) / 4);

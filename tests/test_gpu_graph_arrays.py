@@ -117,3 +117,70 @@ def test_device_output_past_its_allocation_is_refused(oracle, short):
             assert e.value.code == -2  # MEDUSA_ERR_HIP
             assert (A.bytes() == 7).all(), i
             A.free()
+
+
+class _MappedArray:
+    """`nbytes` of device memory behind one address range of two mappings (hipMemMap)."""
+
+    class _Location(ctypes.Structure):
+        _fields_ = [("type", ctypes.c_int), ("id", ctypes.c_int)]
+
+    class _Prop(ctypes.Structure):
+        pass
+
+    class _Access(ctypes.Structure):
+        pass
+
+    _Prop._fields_ = [("type", ctypes.c_int), ("handle_types", ctypes.c_int), ("location", _Location),
+                      ("win32", ctypes.c_void_p), ("flags", ctypes.c_uint32)]
+    _Access._fields_ = [("location", _Location), ("flags", ctypes.c_int)]
+
+    def __init__(self, nbytes):
+        L, size, ull = md.lib(), ctypes.c_size_t, ctypes.c_ulonglong
+        here = self._Location(1, 0)  # hipMemLocationTypeDevice
+        prop = self._Prop(1, 0, here, None, 0)  # hipMemAllocationTypePinned
+        gran = size()
+        assert L.hipMemGetAllocationGranularity(ctypes.byref(gran), ctypes.byref(prop), ctypes.c_int(1)) == 0
+        half = -(-(nbytes // 2) // gran.value) * gran.value
+        assert half < nbytes <= 2 * half
+        va = ctypes.c_void_p()
+        assert L.hipMemAddressReserve(ctypes.byref(va), size(2 * half), size(0), ctypes.c_void_p(), ull(0)) == 0
+        self.base, self.half, self.handles = va.value, half, []
+        for i in range(2):
+            h = ctypes.c_void_p()
+            assert L.hipMemCreate(ctypes.byref(h), size(half), ctypes.byref(prop), ull(0)) == 0
+            assert L.hipMemMap(ctypes.c_void_p(self.base + i * half), size(half), size(0), h, ull(0)) == 0
+            self.handles.append(h)
+        access = self._Access(here, 3)  # hipMemAccessFlagsProtReadWrite
+        assert L.hipMemSetAccess(va, size(2 * half), ctypes.byref(access), size(1)) == 0
+
+    def data_ptr(self):
+        return self.base
+
+    def free(self):
+        L = md.lib()
+        for i, h in enumerate(self.handles):
+            assert L.hipMemUnmap(ctypes.c_void_p(self.base + i * self.half), ctypes.c_size_t(self.half)) == 0
+            assert L.hipMemRelease(h) == 0
+        assert L.hipMemAddressFree(ctypes.c_void_p(self.base), ctypes.c_size_t(2 * self.half)) == 0
+
+
+def test_device_output_over_two_mappings(oracle):
+    """An output over both mappings of an address range, of which HIP names one at a time, is filled."""
+    n, k = 1_048_576, 8
+    rng = np.random.default_rng(5)
+    rp, col, _ = csr_from_edges(n, rng.integers(0, n, (4 * n, 2)))
+    w = rng.integers(1, 1001, len(col)).astype(np.uint32)
+    srcs = rng.integers(0, n, k).astype(np.uint32)
+    calls = [(4 * n, lambda G, o: G.bfs(0, out=o), lambda: oracle.bfs_queue(rp, col, 0)),
+             (4 * n, lambda G, o: G.sssp(0, out=o), lambda: oracle.sssp_dijkstra(rp, col, w, 0)),
+             (4 * n, lambda G, o: G.pagerank(0.85, 3, out=o), lambda: oracle.pagerank_f32(rp, col, 0.85, 3)),
+             (k * n, lambda G, o: G.mbfs(srcs, out=o), lambda: oracle.mbfs(rp, col, srcs))]
+    with md.Graph(rp, col, w) as G:
+        for i, (need, call, want) in enumerate(calls):
+            print(f"[case] call {i}", flush=True)
+            A = _MappedArray(need)
+            call(G, A)
+            got = _d2h(A.data_ptr(), need // 4)
+            assert np.array_equal(got.view(np.uint8), np.ascontiguousarray(want()).view(np.uint8).ravel()), i
+            A.free()
