@@ -20,15 +20,16 @@ MDS_HD inline uint32_t advance_to(uint32_t at, uint32_t off, uint32_t end) {
     return lies_before(at, off, end) ? at + off : end;
 }
 
-// Bounds of part `part` of [begin, begin + count) cut into `parts` parts of equal length but for the last
-// ones, which may be shorter or empty.
+// Bounds of part `part` of [begin, begin + count) cut into `parts` (at most 65535) parts of equal length but
+// for the last ones, which may be shorter or empty.  No product of these passes 2^32.
 struct EdgePart {
     uint32_t lo, hi;
 };
 MDS_HD inline EdgePart edge_part(uint32_t begin, uint32_t count, uint32_t part, uint32_t parts) {
-    const uint32_t per = count / parts + (count % parts ? 1u : 0u);
-    const uint64_t lo = (uint64_t)part * per, hi = lo + per;
-    return {begin + (uint32_t)(lo < count ? lo : count), begin + (uint32_t)(hi < count ? hi : count)};
+    if (!count) return {begin, begin};
+    const uint32_t per = (count - 1) / parts + 1, at = part * per;
+    const uint32_t lo = at < count ? at : count, left = count - lo;
+    return {begin + lo, begin + lo + (left < per ? left : per)};
 }
 
 }  // namespace medusa
