@@ -446,7 +446,8 @@ __device__ __forceinline__ uint32_t wave_min_u32(uint32_t x) {
 // asked for on mean out-degree 8 (2^20) 6.03, 1.68 and 2.72.  Bounds of 32768 and 65536 are level with this one
 // there, but in the 1400^2 lattice without buckets, whose frontier is that wide, they take 31 and 24 ms
 // instead of 8.8 (without any bound 8.8).  The other side of it: 3000^2 without buckets 77 ms unbounded, 159
-// bounded, 146 with the block-wide rounds; with buckets (9.4 ms) it does not get there.
+// bounded, 146 with the block-wide rounds; with buckets (9.4 ms) it does not get there.  And uniform
+// graphs of mean out-degree 2: 2^22 vertices 0.80 and 0.96 (block-wide 1.53), 2^24 3.98 and 3.16 (4.10).
 constexpr uint32_t kRecEdges = 7;
 constexpr uint32_t kRecWords = 4;        // uint4 per record: {out-degree, row_ptr, (target, weight) x 7}
 constexpr uint32_t kRing = 512;          // offers per wave
